@@ -238,6 +238,73 @@ def _layer_forward(s):
     return [q, k, v, o, y]
 
 
+# ---- the same pass in 64 bits ------------------------------------------------------------------------------------------------
+def _weight64(layer):
+    """The frozen weight [n, k] that a 4-bit layer's buffers stand for."""
+    if hasattr(layer, "qweight"):  # eight rows of k per word, eight columns of n per zero-point word
+        shifts = torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)
+        q = ((layer.qweight[:, None, :] >> shifts[None, :, None]) & 15).reshape(-1, layer.qweight.shape[1])
+        z = ((layer.qzeros[:, :, None] >> shifts) & 15).reshape(layer.qzeros.shape[0], -1)
+        group = layer.g_idx.long()
+        return ((q - z[group]).double() * layer.scales[group].double()).t()
+    state = layer.weight.quant_state
+    packed = layer.weight.data.reshape(-1)
+    codes = torch.stack([packed >> 4, packed & 15], -1).reshape(-1, state.blocksize).long()
+    outer = state.state2
+    scale = outer.code.double()[state.absmax.long()] * outer.absmax.double().repeat_interleave(outer.blocksize)[: state.absmax.numel()]
+    return (state.code.double()[codes] * (scale + state.offset.double())[:, None]).reshape(tuple(state.shape))
+
+
+def exact(case, seed):
+    """What run() returns, with every step in fp64 and nothing rounded in between."""
+    s = prepare(case, seed)
+    train, kind = s["train"], case["kind"]
+    if kind == "loss":
+        logits = s["logits"].detach().double().requires_grad_(True)
+        rows, labels = logits[:, :-1].reshape(-1, case["vocab"]), s["labels"][:, 1:].reshape(-1)
+        loss = torch.nn.functional.cross_entropy(rows, labels, ignore_index=-100)
+        loss.backward()
+        return [loss.detach(), logits.grad]
+    leaves = {id(p): p.detach().double().requires_grad_(train) for p in s["params"]}
+
+    def leaf(p):
+        return leaves[id(p)] if id(p) in leaves else p.detach().double()
+
+    def linear(lin, x):
+        if not hasattr(lin, "lora_A"):
+            return x @ _weight64(lin).t()
+        a, b = leaf(lin.lora_A["default"].weight), leaf(lin.lora_B["default"].weight)
+        return x @ _weight64(lin.base_layer).t() + (x @ a.t()) @ b.t() * lin.scaling["default"]
+
+    def norm(module, x):
+        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + module.variance_epsilon) * module.weight.double()
+
+    def rotate(x):
+        half = torch.cat([-x[..., x.shape[-1] // 2:], x[..., : x.shape[-1] // 2]], -1)
+        return x * s["cos"].double()[:, None] + half * s["sin"].double()[:, None]
+
+    def mlp(x):
+        m = s["mlp"]
+        return linear(m.down_proj, torch.nn.functional.silu(linear(m.gate_proj, x)) * linear(m.up_proj, x))
+
+    with torch.set_grad_enabled(train):
+        if kind == "train_linear":
+            outs, grads = [linear(s["o"], leaf(s["x"]))], [s["dy"]]
+        elif kind == "train_mlp":
+            outs, grads = [mlp(leaf(s["x_mlp"]))], [s["dy"]]
+        else:
+            (heads, kv, hd), attn = s["heads"], s["attn"]
+            x = norm(s["norm_attn"], leaf(s["x_attn"]))
+            q, k, v = (linear(p, x).view(*x.shape[:2], h, hd).transpose(1, 2)
+                       for p, h in ((attn.q_proj, heads), (attn.k_proj, kv), (attn.v_proj, kv)))
+            outs = [rotate(q), rotate(k), v, linear(attn.o_proj, leaf(s["x_o"])), mlp(norm(s["norm_mlp"], leaf(s["x_mlp"])))]
+            grads = [s["dq"], s["dk"], s["dv"], s["do"], s["dy"]] if train else []
+    if not train:
+        return outs
+    torch.autograd.backward(outs, [g.double() for g in grads])
+    return [o.detach() for o in outs] + [leaves[id(p)].grad for p in s["params"]]
+
+
 # ---- what a pass cannot do without ------------------------------------------------------------------------------------------
 def work(case):
     m, train = _tokens(case), case["kind"].startswith("train")
