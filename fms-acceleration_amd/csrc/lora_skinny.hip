@@ -19,10 +19,13 @@ namespace {
 // keeps enough bytes in flight.  The NW partial [16 * MTL x r] tiles are summed through LDS in a
 // fixed order: the upper half of the waves hands its tiles to the lower half, whose sums are then
 // added up by all threads.
+// With few tokens one workgroup per 16 of them leaves most CUs idle and every wave with a long serial walk over its slice
+// (40 us at 1100 tokens x 4096, rank 64; 17 us for ONE token), so the columns are also split over gridDim.y workgroups:
+// their fp32 sums go to partial[split][M][r], which lora_down_reduce_kernel adds in index order.
 template <typename T, int RT, int MTL, int NW>
 __global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __restrict__ X, int64_t ldx,
                                                             const uint16_t* __restrict__ Wd, int M, int C, int r,
-                                                            uint16_t* __restrict__ out, int64_t ldo) {
+                                                            uint16_t* __restrict__ out, int64_t ldo, float* __restrict__ partial) {
   constexpr int NH = NW / 2;
   __shared__ float red[NH][MTL][RT][64][4];
   const int tid = threadIdx.x;
@@ -31,9 +34,10 @@ __global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __re
   const int m_base = blockIdx.x * (16 * MTL);
   // slice boundaries in units of 32 columns
   const int n32 = (C + 31) / 32;
-  const int per = (n32 + NW - 1) / NW;
-  const int c_begin = min(C, wave * per * 32);
-  const int c_end = min(C, (wave + 1) * per * 32);
+  const int slice = blockIdx.y * NW + wave, n_slices = gridDim.y * NW;
+  const int per = (n32 + n_slices - 1) / n_slices;
+  const int c_begin = min(C, slice * per * 32);
+  const int c_end = min(C, (slice + 1) * per * 32);
 
   f32x4 acc[MTL][RT];
 #pragma unroll
@@ -92,7 +96,12 @@ __global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __re
     for (int w = 1; w < NH; ++w) v += red[w][u][t][ln][i];
     const int row = m_base + 16 * u + 4 * (ln >> 4) + i;
     const int j = 16 * t + (ln & 15);
-    if (row < M && j < r) out[(size_t)row * ldo + j] = pack1<T>(v);
+    if (row < M && j < r) {
+      if (partial)
+        partial[((size_t)blockIdx.y * M + row) * r + j] = v;
+      else
+        out[(size_t)row * ldo + j] = pack1<T>(v);
+    }
   }
 }
 
@@ -448,6 +457,7 @@ __global__ __launch_bounds__(256) void lora_down_reduce_kernel(const float* __re
   const int m = (int)(q4 / per_row), j = 4 * (int)(q4 % per_row);
   const size_t plane = (size_t)M * r;
   f32x4 v = *reinterpret_cast<const f32x4*>(partial + (size_t)m * r + j);
+#pragma unroll 8
   for (int s = 1; s < n_split; ++s) v += *reinterpret_cast<const f32x4*>(partial + s * plane + (size_t)m * r + j);
   u32x2 o;
   o[0] = pack2<T>(v[0], v[1]);
@@ -753,12 +763,13 @@ int lora_grad_splits(int M, int C) {
   return splits;
 }
 
-int launch_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
-                     int64_t ldo, hipStream_t st) {
+// n_split > 1: the fragment kernel with its columns split over workgroups, sums to `partial` (the caller reduces them)
+static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
+                                  int64_t ldo, float* partial, int n_split, hipStream_t st) {
   // 32 tokens per workgroup once that still leaves a workgroup per CU (halves the re-reads of Wd)
   const int mtl = (M >= 32 * 256 && r <= 64) ? 2 : 1;
   constexpr int NW = 8;  // waves per workgroup: measured best of 4 / 8 / 16 at 8192 tokens
-  dim3 grid((M + 16 * mtl - 1) / (16 * mtl)), block(64 * NW);
+  dim3 grid((M + 16 * mtl - 1) / (16 * mtl), n_split), block(64 * NW);
   const int rt = (r + 15) / 16;
   // staged kernel: 32 (from 8192 tokens) or 16 (from 4096) tokens per workgroup, worth it once that gives every CU a
   // workgroup and the rows are long enough to amortise its pipeline fill (measured at 8192 tokens: 59 -> 48 us at
@@ -798,10 +809,10 @@ int launch_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, i
   do {                                                                                                                       \
     if (mtl == 2)                                                                                                            \
       hipLaunchKernelGGL((lora_down_kernel<TT, RT, (RT > 4 ? 1 : 2), NW>), grid, block, 0, st, (const uint16_t*)X, ldx,       \
-                         (const uint16_t*)Wd, M, C, r, (uint16_t*)out, ldo);                                                 \
+                         (const uint16_t*)Wd, M, C, r, (uint16_t*)out, ldo, partial);                                        \
     else                                                                                                                     \
       hipLaunchKernelGGL((lora_down_kernel<TT, RT, 1, NW>), grid, block, 0, st, (const uint16_t*)X, ldx, (const uint16_t*)Wd, \
-                         M, C, r, (uint16_t*)out, ldo);                                                                      \
+                         M, C, r, (uint16_t*)out, ldo, partial);                                                             \
   } while (0)
 #define DISPATCH(TT)            \
   switch (rt) {                 \
@@ -821,6 +832,11 @@ int launch_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, i
   return FMSA_OK;
 }
 
+int launch_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
+                     int64_t ldo, hipStream_t st) {
+  return launch_lora_down_plain(X, ldx, Wd, M, C, r, act_dtype, out, ldo, nullptr, 1, st);
+}
+
 namespace {
 // Shape of the split launch: row groups per workgroup, column ranges, or g = 0 when the kernels without workspace do as
 // well or the matrix is too small.  (At rank 16 and below Wd is a small part of the traffic; what the split kernel adds there
@@ -829,9 +845,16 @@ namespace {
 struct DownSplit {
   int g, n_tb, n_split;
 };
-DownSplit lora_down_split_shape(int M, int C, int r) {
+DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
   const int rt = (std::min(r, 64) + 15) / 16;  // ranks above 64 go out 64 at a time (accumulator registers)
-  if (M < 2048 || C < 2048) return {0, 0, 0};
+  if (M < 2048 || C < 2048) {
+    if (!few_tokens) return {0, 0, 0};
+    // g = 1: the fragment kernel, columns split until two workgroups per CU are there or a wave is down to two steps of 32
+    const int n_tb = (M + 15) / 16;
+    const int n_split = std::min(512 / n_tb, C / 512);
+    if (n_split < 2) return {0, 0, 0};
+    return {1, n_tb, n_split};
+  }
   if (rt < 2 && M >= 16384) return {0, 0, 0};  // rank 16 and below with a workgroup per CU anyway: the 32-token kernels do as well
   const int g = rt <= 2 ? 2 : 4;  // rank 32: 64 tokens per workgroup; 48 / 64: 128
   const int n_tb = (M + 32 * g - 1) / (32 * g);
@@ -842,25 +865,42 @@ DownSplit lora_down_split_shape(int M, int C, int r) {
 }
 }  // namespace
 
-size_t lora_down_workspace(int M, int C, int r) {
-  const DownSplit d = lora_down_split_shape(M, C, r);
-  return d.g && d.n_split > 1 ? (size_t)d.n_split * (size_t)M * (size_t)std::min(r, 64) * sizeof(float) : 0;
+size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
+  const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
+  const int ranks = d.g == 1 ? r : std::min(r, 64);
+  return d.g && d.n_split > 1 ? (size_t)d.n_split * (size_t)M * (size_t)ranks * sizeof(float) : 0;
 }
 
 // The split kernel where it pays and the caller brought the partial-sum buffer (or none is needed); launch_lora_down otherwise.
 int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
-                        int64_t ldo, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  const DownSplit d = lora_down_split_shape(M, C, r);
-  const size_t need = lora_down_workspace(M, C, r);
+                        int64_t ldo, void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st) {
+  const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
+  const size_t need = lora_down_workspace(M, C, r, few_tokens);
   const bool out_ok = ((uintptr_t)out % 8 == 0) && ldo % 4 == 0;  // the reduce pass stores four ranks at a time
   if (!d.g || (need && (!workspace || workspace_bytes < need || !out_ok)))
     return launch_lora_down(X, ldx, Wd, M, C, r, act_dtype, out, ldo, st);
+  auto reduce = [&]() -> int {
+    const int64_t quads = (int64_t)M * (r / 4);
+    dim3 rgrid((unsigned)((quads + 255) / 256));
+    if (act_dtype == FMSA_BF16)
+      hipLaunchKernelGGL((lora_down_reduce_kernel<bf16_t>), rgrid, dim3(256), 0, st, (const float*)workspace, d.n_split, M, r,
+                         (uint16_t*)out, ldo);
+    else
+      hipLaunchKernelGGL((lora_down_reduce_kernel<f16_t>), rgrid, dim3(256), 0, st, (const float*)workspace, d.n_split, M, r,
+                         (uint16_t*)out, ldo);
+    FMSA_CHECK_LAUNCH();
+    return FMSA_OK;
+  };
+  if (d.g == 1) {
+    if (int rc = launch_lora_down_plain(X, ldx, Wd, M, C, r, act_dtype, out, ldo, (float*)workspace, d.n_split, st)) return rc;
+    return reduce();
+  }
   if (r > 64) {
     // 64 ranks per pass over X (launches on one stream run in order, so the passes share the workspace); cheaper than one
     // pass whose accumulators and double-buffered Wd fragments do not fit the registers
     for (int r0 = 0; r0 < r; r0 += 64) {
       const int rc = launch_lora_down_ws(X, ldx, (const uint16_t*)Wd + (size_t)r0 * C, M, C, std::min(64, r - r0), act_dtype,
-                                         (uint16_t*)out + r0, ldo, workspace, workspace_bytes, st);
+                                         (uint16_t*)out + r0, ldo, workspace, workspace_bytes, few_tokens, st);
       if (rc != FMSA_OK) return rc;
     }
     return FMSA_OK;
@@ -884,17 +924,7 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
 #undef SPLIT_DISPATCH
 #undef SPLIT_LAUNCH
   FMSA_CHECK_LAUNCH();
-  if (d.n_split > 1) {
-    const int64_t quads = (int64_t)M * (r / 4);
-    dim3 rgrid((unsigned)((quads + 255) / 256));
-    if (act_dtype == FMSA_BF16)
-      hipLaunchKernelGGL((lora_down_reduce_kernel<bf16_t>), rgrid, dim3(256), 0, st, (const float*)workspace, d.n_split, M, r,
-                         (uint16_t*)out, ldo);
-    else
-      hipLaunchKernelGGL((lora_down_reduce_kernel<f16_t>), rgrid, dim3(256), 0, st, (const float*)workspace, d.n_split, M, r,
-                         (uint16_t*)out, ldo);
-    FMSA_CHECK_LAUNCH();
-  }
+  if (d.n_split > 1) return reduce();
   return FMSA_OK;
 }
 

@@ -31,6 +31,8 @@ EXPORTED_SYMBOLS = (
     "fmsa_lora_down",
     "fmsa_lora_down_workspace",
     "fmsa_lora_down_ws",
+    "fmsa_lora_down_split_workspace",
+    "fmsa_lora_down_split",
     "fmsa_lora_grad_workspace",
     "fmsa_lora_grad",
     "fmsa_lora_grad_batch_workspace",
@@ -178,7 +180,7 @@ class BwdProj(Structure):
 _lib = None
 
 
-ABI_VERSION = 9  # include/fmsa.h as this binding mirrors it (fmsa_abi_version of the library must agree)
+ABI_VERSION = 10  # include/fmsa.h as this binding mirrors it (fmsa_abi_version of the library must agree)
 
 
 def lib() -> ctypes.CDLL:
@@ -211,6 +213,9 @@ def lib() -> ctypes.CDLL:
     L.fmsa_lora_grad_workspace.argtypes = [c_int, c_int, c_int]
     L.fmsa_lora_grad.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_int, c_int, c_int,
                                  c_void_p, c_void_p, c_size_t, c_void_p]
+    L.fmsa_lora_down_split_workspace.restype = c_size_t
+    L.fmsa_lora_down_split_workspace.argtypes = [c_int, c_int, c_int]
+    L.fmsa_lora_down_split.argtypes = L.fmsa_lora_down_ws.argtypes
     L.fmsa_lora_grad_batch_workspace.restype = c_size_t
     L.fmsa_lora_grad_batch_workspace.argtypes = [POINTER(LoraGradJob), c_int, c_int]
     L.fmsa_lora_grad_batch.argtypes = [POINTER(LoraGradJob), c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]
@@ -347,10 +352,11 @@ def lora_down(x2d, wd, out=None):
     if out is None:
         out = torch.empty((M, r), dtype=x2d.dtype, device=x2d.device)
     assert out.shape == (M, r) and out.stride(1) == 1 and out.dtype == x2d.dtype
-    nbytes = lib().fmsa_lora_down_workspace(M, C, r)
+    nbytes = lib().fmsa_lora_down_split_workspace(M, C, r)
     ws = _workspace(nbytes, x2d.device) if nbytes else None
-    _check("fmsa_lora_down_ws", lib().fmsa_lora_down_ws(_ptr(x2d), x2d.stride(0), _ptr(wd), M, C, r, act_enum(x2d.dtype), _ptr(out),
-                                                        out.stride(0), _ptr(ws), 0 if ws is None else ws.numel(), _stream(out)))
+    _check("fmsa_lora_down_split",
+           lib().fmsa_lora_down_split(_ptr(x2d), x2d.stride(0), _ptr(wd), M, C, r, act_enum(x2d.dtype), _ptr(out), out.stride(0),
+                                      _ptr(ws), 0 if ws is None else ws.numel(), _stream(out)))
     return out
 
 

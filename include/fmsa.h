@@ -128,6 +128,12 @@ size_t fmsa_lora_down_workspace(int M, int C, int r);
 int fmsa_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype,
                       void* out, int64_t ldout, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same with the columns split over workgroups for few tokens too (below 2048, down to one), where the kernels above
+ * leave most of the chip idle. */
+size_t fmsa_lora_down_split_workspace(int M, int C, int r);
+int fmsa_lora_down_split(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype,
+                      void* out, int64_t ldout, void* workspace, size_t workspace_bytes, void* stream);
+
 /* out = scale * L[M, r]^T * R[M, C]   (a reduction over the M tokens; L has row stride ldl >= r), written as
  *   [r, C] when transpose_out == 0   (dA = s * (dY B)^T Xd,  UL/gptq/fast_lora.py:822,824,842)
  *   [C, r] when transpose_out == 1   (dB = s * dY^T (Xd A^T), :823,825,843)

@@ -1,0 +1,29 @@
+"""lora_down with few tokens, where the columns are split over workgroups: against the fp32 product, next to the unsplit
+kernel (fmsa_lora_down)."""
+import pytest
+import torch
+
+from tests.helpers import randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,C,r", [(1, 1024, 8), (1, 14336, 16), (15, 4096, 64), (17, 1056, 128), (300, 8200, 24), (2047, 4096, 64),
+                                   (4000, 1536, 16)])
+def test_lora_down_few_tokens(M, C, r, dtype):
+    import fmsa_hip
+
+    lib = fmsa_hip.lib()
+    x = randn((M, C + 8), 1, dtype).cuda()[:, :C]  # a column slice
+    wd = randn((r, C), 2, dtype, 0.05).cuda()
+    ref = x.float() @ wd.float().t()
+    whole = torch.empty((M, r), dtype=dtype, device="cuda")
+    assert lib.fmsa_lora_down(x.data_ptr(), x.stride(0), wd.data_ptr(), M, C, r, fmsa_hip.act_enum(dtype), whole.data_ptr(), r,
+                              torch.cuda.current_stream().cuda_stream) == 0
+    wide = torch.full((M, r + 16), 3.0, dtype=dtype, device="cuda")
+    out = fmsa_hip.lora_down(x, wd, out=wide[:, 8 : 8 + r])
+    # another order of the fp32 sums meets a few other roundings of the result, no larger ones
+    assert (out.float() - ref).norm() <= 1.02 * (whole.float() - ref).norm() + 1e-6 * ref.norm()
+    assert torch.all(wide[:, :8] == 3.0) and torch.all(wide[:, 8 + r :] == 3.0)
+    assert torch.equal(fmsa_hip.lora_down(x, wd), out)
