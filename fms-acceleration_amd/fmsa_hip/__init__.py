@@ -264,13 +264,17 @@ def _check(fn: str, code: int):
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _raw_stream(index: int) -> int:
+    return torch._C._cuda_getCurrentRawStream(index)  # pylint: disable=protected-access
 
 
 def _stream(t: torch.Tensor):
     if not t.is_cuda:
         raise RuntimeError("libfmsa_hip kernels need tensors on the GPU (there is no CPU implementation)")
-    return c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _raw_stream(t.get_device())
 
 
 def act_enum(dtype: torch.dtype) -> int:
@@ -366,7 +370,7 @@ _ws_cache = {}
 def _workspace(nbytes: int, device) -> torch.Tensor:
     """Partial-sum buffer of the adapter-gradient launches, one per (device, stream): launches on one stream
     are ordered and may share it, launches on two streams of one device must not."""
-    key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, _raw_stream(device.index))
     ws = _ws_cache.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
