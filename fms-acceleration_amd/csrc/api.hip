@@ -17,12 +17,15 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
                         void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st);
 int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st);
 int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
-                         int64_t ldh, const fmsa_rope* rope, int act_dtype, hipStream_t st);
+                         int64_t ldh, const fmsa_rope* rope, int act_dtype, void* workspace, size_t workspace_bytes, hipStream_t st);
+size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode);
+size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M);
 int launch_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e,
                             void* g, void* h_out, int64_t ldeg, int act_dtype, hipStream_t st);
 
 int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e,
-                              void* g, void* h_out, int64_t ldeg, int act_dtype, hipStream_t st);
+                              void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace, size_t workspace_bytes,
+                              hipStream_t st);
 int bwd_dx_twin_flavour(const fmsa_bwd_proj* projs, int n_proj, int act_dtype);
 int launch_gptq_transpose(const int32_t* qweight, int K, int N, int32_t* out, hipStream_t st);
 int launch_gptq_interleave(const int32_t* qweight, int K, int N, int32_t* out, hipStream_t st);
@@ -165,7 +168,7 @@ int fmsa_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, int
 
 size_t fmsa_lora_down_workspace(int M, int C, int r) {
   if (M <= 0 || C <= 0 || r <= 0 || r > 128 || r % 8 != 0 || C % 8 != 0) return 0;
-  return lora_down_workspace(M, C, r);
+  return lora_down_workspace(M, C, r, false);
 }
 
 size_t fmsa_lora_down_split_workspace(int M, int C, int r) {
@@ -310,8 +313,22 @@ static int check_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int6
 
 int fmsa_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
                        int64_t ldh, int act_dtype, void* stream) {
+  return fmsa_gptq_lora_fwd_ws(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype, nullptr, 0, stream);
+}
+
+size_t fmsa_gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return gptq_lora_fwd_workspace(projs, n_proj, M, mode);
+}
+
+int fmsa_gptq_lora_fwd_ws(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
+                          int64_t ldh, int act_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   if (int rc = check_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype)) return rc;
-  return launch_gptq_lora_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, nullptr, act_dtype, (hipStream_t)stream);
+  if (workspace && !aligned16(workspace)) return FMSA_ERR_ALIGN;
+  return launch_gptq_lora_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, nullptr, act_dtype, workspace, workspace_bytes,
+                              (hipStream_t)stream);
 }
 
 int fmsa_gptq_lora_fwd_rope(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, const fmsa_rope* rope,
@@ -335,11 +352,24 @@ int fmsa_gptq_lora_fwd_rope(const fmsa_fwd_proj* projs, int n_proj, const void* 
     if (projs[p].w.nibble_order != 0) return FMSA_ERR_UNSUPPORTED;  // the rotating flavours read the checkpoint's order
   }
   if (K % 64 != 0) return FMSA_ERR_UNSUPPORTED;
-  return launch_gptq_lora_fwd(projs, n_proj, X, ldx, M, FMSA_FWD_LINEAR, nullptr, 0, rope, act_dtype, (hipStream_t)stream);
+  return launch_gptq_lora_fwd(projs, n_proj, X, ldx, M, FMSA_FWD_LINEAR, nullptr, 0, rope, act_dtype, nullptr, 0,
+                              (hipStream_t)stream);
 }
 
 int fmsa_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e,
                           void* g, void* h_out, int64_t ldeg, int act_dtype, void* stream) {
+  return fmsa_gptq_lora_bwd_dx_ws(projs, n_proj, M, mode, dX, lddx, e, g, h_out, ldeg, act_dtype, nullptr, 0, stream);
+}
+
+size_t fmsa_gptq_lora_bwd_dx_workspace(const fmsa_bwd_proj* projs, int n_proj, int M, int act_dtype) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return bwd_dx_twin_flavour(projs, n_proj, act_dtype) ? gptq_lora_bwd_dx_t_workspace(projs, n_proj, M) : 0;
+}
+
+int fmsa_gptq_lora_bwd_dx_ws(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e, void* g,
+                             void* h_out, int64_t ldeg, int act_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   if (!projs) return FMSA_ERR_NULL;
   if (n_proj < 1 || n_proj > 3 || M <= 0) return FMSA_ERR_SHAPE;
   if (mode != FMSA_BWD_LINEAR && mode != FMSA_BWD_SWIGLU) return FMSA_ERR_SHAPE;
@@ -385,13 +415,15 @@ int fmsa_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs, int n_proj, int M, int mod
     if (lddx < K) return FMSA_ERR_SHAPE;
     if (!aligned16(dX) || lddx % 8 != 0) return FMSA_ERR_ALIGN;
   }
+  if (workspace && !aligned16(workspace)) return FMSA_ERR_ALIGN;
   const int twin = bwd_dx_twin_flavour(projs, n_proj, act_dtype);
   // the checkpoint-layout kernel needs every affine projection's fp32 offset table
   if (!twin)
     for (int p = 0; p < n_proj; ++p)
       if (!projs[p].nsz && projs[p].w.format != FMSA_WEIGHT_CODEBOOK) return FMSA_ERR_NULL;
   if (twin)
-    return launch_gptq_lora_bwd_dx_t(projs, n_proj, M, mode, dX, lddx, e, g, h_out, ldeg, act_dtype, (hipStream_t)stream);
+    return launch_gptq_lora_bwd_dx_t(projs, n_proj, M, mode, dX, lddx, e, g, h_out, ldeg, act_dtype, workspace, workspace_bytes,
+                                     (hipStream_t)stream);
   return launch_gptq_lora_bwd_dx(projs, n_proj, M, mode, dX, lddx, e, g, h_out, ldeg, act_dtype, (hipStream_t)stream);
 }
 

@@ -25,6 +25,7 @@
 // ahead, two stage buffers.  Results are bit-identical to the kernel that reads the checkpoint layout
 // (gemm_bwd.hip): same operand values, same MFMA operand roles and contraction order.
 #include "common.h"
+#include "split_tiles.h"
 
 namespace {
 
@@ -63,12 +64,53 @@ struct BwdTArgs {
   int64_t ldeg;
   const uint16_t* mask_src;
   int64_t ldmask;
+  // contraction split (SPLIT flavours): tiles n_whole .. n_whole + n_cut - 1 are cut into n_ranges ranges of the stages
+  // of all projections laid end to end
+  int n_whole, n_cut, n_ranges, n_stages_all;
+  float* partial;
 };
 
 FMSA_DEVI BwdTProjDev select_proj(const BwdTArgs& a, int p) { return p == 0 ? a.p[0] : (p == 1 ? a.p[1] : a.p[2]); }
 
+// token block and column block of tile pid: grouped-M order
+FMSA_DEVI void bwd_tile(const BwdTArgs& a, int pid, int& bm, int& bk) {
+  constexpr int GROUP_M = 4;  // token blocks per group: 4 x 8 tiles in flight per XCD share dY and W tiles in its L2
+  const int width = GROUP_M * a.nbk;
+  const int first_m = (pid / width) * GROUP_M;
+  const int gsz = min(a.nbm - first_m, GROUP_M);
+  bm = first_m + (pid % width) % gsz;
+  bk = (pid % width) / gsz;
+}
+
+// SwiGLU backward of two adjacent columns: e, g, the rounded base and adapter parts of dh, and the mask source in;
+// h, d_g, d_e out.  Every rounding to the storage type is one packed conversion whose two halves are read back as fp32
+// (UL/swiglu.py:69-88 rounds f, h, DW and DW * g to the storage type; their products with fp32 factors are rounded once,
+// on store).  The adapter part of dh is masked by (dropout(h) != 0): `mv` holds dropout(h) when a dropout was applied,
+// otherwise h itself (recomputed here) decides; +-0 count as zero.
+template <typename T>
+FMSA_DEVI void swiglu_bwd_pair(uint32_t ev, uint32_t gv, uint32_t bv, uint32_t lv, uint32_t mv, bool has_mask, uint32_t& h,
+                               uint32_t& dg, uint32_t& de) {
+  const float e0 = unpack_lo<T>(ev), e1 = unpack_hi<T>(ev);
+  const float g0 = unpack_lo<T>(gv), g1 = unpack_hi<T>(gv);
+  const float b0 = unpack_lo<T>(bv), b1 = unpack_hi<T>(bv);
+  const float se0 = sigmoidf_(e0), se1 = sigmoidf_(e1);
+  const uint32_t fp = pack2<T>(se0 * e0, se1 * e1);  // f = silu(e)
+  const float f0 = unpack_lo<T>(fp), f1 = unpack_hi<T>(fp);
+  const uint32_t hp = pack2<T>(f0 * g0, f1 * g1);  // h = f * g
+  const uint32_t sel = has_mask ? mv : hp;
+  const float s0 = b0 + unpack_lo<T>(lv), s1 = b1 + unpack_hi<T>(lv);
+  const uint32_t dwp = pack2<T>((sel & 0x7fffu) ? s0 : b0, (sel & 0x7fff0000u) ? s1 : b1);
+  const float DW0 = unpack_lo<T>(dwp), DW1 = unpack_hi<T>(dwp);
+  const uint32_t tp = pack2<T>(DW0 * g0, DW1 * g1);  // dg = DW * g in storage dtype (:79)
+  h = hp;
+  dg = pack2<T>(DW0 * f0, DW1 * f1);  // d_g ("df", :77)
+  de = pack2<T>(unpack_lo<T>(tp) * se0 * (1.0f + e0 * (1.0f - se0)),  // d_e (:81-83)
+                unpack_hi<T>(tp) * se1 * (1.0f + e1 * (1.0f - se1)));
+}
+
 // CODEBOOK: W = code[q] * block_scale[group, n] instead of the affine scale * q + (-scale * zero).
-template <typename T, bool NTAIL, int MODE, bool CODEBOOK, bool PK16 = false>
+// SPLIT: the tiles that do not fill a round of the chip are cut along the contraction (split_tiles.h).
+template <typename T, bool NTAIL, int MODE, bool CODEBOOK, bool PK16 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs a) {
   static_assert(!PK16 || (std::is_same<T, f16_t>::value && !CODEBOOK), "packed half unpack: fp16 activations, affine weights");
   // separate arrays per stage buffer: every access names its buffer statically, so the compiler can tell fragment
@@ -88,13 +130,19 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
   const int l32 = lane & 31;
   const int half = lane >> 5;
 
-  int pid = xcd_remap(blockIdx.x, a.nbm * a.nbk);
-  constexpr int GROUP_M = 4;  // token blocks per group: 4 x 8 tiles in flight per XCD share dY and W tiles in its L2
-  const int width = GROUP_M * a.nbk;
-  const int first_m = (pid / width) * GROUP_M;
-  const int gsz = min(a.nbm - first_m, GROUP_M);
-  const int bm = first_m + (pid % width) % gsz;
-  const int bk = (pid % width) / gsz;
+  SplitWork work{0, -1, 0};
+  if constexpr (SPLIT) work = split_work(a.n_whole, a.n_cut, a.n_ranges);
+  const int pid = SPLIT ? work.tile : xcd_remap(blockIdx.x, a.nbm * a.nbk);
+  // this workgroup's stages [g_lo, g_hi) of the projections' stages laid end to end (SPLIT)
+  int g_lo = 0, g_hi = 0x7fffffff, g_at = 0;
+  if constexpr (SPLIT) {
+    if (work.range >= 0) {
+      g_lo = (int)((int64_t)work.range * a.n_stages_all / a.n_ranges);
+      g_hi = (int)((int64_t)(work.range + 1) * a.n_stages_all / a.n_ranges);
+    }
+  }
+  int bm, bk;
+  bwd_tile(a, pid, bm, bk);
   const int m0 = bm * BM;
   const int k_tile0 = bk * 256;
 
@@ -133,7 +181,14 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
     const BwdTProjDev P = select_proj(a, p);
     const int N = __builtin_amdgcn_readfirstlane(P.N);
     const int gs = __builtin_amdgcn_readfirstlane(P.group_size);
-    const int n_stages = (N + BK - 1) / BK;
+    int st0 = 0, st_end = (N + BK - 1) / BK;  // this workgroup's stages of the projection
+    if constexpr (SPLIT) {
+      const int n = st_end;
+      st0 = min(max(g_lo - g_at, 0), n);
+      st_end = min(max(g_hi - g_at, 0), n);
+      g_at += n;
+      if (st0 >= st_end) continue;
+    }
     const int n_groups = (K + gs - 1) / gs;
 
     // ---- direct-load addressing: buffer resources + 32-bit lane offsets + scalar offsets ---------
@@ -510,15 +565,15 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
       step(sb_c, I3{}, I1{}, I0{}, NoVmem{}, 0, sb_c);
       __builtin_amdgcn_s_waitcnt(WAIT_VM0);
       __syncthreads();
-      const int st_next = min(s + 2, n_stages - 1);
+      const int st_next = min(s + 2, st_end - 1);
       step(S1{}, I0{}, I0{}, I1{}, WithVmem{}, st_next, sb_c);
     };
 
     __syncthreads();  // the previous projection's last LDS reads are done
-    load_stage(0, I0{});
+    load_stage(st0, I0{});
     __builtin_amdgcn_s_waitcnt(WAIT_VM0);
     __syncthreads();
-    load_stage(min(1, n_stages - 1), I1{});
+    load_stage(min(st0 + 1, st_end - 1), I1{});
     if constexpr (CODEBOOK) {
       prefetch_a(I0{}, I0{}, I0{});
       prefetch_b(I0{});
@@ -526,13 +581,20 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
       prefetch(I0{}, I0{}, I0{});
     }
 
-    const int n_full = n_stages & ~1;
-    int s = 0;
-    for (; s < n_full; s += 2) {
+    const int s_full = st0 + ((st_end - st0) & ~1);
+    int s = st0;
+    for (; s < s_full; s += 2) {
       stage(s, I0{});
       stage(s + 1, I1{});
     }
-    if (s < n_stages) stage(s, I0{});
+    if (s < st_end) stage(s, I0{});
+  }
+  if constexpr (SPLIT) {
+    if (work.range >= 0) {
+      __builtin_amdgcn_s_waitcnt(WAIT_VM0);  // the surplus direct loads of the last stage have landed
+      split_store(acc, a.partial, work.cut, work.range, a.n_ranges);
+      return;
+    }
   }
 
   // ---- epilogue ---------------------------------------------------------------------------
@@ -700,30 +762,14 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
       if constexpr (swiglu) {
         const u32x4 ev = pre_e[it];
         const u32x4 gv = pre_g[it];
-        // Two adjacent columns at a time: every rounding to the storage type is one packed conversion whose two
-        // halves are read back as fp32 (UL/swiglu.py:69-88 rounds f, h, DW and DW * g to the storage type; their
-        // products with fp32 factors are rounded once, on store).
         u32x4 hv, dgv, dev;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          const float e0 = unpack_lo<T>(ev[w]), e1 = unpack_hi<T>(ev[w]);
-          const float g0 = unpack_lo<T>(gv[w]), g1 = unpack_hi<T>(gv[w]);
-          const float b0 = unpack_lo<T>(bv[w]), b1 = unpack_hi<T>(bv[w]);
-          const float se0 = sigmoidf_(e0), se1 = sigmoidf_(e1);
-          const uint32_t fp = pack2<T>(se0 * e0, se1 * e1);  // f = silu(e)
-          const float f0 = unpack_lo<T>(fp), f1 = unpack_hi<T>(fp);
-          const uint32_t hp = pack2<T>(f0 * g0, f1 * g1);  // h = f * g
-          // LoRA part of dh is masked by (dropout(h) != 0): mask_src holds dropout(h) when a dropout was applied,
-          // otherwise h itself (recomputed here) decides; +-0 count as zero
-          const uint32_t sel = has_mask ? mv[w] : hp;
-          const float s0 = b0 + unpack_lo<T>(lv[w]), s1 = b1 + unpack_hi<T>(lv[w]);
-          const uint32_t dwp = pack2<T>((sel & 0x7fffu) ? s0 : b0, (sel & 0x7fff0000u) ? s1 : b1);
-          const float DW0 = unpack_lo<T>(dwp), DW1 = unpack_hi<T>(dwp);
-          const uint32_t tp = pack2<T>(DW0 * g0, DW1 * g1);  // dg = DW * g in storage dtype (:79)
-          hv[w] = hp;
-          dgv[w] = pack2<T>(DW0 * f0, DW1 * f1);  // d_g ("df", :77)
-          dev[w] = pack2<T>(unpack_lo<T>(tp) * se0 * (1.0f + e0 * (1.0f - se0)),   // d_e (:81-83)
-                            unpack_hi<T>(tp) * se1 * (1.0f + e1 * (1.0f - se1)));
+          uint32_t h, dg, de;
+          swiglu_bwd_pair<T>(ev[w], gv[w], bv[w], lv[w], mv[w], has_mask, h, dg, de);
+          hv[w] = h;
+          dgv[w] = dg;
+          dev[w] = de;
         }
         __builtin_amdgcn_raw_buffer_store_b128(hv, h_rsrc, eg_voff, soff_rows * eg_row_bytes, STORE_NT);
         __builtin_amdgcn_raw_buffer_store_b128(dgv, e_rsrc, eg_voff, soff_rows * eg_row_bytes, STORE_NT);
@@ -746,6 +792,97 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
       if (more) issue_loads(q + 1, it_c);
     });
     __syncthreads();
+  }
+}
+
+// Second launch of a split call: workgroup = token tile mt (32 rows) of a cut tile; lane, column and register layout and
+// the rounding points of the kernel above, outputs as 8-byte stores.
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const BwdTArgs a) {
+  constexpr bool swiglu = MODE == FMSA_BWD_SWIGLU;
+  const int cut = blockIdx.x / MT, mt = blockIdx.x % MT;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
+  int bm, bk;
+  bwd_tile(a, a.n_whole + cut, bm, bk);
+  const int m = bm * BM + 32 * mt + l32;
+  if (bm * BM + 32 * mt >= a.M) return;  // the whole workgroup
+  const bool m_ok = m < a.M;
+  f32x4 acc[NT][4];
+  split_load(acc, a.partial, cut, mt, a.n_ranges);
+  f32x16 lora[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lora[j][i] = 0.f;
+  bool any_lora = false;
+  for (int p = 0; p < a.n_proj; ++p) {
+    const BwdTProjDev P = select_proj(a, p);
+    if (P.r <= 0) continue;
+    any_lora = true;
+    f32x16 tmp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tmp[j][i] = 0.f;
+    for (int j0 = 0; j0 < P.r; j0 += 16) {
+      const int ko = j0 + 8 * half;
+      u32x4 tf = {0u, 0u, 0u, 0u}, af[NT];
+      if (m_ok && ko < P.r) tf = *reinterpret_cast<const u32x4*>(P.T + (size_t)m * P.ldt + ko);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int col = bk * 256 + 64 * wave + 32 * j;
+        af[j] = u32x4{0u, 0u, 0u, 0u};
+        if (col < a.K && ko < P.r) af[j] = *reinterpret_cast<const u32x4*>(P.At + (size_t)(col + l32) * P.r + ko);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) tmp[j] = mfma32<T>(af[j], tf, tmp[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lora[j][i] += P.s * tmp[j][i];
+  }
+  if (!m_ok) return;
+  const bool has_mask = a.mask_src != nullptr && any_lora;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int col0 = bk * 256 + 64 * wave + 32 * j;
+    if (col0 >= a.K) continue;
+#pragma unroll
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = col0 + 8 * i0 + 4 * half;
+      const u32x2 bv = {pack2<T>(acc[j][i0][0], acc[j][i0][1]), pack2<T>(acc[j][i0][2], acc[j][i0][3])};
+      u32x2 lv = {0u, 0u}, mv = {0u, 0u};
+      if (any_lora) lv = u32x2{pack2<T>(lora[j][4 * i0], lora[j][4 * i0 + 1]), pack2<T>(lora[j][4 * i0 + 2], lora[j][4 * i0 + 3])};
+      if (has_mask) mv = *reinterpret_cast<const u32x2*>(a.mask_src + (size_t)m * a.ldmask + col);
+      if constexpr (swiglu) {
+        const size_t o = (size_t)m * a.ldeg + col;
+        const u32x2 ev = *reinterpret_cast<const u32x2*>(a.e + o), gv = *reinterpret_cast<const u32x2*>(a.g + o);
+        u32x2 hv, dgv, dev;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          uint32_t h, dg, de;
+          swiglu_bwd_pair<T>(ev[w], gv[w], bv[w], lv[w], mv[w], has_mask, h, dg, de);
+          hv[w] = h;
+          dgv[w] = dg;
+          dev[w] = de;
+        }
+        *reinterpret_cast<u32x2*>(a.h + o) = hv;
+        *reinterpret_cast<u32x2*>(a.e + o) = dgv;
+        *reinterpret_cast<u32x2*>(a.g + o) = dev;
+      } else {
+        u32x2 ov = bv;
+        if (any_lora) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const float l0 = (!has_mask || (mv[w] & 0x7fffu)) ? unpack_lo<T>(lv[w]) : 0.f;
+            const float l1 = (!has_mask || ((mv[w] >> 16) & 0x7fffu)) ? unpack_hi<T>(lv[w]) : 0.f;
+            ov[w] = pack2<T>(unpack_lo<T>(bv[w]) + l0, unpack_hi<T>(bv[w]) + l1);
+          }
+        }
+        *reinterpret_cast<u32x2*>(a.dX + (size_t)m * a.lddx + col) = ov;
+      }
+    }
   }
 }
 
@@ -826,8 +963,21 @@ int bwd_dx_twin_flavour(const fmsa_bwd_proj* projs, int n_proj, int act_dtype) {
   return pk16 ? 2 : (fp32_tables ? 1 : 0);
 }
 
+static int bwd_t_stages(const fmsa_bwd_proj* projs, int n_proj) {
+  int n = 0;
+  for (int p = 0; p < n_proj; ++p) n += (projs[p].w.N + BK - 1) / BK;
+  return n;
+}
+
+static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M) {
+  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj));
+}
+
+size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M) { return bwd_t_split(projs, n_proj, M).bytes(); }
+
 int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx,
-                              void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, hipStream_t st) {
+                              void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace,
+                              size_t workspace_bytes, hipStream_t st) {
   BwdTArgs a{};
   a.n_proj = n_proj;
   a.M = M;
@@ -867,17 +1017,33 @@ int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int
   a.nbm = (M + BM - 1) / BM;
   a.nbk = (a.K + 255) / 256;
   dim3 grid(a.nbm * a.nbk), block(256);
+  // without a workspace that holds it, every tile runs whole
+  SplitPlan plan = bwd_t_split(projs, n_proj, M);
+  if (!workspace || workspace_bytes < plan.bytes()) plan.s = 1;
+  if (plan.s > 1) {
+    a.n_whole = plan.n_whole;
+    a.n_cut = plan.n_split;
+    a.n_ranges = plan.s;
+    a.n_stages_all = bwd_t_stages(projs, n_proj);
+    a.partial = (float*)workspace;
+    grid = dim3(plan.n_whole + plan.n_split * plan.s);
+  }
   const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;  // api.hip: all projections of a launch share the format
   const bool pk16 = bwd_dx_twin_flavour(projs, n_proj, act_dtype) == 2;
+#define LAUNCH_S(TT, NTL, MD, CB, PK)                                                                                       \
+  do {                                                                                                                    \
+    if (plan.s > 1) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<TT, NTL, MD, CB, PK, true>), grid, block, 0, st, a);     \
+    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<TT, NTL, MD, CB, PK>), grid, block, 0, st, a);                      \
+  } while (0)
 #define LAUNCH_PK(MD)                                                                                          \
   do {                                                                                                         \
-    if (ntail) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<f16_t, true, MD, false, true>), grid, block, 0, st, a);  \
-    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<f16_t, false, MD, false, true>), grid, block, 0, st, a);       \
+    if (ntail) LAUNCH_S(f16_t, true, MD, false, true);                                                         \
+    else LAUNCH_S(f16_t, false, MD, false, true);                                                              \
   } while (0)
 #define LAUNCH_C(TT, MD, CB)                                                                             \
   do {                                                                                                   \
-    if (ntail) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<TT, true, MD, CB>), grid, block, 0, st, a);  \
-    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_kernel<TT, false, MD, CB>), grid, block, 0, st, a);       \
+    if (ntail) LAUNCH_S(TT, true, MD, CB, false);                                                        \
+    else LAUNCH_S(TT, false, MD, CB, false);                                                             \
   } while (0)
 #define LAUNCH_M(TT, MD)                  \
   do {                                    \
@@ -901,6 +1067,19 @@ int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int
 #undef LAUNCH_M
 #undef LAUNCH_C
 #undef LAUNCH_PK
+#undef LAUNCH_S
   FMSA_CHECK_LAUNCH();
+  if (plan.s > 1) {
+    const dim3 fgrid(plan.n_split * MT);
+#define FINISH(TT)                                                                                                            \
+  do {                                                                                                                        \
+    if (mode == FMSA_BWD_SWIGLU) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_SWIGLU>), fgrid, block, 0, st, a); \
+    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_LINEAR>), fgrid, block, 0, st, a);                  \
+  } while (0)
+    if (act_dtype == FMSA_BF16) FINISH(bf16_t);
+    else FINISH(f16_t);
+#undef FINISH
+    FMSA_CHECK_LAUNCH();
+  }
   return FMSA_OK;
 }

@@ -18,6 +18,7 @@
 // The rank-r LoRA term is one extra MFMA step per 16 ranks in the epilogue, scaled by s in fp32
 // before the single rounding of the output.
 #include "common.h"
+#include "split_tiles.h"
 
 namespace {
 
@@ -59,11 +60,24 @@ struct FwdArgs {
   const void* rope_sin;
   int64_t rope_ld;
   int rope_rows, rope_head_dim, rope_mask;
+  // contraction split (SPLIT flavours): tiles n_whole .. n_whole + n_cut - 1 are cut into n_ranges ranges of stages
+  int n_whole, n_cut, n_ranges;
+  float* partial;
 };
 
 // a.p[p] for a runtime (wave-uniform) p without dynamic indexing of the kernel-argument struct,
 // which would force a copy of it into scratch memory.
 FMSA_DEVI FwdProjDev select_proj(const FwdArgs& a, int p) { return p == 0 ? a.p[0] : (p == 1 ? a.p[1] : a.p[2]); }
+
+// token block and column block of tile pid: grouped-M order
+FMSA_DEVI void fwd_tile(const FwdArgs& a, int pid, int& bm, int& bn) {
+  constexpr int GROUP_M = 4;  // token blocks per group: 4 x 8 tiles in flight per XCD share X and W tiles in its L2
+  const int width = GROUP_M * a.nbn;
+  const int first_m = (pid / width) * GROUP_M;
+  const int gsz = min(a.nbm - first_m, GROUP_M);
+  bm = first_m + (pid % width) % gsz;
+  bn = (pid % width) / gsz;
+}
 
 // GPS = scale groups per 64-wide K stage: 1 for group_size % 64 == 0, 2 / 4 for group sizes 32 / 16.
 // CODEBOOK (1, 2): the nibbles index a 16-entry table and one fp32 scale per (group, column) multiplies the
@@ -79,7 +93,9 @@ FMSA_DEVI FwdProjDev select_proj(const FwdArgs& a, int p) { return p == 0 ? a.p[
 // 2p + 1 at position 4 + p --, one scale group per stage): a fragment register is (((w >> 4p) & 0x000F000F) | 0x64006400)
 // + (-(1024 + z)) [exact] times the fp16 scale [one rounding] in packed half arithmetic: RNE_fp16(s * (q - z)) bit for bit
 // in 15 instead of 22 instructions per word.
-template <typename T, int GPS, bool KTAIL, int CODEBOOK, int ROPE = 0, bool PK16 = false>
+// SPLIT: the tiles that do not fill a round of the chip are cut along K (split_tiles.h); a template parameter, because the
+// flavours without it are scheduled instruction by instruction.
+template <typename T, int GPS, bool KTAIL, int CODEBOOK, int ROPE = 0, bool PK16 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   static_assert(!PK16 || (std::is_same<T, f16_t>::value && CODEBOOK == 0 && GPS == 1 && ROPE == 0), "packed half unpack");
   // two separate arrays (not one 2-D array): every access names its buffer statically, which is
@@ -101,13 +117,11 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   const int half = lane >> 5;
 
   // ---- tile assignment: XCD-contiguous ranges, then grouped-M order inside the range --------
-  int pid = xcd_remap(blockIdx.x, a.nbm * a.nbn);
-  constexpr int GROUP_M = 4;  // token blocks per group: 4 x 8 tiles in flight per XCD share X and W tiles in its L2
-  const int width = GROUP_M * a.nbn;
-  const int first_m = (pid / width) * GROUP_M;
-  const int gsz = min(a.nbm - first_m, GROUP_M);
-  const int bm = first_m + (pid % width) % gsz;
-  const int bn = (pid % width) / gsz;
+  SplitWork work{0, -1, 0};
+  if constexpr (SPLIT) work = split_work(a.n_whole, a.n_cut, a.n_ranges);
+  const int pid = SPLIT ? work.tile : xcd_remap(blockIdx.x, a.nbm * a.nbn);
+  int bm, bn;
+  fwd_tile(a, pid, bm, bn);
   const int m0 = bm * BM;
 
   int pj[NT], col0[NT];
@@ -167,7 +181,15 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   }
 
   const int K = a.K;
-  const int n_stages = (K + BK - 1) / BK;
+  // this workgroup's stages st0 .. st_end - 1 of the contraction
+  int st0 = 0, st_end = (K + BK - 1) / BK;
+  if constexpr (SPLIT) {
+    if (work.range >= 0) {
+      const int n = st_end;
+      st0 = work.range * n / a.n_ranges;
+      st_end = (work.range + 1) * n / a.n_ranges;
+    }
+  }
 
   f32x16 acc[MT][NT];
 #pragma unroll
@@ -229,7 +251,13 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   // group index of the stage being loaded, advanced without a division when GPS == 1
   int g_ld[NT], k_in_g[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) g_ld[j] = k_in_g[j] = 0;
+  for (int j = 0; j < NT; ++j) {
+    g_ld[j] = k_in_g[j] = 0;
+    if constexpr (SPLIT) {
+      g_ld[j] = __builtin_amdgcn_readfirstlane(st0 * BK / gs[j]);
+      k_in_g[j] = __builtin_amdgcn_readfirstlane(st0 * BK % gs[j]);
+    }
+  }
   // issue the global loads of stage `st` (0 <= st < n_stages) into slot SB; nothing here may read
   // the loaded registers, or the wave would wait for the load on the spot
   auto load_stage = [&](int st, auto sb_c) {
@@ -601,9 +629,9 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     commit_stage(S1{});
     __syncthreads();
     if constexpr (HAND) {
-      step_affine(S1{}, I0{}, I0{}, I1{}, WithVmem{}, min(s + 2, n_stages - 1), sb_c);
+      step_affine(S1{}, I0{}, I0{}, I1{}, WithVmem{}, min(s + 2, st_end - 1), sb_c);
     } else {
-      load_stage(min(s + 2, n_stages - 1), sb_c);
+      load_stage(min(s + 2, st_end - 1), sb_c);
       step(S1{}, I0{}, I0{}, I1{}, WithVmem{});
     }
   };
@@ -638,9 +666,12 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   }
   if constexpr (CODEBOOK == 2) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) zw_raw[0][j][0] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], 0, 0);
+    for (int j = 0; j < NT; ++j) {
+      const int g0 = __builtin_amdgcn_readfirstlane((st0 * BK) >> gshift[j]);
+      zw_raw[0][j][0] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], SPLIT ? (uint32_t)g0 * Np[j] * 4 : 0u, 0);
+    }
   }
-  load_stage(0, I0{});
+  load_stage(st0, I0{});
   __builtin_amdgcn_s_waitcnt(WAIT_VM0);
   commit_stage(I0{});
   if constexpr (CODEBOOK == 2) {  // the first stage's tables, all at once
@@ -650,7 +681,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     build_table_part(I0{}, I3{});
   }
   __syncthreads();
-  load_stage(min(1, n_stages - 1), I1{});
+  load_stage(min(st0 + 1, st_end - 1), I1{});
   if constexpr (CODEBOOK == 1) {
     prefetch_a(I0{}, I0{}, I0{});
     prefetch_b(I0{}, I0{});
@@ -659,13 +690,13 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   }
 
   // whole pairs in a single-exit loop (slots 0, 1), then the odd stage
-  const int n_full = n_stages & ~1;
-  int s = 0;
-  for (; s < n_full; s += NBUF) {
+  const int s_full = st0 + ((st_end - st0) & ~1);
+  int s = st0;
+  for (; s < s_full; s += NBUF) {
     stage(s, I0{});
     stage(s + 1, I1{});
   }
-  if (s < n_stages) stage(s, I0{});
+  if (s < st_end) stage(s, I0{});
 
   // ---- LoRA term as extra contraction steps: acc += U[:, j0..j0+15] x (s * B[:, j0..j0+15])^T -------
   // s * B is rounded to the storage type, the rounding point of the reference's
@@ -692,6 +723,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       u_rsrc[j] = make_rsrc(P.U + (size_t)m0 * P.ldu, rj[j] > 0 ? (size_t)rows_valid * P.ldu * 2 : 0);
       r_max = max(r_max, rj[j]);
     }
+    if (SPLIT && work.range > 0) r_max = 0;  // the adapter's term goes into the first range of a cut tile
     const uint32_t slot = (uint32_t)(2 * l32 + half) * 16;
     const int u_region = a.mode == FMSA_FWD_SWIGLU ? 8 : 0;  // KB between the U blocks of column tiles 0 and 1
     for (int j0 = 0; j0 < r_max; j0 += 16) {
@@ -719,6 +751,13 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[mt][j] = mfma32<T>(bw[j], uf[j][mt], acc[mt][j]);
+    }
+  }
+
+  if constexpr (SPLIT) {
+    if (work.range >= 0) {
+      split_store(acc, a.partial, work.cut, work.range, a.n_ranges);
+      return;
     }
   }
 
@@ -916,10 +955,88 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   (void)active;
 }
 
+// Second launch of a split call: workgroup = token tile mt (32 rows) of a cut tile; lane, column and register layout of
+// the kernel above, outputs as 8-byte stores (a row segment of 64 bytes is completed by four of them in L2).
+template <typename T>
+__global__ __launch_bounds__(256) void gptq_lora_fwd_finish_kernel(const FwdArgs a) {
+  const int cut = blockIdx.x / MT, mt = blockIdx.x % MT;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
+  int bm, bn;
+  fwd_tile(a, a.n_whole + cut, bm, bn);
+  const int m = bm * BM + 32 * mt + l32;
+  if (bm * BM + 32 * mt >= a.M) return;  // the whole workgroup
+  f32x4 acc[NT][4];
+  split_load(acc, a.partial, cut, mt, a.n_ranges);
+  if (m >= a.M) return;
+  const bool swiglu = a.mode == FMSA_FWD_SWIGLU;
+  const int p = swiglu ? 0 : (bn >= a.nblk_start[2] ? 2 : (bn >= a.nblk_start[1] ? 1 : 0));
+  auto biased = [&](const FwdProjDev& P, const f32x4& v, int col) {
+    f32x4 o = v;
+    if (P.bias) {
+      const u32x2 bv = *reinterpret_cast<const u32x2*>(P.bias + col);
+      o += f32x4{unpack_lo<T>(bv[0]), unpack_hi<T>(bv[0]), unpack_lo<T>(bv[1]), unpack_hi<T>(bv[1])};
+    }
+    return u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
+  };
+  if (swiglu) {
+    const int col0 = bn * 128 + 32 * wave + 4 * half;
+    if (bn * 128 + 32 * wave >= a.p[0].N) return;  // N % 32 == 0: a column tile is wholly inside or outside
+#pragma unroll
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = col0 + 8 * i0;
+      const u32x2 ev = biased(a.p[0], acc[0][i0], col), gv = biased(a.p[1], acc[1][i0], col);
+      u32x2 hv;
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {  // f = RNE(e * sigmoid(e)) on the rounded e; h = RNE(f * g) on the rounded g
+        const float e0 = unpack_lo<T>(ev[w]), e1 = unpack_hi<T>(ev[w]);
+        const uint32_t fv = pack2<T>(e0 * sigmoidf_(e0), e1 * sigmoidf_(e1));
+        hv[w] = pack2<T>(unpack_lo<T>(fv) * unpack_lo<T>(gv[w]), unpack_hi<T>(fv) * unpack_hi<T>(gv[w]));
+      }
+      *reinterpret_cast<u32x2*>(a.p[0].Y + (size_t)m * a.p[0].ldy + col) = ev;
+      *reinterpret_cast<u32x2*>(a.p[1].Y + (size_t)m * a.p[1].ldy + col) = gv;
+      *reinterpret_cast<u32x2*>(a.H + (size_t)m * a.ldh + col) = hv;
+    }
+  } else {
+    const FwdProjDev P = select_proj(a, p);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int col0 = (bn - a.nblk_start[p]) * 256 + 64 * wave + 32 * j;
+      if (col0 >= P.N) continue;
+#pragma unroll
+      for (int i0 = 0; i0 < 4; ++i0) {
+        const int col = col0 + 8 * i0 + 4 * half;
+        *reinterpret_cast<u32x2*>(P.Y + (size_t)m * P.ldy + col) = biased(P, acc[j][i0], col);
+      }
+    }
+  }
+}
+
 }  // namespace
 
+// The cut of a launch.  Flavours that are compiled with it: one scale group per stage, no rotary epilogue, and not the
+// gathering code-book unpack.
+static SplitPlan fwd_split(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  int nb = 0;
+  bool ok = true;
+  for (int p = 0; p < n_proj; ++p) {
+    const fmsa_gptq_weight& w = projs[p].w;
+    nb += (w.N + 255) / 256;
+    ok = ok && w.group_size % 64 == 0;
+    if (w.format == FMSA_WEIGHT_CODEBOOK) ok = ok && w.code == projs[0].w.code && (w.group_size & (w.group_size - 1)) == 0;
+  }
+  if (mode == FMSA_FWD_SWIGLU) nb = (projs[0].w.N + 127) / 128;
+  const int tiles = ((M + BM - 1) / BM) * nb;
+  if (!ok) return SplitPlan{tiles, 0, 1};
+  return plan_split(tiles, (projs[0].w.K + BK - 1) / BK);
+}
+
+size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  return fwd_split(projs, n_proj, M, mode).bytes();
+}
+
 int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode,
-                         void* H, int64_t ldh, const fmsa_rope* rope, int act_dtype, hipStream_t st) {
+                         void* H, int64_t ldh, const fmsa_rope* rope, int act_dtype, void* workspace, size_t workspace_bytes,
+                         hipStream_t st) {
   FwdArgs a{};
   if (rope) {
     a.rope_cos = rope->cos;
@@ -965,6 +1082,16 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
   a.nbn = nb;
   a.nbm = (M + BM - 1) / BM;
   dim3 grid(a.nbm * a.nbn), block(256);
+  // without a workspace that holds it, every tile runs whole
+  SplitPlan plan = fwd_split(projs, n_proj, M, mode);
+  if (rope || !workspace || workspace_bytes < plan.bytes()) plan.s = 1;
+  if (plan.s > 1) {
+    a.n_whole = plan.n_whole;
+    a.n_cut = plan.n_split;
+    a.n_ranges = plan.s;
+    a.partial = (float*)workspace;
+    grid = dim3(plan.n_whole + plan.n_split * plan.s);
+  }
   int gps = 1;
   for (int p = 0; p < n_proj; ++p) {
     const int gsz = projs[p].w.group_size;
@@ -979,6 +1106,25 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
   bool table = codebook && gps == 1;
   for (int p = 0; p < n_proj; ++p)
     table = table && projs[p].w.code == projs[0].w.code && (projs[p].w.group_size & (projs[p].w.group_size - 1)) == 0;
+  if (plan.s > 1) {
+#define SPLIT_K(TT, CB, PK)                                                                                         \
+  do {                                                                                                              \
+    if (ktail) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, true, CB, 0, PK, true>), grid, block, 0, st, a);      \
+    else hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, false, CB, 0, PK, true>), grid, block, 0, st, a);           \
+  } while (0)
+    if (pk16) SPLIT_K(f16_t, 0, true);
+    else if (codebook && act_dtype == FMSA_BF16) SPLIT_K(bf16_t, 2, false);
+    else if (codebook) SPLIT_K(f16_t, 2, false);
+    else if (act_dtype == FMSA_BF16) SPLIT_K(bf16_t, 0, false);
+    else SPLIT_K(f16_t, 0, false);
+#undef SPLIT_K
+    FMSA_CHECK_LAUNCH();
+    const dim3 fgrid(plan.n_split * MT);
+    if (act_dtype == FMSA_BF16) hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<bf16_t>), fgrid, block, 0, st, a);
+    else hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<f16_t>), fgrid, block, 0, st, a);
+    FMSA_CHECK_LAUNCH();
+    return FMSA_OK;
+  }
 #define LAUNCH3(TT, KT, CB)                                                                          \
   do {                                                                                               \
     if (rope && rope->dtype == FMSA_F32) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, false, CB, 2>), grid, block, 0, st, a); \

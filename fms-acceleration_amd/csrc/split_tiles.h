@@ -1,0 +1,93 @@
+// Contraction split for launches whose tiles do not fill the chip, shared by the forward and the input-gradient GEMM.
+//
+// A tile of these kernels occupies a CU by itself, so a launch runs in rounds of 256 tiles and a round that holds only R
+// of them costs as much as a full one: 4096 columns at 1100 tokens are 80 tiles, two thirds of the chip idle for the
+// whole launch.  The tiles of whole rounds run as before; each of the R others is cut along its contraction into `s`
+// ranges of stages, one workgroup each, which leave their 256 x 256 fp32 sums in the workspace (256 KB, lane contiguous).
+// A second launch, one workgroup per 32 tokens of a cut tile, adds the ranges in index order (the result does not depend
+// on scheduling) and applies what the kernel's own epilogue does, with the same rounding points.
+// (Adding the ranges in the last workgroup of a tile to arrive, without a second launch, was built first: one CU reads
+// its s x 256 KB at the latency of the memory behind the L2, 90 us per launch at s = 5, more than the split saved.)
+#pragma once
+#include "common.h"
+
+#include <algorithm>
+
+namespace {
+
+constexpr int SPLIT_CUS = 256;
+constexpr int SPLIT_QUADS = 64;  // 16-byte accumulator quads per lane: 8 token tiles x 2 column tiles x 4
+constexpr size_t SPLIT_TILE_BYTES = 4 * 64 * SPLIT_QUADS * 16;
+
+struct SplitPlan {
+  int n_whole;  // tiles that run whole: ids 0 .. n_whole - 1
+  int n_split;  // tiles cut into ranges
+  int s;        // ranges per cut tile (1: nothing is cut)
+  size_t bytes() const { return s > 1 ? (size_t)n_split * s * SPLIT_TILE_BYTES : 0; }
+};
+
+// A stage of 64 contraction elements takes a tile 1.4 us where the chip is not full; the split costs the second launch and
+// the start-up of its ranges (8 us) and the sums' way to memory and back (about 4 TB/s).
+inline SplitPlan plan_split(int tiles, int n_stages) {
+  SplitPlan p{tiles, 0, 1};
+  const int rest = tiles % SPLIT_CUS;
+  if (rest == 0) return p;
+  const float stage_us = 1.4f, fixed_us = 8.0f, range_us = 2.0f * SPLIT_TILE_BYTES / 4.0e6f;
+  float best = n_stages * stage_us - 3.0f;  // not for a gain that the noise of a launch would hide
+  int s_best = 1;
+  for (int s = 2; s <= SPLIT_CUS / rest && 2 * s <= n_stages; ++s) {
+    const float us = n_stages * stage_us / s + fixed_us + rest * s * range_us;
+    if (us < best) {
+      best = us;
+      s_best = s;
+    }
+  }
+  if (s_best > 1) p = SplitPlan{tiles - rest, rest, s_best};
+  return p;
+}
+
+// What a workgroup of a split launch works on.
+struct SplitWork {
+  int tile;    // tile index
+  int range;   // index of the range of a cut tile, -1: whole tile
+  int cut;     // index among the cut tiles
+};
+
+FMSA_DEVI SplitWork split_work(int n_whole, int n_split, int s) {
+  const int id = blockIdx.x;
+  if (id < n_whole) return {xcd_remap(id, n_whole), -1, 0};
+  const int u = xcd_remap(id - n_whole, n_split * s);
+  return {n_whole + u / s, u % s, u / s};
+}
+
+// One range's sums: quad (mt * NT + j) * 4 + i0 of lane l of wave w at [range][w][quad][l]
+template <int MT, int NT>
+FMSA_DEVI void split_store(const f32x16 (&acc)[MT][NT], float* partial, int cut, int range, int s) {
+  static_assert(MT * NT * 4 == SPLIT_QUADS, "a wave's accumulators");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  f32x4* dst = reinterpret_cast<f32x4*>(partial + (size_t)(cut * s + range) * (SPLIT_TILE_BYTES / 4)) + (size_t)wave * SPLIT_QUADS * 64 + lane;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i0 = 0; i0 < 4; ++i0)
+        dst[((mt * NT + j) * 4 + i0) * 64] =
+            f32x4{acc[mt][j][4 * i0], acc[mt][j][4 * i0 + 1], acc[mt][j][4 * i0 + 2], acc[mt][j][4 * i0 + 3]};
+}
+
+// The sums of token tile mt of a cut tile, all ranges in index order: register layout of the GEMM's accumulators
+template <int NT>
+FMSA_DEVI void split_load(f32x4 (&acc)[NT][4], const float* partial, int cut, int mt, int s) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const f32x4* src = reinterpret_cast<const f32x4*>(partial + (size_t)cut * s * (SPLIT_TILE_BYTES / 4)) +
+                     ((size_t)wave * SPLIT_QUADS + mt * NT * 4) * 64 + lane;
+#pragma unroll
+  for (int q = 0; q < NT * 4; ++q) acc[q >> 2][q & 3] = src[q * 64];
+#pragma unroll 4
+  for (int rg = 1; rg < s; ++rg)
+#pragma unroll
+    for (int q = 0; q < NT * 4; ++q) acc[q >> 2][q & 3] += src[(size_t)rg * (SPLIT_TILE_BYTES / 16) + q * 64];
+}
+
+}  // namespace

@@ -231,10 +231,11 @@ def _lora_down_all(projs, Xds, stack):
     return [fmsa_hip.lora_down(Xd, p.A) if p.r else None for p, Xd in zip(projs, Xds)]
 
 
-def _rope_in_epilogue(projs, rope, dtype):
+def _rope_in_epilogue(projs, rope, dtype, M):
     """Whether the forward kernel can apply the rotary embedding itself (fmsa_gptq_lora_fwd_rope): group sizes and
     K in whole 64-wide stages, heads that do not straddle its 256-column tiles, tables of the activation type or
-    fp32 whose rows start on 16-byte boundaries."""
+    fp32 whose rows start on 16-byte boundaries.  Where the launch would be cut along K (few tokens), the plain one and the
+    rotating pass over its small outputs are taken: the rotating flavours are not cut."""
     cos2d, sin2d, head_dim, mask = rope
     K = projs[0].w.K
     esz = cos2d.element_size()
@@ -243,7 +244,8 @@ def _rope_in_epilogue(projs, rope, dtype):
             and cos2d.stride() == sin2d.stride() and (cos2d.stride(0) * esz) % 16 == 0
             and cos2d.data_ptr() % 16 == 0 and sin2d.data_ptr() % 16 == 0
             and all(p.w.group_size % 64 == 0 for p in projs)
-            and all(p.w.N % head_dim == 0 for i, p in enumerate(projs) if (mask >> i) & 1))
+            and all(p.w.N % head_dim == 0 for i, p in enumerate(projs) if (mask >> i) & 1)
+            and not fmsa_hip.gptq_lora_fwd_splits([p.w.struct for p in projs], M))
 
 
 def _interleaved(projs, dtype):
@@ -258,17 +260,17 @@ def _linear_forward(projs, X2, Xds, stack=None, rope=None):
     rope = (cos2d, sin2d, head_dim, mask): the projections named by the mask leave with the rotary embedding
     applied, in the kernel's epilogue where it can, by the in-place kernel otherwise."""
     Us = _lora_down_all(projs, Xds, stack)
-    fused_rope = rope is not None and _rope_in_epilogue(projs, rope, X2.dtype)
+    fused_rope = rope is not None and _rope_in_epilogue(projs, rope, X2.dtype, X2.shape[0])
     if _one_order(projs):
         il = not fused_rope and _interleaved(projs, X2.dtype)  # the rotating flavours read the checkpoint's nibble order
         outs = fmsa_hip.gptq_lora_fwd(projs[0].to_kernel_order(X2), [p.fwd_dict(U, il) for p, U in zip(projs, Us)],
-                                      rope=rope if fused_rope else None)
+                                      rope=rope if fused_rope else None, split=True)
     else:
         outs = []
         for i, (p, U) in enumerate(zip(projs, Us)):
             r1 = (rope[0], rope[1], rope[2], 1) if fused_rope and (rope[3] >> i) & 1 else None
             il = r1 is None and _interleaved([p], X2.dtype)
-            outs.append(fmsa_hip.gptq_lora_fwd(p.to_kernel_order(X2), [p.fwd_dict(U, il)], rope=r1)[0])
+            outs.append(fmsa_hip.gptq_lora_fwd(p.to_kernel_order(X2), [p.fwd_dict(U, il)], rope=r1, split=True)[0])
     if rope is not None and not fused_rope:
         cos2d, sin2d, head_dim, mask = rope
         for i, (p, y) in enumerate(zip(projs, outs)):
@@ -317,11 +319,11 @@ def _linear_backward_dx(projs, dYs, Ts, Xds, M, K):
     one_mask = all(_same(m, masks[0]) for m in masks)
     if one_mask and _one_order(projs):
         permuted = {}
-        dXk = fmsa_hip.gptq_lora_bwd_dx([p.bwd_dict(dY, T, Xd, permuted) for p, dY, T, Xd in zip(projs, dYs, Ts, Xds)], M, K)
+        dXk = fmsa_hip.gptq_lora_bwd_dx([p.bwd_dict(dY, T, Xd, permuted) for p, dY, T, Xd in zip(projs, dYs, Ts, Xds)], M, K, split=True)
         return projs[0].from_kernel_order(dXk)
     dX = None
     for p, dY, T, Xd in zip(projs, dYs, Ts, Xds):
-        part = p.from_kernel_order(fmsa_hip.gptq_lora_bwd_dx([p.bwd_dict(dY, T, Xd)], M, K))
+        part = p.from_kernel_order(fmsa_hip.gptq_lora_bwd_dx([p.bwd_dict(dY, T, Xd)], M, K, split=True))
         dX = part.float() if dX is None else dX.add_(part)  # summed in fp32, rounded once
     return dX.to(dYs[0].dtype) if len(projs) > 1 else part
 
@@ -421,7 +423,8 @@ def mlp_forward(ctx, X, gate, up, down, dropouts, dtype):
     if fused:
         Ug, Uu = _lora_down_all([gate, up], [Xg, Xu], stack)
         il = _interleaved([gate, up], X2.dtype)
-        e, g, h = fmsa_hip.gptq_lora_fwd(gate.to_kernel_order(X2), [gate.fwd_dict(Ug, il), up.fwd_dict(Uu, il)], fmsa_hip.FWD_SWIGLU)
+        e, g, h = fmsa_hip.gptq_lora_fwd(gate.to_kernel_order(X2), [gate.fwd_dict(Ug, il), up.fwd_dict(Uu, il)],
+                                        fmsa_hip.FWD_SWIGLU, split=True)
     else:
         (e, g), (Ug, Uu) = _linear_forward([gate, up], X2, [Xg, Xu], stack)
         h = fmsa_hip.swiglu_fwd(e, g)
@@ -455,13 +458,13 @@ def mlp_backward(ctx, dY):
             (dBd,) = fmsa_hip.lora_grad_batch([(Ud, dY2, down.s, True, down.B_param.dtype, down.Bt, Td)])
     mask_h = hd if ctx.down_dropped else None
     if down.w.perm is None or down.input_ordered:
-        h = fmsa_hip.gptq_lora_bwd_dx([down.bwd_dict(dY2, Td, mask_h)], M, I, fmsa_hip.BWD_SWIGLU, e=e, g=g)
+        h = fmsa_hip.gptq_lora_bwd_dx([down.bwd_dict(dY2, Td, mask_h)], M, I, fmsa_hip.BWD_SWIGLU, e=e, g=g, split=True)
     else:
         # un-fused epilogue for a repacked (act-order) weight: dh in kernel order, scatter back,
         # then the standalone SwiGLU backward.  The mask of the LoRA part is (dropout(h) != 0).
         h_now = fmsa_hip.swiglu_fwd(e, g)
         dh = down.from_kernel_order(
-            fmsa_hip.gptq_lora_bwd_dx([down.bwd_dict(dY2, Td, mask_h if mask_h is not None else h_now)], M, I))
+            fmsa_hip.gptq_lora_bwd_dx([down.bwd_dict(dY2, Td, mask_h if mask_h is not None else h_now)], M, I, split=True))
         h = fmsa_hip.swiglu_bwd(dh, e, g)
     d_g, d_e = e, g
     if down.r:

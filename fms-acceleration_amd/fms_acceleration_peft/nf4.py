@@ -130,7 +130,7 @@ class Linear4bitFunction(torch.autograd.Function):
         w = prepare(weight, quant_state)
         ctx.w = w
         x2 = x if x.is_contiguous() else x.contiguous()
-        (y,) = fmsa_hip.gptq_lora_fwd(x2, [{"w": w.struct, "U": None, "B": None, "bias": None, "r": 0, "s": 0.0}])
+        (y,) = fmsa_hip.gptq_lora_fwd(x2, [{"w": w.struct, "U": None, "B": None, "bias": None, "r": 0, "s": 0.0}], split=True)
         return y
 
     @staticmethod
@@ -141,7 +141,7 @@ class Linear4bitFunction(torch.autograd.Function):
         dy2 = dy if dy.is_contiguous() else dy.contiguous()
         dx = fmsa_hip.gptq_lora_bwd_dx(
             [{"w": w.struct, "nsz": w.nsz, "dY": dy2, "T": None, "At": None, "mask_src": None, "r": 0, "s": 0.0,
-              "qweight_t": w.twin[0], "scale_f32": w.twin[1], "negzp_f16": w.twin[2]}], dy2.shape[0], w.K)
+              "qweight_t": w.twin[0], "scale_f32": w.twin[1], "negzp_f16": w.twin[2]}], dy2.shape[0], w.K, split=True)
         return dx, None, None
 
 

@@ -39,8 +39,12 @@ EXPORTED_SYMBOLS = (
     "fmsa_lora_grad_batch",
     "fmsa_lora_grad_static",
     "fmsa_gptq_lora_fwd",
+    "fmsa_gptq_lora_fwd_workspace",
+    "fmsa_gptq_lora_fwd_ws",
     "fmsa_gptq_lora_fwd_rope",
     "fmsa_gptq_lora_bwd_dx",
+    "fmsa_gptq_lora_bwd_dx_workspace",
+    "fmsa_gptq_lora_bwd_dx_ws",
     "fmsa_swiglu_fwd",
     "fmsa_swiglu_bwd",
     "fmsa_gptq_make_nsz",
@@ -209,13 +213,13 @@ def lib() -> ctypes.CDLL:
     L.fmsa_lora_down_workspace.argtypes = [c_int, c_int, c_int]
     L.fmsa_lora_down_ws.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_size_t,
                                     c_void_p]
+    L.fmsa_lora_down_split_workspace.restype = c_size_t
+    L.fmsa_lora_down_split_workspace.argtypes = [c_int, c_int, c_int]
+    L.fmsa_lora_down_split.argtypes = L.fmsa_lora_down_ws.argtypes
     L.fmsa_lora_grad_workspace.restype = c_size_t
     L.fmsa_lora_grad_workspace.argtypes = [c_int, c_int, c_int]
     L.fmsa_lora_grad.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_int, c_int, c_int,
                                  c_void_p, c_void_p, c_size_t, c_void_p]
-    L.fmsa_lora_down_split_workspace.restype = c_size_t
-    L.fmsa_lora_down_split_workspace.argtypes = [c_int, c_int, c_int]
-    L.fmsa_lora_down_split.argtypes = L.fmsa_lora_down_ws.argtypes
     L.fmsa_lora_grad_batch_workspace.restype = c_size_t
     L.fmsa_lora_grad_batch_workspace.argtypes = [POINTER(LoraGradJob), c_int, c_int]
     L.fmsa_lora_grad_batch.argtypes = [POINTER(LoraGradJob), c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]
@@ -223,6 +227,14 @@ def lib() -> ctypes.CDLL:
                                         c_void_p, c_void_p]
     L.fmsa_gptq_lora_fwd.argtypes = [POINTER(FwdProj), c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_int64,
                                      c_int, c_void_p]
+    L.fmsa_gptq_lora_fwd_workspace.restype = c_size_t
+    L.fmsa_gptq_lora_fwd_workspace.argtypes = [POINTER(FwdProj), c_int, c_int, c_int]
+    L.fmsa_gptq_lora_fwd_ws.argtypes = [POINTER(FwdProj), c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p,
+                                        c_size_t, c_void_p]
+    L.fmsa_gptq_lora_bwd_dx_workspace.restype = c_size_t
+    L.fmsa_gptq_lora_bwd_dx_workspace.argtypes = [POINTER(BwdProj), c_int, c_int, c_int]
+    L.fmsa_gptq_lora_bwd_dx_ws.argtypes = [POINTER(BwdProj), c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
+                                           c_int64, c_int, c_void_p, c_size_t, c_void_p]
     L.fmsa_gptq_lora_fwd_rope.argtypes = [POINTER(FwdProj), c_int, c_void_p, c_int64, c_int, POINTER(Rope), c_int, c_void_p]
     L.fmsa_gptq_lora_bwd_dx.argtypes = [POINTER(BwdProj), c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p,
                                         c_void_p, c_int64, c_int, c_void_p]
@@ -263,6 +275,8 @@ def _check(fn: str, code: int):
         raise FmsaError(fn, code)
 
 
+# A small launch costs the host as much as the GPU, so pointers and streams go to ctypes as plain integers (it makes its own
+# c_void_p from the argument types) and the stream is asked for by its raw handle, without a Stream object per launch.
 def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -447,11 +461,12 @@ def lora_grad_batch(jobs):
     return outs
 
 
-def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None):
+def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None, split: bool = False):
     """projs: dicts with keys w (GptqWeight), U, B, bias (tensors or None), r, s.
     Returns the list of outputs Y_p [M, N_p]; in SWIGLU mode returns (e, g, h).
     rope = (cos2d, sin2d, head_dim, proj_mask): LINEAR mode only; the projections whose bit is set in proj_mask
-    leave with the rotary embedding applied (token row m takes row m % cos2d.shape[0] of the tables)."""
+    leave with the rotary embedding applied (token row m takes row m % cos2d.shape[0] of the tables).
+    split=True lets the call cut tiles that do not fill the chip along K (another, still fixed, order of the fp32 sums)."""
     M = x2d.shape[0]
     arr = (FwdProj * len(projs))()
     outs = []
@@ -477,18 +492,30 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None)
                lib().fmsa_gptq_lora_fwd_rope(arr, len(projs), _ptr(x2d), x2d.stride(0), M, ctypes.byref(desc),
                                              act_enum(x2d.dtype), _stream(x2d)))
         return outs
-    _check("fmsa_gptq_lora_fwd",
-           lib().fmsa_gptq_lora_fwd(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
-                                    0 if h is None else h.stride(0), act_enum(x2d.dtype), _stream(x2d)))
+    nbytes = lib().fmsa_gptq_lora_fwd_workspace(arr, len(projs), M, mode) if split else 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x2d.device) if nbytes else None
+    _check("fmsa_gptq_lora_fwd_ws",
+           lib().fmsa_gptq_lora_fwd_ws(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
+                                       0 if h is None else h.stride(0), act_enum(x2d.dtype), _ptr(ws), nbytes, _stream(x2d)))
     if mode == FWD_SWIGLU:
         return outs[0], outs[1], h
     return outs
 
 
-def gptq_lora_bwd_dx(projs: Sequence[dict], M: int, K: int, mode: int = BWD_LINEAR, e=None, g=None):
+def gptq_lora_fwd_splits(weights, M: int) -> bool:
+    """Whether gptq_lora_fwd(split=True) cuts the tiles of a LINEAR launch of these weights over M tokens."""
+    arr = (FwdProj * len(weights))()
+    for i, w in enumerate(weights):
+        arr[i].w = w
+    return lib().fmsa_gptq_lora_fwd_workspace(arr, len(weights), M, FWD_LINEAR) > 0
+
+
+def gptq_lora_bwd_dx(projs: Sequence[dict], M: int, K: int, mode: int = BWD_LINEAR, e=None, g=None, split: bool = False):
     """projs: dicts with keys w, nsz, dY, T, At, mask_src, r, s and optionally qweight_t, scale_f32, negzp_f16 (the
     weight's transposed twin and its tables, see gptq_transpose and gptq_negzp_f16).  LINEAR mode returns dX [M, K]; SWIGLU mode overwrites e <- d_g,
-    g <- d_e and returns h."""
+    g <- d_e and returns h.
+    split=True lets a call on the twins cut tiles that do not fill the chip along the contraction (another, still fixed,
+    order of the fp32 sums: the checkpoint layout's results, which run whole, then differ in their last bits)."""
     arr = (BwdProj * len(projs))()
     ref = projs[0]["dY"]
     for i, p in enumerate(projs):
@@ -501,16 +528,18 @@ def gptq_lora_bwd_dx(projs: Sequence[dict], M: int, K: int, mode: int = BWD_LINE
                          _ptr(p.get("At")) if p["r"] else None, _ptr(ms), 0 if ms is None else ms.stride(0),
                          int(p["r"]), float(p["s"] or 0.0), _ptr(p.get("qweight_t")), _ptr(p.get("scale_f32")),
                          _ptr(p.get("negzp_f16")))
+    nbytes = lib().fmsa_gptq_lora_bwd_dx_workspace(arr, len(projs), M, act_enum(ref.dtype)) if split else 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=ref.device) if nbytes else None
     if mode == BWD_SWIGLU:
         h = torch.empty_like(e)
-        _check("fmsa_gptq_lora_bwd_dx",
-               lib().fmsa_gptq_lora_bwd_dx(arr, len(projs), M, mode, None, 0, _ptr(e), _ptr(g), _ptr(h), e.stride(0),
-                                           act_enum(ref.dtype), _stream(ref)))
+        _check("fmsa_gptq_lora_bwd_dx_ws",
+               lib().fmsa_gptq_lora_bwd_dx_ws(arr, len(projs), M, mode, None, 0, _ptr(e), _ptr(g), _ptr(h), e.stride(0),
+                                              act_enum(ref.dtype), _ptr(ws), nbytes, _stream(ref)))
         return h
     dx = torch.empty((M, K), dtype=ref.dtype, device=ref.device)
-    _check("fmsa_gptq_lora_bwd_dx",
-           lib().fmsa_gptq_lora_bwd_dx(arr, len(projs), M, mode, _ptr(dx), dx.stride(0), None, None, None, 0,
-                                       act_enum(ref.dtype), _stream(ref)))
+    _check("fmsa_gptq_lora_bwd_dx_ws",
+           lib().fmsa_gptq_lora_bwd_dx_ws(arr, len(projs), M, mode, _ptr(dx), dx.stride(0), None, None, None, 0,
+                                          act_enum(ref.dtype), _ptr(ws), nbytes, _stream(ref)))
     return dx
 
 

@@ -238,6 +238,15 @@ enum fmsa_fwd_mode { FMSA_FWD_LINEAR = 0, FMSA_FWD_SWIGLU = 1 };
 int fmsa_gptq_lora_fwd(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx,
                        int M, int mode, void* H, int64_t ldh, int act_dtype, void* stream);
 
+/* The same forward with a partial-sum buffer at hand: where the tiles do not fill the chip (few tokens, few columns, or
+ * the rest of a launch), they are cut along K over the idle CUs; the ranges' fp32 sums are added in index order, so the
+ * result does not depend on scheduling.  fmsa_gptq_lora_fwd_workspace gives the bytes (0: nothing is cut); with a smaller
+ * or no workspace the call runs as fmsa_gptq_lora_fwd does.  16-byte aligned; calls that may overlap in time need separate
+ * workspaces. */
+size_t fmsa_gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M, int mode);
+int fmsa_gptq_lora_fwd_ws(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M, int mode,
+                          void* H, int64_t ldh, int act_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The same forward (FMSA_FWD_LINEAR) with the rotary position embedding of the attention block applied in the
  * epilogue of the projections named by `proj_mask` (bit p = projection p; q and k of LoRA_QKV): replaces the
  * separate in-place pass of kernels/unsloth/rope_embedding.py:36-65, 68-103 over Q and K,
@@ -314,6 +323,12 @@ int fmsa_gptq_transpose(const int32_t* qweight, int K, int N, int32_t* qweight_t
 int fmsa_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int mode,
                           void* dX, int64_t lddx, void* e, void* g, void* h_out, int64_t ldeg,
                           int act_dtype, void* stream);
+
+/* The same with a partial-sum buffer (see fmsa_gptq_lora_fwd_ws); calls that run on the transposed twin use it. */
+size_t fmsa_gptq_lora_bwd_dx_workspace(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int act_dtype);
+int fmsa_gptq_lora_bwd_dx_ws(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int mode, void* dX, int64_t lddx,
+                             void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace,
+                             size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Standalone SwiGLU (UL/swiglu.py:20-47 and :50-98) for the paths whose GEMM epilogue cannot
