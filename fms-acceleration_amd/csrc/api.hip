@@ -41,6 +41,10 @@ int launch_ce_fwd(const void* logits, int64_t ld, const int64_t* labels, int M, 
                   hipStream_t st);
 int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse, const int64_t* labels, int M,
                   int V, int dtype, int vec, hipStream_t st);
+int launch_ce_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype,
+                       float* losses, float* lse, hipStream_t st);
+int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse,
+                       const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st);
 int launch_ce_fused(void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, int vec, int64_t ignore_index,
                     const float* scale, float smoothing, float* losses, hipStream_t st);
 int launch_nf4_dequant(const fmsa_nf4_weight* w, int out_dtype, void* out, hipStream_t st);
@@ -559,6 +563,33 @@ int fmsa_cross_entropy_bwd(void* logits, int64_t ld, const float* dloss, int64_t
   if (!is_float_dtype(dtype)) return FMSA_ERR_DTYPE;
   const int vec = (V % 8 == 0) && aligned_rows(logits, ld, dtype);
   return launch_ce_bwd(logits, ld, dloss, dloss_stride, logsumexp, labels, M, V, dtype, vec, (hipStream_t)stream);
+}
+
+static int check_ce_rows(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype) {
+  if (!logits || !labels) return FMSA_ERR_NULL;
+  if (n_seq <= 0 || seq_out <= 0 || seq_in < seq_out || V <= 0 || ld < V) return FMSA_ERR_SHAPE;
+  if ((int64_t)n_seq * seq_in > 0x7fffffff) return FMSA_ERR_SHAPE;
+  if (!is_act(dtype)) return FMSA_ERR_DTYPE;
+  if (reinterpret_cast<uintptr_t>(logits) & 1u) return FMSA_ERR_ALIGN;
+  return FMSA_OK;
+}
+
+int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
+                                int dtype, float* losses, float* logsumexp, void* stream) {
+  if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
+  if (!losses || !logsumexp) return FMSA_ERR_NULL;
+  return launch_ce_rows_fwd(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
+}
+
+int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride,
+                                const float* logsumexp, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype,
+                                void* stream) {
+  if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
+  if (!grad || !dloss || !logsumexp) return FMSA_ERR_NULL;
+  if (dloss_stride < 0) return FMSA_ERR_SHAPE;
+  if (reinterpret_cast<uintptr_t>(grad) & 1u) return FMSA_ERR_ALIGN;
+  return launch_ce_rows_bwd(logits, grad, ld, dloss, dloss_stride, logsumexp, labels, n_seq, seq_in, seq_out, V, dtype,
+                            (hipStream_t)stream);
 }
 
 int fmsa_cross_entropy_fused(void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, int64_t ignore_index,

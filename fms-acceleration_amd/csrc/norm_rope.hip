@@ -454,6 +454,144 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(void* __restrict__ logits, 
 }
 
 
+// The causal-LM loss straight on the model's 16-bit logits [sequences, seq_in, V]: rows 0 .. seq_out - 1 of every sequence
+// count (seq_out = seq_in - 1 where the labels are shifted against the logits).  Forward: one read of the logits.
+// Backward: one read, and one write of a gradient of its own, whole: the rows past seq_out and the rows without a label are
+// written as zeros and not read.  Both are bound by HBM.  The widening copy to fp32, the copy that drops every sequence's
+// last row, the pass over the fp32 gradient and its narrowing and padding copies took 1040 us at 1024 x 128256 bf16 (4.2 GB
+// of traffic); the two kernels move 0.55 - 0.79 GB.
+// Rows are walked in 16-byte chunks from the first aligned element on (V need not be a multiple of 8, so every row of a
+// contiguous matrix may begin elsewhere), with four chunks per thread in flight; the ends are element accesses.
+struct RowSpan {
+  int head, n_vec;  // elements in front of the first 16-byte chunk; chunks
+};
+FMSA_DEVI RowSpan row_span(const uint16_t* x, int V, bool vec) {
+  RowSpan r{V, 0};
+  if (vec) {
+    r.head = min(V, (int)(((16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15) >> 1));
+    r.n_vec = (V - r.head) >> 3;
+  }
+  return r;
+}
+FMSA_DEVI int64_t logits_row(int row, int seq_in, int seq_out) { return (int64_t)(row / seq_out) * seq_in + row % seq_out; }
+
+template <int D>
+__global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels,
+                                                          int seq_in, int seq_out, int V, int vec, float* __restrict__ losses,
+                                                          float* __restrict__ lse_out) {
+  __shared__ float red_m[256], red_s[256];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const int64_t label = labels[row];
+  if (label < 0 || label >= V) {  // ignored (or a caller error, treated as such): uniform over the workgroup
+    if (tid == 0) losses[row] = lse_out[row] = 0.f;
+    return;
+  }
+  const uint16_t* x = logits + logits_row(row, seq_in, seq_out) * ld;
+  const RowSpan sp = row_span(x, V, vec != 0);
+  float m = -INFINITY, s = 0.f;
+  for (int c = tid; c < sp.head; c += 256) online_add(m, s, load1<D>(x, c));
+  for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) online_add(m, s, load1<D>(x, c));
+  const uint16_t* xv = x + sp.head;
+  for (int i = tid; i < sp.n_vec; i += 1024) {
+    float v[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) Vec8<D>::load(xv, 8 * (int64_t)min(i + 256 * u, sp.n_vec - 1), v[u]);
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) mn = fmaxf(mn, v[u][k]);  // (a chunk past the end repeats the last one)
+    if (mn == -INFINITY) continue;  // nothing finite yet: (m, s) stays (-inf, 0), see online_add
+    s *= __builtin_amdgcn_exp2f((m - mn) * kLog2e);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc += __builtin_amdgcn_exp2f((v[u][k] - mn) * kLog2e);
+      s += i + 256 * u < sp.n_vec ? acc : 0.f;
+    }
+    m = mn;
+  }
+  red_m[tid] = m;
+  red_s[tid] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (tid < o) {
+      const float m2 = red_m[tid + o], s2 = red_s[tid + o];
+      const float mn = fmaxf(red_m[tid], m2);
+      const float a = red_m[tid] == -INFINITY ? 0.f : red_s[tid] * __builtin_amdgcn_exp2f((red_m[tid] - mn) * kLog2e);
+      const float b = m2 == -INFINITY ? 0.f : s2 * __builtin_amdgcn_exp2f((m2 - mn) * kLog2e);
+      red_m[tid] = mn;
+      red_s[tid] = a + b;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    const float lse = red_m[0] + __builtin_amdgcn_logf(red_s[0]) * kLn2;
+    lse_out[row] = lse;
+    losses[row] = lse - load1<D>(x, label);
+  }
+}
+
+constexpr int CE_CHUNKS = 4;  // 16-byte chunks per thread of the backward
+
+// grad has the logits' shape, row stride and alignment modulo 16 (vec; otherwise element accesses)
+template <int D>
+__global__ __launch_bounds__(256) void ce_rows_bwd_kernel(const uint16_t* __restrict__ logits, uint16_t* __restrict__ grad, int64_t ld,
+                                                          const float* __restrict__ dloss, int64_t dloss_stride,
+                                                          const float* __restrict__ lse, const int64_t* __restrict__ labels, int seq_in,
+                                                          int seq_out, int V, int vec) {
+  const int seq = blockIdx.x / seq_in, t = blockIdx.x % seq_in;
+  const uint16_t* x = logits + (int64_t)blockIdx.x * ld;
+  uint16_t* g = grad + (int64_t)blockIdx.x * ld;
+  const int row = seq * seq_out + t;
+  const int64_t label = t < seq_out ? labels[row] : -100;
+  const bool live = label >= 0 && label < V;  // uniform over the workgroup
+  const float dl = live ? dloss[(int64_t)row * dloss_stride] : 0.f;
+  const float l = live ? lse[row] : 0.f;
+  const RowSpan sp = row_span(x, V, vec != 0);
+  auto element = [&](int c) {
+    float p = 0.f;
+    if (live) {
+      p = __builtin_amdgcn_exp2f((load1<D>(x, c) - l) * kLog2e);
+      if (c == label) p -= 1.0f;
+      p *= dl;
+    }
+    store1<D>(g, c, p);
+  };
+  const int step = 256 * gridDim.y, first = blockIdx.y * 256 + threadIdx.x;
+  for (int c = first; c < sp.head; c += step) element(c);
+  for (int c = sp.head + 8 * sp.n_vec + first; c < V; c += step) element(c);
+  const int i0 = blockIdx.y * (256 * CE_CHUNKS) + threadIdx.x;
+  const uint16_t* xv = x + sp.head;
+  uint16_t* gv = g + sp.head;
+  if (i0 >= sp.n_vec) return;
+  if (!live) {
+    const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < CE_CHUNKS; ++u)
+      if (i0 + 256 * u < sp.n_vec) Vec8<D>::store(gv, 8 * (int64_t)(i0 + 256 * u), z);
+    return;
+  }
+  float v[CE_CHUNKS][8];
+#pragma unroll
+  for (int u = 0; u < CE_CHUNKS; ++u) Vec8<D>::load(xv, 8 * (int64_t)min(i0 + 256 * u, sp.n_vec - 1), v[u]);
+#pragma unroll
+  for (int u = 0; u < CE_CHUNKS; ++u) {
+    const int i = i0 + 256 * u;
+    if (i >= sp.n_vec) break;
+    const int64_t c = sp.head + 8 * (int64_t)i;
+    float y[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float p = __builtin_amdgcn_exp2f((v[u][k] - l) * kLog2e);
+      if (c + k == label) p -= 1.0f;
+      y[k] = dl * p;
+    }
+    Vec8<D>::store(gv, 8 * (int64_t)i, y);
+  }
+}
+
 // Loss and logits gradient in one launch (reference: fused_ops/liger_ce/cross_entropy.py:33-186): the
 // loss head calls this on each freshly computed chunk of logits, so nothing is saved for a backward
 // pass.  One workgroup per row: pass 1 streams the row (online max / sum exp, and sum x for label
@@ -574,6 +712,33 @@ int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_st
     else
       hipLaunchKernelGGL((ce_bwd_kernel<D, false>), grid, block, 0, st, logits, ld, dloss, dloss_stride, lse, labels, V);
   })
+  FMSA_CHECK_LAUNCH();
+  return FMSA_OK;
+}
+
+int launch_ce_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype,
+                       float* losses, float* lse, hipStream_t st) {
+  const dim3 grid(n_seq * seq_out), block(256);
+  const uint16_t* x = (const uint16_t*)logits;
+  if (dtype == FMSA_BF16)
+    hipLaunchKernelGGL((ce_rows_fwd_kernel<FMSA_BF16>), grid, block, 0, st, x, ld, labels, seq_in, seq_out, V, 1, losses, lse);
+  else
+    hipLaunchKernelGGL((ce_rows_fwd_kernel<FMSA_F16>), grid, block, 0, st, x, ld, labels, seq_in, seq_out, V, 1, losses, lse);
+  FMSA_CHECK_LAUNCH();
+  return FMSA_OK;
+}
+
+int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse,
+                       const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st) {
+  const int per_block = 256 * CE_CHUNKS * 8;
+  const dim3 grid(n_seq * seq_in, (V + per_block - 1) / per_block), block(256);
+  const uint16_t* x = (const uint16_t*)logits;
+  uint16_t* g = (uint16_t*)grad;
+  const int vec = ((reinterpret_cast<uintptr_t>(x) ^ reinterpret_cast<uintptr_t>(g)) & 15) == 0;
+  if (dtype == FMSA_BF16)
+    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_BF16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, lse, labels, seq_in, seq_out, V, vec);
+  else
+    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_F16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, lse, labels, seq_in, seq_out, V, vec);
   FMSA_CHECK_LAUNCH();
   return FMSA_OK;
 }

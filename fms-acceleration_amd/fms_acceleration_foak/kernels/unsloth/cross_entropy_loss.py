@@ -27,6 +27,32 @@ class Fast_CrossEntropyLoss(torch.autograd.Function):
         return logits, None, None
 
 
+class Fast_CausalLMLossRows(torch.autograd.Function):
+    """Losses of rows 0 .. seq_out - 1 of every sequence, read from the 16-bit logits where they are; the gradient is a
+    tensor of its own, so the logits stay as the caller sees them."""
+
+    @staticmethod
+    def forward(ctx, logits, labels, seq_out):
+        losses, logsumexp = fmsa_hip.cross_entropy_rows_fwd(logits, labels, seq_out)
+        ctx.save_for_backward(logits, logsumexp, labels)
+        ctx.seq_out = seq_out
+        return losses
+
+    @staticmethod
+    def backward(ctx, dlosses):
+        logits, logsumexp, labels = ctx.saved_tensors
+        return fmsa_hip.cross_entropy_rows_bwd(logits, dlosses.float(), logsumexp, labels, ctx.seq_out), None, None
+
+
+def _rows_in_place(logits, labels, vocab_size, shifted):
+    """Whether the loss can be taken from the logits as they are: 16-bit, contiguous [batch, seq, vocab] on the GPU, with a
+    label per token (or per token after the shift).  Anything else goes the general way, through an fp32 copy."""
+    return (logits.is_cuda and logits.dtype in (torch.float16, torch.bfloat16) and logits.dim() == 3 and logits.is_contiguous()
+            and logits.shape[2] == vocab_size and 0 not in logits.shape and logits.shape[1] > (0 if shifted else 1)
+            and (labels.numel() == logits.shape[0] * logits.shape[1] if shifted else labels.shape == logits.shape[:2])
+            and not labels.is_floating_point())
+
+
 def fast_cross_entropy_loss(logits, labels):
     """logits (batch, seq_len, vocab), labels (batch, seq_len) -> mean loss over labels != -100."""
     batch, seq_len, d = logits.shape
@@ -49,6 +75,14 @@ class FastCrossEntropyLoss(torch.nn.CrossEntropyLoss):
 def FastForCausalLMLoss(logits, labels, vocab_size: int, num_items_in_batch: int = None, ignore_index: int = -100,
                         shift_labels=None, **kwargs):
     """Counterpart of transformers.loss.loss_utils.ForCausalLMLoss on the fused kernel."""
+    if ignore_index == -100 and _rows_in_place(logits, labels if shift_labels is None else shift_labels, vocab_size, shift_labels is not None):
+        # the fp32 copy, the shifted copy and their gradients' copies cost five times the two kernels
+        seq_out = logits.shape[1] - (shift_labels is None)
+        target = labels[:, 1:] if shift_labels is None else shift_labels
+        target = target.to(device=logits.device, dtype=torch.int64).reshape(-1)
+        loss = Fast_CausalLMLossRows.apply(logits, target, seq_out)
+        n_items = num_items_in_batch if num_items_in_batch is not None else torch.count_nonzero(target != -100)
+        return loss.sum() / n_items
     logits = logits.float()
     if shift_labels is None:
         labels = labels.to(logits.device)

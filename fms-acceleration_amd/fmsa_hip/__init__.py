@@ -59,6 +59,8 @@ EXPORTED_SYMBOLS = (
     "fmsa_rope_embedding",
     "fmsa_cross_entropy_fwd",
     "fmsa_cross_entropy_bwd",
+    "fmsa_cross_entropy_rows_fwd",
+    "fmsa_cross_entropy_rows_bwd",
     "fmsa_cross_entropy_fused",
 )
 
@@ -256,6 +258,9 @@ def lib() -> ctypes.CDLL:
                                       c_int, c_void_p]
     L.fmsa_cross_entropy_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
     L.fmsa_cross_entropy_bwd.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
+    L.fmsa_cross_entropy_rows_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
+    L.fmsa_cross_entropy_rows_bwd.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                              c_int, c_void_p]
     L.fmsa_cross_entropy_fused.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int64, c_void_p, c_float, c_void_p, c_void_p]
     for name in EXPORTED_SYMBOLS:
         getattr(L, name)  # AttributeError here means the library is stale: rebuild it
@@ -726,6 +731,31 @@ def cross_entropy_bwd_(logits2d, dlosses, lse, labels):
                                                                   _ptr(lse), _ptr(labels), M, V, _DTYPE_ENUM[logits2d.dtype],
                                                                   _stream(logits2d)))
     return logits2d
+
+
+def cross_entropy_rows_fwd(logits3d, labels, seq_out: int):
+    """(losses, logsumexp), fp32 [n_seq * seq_out], of rows 0 .. seq_out - 1 of every sequence of contiguous 16-bit logits
+    [n_seq, seq_in, V]; labels int64 [n_seq * seq_out], -100 ignored."""
+    n_seq, seq_in, V = logits3d.shape
+    rows = n_seq * seq_out
+    assert logits3d.is_contiguous() and labels.dtype == torch.int64 and labels.is_contiguous() and labels.numel() == rows
+    losses = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
+    lse = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
+    _check("fmsa_cross_entropy_rows_fwd",
+           lib().fmsa_cross_entropy_rows_fwd(_ptr(logits3d), V, _ptr(labels), n_seq, seq_in, seq_out, V, act_enum(logits3d.dtype),
+                                             _ptr(losses), _ptr(lse), _stream(logits3d)))
+    return losses, lse
+
+
+def cross_entropy_rows_bwd(logits3d, dlosses, lse, labels, seq_out: int):
+    """Gradient of cross_entropy_rows_fwd's losses, a tensor of its own; dlosses fp32 (any stride, 0 included)."""
+    n_seq, seq_in, V = logits3d.shape
+    assert dlosses.dtype == torch.float32 and dlosses.dim() == 1 and dlosses.numel() == n_seq * seq_out
+    grad = torch.empty_like(logits3d)
+    _check("fmsa_cross_entropy_rows_bwd",
+           lib().fmsa_cross_entropy_rows_bwd(_ptr(logits3d), _ptr(grad), V, _ptr(dlosses), dlosses.stride(0), _ptr(lse), _ptr(labels),
+                                             n_seq, seq_in, seq_out, V, act_enum(logits3d.dtype), _stream(logits3d)))
+    return grad
 
 
 def cross_entropy_fused_(logits2d, labels, scale=None, label_smoothing=0.0, ignore_index=-100, losses_out=None):

@@ -408,6 +408,17 @@ int fmsa_cross_entropy_bwd(void* logits, int64_t ld, const float* dloss, int64_t
                            const float* logsumexp, const int64_t* labels, int M, int V, int dtype,
                            void* stream);
 
+/* The same loss straight on 16-bit logits [n_seq, seq_in, V] (row stride ld) of which rows 0 .. seq_out - 1 of every
+ * sequence count: seq_out = seq_in - 1 with labels [n_seq, seq_out] shifted by one token is the causal-LM loss
+ * (kernels/unsloth/cross_entropy_loss.py:302-327) without a copy of the logits.  losses, logsumexp: [n_seq * seq_out].
+ * The backward writes a gradient of its own, all of [n_seq, seq_in, V] (row stride ld; rows past seq_out and rows without
+ * a label are zeros), and leaves the logits alone. */
+int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out,
+                                int V, int dtype, float* losses, float* logsumexp, void* stream);
+int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride,
+                                const float* logsumexp, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
+                                int dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Loss and logits gradient in one launch, for a loss head that consumes its logits chunk by chunk
  * (fused_ops/liger_ce/cross_entropy.py:33-186, called from

@@ -1,0 +1,53 @@
+"""FastForCausalLMLoss on 16-bit logits read in place, against the same function on the fp32 copy of them (which goes through
+the general kernels): edges of the 16-byte chunks, odd vocabularies, rows that begin anywhere, ignored rows."""
+import pytest
+import torch
+
+from tests.helpers import randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,s,V,offset", [(1, 2, 3, 0), (2, 9, 8, 8), (3, 5, 17, 1), (2, 7, 8195, 3), (2, 3, 32003, 0), (1, 4, 40960, 5)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_rows_in_place(b, s, V, offset, shifted, dtype):
+    from fms_acceleration_foak.kernels.unsloth import FastForCausalLMLoss
+
+    gen = torch.Generator().manual_seed(V)
+    store = torch.empty(offset + b * s * V, dtype=dtype, device="cuda")
+    store[offset:] = randn((b * s * V,), 5, dtype, scale=3.0).cuda()
+    x = store[offset:].view(b, s, V)
+    labels = torch.randint(0, V, (b, s), generator=gen)
+    labels[:, 0] = labels[:, 1] = V - 1
+    if s > 3:
+        labels[b - 1, 2:4] = -100
+        x[b - 1, 1 if not shifted else 2, V // 2] = float("inf")  # in a row without a label: not part of the loss
+    labels = labels.cuda()
+    kw = {"shift_labels": labels} if shifted else {}
+    keep = x.clone()
+    xa = x.detach().requires_grad_(True)
+    la = FastForCausalLMLoss(xa, labels, V, **kw)
+    (2.5 * la).backward()
+    clean = torch.where(torch.isinf(keep), torch.zeros_like(keep), keep)  # the general backward multiplies such a row by zero
+    xb = clean.float().requires_grad_(True)
+    lb = FastForCausalLMLoss(xb * 1.0, labels, V, **kw)
+    (2.5 * lb).backward()
+    assert torch.equal(x, keep)  # the logits are left alone
+    assert abs(la.item() - lb.item()) <= 2e-6 * max(1.0, abs(lb.item()))  # fp32 sums in another order
+    # the gradients agree to fp32 rounding before their one rounding to the storage type: at most one unit apart
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    tiny = 1e-30 if dtype == torch.bfloat16 else 2.0 ** -24
+    diff = (xa.grad.float() - xb.grad).abs()
+    assert bool((diff <= ulp * xb.grad.abs() + tiny).all())
+    if not shifted:
+        assert bool((xa.grad[:, -1] == 0).all())
+
+
+def test_all_labels_ignored():
+    from fms_acceleration_foak.kernels.unsloth import FastForCausalLMLoss
+
+    x = randn((2, 5, 1000), 1, torch.bfloat16).cuda().requires_grad_(True)
+    loss = FastForCausalLMLoss(x, torch.full((2, 5), -100, device="cuda"), 1000, num_items_in_batch=7)
+    loss.backward()
+    assert loss.item() == 0.0 and bool((x.grad == 0).all())
