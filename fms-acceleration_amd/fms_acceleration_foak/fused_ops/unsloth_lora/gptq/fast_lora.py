@@ -38,6 +38,7 @@ from fmsa_hip.gptq_prepared import prepare as _prepare  # per-weight C-ABI view,
 
 from .. import fused_core as core
 from ..fused_core import _act_dtype, _Proj
+from ..utils import active_adapter_parts, member
 
 
 # ----------------------------------------------------------------------------------------------
@@ -75,18 +76,17 @@ def _nonzero_bias(qmodule):
 
 
 def extract_gptq_state(qmodule):
-    if hasattr(qmodule, "base_layer"):
-        qmodule = qmodule.base_layer
+    qmodule = member(qmodule, "_modules", "base_layer", qmodule)
     return GPTQuantState(
         infeatures=qmodule.infeatures,
         outfeatures=qmodule.outfeatures,
         bits=qmodule.bits,
         group_size=qmodule.group_size,
         maxq=qmodule.maxq,
-        qweight=qmodule.qweight,
-        qzeros=qmodule.qzeros,
-        scales=qmodule.scales,
-        g_idx=qmodule.g_idx,
+        qweight=member(qmodule, "_buffers", "qweight"),
+        qzeros=member(qmodule, "_buffers", "qzeros"),
+        scales=member(qmodule, "_buffers", "scales"),
+        g_idx=member(qmodule, "_buffers", "g_idx"),
         bias=_nonzero_bias(qmodule),
     )
 
@@ -94,7 +94,7 @@ def extract_gptq_state(qmodule):
 def get_lora_parameters(proj):
     """(qstate, bias, A, B, s, dropout) of a LoRA-wrapped (or bare) GPTQ linear; A = B = s = None
     when the adapters are disabled or merged (:94-116)."""
-    base_layer = proj.base_layer if hasattr(proj, "base_layer") else proj
+    base_layer = member(proj, "_modules", "base_layer", proj)
     qstate = extract_gptq_state(base_layer)
     bias = qstate.bias
     if base_layer.__module__.startswith("auto_gptq"):
@@ -102,12 +102,7 @@ def get_lora_parameters(proj):
         setattr(qstate.qzeros, "offset", 1)
     if not hasattr(proj, "disable_adapters") or proj.disable_adapters or proj.merged:
         return qstate, bias, None, None, None, None
-    active = proj.active_adapters[0] if hasattr(proj, "active_adapters") else proj.active_adapter
-    A = proj.lora_A[active].weight
-    B = proj.lora_B[active].weight
-    s = proj.scaling[active]
-    dropout = proj.lora_dropout[active] if hasattr(proj, "lora_dropout") else None
-    return qstate, bias, A, B, s, dropout
+    return (qstate, bias) + active_adapter_parts(proj)
 
 
 

@@ -17,18 +17,38 @@ def QUANT_STATE(W, base_layer):
     return getattr(base_layer, "quant_state", None)
 
 
+_RAISE = object()
+
+
+def member(module, kind, name, default=_RAISE):
+    """getattr(module, name) for what a module keeps in its `kind` dictionary (_modules, _buffers, _parameters), asked for
+    there first: nn.Module.__getattr__ runs after a failed lookup and searches all three, which a layer pass of seven
+    adapted projections pays for a hundred times.  Anything kept elsewhere (a property, a plain attribute) is found as
+    getattr finds it."""
+    found = module.__dict__.get(kind)
+    if found is not None:
+        found = found.get(name)
+        if found is not None:
+            return found
+    return getattr(module, name) if default is _RAISE else getattr(module, name, default)
+
+
+def active_adapter_parts(proj):
+    """(A, B, scaling, dropout) of the active adapter of a LoRA layer."""
+    active = proj.active_adapters[0] if hasattr(proj, "active_adapters") else proj.active_adapter
+    A = member(member(proj, "_modules", "lora_A")[active], "_parameters", "weight")
+    B = member(member(proj, "_modules", "lora_B")[active], "_parameters", "weight")
+    dropout = member(proj, "_modules", "lora_dropout", None)
+    return A, B, proj.scaling[active], None if dropout is None else dropout[active]
+
+
 def get_lora_parameters(proj):
-    base_layer = proj.base_layer if hasattr(proj, "base_layer") else proj
-    W = base_layer.weight
-    bias = base_layer.bias if hasattr(base_layer, "bias") else None
+    base_layer = member(proj, "_modules", "base_layer", proj)
+    W = member(base_layer, "_parameters", "weight")
+    bias = getattr(base_layer, "bias", None)
     if not hasattr(proj, "disable_adapters") or proj.disable_adapters or proj.merged:
         return W, QUANT_STATE(W, base_layer), bias, None, None, None, None
-    active = proj.active_adapters[0] if hasattr(proj, "active_adapters") else proj.active_adapter
-    A = proj.lora_A[active].weight
-    B = proj.lora_B[active].weight
-    s = proj.scaling[active]
-    dropout = proj.lora_dropout[active] if hasattr(proj, "lora_dropout") else None
-    return W, QUANT_STATE(W, base_layer), bias, A, B, s, dropout
+    return (W, QUANT_STATE(W, base_layer), bias) + active_adapter_parts(proj)
 
 
 def fast_dequantize(W, quant_state=None, out_dtype=None):

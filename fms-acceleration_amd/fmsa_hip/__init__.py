@@ -373,7 +373,7 @@ def lora_down(x2d, wd, out=None):
     r = wd.shape[0]
     assert wd.shape[1] == C and wd.is_contiguous() and wd.dtype == x2d.dtype and x2d.stride(1) == 1
     if out is None:
-        out = torch.empty((M, r), dtype=x2d.dtype, device=x2d.device)
+        out = x2d.new_empty((M, r))
     assert out.shape == (M, r) and out.stride(1) == 1 and out.dtype == x2d.dtype
     nbytes = lib().fmsa_lora_down_split_workspace(M, C, r)
     ws = _workspace(nbytes, x2d.device) if nbytes else None
@@ -477,7 +477,7 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None,
     outs = []
     for i, p in enumerate(projs):
         w = p["w"]
-        y = torch.empty((M, w.N), dtype=x2d.dtype, device=x2d.device)
+        y = x2d.new_empty((M, w.N))
         outs.append(y)
         U = p.get("U") if p["r"] else None
         assert U is None or U.stride(1) == 1
@@ -643,22 +643,21 @@ def lora_pack_batch(adapters, act_dtype):
     for A, B, A16_out in adapters:
         if not (A.is_cuda and B.is_cuda):
             raise RuntimeError("fmsa_hip needs GPU tensors")
-        A, B = A.detach(), B.detach()
         if A.dtype != B.dtype:
-            B = B.to(A.dtype)
-        A = A if A.is_contiguous() else A.contiguous()
-        B = B if B.is_contiguous() else B.contiguous()
+            B = B.detach().to(A.dtype)
+        A = A if A.is_contiguous() else A.detach().contiguous()
+        B = B if B.is_contiguous() else B.detach().contiguous()
         r, K = A.shape
         N = B.shape[0]
-        own_a = A16_out is None
-        buf = torch.empty(r * K * (2 if own_a else 1) + 2 * r * N, dtype=act_dtype, device=A.device)
-        o = 0
-        if own_a:
-            A16_out, o = buf[: r * K].view(r, K), r * K
-        assert A16_out.shape == (r, K) and A16_out.is_contiguous() and A16_out.dtype == act_dtype
-        At16 = buf[o : o + r * K].view(K, r)
-        B16 = buf[o + r * K : o + r * K + N * r].view(N, r)
-        Bt16 = buf[o + r * K + N * r :].view(r, N)
+        # an allocation each: four cost the host less than one and its four views
+        dev = A.device
+        if A16_out is None:
+            A16_out = torch.empty((r, K), dtype=act_dtype, device=dev)
+        else:
+            assert A16_out.shape == (r, K) and A16_out.is_contiguous() and A16_out.dtype == act_dtype
+        At16 = torch.empty((K, r), dtype=act_dtype, device=dev)
+        B16 = torch.empty((N, r), dtype=act_dtype, device=dev)
+        Bt16 = torch.empty((r, N), dtype=act_dtype, device=dev)
         outs.append((A16_out, At16, B16, Bt16))
         jobs.append((A, B, LoraPackJob(_ptr(A), _ptr(B), _ptr(A16_out), _ptr(At16), _ptr(B16), _ptr(Bt16), r, K, N,
                                        _DTYPE_ENUM[A.dtype])))
