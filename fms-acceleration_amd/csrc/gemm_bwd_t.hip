@@ -969,11 +969,15 @@ static int bwd_t_stages(const fmsa_bwd_proj* projs, int n_proj) {
   return n;
 }
 
-static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M) {
-  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj));
+static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M, int mode) {
+  const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;
+  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), codebook ? 1.7f : 1.4f,
+                    mode == FMSA_BWD_SWIGLU ? 0.12f : 0.f);
 }
 
-size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M) { return bwd_t_split(projs, n_proj, M).bytes(); }
+size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M) {
+  return std::max(bwd_t_split(projs, n_proj, M, FMSA_BWD_LINEAR).bytes(), bwd_t_split(projs, n_proj, M, FMSA_BWD_SWIGLU).bytes());
+}
 
 int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx,
                               void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace,
@@ -1018,7 +1022,7 @@ int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int
   a.nbk = (a.K + 255) / 256;
   dim3 grid(a.nbm * a.nbk), block(256);
   // without a workspace that holds it, every tile runs whole
-  SplitPlan plan = bwd_t_split(projs, n_proj, M);
+  SplitPlan plan = bwd_t_split(projs, n_proj, M, mode);
   if (!workspace || workspace_bytes < plan.bytes()) plan.s = 1;
   if (plan.s > 1) {
     a.n_whole = plan.n_whole;
