@@ -807,6 +807,21 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const Bw
   const int m = bm * BM + 32 * mt + l32;
   if (bm * BM + 32 * mt >= a.M) return;  // the whole workgroup
   const bool m_ok = m < a.M;
+  // A workgroup is short and few are resident, so its time is its chain of memory latencies: the mask, four rank steps of
+  // every projection and the sums are each asked for in one go (one step and one load after the other: 32 us at 80 tiles,
+  // rank 64).
+  bool any_lora = false;
+  for (int p = 0; p < a.n_proj; ++p) any_lora = any_lora || select_proj(a, p).r > 0;
+  const bool has_mask = a.mask_src != nullptr && any_lora;
+  u32x2 mask[NT][4];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = bk * 256 + 64 * wave + 32 * j + 8 * i0 + 4 * half;
+      mask[j][i0] = u32x2{0u, 0u};
+      if (has_mask && m_ok && col < a.K) mask[j][i0] = *reinterpret_cast<const u32x2*>(a.mask_src + (size_t)m * a.ldmask + col);
+    }
   f32x4 acc[NT][4];
   split_load(acc, a.partial, cut, mt, a.n_ranges);
   f32x16 lora[NT];
@@ -814,28 +829,34 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const Bw
   for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i) lora[j][i] = 0.f;
-  bool any_lora = false;
   for (int p = 0; p < a.n_proj; ++p) {
     const BwdTProjDev P = select_proj(a, p);
     if (P.r <= 0) continue;
-    any_lora = true;
     f32x16 tmp[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int i = 0; i < 16; ++i) tmp[j][i] = 0.f;
-    for (int j0 = 0; j0 < P.r; j0 += 16) {
-      const int ko = j0 + 8 * half;
-      u32x4 tf = {0u, 0u, 0u, 0u}, af[NT];
-      if (m_ok && ko < P.r) tf = *reinterpret_cast<const u32x4*>(P.T + (size_t)m * P.ldt + ko);
+    for (int j0 = 0; j0 < P.r; j0 += 64) {
+      u32x4 tf[4], af[4][NT];
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const int col = bk * 256 + 64 * wave + 32 * j;
-        af[j] = u32x4{0u, 0u, 0u, 0u};
-        if (col < a.K && ko < P.r) af[j] = *reinterpret_cast<const u32x4*>(P.At + (size_t)(col + l32) * P.r + ko);
+      for (int st = 0; st < 4; ++st) {
+        const int ko = j0 + 16 * st + 8 * half;
+        tf[st] = u32x4{0u, 0u, 0u, 0u};
+        if (m_ok && ko < P.r) tf[st] = *reinterpret_cast<const u32x4*>(P.T + (size_t)m * P.ldt + ko);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const int col = bk * 256 + 64 * wave + 32 * j;
+          af[st][j] = u32x4{0u, 0u, 0u, 0u};
+          if (col < a.K && ko < P.r) af[st][j] = *reinterpret_cast<const u32x4*>(P.At + (size_t)(col + l32) * P.r + ko);
+        }
       }
 #pragma unroll
-      for (int j = 0; j < NT; ++j) tmp[j] = mfma32<T>(af[j], tf, tmp[j]);
+      for (int st = 0; st < 4; ++st)
+        if (j0 + 16 * st < P.r) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) tmp[j] = mfma32<T>(af[st][j], tf[st], tmp[j]);
+        }
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j)
@@ -843,7 +864,6 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const Bw
       for (int i = 0; i < 16; ++i) lora[j][i] += P.s * tmp[j][i];
   }
   if (!m_ok) return;
-  const bool has_mask = a.mask_src != nullptr && any_lora;
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int col0 = bk * 256 + 64 * wave + 32 * j;
@@ -852,9 +872,9 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const Bw
     for (int i0 = 0; i0 < 4; ++i0) {
       const int col = col0 + 8 * i0 + 4 * half;
       const u32x2 bv = {pack2<T>(acc[j][i0][0], acc[j][i0][1]), pack2<T>(acc[j][i0][2], acc[j][i0][3])};
-      u32x2 lv = {0u, 0u}, mv = {0u, 0u};
+      const u32x2 mv = mask[j][i0];
+      u32x2 lv = {0u, 0u};
       if (any_lora) lv = u32x2{pack2<T>(lora[j][4 * i0], lora[j][4 * i0 + 1]), pack2<T>(lora[j][4 * i0 + 2], lora[j][4 * i0 + 3])};
-      if (has_mask) mv = *reinterpret_cast<const u32x2*>(a.mask_src + (size_t)m * a.ldmask + col);
       if constexpr (swiglu) {
         const size_t o = (size_t)m * a.ldeg + col;
         const u32x2 ev = *reinterpret_cast<const u32x2*>(a.e + o), gv = *reinterpret_cast<const u32x2*>(a.g + o);
