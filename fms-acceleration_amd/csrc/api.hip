@@ -37,6 +37,9 @@ int launch_rms_bwd(void* dY, int64_t lddy, const void* X, int64_t ldx, const voi
                    int x_dtype, int w_dtype, hipStream_t st);
 int launch_rope(void* Q, int64_t ldq, const void* cosp, const void* sinp, int64_t ldcs, int M, int n_heads, int head_dim, int cs_rows,
                 int backward, int q_dtype, int cs_dtype, hipStream_t st);
+int launch_rope_strided(const void* src, int64_t s_batch, int64_t s_tok, int64_t s_head, void* dst, const void* cosp, const void* sinp,
+                        int64_t ldcs, int batch, int seq, int n_heads, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype,
+                        hipStream_t st);
 int launch_ce_fwd(const void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, int vec, float* losses, float* lse,
                   hipStream_t st);
 int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse, const int64_t* labels, int M,
@@ -545,6 +548,22 @@ int fmsa_rope_embedding(void* Q, int64_t ldq, const void* cos, const void* sin, 
   if (!aligned_rows(Q, ldq, q_dtype) || !aligned_rows(cos, ldcs, cs_dtype) || !aligned_rows(sin, ldcs, cs_dtype))
     return FMSA_ERR_ALIGN;
   return launch_rope(Q, ldq, cos, sin, ldcs, M, n_heads, head_dim, cs_rows, backward, q_dtype, cs_dtype, (hipStream_t)stream);
+}
+
+int fmsa_rope_embedding_strided(const void* src, int64_t stride_batch, int64_t stride_token, int64_t stride_head, void* dst,
+                                const void* cos, const void* sin, int64_t ldcs, int batch, int seq, int n_heads, int head_dim,
+                                int cs_rows, int backward, int q_dtype, int cs_dtype, void* stream) {
+  if (!src || !dst || !cos || !sin) return FMSA_ERR_NULL;
+  if (batch <= 0 || seq <= 0 || n_heads <= 0 || head_dim <= 0 || head_dim % 16 != 0 || cs_rows <= 0) return FMSA_ERR_SHAPE;
+  if ((int64_t)batch * seq > 0x7fffffff || ldcs < head_dim / 2) return FMSA_ERR_SHAPE;
+  if (stride_batch < 0 || stride_token < 0 || stride_head < 0) return FMSA_ERR_SHAPE;
+  if (!is_float_dtype(q_dtype) || !is_float_dtype(cs_dtype)) return FMSA_ERR_DTYPE;
+  const int64_t row = (int64_t)n_heads * head_dim;
+  if (!aligned_rows(src, stride_batch, q_dtype) || !aligned_rows(src, stride_token, q_dtype) || !aligned_rows(src, stride_head, q_dtype) ||
+      !aligned_rows(dst, row, q_dtype) || !aligned_rows(cos, ldcs, cs_dtype) || !aligned_rows(sin, ldcs, cs_dtype))
+    return FMSA_ERR_ALIGN;
+  return launch_rope_strided(src, stride_batch, stride_token, stride_head, dst, cos, sin, ldcs, batch, seq, n_heads, head_dim, cs_rows,
+                             backward, q_dtype, cs_dtype, (hipStream_t)stream);
 }
 
 int fmsa_cross_entropy_fwd(const void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, float* losses,

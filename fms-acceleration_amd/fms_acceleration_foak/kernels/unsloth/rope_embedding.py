@@ -42,6 +42,10 @@ class Fast_RoPE_Embedding(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dY):
         batch, seq_len, n_heads, head_dim = dY.shape
+        if not dY.is_contiguous() and fmsa_hip.rope_strided_ok(dY, ctx.cos, ctx.sin):
+            # attention's [batch, heads, seq, head_dim] seen token by token: read where it lies instead of copied into rows
+            dX = fmsa_hip.rope_embedding_(dY, ctx.cos, ctx.sin, n_heads, head_dim, backward=True, strided=True)
+            return dX.view(batch, seq_len, n_heads, head_dim), None, None
         dY2 = dY.reshape(batch * seq_len, n_heads * head_dim)  # reshape: dY may be non-contiguous (:111-112)
         dY2 = dY2 if dY2.stride(1) == 1 else dY2.contiguous()
         fmsa_hip.rope_embedding_(dY2, ctx.cos, ctx.sin, n_heads, head_dim, backward=True)

@@ -57,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "fmsa_rms_layernorm_fwd",
     "fmsa_rms_layernorm_bwd",
     "fmsa_rope_embedding",
+    "fmsa_rope_embedding_strided",
     "fmsa_cross_entropy_fwd",
     "fmsa_cross_entropy_bwd",
     "fmsa_cross_entropy_rows_fwd",
@@ -256,6 +257,8 @@ def lib() -> ctypes.CDLL:
                                          c_int, c_void_p]
     L.fmsa_rope_embedding.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int,
                                       c_int, c_void_p]
+    L.fmsa_rope_embedding_strided.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                              c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]
     L.fmsa_cross_entropy_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
     L.fmsa_cross_entropy_bwd.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
     L.fmsa_cross_entropy_rows_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
@@ -697,8 +700,12 @@ def rms_layernorm_bwd(dy2d, x2d, weight, r, gemma: bool = False):
     return dy2d
 
 
-def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bool = False):
-    """In place on q2d [M, n_heads * head_dim]; row m uses row m % cos2d.shape[0] of cos / sin."""
+def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bool = False, strided: bool = False):
+    """In place on q2d [M, n_heads * head_dim]; row m uses row m % cos2d.shape[0] of cos / sin.  strided=True takes
+    [batch, seq, n_heads, head_dim] of any strides instead and returns new rows (rope_embedding_strided)."""
+    if strided:
+        assert q2d.shape[2:] == (n_heads, head_dim)
+        return rope_embedding_strided(q2d, cos2d, sin2d, backward)
     if not (q2d.is_cuda and cos2d.is_cuda and sin2d.is_cuda):
         raise RuntimeError("fmsa_hip needs GPU tensors")
     assert q2d.stride(1) == 1 and cos2d.stride(1) == 1 and cos2d.stride() == sin2d.stride() and cos2d.dtype == sin2d.dtype
@@ -707,6 +714,29 @@ def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bo
                                      head_dim, cos2d.shape[0], int(backward), _DTYPE_ENUM[q2d.dtype], _DTYPE_ENUM[cos2d.dtype],
                                      _stream(q2d)))
     return q2d
+
+
+def rope_strided_ok(q4d, cos2d, sin2d) -> bool:
+    """Whether rope_embedding_strided takes q4d [batch, seq, heads, head_dim] as it lies in memory."""
+    esz, csz = q4d.element_size(), cos2d.element_size()
+    return (q4d.is_cuda and q4d.numel() > 0 and q4d.dtype in _DTYPE_ENUM and q4d.stride(3) == 1 and q4d.shape[3] % 16 == 0
+            and q4d.data_ptr() % 16 == 0 and all(q4d.stride(i) >= 0 and q4d.stride(i) * esz % 16 == 0 for i in range(3))
+            and cos2d.data_ptr() % 16 == 0 and sin2d.data_ptr() % 16 == 0 and cos2d.stride(0) * csz % 16 == 0)
+
+
+def rope_embedding_strided(q4d, cos2d, sin2d, backward: bool = False):
+    """The rotation of q4d [batch, seq, heads, head_dim], any strides (see rope_strided_ok), as contiguous rows
+    [batch * seq, heads * head_dim]; row m uses row m % cos2d.shape[0] of cos / sin.  q4d is left alone."""
+    if not (q4d.is_cuda and cos2d.is_cuda and sin2d.is_cuda):
+        raise RuntimeError("fmsa_hip needs GPU tensors")
+    b, t, h, d = q4d.shape
+    assert q4d.stride(3) == 1 and cos2d.stride(1) == 1 and cos2d.stride() == sin2d.stride() and cos2d.dtype == sin2d.dtype
+    out = q4d.new_empty((b * t, h * d))
+    _check("fmsa_rope_embedding_strided",
+           lib().fmsa_rope_embedding_strided(_ptr(q4d), q4d.stride(0), q4d.stride(1), q4d.stride(2), _ptr(out), _ptr(cos2d), _ptr(sin2d),
+                                             cos2d.stride(0), b, t, h, d, cos2d.shape[0], int(backward), _DTYPE_ENUM[q4d.dtype],
+                                             _DTYPE_ENUM[cos2d.dtype], _stream(q4d)))
+    return out
 
 
 def cross_entropy_fwd(logits2d, labels):
