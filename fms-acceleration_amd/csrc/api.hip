@@ -15,6 +15,8 @@ size_t lora_grad_batch_workspace(const fmsa_lora_grad_job* jobs, int n_jobs, int
 size_t lora_down_workspace(int M, int C, int r, bool few_tokens);
 int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out, int64_t ldo,
                         void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st);
+size_t lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M);
+int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st);
 int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st);
 int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
                          int64_t ldh, const fmsa_rope* rope, int act_dtype, void* workspace, size_t workspace_bytes, hipStream_t st);
@@ -203,6 +205,37 @@ int fmsa_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, 
 int fmsa_lora_down_split(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
                       int64_t ldout, void* workspace, size_t workspace_bytes, void* stream) {
   return lora_down_ws(X, ldx, Wd, M, C, r, act_dtype, out, ldout, workspace, workspace_bytes, true, stream);
+}
+
+static int check_down_jobs(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
+  if (!jobs) return FMSA_ERR_NULL;
+  if (n_jobs < 1 || n_jobs > FMSA_LORA_DOWN_MAX_JOBS || M <= 0) return FMSA_ERR_SHAPE;
+  for (int q = 0; q < n_jobs; ++q) {
+    const fmsa_lora_down_job& s = jobs[q];
+    if (s.C <= 0 || s.C % 8 != 0 || s.r <= 0 || s.ldx < s.C || s.ldout < s.r) return FMSA_ERR_SHAPE;
+    if (int rc = check_rank(s.r)) return rc;
+  }
+  return FMSA_OK;
+}
+
+size_t fmsa_lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
+  return check_down_jobs(jobs, n_jobs, M) == FMSA_OK ? lora_down_batch_workspace(jobs, n_jobs, M) : 0;
+}
+
+int fmsa_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+  if (int rc = check_down_jobs(jobs, n_jobs, M)) return rc;
+  if (!is_act(act_dtype)) return FMSA_ERR_DTYPE;
+  for (int q = 0; q < n_jobs; ++q) {
+    const fmsa_lora_down_job& s = jobs[q];
+    if (!s.X || !s.Wd || !s.out) return FMSA_ERR_NULL;
+    if (!aligned16(s.X) || !aligned16(s.Wd) || s.ldx % 8 != 0 || (reinterpret_cast<uintptr_t>(s.out) & 7u) || s.ldout % 4 != 0)
+      return FMSA_ERR_ALIGN;
+  }
+  if (!workspace) return FMSA_ERR_NULL;
+  if (!aligned16(workspace)) return FMSA_ERR_ALIGN;
+  if (workspace_bytes < lora_down_batch_workspace(jobs, n_jobs, M)) return FMSA_ERR_SHAPE;
+  return launch_lora_down_batch(jobs, n_jobs, M, act_dtype, workspace, (hipStream_t)stream);
 }
 
 size_t fmsa_lora_grad_workspace(int M, int C, int r) {

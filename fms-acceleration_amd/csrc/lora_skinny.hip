@@ -23,9 +23,8 @@ namespace {
 // (40 us at 1100 tokens x 4096, rank 64; 17 us for ONE token), so the columns are also split over gridDim.y workgroups:
 // their fp32 sums go to partial[split][M][r], which lora_down_reduce_kernel adds in index order.
 template <typename T, int RT, int MTL, int NW>
-__global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __restrict__ X, int64_t ldx,
-                                                            const uint16_t* __restrict__ Wd, int M, int C, int r,
-                                                            uint16_t* __restrict__ out, int64_t ldo, float* __restrict__ partial) {
+FMSA_DEVI void lora_down_tile(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ Wd, int M, int C, int r,
+                              uint16_t* __restrict__ out, int64_t ldo, float* __restrict__ partial, int n_split) {
   constexpr int NH = NW / 2;
   __shared__ float red[NH][MTL][RT][64][4];
   const int tid = threadIdx.x;
@@ -34,7 +33,7 @@ __global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __re
   const int m_base = blockIdx.x * (16 * MTL);
   // slice boundaries in units of 32 columns
   const int n32 = (C + 31) / 32;
-  const int slice = blockIdx.y * NW + wave, n_slices = gridDim.y * NW;
+  const int slice = blockIdx.y * NW + wave, n_slices = n_split * NW;
   const int per = (n32 + n_slices - 1) / n_slices;
   const int c_begin = min(C, slice * per * 32);
   const int c_end = min(C, (slice + 1) * per * 32);
@@ -103,6 +102,36 @@ __global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __re
         out[(size_t)row * ldo + j] = pack1<T>(v);
     }
   }
+}
+
+template <typename T, int RT, int MTL, int NW>
+__global__ __launch_bounds__(64 * NW) void lora_down_kernel(const uint16_t* __restrict__ X, int64_t ldx,
+                                                            const uint16_t* __restrict__ Wd, int M, int C, int r,
+                                                            uint16_t* __restrict__ out, int64_t ldo, float* __restrict__ partial) {
+  lora_down_tile<T, RT, MTL, NW>(X, ldx, Wd, M, C, r, out, ldo, partial, gridDim.y);
+}
+
+// Several products over the same few tokens in one launch (q, k, v; gate, up): blockIdx.z names the job.  A launch of one
+// of them is 14 us at 1100 tokens, rank 64, most of it ramp and latency; its column sums are another launch.
+struct LoraDownJobDev {
+  const uint16_t* X;
+  const uint16_t* Wd;
+  uint16_t* out;
+  float* partial;
+  int64_t ldx, ldo;
+  int C, r, n_split;
+};
+struct LoraDownArgs {
+  LoraDownJobDev j[FMSA_LORA_DOWN_MAX_JOBS];
+  int M;
+};
+FMSA_DEVI LoraDownJobDev select_down_job(const LoraDownArgs& a, int q) { return q == 0 ? a.j[0] : (q == 1 ? a.j[1] : a.j[2]); }
+
+template <typename T, int RT, int NW>
+__global__ __launch_bounds__(64 * NW) void lora_down_batch_kernel(const LoraDownArgs a) {
+  const LoraDownJobDev J = select_down_job(a, blockIdx.z);
+  if ((int)blockIdx.y >= J.n_split) return;
+  lora_down_tile<T, RT, 1, NW>(J.X, J.ldx, J.Wd, a.M, J.C, J.r, J.out, J.ldo, J.partial, J.n_split);
 }
 
 // ---- lora_down, staged ----------------------------------------------------------------------------
@@ -449,8 +478,7 @@ __global__ __launch_bounds__(512) void lora_down_split_kernel(const uint16_t* __
 
 // out[m, j] = round(sum over splits, in index order, of partial[split][m][j]); r % 8 == 0: four ranks per thread
 template <typename T>
-__global__ __launch_bounds__(256) void lora_down_reduce_kernel(const float* __restrict__ partial, int n_split, int M, int r,
-                                                               uint16_t* __restrict__ out, int64_t ldo) {
+FMSA_DEVI void lora_down_reduce(const float* __restrict__ partial, int n_split, int M, int r, uint16_t* __restrict__ out, int64_t ldo) {
   const int64_t q4 = (int64_t)blockIdx.x * 256 + threadIdx.x;  // quad of ranks
   const int per_row = r / 4;
   if (q4 >= (int64_t)M * per_row) return;
@@ -463,6 +491,17 @@ __global__ __launch_bounds__(256) void lora_down_reduce_kernel(const float* __re
   o[0] = pack2<T>(v[0], v[1]);
   o[1] = pack2<T>(v[2], v[3]);
   *reinterpret_cast<u32x2*>(out + (size_t)m * ldo + j) = o;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void lora_down_reduce_kernel(const float* __restrict__ partial, int n_split, int M, int r,
+                                                               uint16_t* __restrict__ out, int64_t ldo) {
+  lora_down_reduce<T>(partial, n_split, M, r, out, ldo);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void lora_down_reduce_batch_kernel(const LoraDownArgs a) {
+  const LoraDownJobDev J = select_down_job(a, blockIdx.y);
+  lora_down_reduce<T>(J.partial, J.n_split, a.M, J.r, J.out, J.ldo);
 }
 
 // ---- lora_grad ----------------------------------------------------------------------------------
@@ -925,6 +964,55 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
 #undef SPLIT_LAUNCH
   FMSA_CHECK_LAUNCH();
   if (d.n_split > 1) return reduce();
+  return FMSA_OK;
+}
+
+// One launch for up to FMSA_LORA_DOWN_MAX_JOBS products over the same tokens, for few tokens (the rule of the g = 1 split).
+static int down_batch_split(int M, int C, int n_jobs) { return std::max(1, std::min(512 / (((M + 15) / 16) * n_jobs), C / 512)); }
+
+size_t lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
+  size_t bytes = 0;
+  for (int q = 0; q < n_jobs; ++q) bytes += (size_t)down_batch_split(M, jobs[q].C, n_jobs) * M * jobs[q].r * sizeof(float);
+  return bytes;
+}
+
+int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st) {
+  LoraDownArgs a{};
+  a.M = M;
+  int r_max = 0, split_max = 1;
+  float* p = (float*)workspace;
+  for (int q = 0; q < n_jobs; ++q) {
+    const fmsa_lora_down_job& s = jobs[q];
+    LoraDownJobDev& d = a.j[q];
+    d.X = (const uint16_t*)s.X;
+    d.Wd = (const uint16_t*)s.Wd;
+    d.out = (uint16_t*)s.out;
+    d.ldx = s.ldx;
+    d.ldo = s.ldout;
+    d.C = s.C;
+    d.r = s.r;
+    d.n_split = down_batch_split(M, s.C, n_jobs);
+    d.partial = p;
+    p += (size_t)d.n_split * M * s.r;
+    r_max = std::max(r_max, s.r);
+    split_max = std::max(split_max, d.n_split);
+  }
+  constexpr int NW = 8;
+  const dim3 grid((M + 15) / 16, split_max, n_jobs), block(64 * NW);
+  const dim3 rgrid((unsigned)(((int64_t)M * (r_max / 4) + 255) / 256), n_jobs);
+  const int rt = (r_max + 15) / 16;
+#define BATCH(TT)                                                                                            \
+  do {                                                                                                       \
+    if (rt <= 1) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 1, NW>), grid, block, 0, st, a);              \
+    else if (rt <= 2) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 2, NW>), grid, block, 0, st, a);         \
+    else if (rt <= 4) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 4, NW>), grid, block, 0, st, a);         \
+    else hipLaunchKernelGGL((lora_down_batch_kernel<TT, 8, NW>), grid, block, 0, st, a);                      \
+    hipLaunchKernelGGL((lora_down_reduce_batch_kernel<TT>), rgrid, dim3(256), 0, st, a);                      \
+  } while (0)
+  if (act_dtype == FMSA_BF16) BATCH(bf16_t);
+  else BATCH(f16_t);
+#undef BATCH
+  FMSA_CHECK_LAUNCH();
   return FMSA_OK;
 }
 

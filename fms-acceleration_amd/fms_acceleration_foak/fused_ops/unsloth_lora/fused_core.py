@@ -232,7 +232,9 @@ def _lora_down_all(projs, Xds, stack):
     if stack is not None:
         U_cat = fmsa_hip.lora_down(Xds[0], stack.A_cat)
         return [U_cat[:, a:b] for a, b in stack.cols]
-    return [fmsa_hip.lora_down(Xd, p.A) if p.r else None for p, Xd in zip(projs, Xds)]
+    live = [(Xd, p.A, None) for p, Xd in zip(projs, Xds) if p.r]
+    outs = iter(fmsa_hip.lora_down_batch(live) if live else [])
+    return [next(outs) if p.r else None for p in projs]
 
 
 def _rope_in_epilogue(projs, rope, dtype, M):
@@ -300,14 +302,20 @@ def _adapter_grads(projs, dYs, Xds, Us, stack):
                                             for p, dY, U, T in zip(projs, dYs, Us, Ts)])
             dAs = fmsa_hip.lora_grad_batch(dA_jobs)
         else:
-            for p, dY, T in zip(projs, dYs, Ts):
-                fmsa_hip.lora_down(dY, p.Bt, out=T)
+            fmsa_hip.lora_down_batch([(dY, p.Bt, T) for p, dY, T in zip(projs, dYs, Ts)])
             outs = fmsa_hip.lora_grad_batch(dA_jobs + [(U, dY, p.s, True, p.B_param.dtype) for p, dY, U in zip(projs, dYs, Us)])
             dAs, dBs = outs[: len(dA_jobs)], outs[len(dA_jobs) :]
         if stacked_dA:
             dAs = [dAs[0][a:b] for a, b in stack.cols]
         return Ts, list(zip(dAs, dBs))
     Ts, grads = [], []
+    live = [(p, dY, Xd, U) for p, dY, Xd, U in zip(projs, dYs, Xds, Us) if p.r]
+    if (len(live) == len(projs) > 1 and dYs[0].shape[0] <= fmsa_hip.LORA_DOWN_BATCH_TOKENS and 2 * len(live) <= fmsa_hip.LORA_GRAD_MAX_JOBS):
+        # few tokens: every T in one launch, then every dA and dB in one
+        Ts = fmsa_hip.lora_down_batch([(dY, p.Bt, None) for p, dY, _, _ in live])
+        outs = fmsa_hip.lora_grad_batch([(T, Xd, p.s, False, p.A_param.dtype) for (p, _, Xd, _), T in zip(live, Ts)]
+                                        + [(U, dY, p.s, True, p.B_param.dtype) for p, dY, _, U in live])
+        return Ts, list(zip(outs[: len(live)], outs[len(live) :]))
     for p, dY, Xd, U in zip(projs, dYs, Xds, Us):
         T, dA, dB = p.t_and_grads(Xd, U, dY)
         Ts.append(T)

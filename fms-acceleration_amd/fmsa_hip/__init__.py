@@ -33,6 +33,8 @@ EXPORTED_SYMBOLS = (
     "fmsa_lora_down_ws",
     "fmsa_lora_down_split_workspace",
     "fmsa_lora_down_split",
+    "fmsa_lora_down_batch_workspace",
+    "fmsa_lora_down_batch",
     "fmsa_lora_grad_workspace",
     "fmsa_lora_grad",
     "fmsa_lora_grad_batch_workspace",
@@ -134,6 +136,20 @@ class LoraGradJob(Structure):
     ]
 
 
+class LoraDownJob(Structure):
+    """fmsa_lora_down_job: one product of a batch."""
+
+    _fields_ = [
+        ("X", c_void_p),
+        ("Wd", c_void_p),
+        ("out", c_void_p),
+        ("ldx", c_int64),
+        ("ldout", c_int64),
+        ("C", c_int32),
+        ("r", c_int32),
+    ]
+
+
 class LoraPackJob(Structure):
     """fmsa_lora_pack_job: one adapter of a batched pack."""
 
@@ -219,6 +235,9 @@ def lib() -> ctypes.CDLL:
     L.fmsa_lora_down_split_workspace.restype = c_size_t
     L.fmsa_lora_down_split_workspace.argtypes = [c_int, c_int, c_int]
     L.fmsa_lora_down_split.argtypes = L.fmsa_lora_down_ws.argtypes
+    L.fmsa_lora_down_batch_workspace.restype = c_size_t
+    L.fmsa_lora_down_batch_workspace.argtypes = [POINTER(LoraDownJob), c_int, c_int]
+    L.fmsa_lora_down_batch.argtypes = [POINTER(LoraDownJob), c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]
     L.fmsa_lora_grad_workspace.restype = c_size_t
     L.fmsa_lora_grad_workspace.argtypes = [c_int, c_int, c_int]
     L.fmsa_lora_grad.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_int, c_int, c_int,
@@ -384,6 +403,37 @@ def lora_down(x2d, wd, out=None):
            lib().fmsa_lora_down_split(_ptr(x2d), x2d.stride(0), _ptr(wd), M, C, r, act_enum(x2d.dtype), _ptr(out), out.stride(0),
                                       _ptr(ws), 0 if ws is None else ws.numel(), _stream(out)))
     return out
+
+
+LORA_DOWN_MAX_JOBS = 3
+LORA_DOWN_BATCH_TOKENS = 2047  # from 2048 tokens on a product fills the chip by itself (and takes another kernel)
+
+
+def lora_down_batch(jobs):
+    """jobs: (x2d, wd, out or None) triples over the same M tokens; the list of lora_down(x2d, wd, out).  With few tokens
+    one launch (and one of column sums) per LORA_DOWN_MAX_JOBS of them, single calls otherwise."""
+    M = jobs[0][0].shape[0]
+    if len(jobs) < 2 or M > LORA_DOWN_BATCH_TOKENS or any(
+            x.shape[1] % 8 or (o is not None and (o.data_ptr() % 8 or o.stride(0) % 4)) for x, _, o in jobs):
+        return [lora_down(x, wd, out=o) for x, wd, o in jobs]
+    outs = []
+    for i in range(0, len(jobs), LORA_DOWN_MAX_JOBS):
+        chunk = jobs[i : i + LORA_DOWN_MAX_JOBS]
+        arr = (LoraDownJob * len(chunk))()
+        for q, (x, wd, out) in enumerate(chunk):
+            r, C = wd.shape
+            assert x.shape == (M, C) and wd.is_contiguous() and wd.dtype == x.dtype == chunk[0][0].dtype and x.stride(1) == 1
+            if out is None:
+                out = x.new_empty((M, r))
+            assert out.shape == (M, r) and out.stride(1) == 1 and out.dtype == x.dtype
+            outs.append(out)
+            arr[q] = LoraDownJob(_ptr(x), _ptr(wd), _ptr(out), x.stride(0), out.stride(0), C, r)
+        x0 = chunk[0][0]
+        nbytes = lib().fmsa_lora_down_batch_workspace(arr, len(chunk), M)
+        ws = _workspace(max(nbytes, 1), x0.device)
+        _check("fmsa_lora_down_batch",
+               lib().fmsa_lora_down_batch(arr, len(chunk), M, act_enum(x0.dtype), _ptr(ws), ws.numel(), _stream(x0)))
+    return outs
 
 
 _ws_cache = {}

@@ -134,6 +134,22 @@ size_t fmsa_lora_down_split_workspace(int M, int C, int r);
 int fmsa_lora_down_split(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype,
                       void* out, int64_t ldout, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Up to FMSA_LORA_DOWN_MAX_JOBS of these products over the same M tokens in one launch and one launch of column sums, for
+ * few tokens, where a launch is mostly ramp and latency.  The workspace is always needed. */
+#define FMSA_LORA_DOWN_MAX_JOBS 3
+typedef struct fmsa_lora_down_job {
+  const void* X;   /* [M, C] act_dtype, row stride ldx % 8 == 0 */
+  const void* Wd;  /* [r, C] act_dtype */
+  void* out;       /* [M, r] act_dtype, 8-byte aligned, row stride ldout % 4 == 0 */
+  int64_t ldx;
+  int64_t ldout;
+  int32_t C;       /* % 8 == 0 */
+  int32_t r;       /* % 8 == 0, <= 128 */
+} fmsa_lora_down_job;
+size_t fmsa_lora_down_batch_workspace(const fmsa_lora_down_job* jobs /*host*/, int n_jobs, int M);
+int fmsa_lora_down_batch(const fmsa_lora_down_job* jobs /*host*/, int n_jobs, int M, int act_dtype, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* out = scale * L[M, r]^T * R[M, C]   (a reduction over the M tokens; L has row stride ldl >= r), written as
  *   [r, C] when transpose_out == 0   (dA = s * (dY B)^T Xd,  UL/gptq/fast_lora.py:822,824,842)
  *   [C, r] when transpose_out == 1   (dB = s * dY^T (Xd A^T), :823,825,843)

@@ -27,3 +27,25 @@ def test_lora_down_few_tokens(M, C, r, dtype):
     assert (out.float() - ref).norm() <= 1.02 * (whole.float() - ref).norm() + 1e-6 * ref.norm()
     assert torch.all(wide[:, :8] == 3.0) and torch.all(wide[:, 8 + r :] == 3.0)
     assert torch.equal(fmsa_hip.lora_down(x, wd), out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,shapes", [(1, [(1024, 8), (14336, 16)]), (33, [(4096, 64), (1024, 64), (520, 64)]),
+                                      (2047, [(96, 8), (4096, 128), (1056, 24)]), (300, [(2048, 16)] * 4)])
+def test_lora_down_batch(M, shapes, dtype):
+    """Products of different widths and ranks in one launch, the last one into a column slice."""
+    import fmsa_hip
+
+    jobs, refs = [], []
+    for i, (C, r) in enumerate(shapes):
+        x = randn((M, C + 8), 10 + i, dtype).cuda()[:, :C]
+        wd = randn((r, C), 20 + i, dtype, 0.05).cuda()
+        wide = torch.full((M, r + 16), 3.0, dtype=dtype, device="cuda")
+        jobs.append((x, wd, wide[:, 8 : 8 + r] if i + 1 == len(shapes) else None))
+        refs.append(x.float() @ wd.float().t())
+    outs = fmsa_hip.lora_down_batch(jobs)
+    for (x, wd, _), out, ref in zip(jobs, outs, refs):
+        single = fmsa_hip.lora_down(x, wd)
+        assert (out.float() - ref).norm() <= 1.02 * (single.float() - ref).norm() + 1e-6 * ref.norm()
+    assert torch.all(wide[:, :8] == 3.0) and torch.all(wide[:, 8 + wd.shape[0] :] == 3.0)
+    assert all(torch.equal(a, b) for a, b in zip(outs, fmsa_hip.lora_down_batch(jobs)))
