@@ -79,7 +79,7 @@ def FastForCausalLMLoss(logits, labels, vocab_size: int, num_items_in_batch: int
         # the fp32 copy, the shifted copy and their gradients' copies cost five times the two kernels
         seq_out = logits.shape[1] - (shift_labels is None)
         target = labels[:, 1:] if shift_labels is None else shift_labels
-        target = target.to(device=logits.device, dtype=torch.int64).reshape(-1)
+        target = target.to(device=logits.device, dtype=torch.int64).reshape(-1).contiguous()  # a row of a strided view stays strided
         loss = Fast_CausalLMLossRows.apply(logits, target, seq_out)
         n_items = num_items_in_batch if num_items_in_batch is not None else torch.count_nonzero(target != -100)
         return loss.sum() / n_items

@@ -51,3 +51,16 @@ def test_all_labels_ignored():
     loss = FastForCausalLMLoss(x, torch.full((2, 5), -100, device="cuda"), 1000, num_items_in_batch=7)
     loss.backward()
     assert loss.item() == 0.0 and bool((x.grad == 0).all())
+
+
+@pytest.mark.parametrize("shifted", [False, True])
+def test_strided_labels(shifted):
+    """Labels of one sequence that are a strided view: flattening them does not copy."""
+    from fms_acceleration_foak.kernels.unsloth import FastForCausalLMLoss
+
+    x = randn((1, 6, 100), 2, torch.bfloat16).cuda()
+    labels = torch.arange(12, device="cuda").view(1, 12)[:, ::2]
+    packed = labels.contiguous()
+    kw = ({"shift_labels": labels}, {"shift_labels": packed}) if shifted else ({}, {})
+    la, lb = FastForCausalLMLoss(x, labels, 100, **kw[0]), FastForCausalLMLoss(x, packed, 100, **kw[1])
+    assert not labels.is_contiguous() and torch.equal(la, lb)
