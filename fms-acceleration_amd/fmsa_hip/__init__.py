@@ -430,24 +430,17 @@ def lora_down_batch(jobs):
             arr[q] = LoraDownJob(_ptr(x), _ptr(wd), _ptr(out), x.stride(0), out.stride(0), C, r)
         x0 = chunk[0][0]
         nbytes = lib().fmsa_lora_down_batch_workspace(arr, len(chunk), M)
-        ws = _workspace(max(nbytes, 1), x0.device)
+        ws = _workspace(nbytes, x0.device)
         _check("fmsa_lora_down_batch",
                lib().fmsa_lora_down_batch(arr, len(chunk), M, act_enum(x0.dtype), _ptr(ws), ws.numel(), _stream(x0)))
     return outs
 
 
-_ws_cache = {}
-
-
 def _workspace(nbytes: int, device) -> torch.Tensor:
-    """Partial-sum buffer of the adapter-gradient launches, one per (device, stream): launches on one stream
-    are ordered and may share it, launches on two streams of one device must not."""
-    key = (device.index, _raw_stream(device.index))
-    ws = _ws_cache.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _ws_cache[key] = ws
-    return ws
+    """Partial-sum buffer of one call.  A call is two launches, one writing the sums and one reading them, and another
+    thread's call on the same stream may come between them; a captured graph keeps its address.  So no two calls share
+    one: torch's allocator hands it out in stream order, or from the graph's own pool under capture."""
+    return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
 
 
 def lora_grad(L, R, scale: float, transpose_out: bool, out_dtype=torch.float32):

@@ -49,3 +49,26 @@ def test_lora_down_batch(M, shapes, dtype):
         assert (out.float() - ref).norm() <= 1.02 * (single.float() - ref).norm() + 1e-6 * ref.norm()
     assert torch.all(wide[:, :8] == 3.0) and torch.all(wide[:, 8 + wd.shape[0] :] == 3.0)
     assert all(torch.equal(a, b) for a, b in zip(outs, fmsa_hip.lora_down_batch(jobs)))
+
+
+def test_calls_do_not_share_partial_sums():
+    """Two calls on one stream may interleave their launches (threads), and a captured one is replayed after the next has
+    asked for more: the buffers of partial sums are the calls' own."""
+    import fmsa_hip
+
+    a, b = fmsa_hip._workspace(1 << 20, torch.device("cuda:0")), fmsa_hip._workspace(1 << 20, torch.device("cuda:0"))
+    assert a.data_ptr() != b.data_ptr()
+    x, wd = randn((3, 4096), 1, torch.bfloat16).cuda(), randn((16, 4096), 2, torch.bfloat16, 0.05).cuda()
+    big = randn((1500, 8192), 3, torch.bfloat16).cuda()
+    wb = randn((64, 8192), 4, torch.bfloat16, 0.05).cuda()
+    ref, ref_b = fmsa_hip.lora_down(x, wd), fmsa_hip.lora_down(big, wb)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = fmsa_hip.lora_down(x, wd)
+    for _ in range(3):
+        assert torch.equal(fmsa_hip.lora_down(big, wb), ref_b)  # eager work of its own between the replays
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
