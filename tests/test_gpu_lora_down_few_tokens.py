@@ -31,7 +31,9 @@ def test_lora_down_few_tokens(M, C, r, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,shapes", [(1, [(1024, 8), (14336, 16)]), (33, [(4096, 64), (1024, 64), (520, 64)]),
-                                      (2047, [(96, 8), (4096, 128), (1056, 24)]), (300, [(2048, 16)] * 4)])
+                                      (2047, [(96, 8), (4096, 128), (1056, 24)]), (300, [(2048, 16)] * 4),
+                                      (1023, [(4096, 64), (1056, 24)]), (1024, [(4096, 64), (1056, 8)]), (1100, [(14336, 64), (520, 32)]),
+                                      (1041, [(1032, 24), (2048, 32)])])
 def test_lora_down_batch(M, shapes, dtype):
     """Products of different widths and ranks in one launch, the last one into a column slice."""
     import fmsa_hip
