@@ -414,12 +414,24 @@ constexpr float kLn2 = 0.69314718055994531f;
 
 // (m, s) <- (m, s) (+) (x): running maximum and sum of exp(. - m)
 // While everything seen so far is -inf (a masked vocabulary span) the pair stays (-inf, 0): the update
-// would form (-inf) - (-inf) = NaN, which no later finite logit could remove from s.
+// would form (-inf) - (-inf) = NaN, which no later finite logit could remove from s.  A NaN among the logits has to stay,
+// though, and the maximum passes it over: with nothing finite beside it, it is put into s here.
 FMSA_DEVI void online_add(float& m, float& s, float x) {
   const float mn = fmaxf(m, x);
   if (mn != -INFINITY) s = s * __builtin_amdgcn_exp2f((m - mn) * kLog2e) + __builtin_amdgcn_exp2f((x - mn) * kLog2e);
+  else if (x != x) s = x;
   m = mn;
 }
+
+// the same for eight logits none of which is above -inf
+FMSA_DEVI void keep_nan(float& s, const float (&x)[8]) {
+  const float t = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));  // -inf, or NaN if one of them is
+  if (t != t) s = t;
+}
+
+// s against the maximum mn of a merge: a thread that saw nothing finite holds (-inf, 0), whose term must not turn into
+// NaN, or (-inf, NaN), whose term must
+FMSA_DEVI float merge_term(float m, float s, float mn) { return s == 0.f ? 0.f : s * __builtin_amdgcn_exp2f((m - mn) * kLog2e); }
 
 template <int D, bool VEC>
 __global__ __launch_bounds__(256) void ce_fwd_kernel(const void* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels,
@@ -436,7 +448,10 @@ __global__ __launch_bounds__(256) void ce_fwd_kernel(const void* __restrict__ lo
 #pragma unroll
       for (int k = 1; k < 8; ++k) mx = fmaxf(mx, x[k]);
       const float mn = fmaxf(m, mx);
-      if (mn == -INFINITY) continue;  // nothing finite yet: (m, s) stays (-inf, 0), see online_add
+      if (mn == -INFINITY) {  // nothing finite yet: see online_add
+        keep_nan(s, x);
+        continue;
+      }
       float acc = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc += __builtin_amdgcn_exp2f((x[k] - mn) * kLog2e);
@@ -453,11 +468,8 @@ __global__ __launch_bounds__(256) void ce_fwd_kernel(const void* __restrict__ lo
     if (tid < o) {
       const float m2 = red_m[tid + o], s2 = red_s[tid + o];
       const float mn = fmaxf(red_m[tid], m2);
-      // a thread that saw no element holds (-inf, 0): its term must not turn into NaN
-      const float a = red_m[tid] == -INFINITY ? 0.f : red_s[tid] * __builtin_amdgcn_exp2f((red_m[tid] - mn) * kLog2e);
-      const float b = m2 == -INFINITY ? 0.f : s2 * __builtin_amdgcn_exp2f((m2 - mn) * kLog2e);
+      red_s[tid] = merge_term(red_m[tid], red_s[tid], mn) + merge_term(m2, s2, mn);
       red_m[tid] = mn;
-      red_s[tid] = a + b;
     }
     __syncthreads();
   }
@@ -549,7 +561,11 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __rest
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int k = 0; k < 8; ++k) mn = fmaxf(mn, v[u][k]);  // (a chunk past the end repeats the last one)
-    if (mn == -INFINITY) continue;  // nothing finite yet: (m, s) stays (-inf, 0), see online_add
+    if (mn == -INFINITY) {  // nothing finite yet: see online_add
+#pragma unroll
+      for (int u = 0; u < 4; ++u) keep_nan(s, v[u]);
+      continue;
+    }
     s *= __builtin_amdgcn_exp2f((m - mn) * kLog2e);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -567,10 +583,8 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __rest
     if (tid < o) {
       const float m2 = red_m[tid + o], s2 = red_s[tid + o];
       const float mn = fmaxf(red_m[tid], m2);
-      const float a = red_m[tid] == -INFINITY ? 0.f : red_s[tid] * __builtin_amdgcn_exp2f((red_m[tid] - mn) * kLog2e);
-      const float b = m2 == -INFINITY ? 0.f : s2 * __builtin_amdgcn_exp2f((m2 - mn) * kLog2e);
+      red_s[tid] = merge_term(red_m[tid], red_s[tid], mn) + merge_term(m2, s2, mn);
       red_m[tid] = mn;
-      red_s[tid] = a + b;
     }
     __syncthreads();
   }
@@ -679,7 +693,10 @@ __global__ __launch_bounds__(256) void ce_fused_kernel(void* __restrict__ logits
       const float mn = fmaxf(m, mx);
 #pragma unroll
       for (int k = 0; k < 8; ++k) sx += x[k];
-      if (mn == -INFINITY) continue;  // nothing finite yet: (m, s) stays (-inf, 0), see online_add
+      if (mn == -INFINITY) {  // nothing finite yet: see online_add
+        keep_nan(s, x);
+        continue;
+      }
       float acc = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc += __builtin_amdgcn_exp2f((x[k] - mn) * kLog2e);
@@ -701,10 +718,8 @@ __global__ __launch_bounds__(256) void ce_fused_kernel(void* __restrict__ logits
     if (tid < o) {
       const float m2 = red_m[tid + o], s2 = red_s[tid + o];
       const float mn = fmaxf(red_m[tid], m2);
-      const float a = red_m[tid] == -INFINITY ? 0.f : red_s[tid] * __builtin_amdgcn_exp2f((red_m[tid] - mn) * kLog2e);
-      const float b = m2 == -INFINITY ? 0.f : s2 * __builtin_amdgcn_exp2f((m2 - mn) * kLog2e);
+      red_s[tid] = merge_term(red_m[tid], red_s[tid], mn) + merge_term(m2, s2, mn);
       red_m[tid] = mn;
-      red_s[tid] = a + b;
       red_x[tid] += red_x[tid + o];
     }
     __syncthreads();

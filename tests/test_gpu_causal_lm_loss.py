@@ -64,3 +64,29 @@ def test_strided_labels(shifted):
     kw = ({"shift_labels": labels}, {"shift_labels": packed}) if shifted else ({}, {})
     la, lb = FastForCausalLMLoss(x, labels, 100, **kw[0]), FastForCausalLMLoss(x, packed, 100, **kw[1])
     assert not labels.is_contiguous() and torch.equal(la, lb)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [3, 17, 1024, 8195, 32003])
+def test_a_nan_logit_stays(V, dtype):
+    """One NaN anywhere in a row, also where a thread sees nothing finite before it: that row's loss and gradient are NaN
+    and no other row's.  16-bit logits are read in place, fp32 ones by the general kernels (rows of whole chunks and not)."""
+    import fmsa_hip
+
+    columns = sorted({0, 1, V // 2, max(0, V - 9), V - 2, V - 1})
+    x = randn((1, len(columns) + 1, V), V, dtype, scale=2.0).cuda()
+    for row, c in enumerate(columns):
+        x[0, row, c] = float("nan")
+    labels = torch.full((len(columns) + 1,), V // 3, dtype=torch.int64, device="cuda")
+    dloss = torch.ones(len(columns) + 1, device="cuda")
+    if dtype == torch.float32:
+        losses, lse = fmsa_hip.cross_entropy_fwd(x[0], labels)
+        grad = fmsa_hip.cross_entropy_bwd_(x[0].clone(), dloss, lse, labels)
+    else:
+        losses, lse = fmsa_hip.cross_entropy_rows_fwd(x, labels, x.shape[1])
+        grad = fmsa_hip.cross_entropy_rows_bwd(x, dloss, lse, labels, x.shape[1])[0]
+    fused, fused_grad = fmsa_hip.cross_entropy_fused_(x[0].clone(), labels)
+    for per_row in (losses, fused):
+        assert bool(per_row[:-1].isnan().all()) and bool(per_row[-1].isfinite())
+    for g in (grad, fused_grad):
+        assert bool(g[:-1].isnan().all()) and bool(g[-1].isfinite().all())
