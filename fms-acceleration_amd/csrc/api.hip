@@ -46,8 +46,8 @@ int launch_ce_fwd(const void* logits, int64_t ld, const int64_t* labels, int M, 
                   hipStream_t st);
 int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse, const int64_t* labels, int M,
                   int V, int dtype, int vec, hipStream_t st);
-int launch_ce_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype,
-                       float* losses, float* lse, hipStream_t st);
+int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
+                       int dtype, float* losses, float* lse, hipStream_t st);
 int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse,
                        const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st);
 int launch_ce_fused(void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, int vec, int64_t ignore_index,
@@ -630,7 +630,15 @@ int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* l
                                 int dtype, float* losses, float* logsumexp, void* stream) {
   if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
   if (!losses || !logsumexp) return FMSA_ERR_NULL;
-  return launch_ce_rows_fwd(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
+  return launch_ce_rows_fwd(logits, nullptr, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
+}
+
+int fmsa_cross_entropy_rows_fwd_keep(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in,
+                                     int seq_out, int V, int dtype, float* losses, float* logsumexp, void* stream) {
+  if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
+  if (!kept || !losses || !logsumexp) return FMSA_ERR_NULL;
+  if ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(kept)) & 15u) return FMSA_ERR_ALIGN;
+  return launch_ce_rows_fwd(logits, kept, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
 }
 
 int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride,

@@ -9,13 +9,15 @@ namespace {
 // eight consecutive elements of a row as fp32, for the three storage types (tag = fmsa_dtype)
 template <int D> struct Vec8;
 template <> struct Vec8<FMSA_BF16> {
-  static FMSA_DEVI void load(const void* p, int64_t i, float (&v)[8]) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p) + i);
+  static FMSA_DEVI void unpack(u32x4 w, float (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       v[2 * k] = unpack_lo<bf16_t>(w[k]);
       v[2 * k + 1] = unpack_hi<bf16_t>(w[k]);
     }
+  }
+  static FMSA_DEVI void load(const void* p, int64_t i, float (&v)[8]) {
+    unpack(*reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p) + i), v);
   }
   static FMSA_DEVI void store(void* p, int64_t i, const float (&v)[8]) {
     u32x4 w;
@@ -26,13 +28,15 @@ template <> struct Vec8<FMSA_BF16> {
   static FMSA_DEVI float round(float x) { return unpack1<bf16_t>(pack1<bf16_t>(x)); }
 };
 template <> struct Vec8<FMSA_F16> {
-  static FMSA_DEVI void load(const void* p, int64_t i, float (&v)[8]) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p) + i);
+  static FMSA_DEVI void unpack(u32x4 w, float (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       v[2 * k] = unpack_lo<f16_t>(w[k]);
       v[2 * k + 1] = unpack_hi<f16_t>(w[k]);
     }
+  }
+  static FMSA_DEVI void load(const void* p, int64_t i, float (&v)[8]) {
+    unpack(*reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p) + i), v);
   }
   static FMSA_DEVI void store(void* p, int64_t i, const float (&v)[8]) {
     u32x4 w;
@@ -519,7 +523,9 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(void* __restrict__ logits, 
 // Backward: one read, and one write of a gradient of its own, whole: the rows past seq_out and the rows without a label are
 // written as zeros and not read.  Both are bound by HBM.  The widening copy to fp32, the copy that drops every sequence's
 // last row, the pass over the fp32 gradient and its narrowing and padding copies took 1040 us at 1024 x 128256 bf16 (4.2 GB
-// of traffic); the two kernels move 0.55 - 0.79 GB.
+// of traffic); the two kernels move 0.55 - 0.79 GB, and 0.18 - 0.26 GB more where the forward keeps the live rows for the
+// backward (KEEP), so that the caller may overwrite the logits in between (loss and gradient of 1024 x 128256, three rows in
+// ten without a label: 159 us a pass where the backward reads the caller's logits, 204 us with the rows kept).
 // Rows are walked in 16-byte chunks from the first aligned element on (V need not be a multiple of 8, so every row of a
 // contiguous matrix may begin elsewhere), with four chunks per thread in flight; the ends are element accesses.
 struct RowSpan {
@@ -535,10 +541,11 @@ FMSA_DEVI RowSpan row_span(const uint16_t* x, int V, bool vec) {
 }
 FMSA_DEVI int64_t logits_row(int row, int seq_in, int seq_out) { return (int64_t)(row / seq_out) * seq_in + row % seq_out; }
 
-template <int D>
-__global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels,
-                                                          int seq_in, int seq_out, int V, int vec, float* __restrict__ losses,
-                                                          float* __restrict__ lse_out) {
+// KEEP: the live rows also go to `kept`, laid out and aligned (modulo 16) as the logits
+template <int D, bool KEEP>
+__global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __restrict__ logits, uint16_t* __restrict__ kept, int64_t ld,
+                                                          const int64_t* __restrict__ labels, int seq_in, int seq_out, int V,
+                                                          float* __restrict__ losses, float* __restrict__ lse_out) {
   __shared__ float red_m[256], red_s[256];
   const int row = blockIdx.x, tid = threadIdx.x;
   const int64_t label = labels[row];
@@ -546,16 +553,30 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __rest
     if (tid == 0) losses[row] = lse_out[row] = 0.f;
     return;
   }
-  const uint16_t* x = logits + logits_row(row, seq_in, seq_out) * ld;
-  const RowSpan sp = row_span(x, V, vec != 0);
+  const int64_t row0 = logits_row(row, seq_in, seq_out) * ld;
+  const uint16_t* x = logits + row0;
+  const RowSpan sp = row_span(x, V, true);
   float m = -INFINITY, s = 0.f;
-  for (int c = tid; c < sp.head; c += 256) online_add(m, s, load1<D>(x, c));
-  for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) online_add(m, s, load1<D>(x, c));
-  const uint16_t* xv = x + sp.head;
+  auto element = [&](int c) {
+    online_add(m, s, load1<D>(x, c));
+    if constexpr (KEEP) kept[row0 + c] = x[c];
+  };
+  for (int c = tid; c < sp.head; c += 256) element(c);
+  for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) element(c);
+  const u32x4* xv = reinterpret_cast<const u32x4*>(x + sp.head);
   for (int i = tid; i < sp.n_vec; i += 1024) {
+    u32x4 w[4];
     float v[4][8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) Vec8<D>::load(xv, 8 * (int64_t)min(i + 256 * u, sp.n_vec - 1), v[u]);
+    for (int u = 0; u < 4; ++u) w[u] = xv[min(i + 256 * u, sp.n_vec - 1)];
+    if constexpr (KEEP) {
+      u32x4* kv = reinterpret_cast<u32x4*>(kept + row0 + sp.head);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i + 256 * u < sp.n_vec) kv[i + 256 * u] = w[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) Vec8<D>::unpack(w[u], v[u]);
     float mn = m;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -779,14 +800,20 @@ int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_st
   return FMSA_OK;
 }
 
-int launch_ce_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype,
-                       float* losses, float* lse, hipStream_t st) {
+int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
+                       int dtype, float* losses, float* lse, hipStream_t st) {
   const dim3 grid(n_seq * seq_out), block(256);
   const uint16_t* x = (const uint16_t*)logits;
-  if (dtype == FMSA_BF16)
-    hipLaunchKernelGGL((ce_rows_fwd_kernel<FMSA_BF16>), grid, block, 0, st, x, ld, labels, seq_in, seq_out, V, 1, losses, lse);
-  else
-    hipLaunchKernelGGL((ce_rows_fwd_kernel<FMSA_F16>), grid, block, 0, st, x, ld, labels, seq_in, seq_out, V, 1, losses, lse);
+  uint16_t* k = (uint16_t*)kept;
+#define ROWS_FWD(D, KEEP) hipLaunchKernelGGL((ce_rows_fwd_kernel<D, KEEP>), grid, block, 0, st, x, k, ld, labels, seq_in, seq_out, V, losses, lse)
+  if (dtype == FMSA_BF16) {
+    if (k) ROWS_FWD(FMSA_BF16, true);
+    else ROWS_FWD(FMSA_BF16, false);
+  } else {
+    if (k) ROWS_FWD(FMSA_F16, true);
+    else ROWS_FWD(FMSA_F16, false);
+  }
+#undef ROWS_FWD
   FMSA_CHECK_LAUNCH();
   return FMSA_OK;
 }

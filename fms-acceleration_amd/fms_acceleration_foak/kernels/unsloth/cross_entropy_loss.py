@@ -29,19 +29,23 @@ class Fast_CrossEntropyLoss(torch.autograd.Function):
 
 class Fast_CausalLMLossRows(torch.autograd.Function):
     """Losses of rows 0 .. seq_out - 1 of every sequence, read from the 16-bit logits where they are; the gradient is a
-    tensor of its own, so the logits stay as the caller sees them."""
+    tensor of its own, so the logits stay as the caller sees them.  keep (a backward may follow): the forward leaves the
+    rows it read in a copy for the backward, so the caller may overwrite the logits before it, as with the fp32 copy of
+    the general way."""
 
     @staticmethod
-    def forward(ctx, logits, labels, seq_out):
-        losses, logsumexp = fmsa_hip.cross_entropy_rows_fwd(logits, labels, seq_out)
-        ctx.save_for_backward(logits, logsumexp, labels)
+    def forward(ctx, logits, labels, seq_out, keep):
+        if not keep:
+            return fmsa_hip.cross_entropy_rows_fwd(logits, labels, seq_out)[0]
+        losses, logsumexp, kept = fmsa_hip.cross_entropy_rows_fwd_keep(logits, labels, seq_out)
+        ctx.save_for_backward(kept, logsumexp, labels)
         ctx.seq_out = seq_out
         return losses
 
     @staticmethod
     def backward(ctx, dlosses):
-        logits, logsumexp, labels = ctx.saved_tensors
-        return fmsa_hip.cross_entropy_rows_bwd(logits, dlosses.float(), logsumexp, labels, ctx.seq_out), None, None
+        kept, logsumexp, labels = ctx.saved_tensors
+        return fmsa_hip.cross_entropy_rows_bwd(kept, dlosses.float(), logsumexp, labels, ctx.seq_out), None, None, None
 
 
 def _rows_in_place(logits, labels, vocab_size, shifted):
@@ -80,7 +84,7 @@ def FastForCausalLMLoss(logits, labels, vocab_size: int, num_items_in_batch: int
         seq_out = logits.shape[1] - (shift_labels is None)
         target = labels[:, 1:] if shift_labels is None else shift_labels
         target = target.to(device=logits.device, dtype=torch.int64).reshape(-1).contiguous()  # a row of a strided view stays strided
-        loss = Fast_CausalLMLossRows.apply(logits, target, seq_out)
+        loss = Fast_CausalLMLossRows.apply(logits, target, seq_out, torch.is_grad_enabled() and logits.requires_grad)
         n_items = num_items_in_batch if num_items_in_batch is not None else torch.count_nonzero(target != -100)
         return loss.sum() / n_items
     logits = logits.float()

@@ -63,6 +63,7 @@ EXPORTED_SYMBOLS = (
     "fmsa_cross_entropy_fwd",
     "fmsa_cross_entropy_bwd",
     "fmsa_cross_entropy_rows_fwd",
+    "fmsa_cross_entropy_rows_fwd_keep",
     "fmsa_cross_entropy_rows_bwd",
     "fmsa_cross_entropy_fused",
 )
@@ -281,6 +282,8 @@ def lib() -> ctypes.CDLL:
     L.fmsa_cross_entropy_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
     L.fmsa_cross_entropy_bwd.argtypes = [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
     L.fmsa_cross_entropy_rows_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
+    L.fmsa_cross_entropy_rows_fwd_keep.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                                                   c_void_p, c_void_p]
     L.fmsa_cross_entropy_rows_bwd.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                               c_int, c_void_p]
     L.fmsa_cross_entropy_fused.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int64, c_void_p, c_float, c_void_p, c_void_p]
@@ -817,6 +820,22 @@ def cross_entropy_rows_fwd(logits3d, labels, seq_out: int):
            lib().fmsa_cross_entropy_rows_fwd(_ptr(logits3d), V, _ptr(labels), n_seq, seq_in, seq_out, V, act_enum(logits3d.dtype),
                                              _ptr(losses), _ptr(lse), _stream(logits3d)))
     return losses, lse
+
+
+def cross_entropy_rows_fwd_keep(logits3d, labels, seq_out: int):
+    """(losses, logsumexp, kept): cross_entropy_rows_fwd that leaves the rows with a label in a tensor of its own too, for a
+    backward that must not depend on what the caller does to the logits in the meantime."""
+    n_seq, seq_in, V = logits3d.shape
+    rows = n_seq * seq_out
+    assert logits3d.is_contiguous() and labels.dtype == torch.int64 and labels.is_contiguous() and labels.numel() == rows
+    losses = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
+    lse = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
+    offset = logits3d.data_ptr() % 16 // logits3d.element_size()  # a row begins where it does in the logits, modulo 16 bytes
+    kept = logits3d.new_empty(offset + logits3d.numel())[offset:].view(logits3d.shape)
+    _check("fmsa_cross_entropy_rows_fwd_keep",
+           lib().fmsa_cross_entropy_rows_fwd_keep(_ptr(logits3d), _ptr(kept), V, _ptr(labels), n_seq, seq_in, seq_out, V,
+                                                  act_enum(logits3d.dtype), _ptr(losses), _ptr(lse), _stream(logits3d)))
+    return losses, lse, kept
 
 
 def cross_entropy_rows_bwd(logits3d, dlosses, lse, labels, seq_out: int):

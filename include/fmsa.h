@@ -436,6 +436,12 @@ int fmsa_cross_entropy_bwd(void* logits, int64_t ld, const float* dloss, int64_t
  * a label are zeros), and leaves the logits alone. */
 int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out,
                                 int V, int dtype, float* losses, float* logsumexp, void* stream);
+/* The same forward, leaving the rows that have a label in `kept` as well (the logits' layout and row stride, and their
+ * alignment modulo 16 bytes; the other rows are not written): the backward may then read `kept` while the caller
+ * overwrites the logits. */
+int fmsa_cross_entropy_rows_fwd_keep(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq,
+                                     int seq_in, int seq_out, int V, int dtype, float* losses, float* logsumexp,
+                                     void* stream);
 int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride,
                                 const float* logsumexp, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
                                 int dtype, void* stream);

@@ -296,3 +296,12 @@ def test_cross_entropy_validation():
     assert u(0x1000, 32, 0x4000, 8, 64, 2, -100, None, 0.0, 0x2000, None) == -2   # ld < V
     assert u(0x1000, 64, 0x4000, 8, 64, 2, -100, None, 1.5, 0x2000, None) == -2   # smoothing outside [0, 1]
     assert u(0x1000, 64, 0x4000, 8, 64, 7, -100, None, 0.0, 0x2000, None) == -4
+
+
+def test_cross_entropy_rows_keep_validation():
+    f = fmsa_hip.lib().fmsa_cross_entropy_rows_fwd_keep
+    args = lambda logits=0x1002, kept=0x2002, ld=9, n_seq=2, seq_in=5, seq_out=4, V=9: (  # noqa: E731
+        logits, kept, ld, 0x3000, n_seq, seq_in, seq_out, V, 1, 0x4000, 0x5000, None)
+    assert f(*args(kept=None)) == -1 and f(*args(logits=None)) == -1
+    assert f(*args(seq_out=6)) == -2 and f(*args(ld=8)) == -2
+    assert f(*args(kept=0x2000)) == -3 and f(*args(logits=0x1004)) == -3  # not congruent modulo 16 bytes

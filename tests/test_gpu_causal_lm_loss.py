@@ -90,3 +90,30 @@ def test_a_nan_logit_stays(V, dtype):
         assert bool(per_row[:-1].isnan().all()) and bool(per_row[-1].isfinite())
     for g in (grad, fused_grad):
         assert bool(g[:-1].isnan().all()) and bool(g[-1].isfinite().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,s,V,offset", [(1, 3, 3, 1), (2, 9, 8, 0), (3, 5, 17, 1), (2, 7, 8195, 3), (2, 4, 40960, 0)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_logits_overwritten_before_the_backward(b, s, V, offset, shifted, dtype):
+    """The gradient belongs to the logits the loss was taken of, whatever the caller writes over them afterwards."""
+    from fms_acceleration_foak.kernels.unsloth import FastForCausalLMLoss
+
+    store = torch.zeros(offset + b * s * V, dtype=dtype, device="cuda")
+    store[offset:] = randn((b * s * V,), 7, dtype, scale=3.0).cuda()
+    labels = torch.randint(0, V, (b, s), generator=torch.Generator().manual_seed(V)).cuda()
+    labels[b - 1, s - 1] = -100
+    kw = {"shift_labels": labels} if shifted else {}
+    grads = []
+    for overwrite in (False, True):
+        leaf = store.clone().requires_grad_(True)
+        x = (leaf * 1.0)[offset:].view(b, s, V)  # what a model hands over: not a leaf
+        loss = FastForCausalLMLoss(x, labels, V, **kw)
+        if overwrite:
+            with torch.no_grad():
+                x.mul_(0.5).add_(1.0)
+        loss.backward()
+        grads.append(leaf.grad)
+    assert torch.equal(*grads) and bool((grads[0] != 0).any())
+    with torch.no_grad():  # nothing is kept where no backward can follow
+        assert torch.equal(FastForCausalLMLoss(store[offset:].view(b, s, V), labels, V, **kw), loss)
