@@ -24,12 +24,12 @@ def member(module, kind, name, default=_RAISE):
     """getattr(module, name) for what a module keeps in its `kind` dictionary (_modules, _buffers, _parameters), asked for
     there first: nn.Module.__getattr__ runs after a failed lookup and searches all three, which a layer pass of seven
     adapted projections pays for a hundred times.  Anything kept elsewhere (a property, a plain attribute) is found as
-    getattr finds it."""
-    found = module.__dict__.get(kind)
-    if found is not None:
-        found = found.get(name)
-        if found is not None:
-            return found
+    getattr finds it, and a plain attribute goes first, as there.  The dictionary is asked by subscript, as
+    nn.Module.__getattr__ does: one that gathers a partitioned parameter on access does it there, and not in get()."""
+    own = module.__dict__
+    found = own.get(kind)
+    if found is not None and name in found and name not in own:
+        return found[name]
     return getattr(module, name) if default is _RAISE else getattr(module, name, default)
 
 
