@@ -814,7 +814,8 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
   // workgroup and the rows are long enough to amortise its pipeline fill (measured at 8192 tokens: 59 -> 48 us at
   // C = 14336, r = 16; 32 -> 28 us at C = 4096, r = 48; 20 -> 21 us at C = 4096, r = 16; at 4096 tokens, C = 28672,
   // r = 64: 205 us with the fragment loads above)
-  const bool staged = M >= 16 * 256 && rt <= 8 && (C >= 8192 || (rt >= 2 && C >= 2048));
+  // (the staged kernel walks all columns: it leaves no partial sums)
+  const bool staged = n_split == 1 && M >= 16 * 256 && rt <= 8 && (C >= 8192 || (rt >= 2 && C >= 2048));
   if (staged) {
     const int smtl = M >= 32 * 256 ? 2 : 1;
     dim3 sgrid((M + 16 * smtl - 1) / (16 * smtl)), sblock(512);
