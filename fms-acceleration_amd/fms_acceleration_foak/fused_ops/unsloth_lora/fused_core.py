@@ -165,19 +165,17 @@ class _Proj:
 
 
 FUSE_T_MIN_BYTES = 96 << 20
-FUSE_T_FEW_TOKENS = 512
 
 
 def _fuse_t(projs, dYs):
     """Whether T_p = dY_p B_p should come out of the dB launch (one pass over dY_p instead of two).  The
     dependent dA launch then cannot share the dB launch any more, which costs about 15 us of launch ramp
     and tail: measured to pay from about 100 MB of dY (q, k, v together; gate and up), not for one
-    4096-wide projection.  With few tokens the launches themselves are the cost: one pair more for the dA instead of a
-    pair (product, column sums) per projection."""
+    4096-wide projection.  Nor for few tokens: the batched products take two launches as the dependent dA does, and the
+    GPU's time for T, dA and dB (stacked; q k v and gate, up of hidden 2048 to 8192, ranks 8 to 64) is 1.0 to 1.2 times as
+    long this way at 1 to 64 tokens and up to 1.6 times as long at 512."""
     if any(p.r > fmsa_hip.LORA_GRAD_T_MAX_RANK for p in projs):
         return False
-    if len(projs) > 1 and dYs[0].shape[0] <= FUSE_T_FEW_TOKENS:
-        return True
     return sum(dY.numel() * dY.element_size() for dY in dYs) >= FUSE_T_MIN_BYTES
 
 

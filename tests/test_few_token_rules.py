@@ -1,0 +1,35 @@
+"""Which launches the rank-r products and adapter gradients of few tokens take: host-side rules, asked without a GPU."""
+import pytest
+import torch
+
+import fmsa_hip
+from fms_acceleration_foak.fused_ops.unsloth_lora import fused_core as core
+
+
+class _Weight:
+    perm = perm_key = None
+
+    def __init__(self, K, N):
+        self.K, self.N = K, N
+
+
+def _projs(K, Ns, r):
+    projs = []
+    for N in Ns:
+        p = core._Proj(_Weight(K, N), None, torch.empty(r, K, device="meta"), torch.empty(N, r, device="meta"), 2.0, torch.bfloat16)
+        p.Bt = torch.empty(r, N, device="meta", dtype=torch.bfloat16)
+        projs.append(p)
+    return projs
+
+
+def _meta(*shape):
+    return torch.empty(*shape, device="meta", dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("M", [1, 300, 512, 513])
+def test_t_has_its_own_launch_for_few_tokens(M):
+    """T out of the gradient launch pays from 96 MB of dY on, however many projections share the launch."""
+    projs = _projs(4096, (4096, 1024, 1024), 16)
+    assert not core._fuse_t(projs, [_meta(M, p.w.N) for p in projs])
+    wide = _projs(8192, (28672, 28672), 16)
+    assert core._fuse_t(wide, [_meta(1024, p.w.N) for p in wide])
