@@ -308,8 +308,11 @@ def _adapter_grads(projs, dYs, Xds, Us, stack):
         return Ts, list(zip(dAs, dBs))
     Ts, grads = [], []
     live = [(p, dY, Xd, U) for p, dY, Xd, U in zip(projs, dYs, Xds, Us) if p.r]
-    if (len(live) == len(projs) > 1 and dYs[0].shape[0] <= fmsa_hip.LORA_DOWN_BATCH_TOKENS and 2 * len(live) <= fmsa_hip.LORA_GRAD_MAX_JOBS):
-        # few tokens: every T in one launch, then every dA and dB in one
+    if (len(live) == len(projs) > 1 and dYs[0].shape[0] <= fmsa_hip.LORA_DOWN_BATCH_TOKENS and 2 * len(live) <= fmsa_hip.LORA_GRAD_MAX_JOBS
+            and not any(p.r <= 16 and _fuse_t([p], [dY]) for p, dY, _, _ in live)):
+        # few tokens: every T in one launch, then every dA and dB in one.  Not where ranks up to 16 meet a dY that pays for
+        # T in its own gradient launch: gate and up of 8192 -> 28672 at 2047 tokens take 126 and 140 us that way at rank 8
+        # and 16, 135 and 160 here; from rank 32 on this is the faster way (175 against 191 us, rank 64: 229 against 295)
         Ts = fmsa_hip.lora_down_batch([(dY, p.Bt, None) for p, dY, _, _ in live])
         outs = fmsa_hip.lora_grad_batch([(T, Xd, p.s, False, p.A_param.dtype) for (p, _, Xd, _), T in zip(live, Ts)]
                                         + [(U, dY, p.s, True, p.B_param.dtype) for p, dY, _, U in live])

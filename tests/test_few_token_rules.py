@@ -33,3 +33,16 @@ def test_t_has_its_own_launch_for_few_tokens(M):
     assert not core._fuse_t(projs, [_meta(M, p.w.N) for p in projs])
     wide = _projs(8192, (28672, 28672), 16)
     assert core._fuse_t(wide, [_meta(1024, p.w.N) for p in wide])
+
+
+@pytest.mark.parametrize("M,N,r,batched", [(2047, 28672, 16, False), (2047, 28672, 8, False), (2047, 28672, 32, True), (1536, 28672, 16, True),
+                                           (2047, 14336, 16, True)])
+def test_unstacked_projections_keep_t_in_the_gradient_launch_where_it_pays(monkeypatch, M, N, r, batched):
+    calls = []
+    monkeypatch.setattr(fmsa_hip, "lora_down_batch", lambda jobs: calls.append("down_batch") or [_meta(M, r) for _ in jobs])
+    monkeypatch.setattr(fmsa_hip, "lora_down", lambda *a, **k: calls.append("down") or _meta(M, r))
+    monkeypatch.setattr(fmsa_hip, "lora_grad_batch", lambda jobs: calls.append("grad") or [_meta(1, 1) for _ in jobs])
+    projs = _projs(8192, (N, N), r)
+    Ts, grads = core._adapter_grads(projs, [_meta(M, N)] * 2, [_meta(M, 8192)] * 2, [_meta(M, r)] * 2, None)
+    assert len(Ts) == len(grads) == 2
+    assert calls == (["down_batch", "grad"] if batched else ["grad"] * 4)
