@@ -888,7 +888,11 @@ struct DownSplit {
 DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
   const int rt = (std::min(r, 64) + 15) / 16;  // ranks above 64 go out 64 at a time (accumulator registers)
   if (M < 2048 || C < 2048) {
-    if (!few_tokens) return {0, 0, 0};
+    // The columns of few tokens, where a wave has enough to walk through that the second launch pays: columns times rank
+    // tiles of 4096 and more (us whole / split at 300 tokens: 1024 columns 4.4 / 5.5 at rank 16, 7.2 / 7.1 at 64,
+    // 11.3 / 9.5 at 128; 2048 columns 6.1 / 6.1 at rank 16, 7.9 / 6.5 at 32; 4096 columns 9.5 / 7.1 at rank 16).
+    // From 2048 tokens on the token blocks fill the chip (1024 columns, rank 64, 3000 tokens: 7.5 / 9.9).
+    if (!few_tokens || M >= 2048 || (int64_t)C * ((r + 15) / 16) < 4096) return {0, 0, 0};
     // g = 1: the fragment kernel, columns split until two workgroups per CU are there or a wave is down to two steps of 32
     const int n_tb = (M + 15) / 16;
     const int n_split = std::min(512 / n_tb, C / 512);

@@ -46,3 +46,10 @@ def test_unstacked_projections_keep_t_in_the_gradient_launch_where_it_pays(monke
     Ts, grads = core._adapter_grads(projs, [_meta(M, N)] * 2, [_meta(M, 8192)] * 2, [_meta(M, r)] * 2, None)
     assert len(Ts) == len(grads) == 2
     assert calls == (["down_batch", "grad"] if batched else ["grad"] * 4)
+
+
+@pytest.mark.parametrize("M,C,r,split", [(300, 1024, 16, False), (1, 1024, 32, False), (300, 1024, 64, True), (300, 1024, 128, True),
+                                         (1, 2048, 16, False), (300, 2048, 24, True), (1, 4096, 8, True), (2047, 4096, 8, True),
+                                         (2048, 1024, 128, False), (3000, 1536, 64, False), (2048, 2048, 64, True)])
+def test_columns_are_split_where_the_second_launch_pays(M, C, r, split):
+    assert (fmsa_hip.lib().fmsa_lora_down_split_workspace(M, C, r) > 0) == split
