@@ -991,8 +991,12 @@ static int bwd_t_stages(const fmsa_bwd_proj* projs, int n_proj) {
 
 static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M, int mode) {
   const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;
-  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), codebook ? 1.7f : 1.4f,
-                    mode == FMSA_BWD_SWIGLU ? 0.12f : 0.f);
+  const bool swiglu = mode == FMSA_BWD_SWIGLU;
+  // measured per whole round, over 1 to 6 of them: 11 to 13 % of its time, 15 to 16 % with the SwiGLU epilogue; from a code
+  // book, where the gathers hide some of it, 6 to 9 and 12 to 15 %
+  const float whole_slow = codebook ? (swiglu ? 0.15f : 0.09f) : (swiglu ? 0.16f : 0.13f);
+  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), whole_slow, codebook ? 1.7f : 1.4f,
+                    swiglu ? 0.12f : 0.f);
 }
 
 size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M) {

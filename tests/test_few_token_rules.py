@@ -53,3 +53,36 @@ def test_unstacked_projections_keep_t_in_the_gradient_launch_where_it_pays(monke
                                          (2048, 1024, 128, False), (3000, 1536, 64, False), (2048, 2048, 64, True)])
 def test_columns_are_split_where_the_second_launch_pays(M, C, r, split):
     assert (fmsa_hip.lib().fmsa_lora_down_split_workspace(M, C, r) > 0) == split
+
+
+def _struct(K, N, codebook=False, group=128):
+    return fmsa_hip.GptqWeight(0x1000, None if codebook else 0x2000, None if codebook else 0x3000, None, K, N, 64 if codebook else group, 0,
+                               fmsa_hip.WEIGHT_CODEBOOK if codebook else fmsa_hip.WEIGHT_AFFINE, 0, 0x7000 if codebook else None,
+                               0x8000 if codebook else None)
+
+
+def _cut_fwd(M, K, Ns, swiglu=False, **kw):
+    arr = (fmsa_hip.FwdProj * len(Ns))()
+    for i, N in enumerate(Ns):
+        arr[i].w = _struct(K, N, **kw)
+    return fmsa_hip.lib().fmsa_gptq_lora_fwd_workspace(arr, len(Ns), M, fmsa_hip.FWD_SWIGLU if swiglu else fmsa_hip.FWD_LINEAR) > 0
+
+
+def _cut_bwd(M, K, Ns, **kw):
+    arr = (fmsa_hip.BwdProj * len(Ns))()
+    for i, N in enumerate(Ns):
+        arr[i].w, arr[i].nsz, arr[i].qweight_t, arr[i].scale_f32 = _struct(K, N, **kw), 0x4000, 0x5000, 0x6000
+    return fmsa_hip.lib().fmsa_gptq_lora_bwd_dx_workspace(arr, len(Ns), M, 1) > 0
+
+
+def test_tiles_are_cut_where_that_pays():
+    """Few tiles are cut; so is the rest behind whole rounds while those cost less on the flavour that cuts than it gives."""
+    assert _cut_fwd(1, 4096, [4096, 1024, 1024]) and _cut_fwd(200, 4096, [14336, 14336], swiglu=True)
+    assert not _cut_fwd(1536, 2048, [4096, 4096], swiglu=True)     # 192 tiles: no CUs to cut for
+    assert _cut_fwd(4400, 4096, [4096]) and _cut_fwd(6144, 14336, [4096])      # 288 and 384 tiles
+    assert not _cut_fwd(7131, 4096, [14336, 14336], swiglu=True)   # 12 whole rounds and 64 tiles: 1359 us whole, 1394 cut
+    assert _cut_bwd(1, 4096, [4096]) and _cut_bwd(300, 14336, [4096])
+    assert _cut_bwd(4352, 4096, [14336]) and _cut_bwd(4352, 4096, [14336], codebook=True)  # 272 tiles, long contraction
+    for M in (6107, 7131, 7387):  # five or six whole rounds in front: 617 / 656, 727 / 767, 729 / 796 us whole / cut
+        assert not _cut_bwd(M, 14336, [4096])
+    assert not _cut_bwd(7131, 8192, [8192, 1024, 1024])            # three rounds and 128 tiles: 941 / 986
