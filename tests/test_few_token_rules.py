@@ -86,3 +86,23 @@ def test_tiles_are_cut_where_that_pays():
     for M in (6107, 7131, 7387):  # five or six whole rounds in front: 617 / 656, 727 / 767, 729 / 796 us whole / cut
         assert not _cut_bwd(M, 14336, [4096])
     assert not _cut_bwd(7131, 8192, [8192, 1024, 1024])            # three rounds and 128 tiles: 941 / 986
+
+
+@pytest.mark.parametrize("cut,rotating", [((), (True, True)), (("k",), (True, False)), (("q",), (False, True)), (("q", "k"), (False, False))])
+def test_rotation_is_decided_per_launch(monkeypatch, cut, rotating):
+    """Projections that walk K in orders of their own are launched one by one: each is asked whether its launch is cut."""
+    launches, passes, M = [], [], 40
+    monkeypatch.setattr(fmsa_hip, "gptq_lora_fwd_splits", lambda weights, m: weights[0] in cut if len(weights) == 1 else "joint" in cut)
+    monkeypatch.setattr(fmsa_hip, "permute_cols", lambda x, *a, **k: x)
+    monkeypatch.setattr(fmsa_hip, "gptq_lora_fwd", lambda x, projs, *a, rope=None, **k: launches.append((projs[0]["w"], rope is not None))
+                        or [_meta(M, 256) for _ in projs])
+    monkeypatch.setattr(fmsa_hip, "rope_embedding_", lambda y, *a, **k: passes.append(1))
+    projs = []
+    for i, name in enumerate("qkv"):
+        w = _Weight(256, 256)
+        w.struct, w.perm, w.perm_key, w.group_size = name, torch.empty(256, device="meta"), i, 128
+        projs.append(core._Proj(w, None, None, None, None, torch.bfloat16))
+    table = _meta(M, 64)
+    outs, _ = core._linear_forward(projs, _meta(M, 256), [_meta(M, 256)] * 3, None, (table, table, 64, 0b011))
+    assert len(outs) == 3 and launches == [("q", rotating[0]), ("k", rotating[1]), ("v", False)]
+    assert len(passes) == 2 - sum(rotating)
