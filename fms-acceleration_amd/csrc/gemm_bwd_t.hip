@@ -22,8 +22,9 @@
 //
 // Tiling as in the forward: workgroup = 4 waves = 256 tokens x 256 output columns, wave = 256 x 64 (8 x 2 MFMA
 // 32x32x16 tiles), contraction walked in stages of 64 with the dY tile loaded global -> LDS directly, one stage
-// ahead, two stage buffers.  Results are bit-identical to the kernel that reads the checkpoint layout
-// (gemm_bwd.hip): same operand values, same MFMA operand roles and contraction order.
+// ahead, two stage buffers.  Where every tile runs whole, results are bit-identical to the kernel that reads the
+// checkpoint layout (gemm_bwd.hip): same operand values, same MFMA operand roles and contraction order.  Tiles cut along the
+// contraction (SPLIT, split_tiles.h) add the same products in another order, the same one on every run.
 #include "common.h"
 #include "split_tiles.h"
 

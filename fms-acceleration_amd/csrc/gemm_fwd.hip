@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       k_in_g[j] = __builtin_amdgcn_readfirstlane(st0 * BK % gs[j]);
     }
   }
-  // issue the global loads of stage `st` (0 <= st < n_stages) into slot SB; nothing here may read
+  // issue the global loads of stage `st` (st0 <= st < st_end) into slot SB; nothing here may read
   // the loaded registers, or the wave would wait for the load on the spot
   auto load_stage = [&](int st, auto sb_c) {
     constexpr int SB = decltype(sb_c)::value;

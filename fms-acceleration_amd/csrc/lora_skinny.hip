@@ -976,8 +976,10 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
 // Token tiles of 16 per workgroup.  Every workgroup reads its columns of all r rows of Wd out of L2, which at rank 64 is four
 // times what it reads of X: two tiles halve that.  Three launches at 1100 tokens, rank 64 (q k v; gate, up of 14336 columns;
 // 4096 columns): 34.4 us each on average with one tile, 23.3 with two, 20.4 with four (which leaves a quarter of the token blocks
-// to split for).  Below 1024 tokens the narrow projections would run out of workgroups; rank 16 and below reads less of Wd
-// than of X.
+// to split for).  The line at 1024 tokens: two tiles against one, ranks 24 to 64, take 0.58 - 0.98 of the time from 1536 tokens
+// on for q k v and gate, up of hidden 1024 to 8192; at 1024 - 1280 tokens 0.71 - 0.92 from hidden 4096 on and 0.97 - 1.07
+// below; at 64 tokens 1.03 - 1.20 (28672 columns 0.9), where the narrow projections run out of workgroups.  Rank 16 and
+// below reads less of Wd than of X.
 static int down_batch_tiles(int M, int r_max) { return M >= 1024 && r_max > 16 && r_max <= 64 ? 2 : 1; }
 static int down_batch_split(int M, int C, int n_jobs, int mtl) {
   const int n_tb = (M + 16 * mtl - 1) / (16 * mtl);

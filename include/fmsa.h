@@ -340,7 +340,8 @@ int fmsa_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M
                           void* dX, int64_t lddx, void* e, void* g, void* h_out, int64_t ldeg,
                           int act_dtype, void* stream);
 
-/* The same with a partial-sum buffer (see fmsa_gptq_lora_fwd_ws); calls that run on the transposed twin use it. */
+/* The same with a partial-sum buffer (see fmsa_gptq_lora_fwd_ws); calls that run on the transposed twin use it.  The bytes
+ * are those of the mode that needs more. */
 size_t fmsa_gptq_lora_bwd_dx_workspace(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int act_dtype);
 int fmsa_gptq_lora_bwd_dx_ws(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int mode, void* dX, int64_t lddx,
                              void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace,
