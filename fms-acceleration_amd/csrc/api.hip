@@ -20,6 +20,12 @@ int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, in
 int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st);
 int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
                          int64_t ldh, const fmsa_rope* rope, int act_dtype, void* workspace, size_t workspace_bytes, hipStream_t st);
+int launch_gptq_lora_fwd_few(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H, int64_t ldh,
+                             int act_dtype, hipStream_t st);
+bool gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int mode);
+size_t lora_few_workspace(const fmsa_few_proj* projs, int n_proj, int M);
+int launch_lora_few(const fmsa_few_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H, int64_t ldh,
+                    int act_dtype, void* workspace, hipStream_t st);
 size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode);
 size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M);
 int launch_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e,
@@ -137,7 +143,7 @@ const char* fmsa_strerror(int code) {
   }
 }
 
-int fmsa_abi_version(void) { return 10; }
+int fmsa_abi_version(void) { return 11; }
 
 int fmsa_gptq_dequant(const fmsa_gptq_weight* w, int out_dtype, void* out, void* stream) {
   if (!w || !out) return FMSA_ERR_NULL;
@@ -369,6 +375,72 @@ int fmsa_gptq_lora_fwd_ws(const fmsa_fwd_proj* projs, int n_proj, const void* X,
   if (workspace && !aligned16(workspace)) return FMSA_ERR_ALIGN;
   return launch_gptq_lora_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, nullptr, act_dtype, workspace, workspace_bytes,
                               (hipStream_t)stream);
+}
+
+int fmsa_gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return gptq_lora_fwd_is_few(projs, n_proj, M, mode) ? 1 : 0;
+}
+
+int fmsa_gptq_lora_fwd_few(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
+                           int64_t ldh, int act_dtype, void* stream) {
+  if (int rc = check_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype)) return rc;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.group_size % 64 != 0) return FMSA_ERR_UNSUPPORTED;
+  return launch_gptq_lora_fwd_few(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype, (hipStream_t)stream);
+}
+
+int fmsa_lora_few_is_few(const fmsa_few_proj* projs, int n_proj, int M, int mode) {
+  if (!projs || n_proj < 1 || n_proj > 3) return 0;
+  fmsa_fwd_proj q[3] = {};
+  for (int p = 0; p < n_proj; ++p) q[p].w = projs[p].w;
+  return fmsa_gptq_lora_fwd_is_few(q, n_proj, M, mode);
+}
+
+size_t fmsa_lora_few_workspace(const fmsa_few_proj* projs, int n_proj, int M) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].r < 0) return 0;
+  return lora_few_workspace(projs, n_proj, M);
+}
+
+int fmsa_lora_few_fwd(const fmsa_few_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H, int64_t ldh,
+                      int act_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!projs || !X) return FMSA_ERR_NULL;
+  if (n_proj < 1 || n_proj > 3 || M <= 0) return FMSA_ERR_SHAPE;
+  if (mode != FMSA_FWD_LINEAR && mode != FMSA_FWD_SWIGLU) return FMSA_ERR_SHAPE;
+  if (!is_act(act_dtype)) return FMSA_ERR_DTYPE;
+  const int K = projs[0].w.K;
+  if (ldx < K) return FMSA_ERR_SHAPE;
+  if (!aligned16(X) || ldx % 8 != 0) return FMSA_ERR_ALIGN;
+  for (int p = 0; p < n_proj; ++p) {
+    const fmsa_few_proj& s = projs[p];
+    if (int rc = check_weight(&s.w, 64, act_dtype == FMSA_F16)) return rc;
+    if (s.w.format != projs[0].w.format || s.w.nibble_order != projs[0].w.nibble_order) return FMSA_ERR_UNSUPPORTED;
+    if (s.w.K != K) return FMSA_ERR_SHAPE;
+    if (!s.Y && mode != FMSA_FWD_SWIGLU) return FMSA_ERR_NULL;
+    if (s.Y && s.ldy < s.w.N) return FMSA_ERR_SHAPE;
+    if (s.Y && (!aligned16(s.Y) || s.ldy % 8 != 0)) return FMSA_ERR_ALIGN;
+    if (int rc = check_rank(s.r)) return rc;
+    if (s.r > 0) {
+      if (!s.A || !s.B) return FMSA_ERR_NULL;
+      if (s.param_dtype != FMSA_F32 && s.param_dtype != act_dtype) return FMSA_ERR_DTYPE;
+      if (!aligned16(s.A) || !aligned16(s.B)) return FMSA_ERR_ALIGN;
+    }
+    if (s.bias && !aligned16(s.bias)) return FMSA_ERR_ALIGN;
+  }
+  if (mode == FMSA_FWD_SWIGLU) {
+    if (n_proj != 2 || projs[0].w.N != projs[1].w.N) return FMSA_ERR_SHAPE;
+    if (!H) return FMSA_ERR_NULL;
+    if (ldh < projs[0].w.N) return FMSA_ERR_SHAPE;
+    if (!aligned16(H) || ldh % 8 != 0) return FMSA_ERR_ALIGN;
+  }
+  const size_t need = lora_few_workspace(projs, n_proj, M);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return FMSA_ERR_WORKSPACE;
+  if (workspace && !aligned16(workspace)) return FMSA_ERR_ALIGN;
+  return launch_lora_few(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype, workspace, (hipStream_t)stream);
 }
 
 int fmsa_gptq_lora_fwd_rope(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, const fmsa_rope* rope,

@@ -20,6 +20,8 @@
 #include "common.h"
 #include "split_tiles.h"
 
+float few_us(const fmsa_fwd_proj* projs, int n_proj, int M, int mode);  // gemm_few.hip
+
 namespace {
 
 constexpr int BM = 256;
@@ -1026,9 +1028,23 @@ static SplitPlan fwd_split(const fmsa_fwd_proj* projs, int n_proj, int M, int mo
   }
   if (mode == FMSA_FWD_SWIGLU) nb = (projs[0].w.N + 127) / 128;
   const int tiles = ((M + BM - 1) / BM) * nb;
-  if (!ok) return SplitPlan{tiles, 0, 1};
+  if (!ok) return SplitPlan{tiles, 0, 1, 1e9f};
   // measured per whole round, over 1 to 12 of them: nothing to 1 % of its time, 3 to 5 % with the SwiGLU epilogue
   return plan_split(tiles, (projs[0].w.K + BK - 1) / BK, mode == FMSA_FWD_SWIGLU ? 0.05f : 0.01f);
+}
+
+// Whether a launch is expected to take less time on the kernel for few tokens than in 256-token tiles, cut or not.  A linear
+// launch that small tiles do whole (a few stages of K) stays there, where the rotating epilogue's sums are the same.
+bool gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  if (M > FMSA_FEW_MAX_TOKENS) return false;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.group_size % 64 != 0) return false;
+  const SplitPlan plan = fwd_split(projs, n_proj, M, mode);
+  if (mode != FMSA_FWD_SWIGLU && plan.s == 1 && plan.n_whole <= SPLIT_CUS / 2) return false;
+  // the estimate of the cut tiles is high by a tenth (SwiGLU) to a quarter: 4096 x 4096 at 300 / 400 / 513 tokens takes 31 / 39
+  // / 52 us this way and 39 / 39 / 41 in tiles, 2048 x 2048 at 700 22 and 29, 4096 of 2048 with the SwiGLU at 300 / 513 33 / 53
+  // and 49 / 50
+  return few_us(projs, n_proj, M, mode) < (mode == FMSA_FWD_SWIGLU ? 0.9f : 0.8f) * plan.us;
 }
 
 size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {

@@ -991,6 +991,13 @@ static int max_rank(const fmsa_lora_down_job* jobs, int n_jobs) {
   return r;
 }
 
+// Column ranges of lora_down (one job) and of the batched launch over few tokens
+int lora_down_few_splits(int M, int C, int r, int n_jobs) {
+  if (n_jobs > 1) return down_batch_split(M, C, n_jobs, 1);
+  const DownSplit d = lora_down_split_shape(M, C, r, true);
+  return d.g == 1 ? d.n_split : 1;
+}
+
 size_t lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
   const int mtl = down_batch_tiles(M, max_rank(jobs, n_jobs));
   size_t bytes = 0;

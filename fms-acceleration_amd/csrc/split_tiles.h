@@ -23,6 +23,7 @@ struct SplitPlan {
   int n_whole;  // tiles that run whole: ids 0 .. n_whole - 1
   int n_split;  // tiles cut into ranges
   int s;        // ranges per cut tile (1: nothing is cut)
+  float us;     // estimate of the launch
   size_t bytes() const { return s > 1 ? (size_t)n_split * s * SPLIT_TILE_BYTES : 0; }
 };
 
@@ -34,11 +35,11 @@ struct SplitPlan {
 // cannot: with whole rounds enough in front, that is more than the cut gives (SwiGLU backward 4096 -> 14336, 6107 tokens,
 // five rounds and 64 tiles: 696 us whole, 766 us cut; at 256 tokens, 56 tiles: 96 and 63 us).
 inline SplitPlan plan_split(int tiles, int n_stages, float whole_slow, float stage_us = 1.4f, float finish_us = 0.f) {
-  SplitPlan p{tiles, 0, 1};
-  const int rest = tiles % SPLIT_CUS;
+  const int rest = tiles % SPLIT_CUS, rounds = tiles / SPLIT_CUS;
+  SplitPlan p{tiles, 0, 1, (rounds + (rest > 0)) * n_stages * stage_us + 8.0f};
   if (rest == 0) return p;
   const float range_us = 2.0f * SPLIT_TILE_BYTES / 4.0e6f;
-  const float fixed_us = 8.0f + rest * finish_us + whole_slow * (tiles / SPLIT_CUS) * n_stages * 1.4f;
+  const float fixed_us = 8.0f + rest * finish_us + whole_slow * rounds * n_stages * 1.4f;
   float best = n_stages * stage_us * (tiles > rest ? 0.9f : 1.0f) - 3.0f;  // not for a gain that the noise of a launch would hide
   int s_best = 1;
   for (int s = 2; s <= SPLIT_CUS / rest && 2 * s <= n_stages; ++s) {
@@ -48,7 +49,7 @@ inline SplitPlan plan_split(int tiles, int n_stages, float whole_slow, float sta
       s_best = s;
     }
   }
-  if (s_best > 1) p = SplitPlan{tiles - rest, rest, s_best};
+  if (s_best > 1) p = SplitPlan{tiles - rest, rest, s_best, rounds * n_stages * stage_us + best};
   return p;
 }
 

@@ -146,23 +146,23 @@ def apply_lora_mlp_swiglu(self, X):
     gateW, gateW_quant, gate_bias, gateA, gateB, gateS, dropout_gate = get_lora_parameters(self.gate_proj)
     upW, upW_quant, up_bias, upA, upB, upS, dropout_up = get_lora_parameters(self.up_proj)
     downW, downW_quant, down_bias, downA, downB, downS, dropout_down = get_lora_parameters(self.down_proj)
-    return LoRA_MLP.apply(X,
-                          gateW, gateW_quant, gate_bias, gateA, gateB, gateS,
-                          upW, upW_quant, up_bias, upA, upB, upS,
-                          downW, downW_quant, down_bias, downA, downB, downS,
-                          swiglu_fg_kernel, swiglu_DWf_DW_dfg_kernel,
-                          dropout_gate, dropout_up, dropout_down)
+    return core.run(LoRA_MLP, X,
+                    gateW, gateW_quant, gate_bias, gateA, gateB, gateS,
+                    upW, upW_quant, up_bias, upA, upB, upS,
+                    downW, downW_quant, down_bias, downA, downB, downS,
+                    swiglu_fg_kernel, swiglu_DWf_DW_dfg_kernel,
+                    dropout_gate, dropout_up, dropout_down)
 
 
 def apply_lora_qkv(self, X):
     QW, QW_quant, Q_bias, QA, QB, QS, dropoutQ = get_lora_parameters(self.q_proj)
     KW, KW_quant, K_bias, KA, KB, KS, dropoutK = get_lora_parameters(self.k_proj)
     VW, VW_quant, V_bias, VA, VB, VS, dropoutV = get_lora_parameters(self.v_proj)
-    return LoRA_QKV.apply(X,
-                          QW, QW_quant, Q_bias, QA, QB, QS,
-                          KW, KW_quant, K_bias, KA, KB, KS,
-                          VW, VW_quant, V_bias, VA, VB, VS,
-                          dropoutQ, dropoutK, dropoutV)
+    return core.run(LoRA_QKV, X,
+                    QW, QW_quant, Q_bias, QA, QB, QS,
+                    KW, KW_quant, K_bias, KA, KB, KS,
+                    VW, VW_quant, V_bias, VA, VB, VS,
+                    dropoutQ, dropoutK, dropoutV)
 
 
 def apply_lora_qkv_rope(self, X, cos, sin):
@@ -175,18 +175,18 @@ def apply_lora_qkv_rope(self, X, cos, sin):
     batch, seq_len = (X.shape[0], X.shape[1]) if X.dim() == 3 else (1, X.shape[0])
     cos2d, sin2d = rope_tables(cos, sin, batch, seq_len)
     head_dim = getattr(self, "head_dim", None) or self.config.head_dim
-    return LoRA_QKV_RoPE.apply(X, cos2d, sin2d, head_dim,
-                               QW, QW_quant, Q_bias, QA, QB, QS,
-                               KW, KW_quant, K_bias, KA, KB, KS,
-                               VW, VW_quant, V_bias, VA, VB, VS,
-                               dropoutQ, dropoutK, dropoutV)
+    return core.run(LoRA_QKV_RoPE, X, cos2d, sin2d, head_dim,
+                    QW, QW_quant, Q_bias, QA, QB, QS,
+                    KW, KW_quant, K_bias, KA, KB, KS,
+                    VW, VW_quant, V_bias, VA, VB, VS,
+                    dropoutQ, dropoutK, dropoutV)
 
 
 def apply_lora_o(self, X):
     OW, OW_quant, O_bias, OA, OB, OS, dropout = get_lora_parameters(self.o_proj)
-    return LoRA_W.apply(X, OW, OW_quant, O_bias, OA, OB, OS, dropout)
+    return core.run(LoRA_W, X, OW, OW_quant, O_bias, OA, OB, OS, dropout)
 
 
 def apply_lora_o_v2(self, X):
     OW, OW_quant, O_bias, OA, OB, OS, dropout = get_lora_parameters(self)
-    return LoRA_W.apply(X, OW, OW_quant, O_bias, OA, OB, OS, dropout)
+    return core.run(LoRA_W, X, OW, OW_quant, O_bias, OA, OB, OS, dropout)

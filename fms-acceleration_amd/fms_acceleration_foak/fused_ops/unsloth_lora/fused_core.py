@@ -18,6 +18,8 @@ import torch
 
 import fmsa_hip
 
+from ...autograd import NoGraph, run  # noqa: F401  (run: for the entry points)
+
 
 # ----------------------------------------------------------------------------------------------
 # small helpers shared by the three functions
@@ -59,6 +61,18 @@ def _dropped_inputs(X2, projs, dropouts):
     """Post-dropout input of each projection's LoRA branch; X2 itself (the same object) where no
     dropout applies, which is what lets projections share passes over it."""
     return [_apply_dropout(X2, d) if p.r else X2 for p, d in zip(projs, dropouts)]
+
+
+def _few_tokens(ctx, X2, projs, dropouts, mode=fmsa_hip.FWD_LINEAR):
+    """The outputs (SWIGLU mode: h) straight from the adapters' parameters where nothing is kept and the tokens are few; None
+    where the general way is to be gone: more tokens, a column order of an act-order weight or a dropout in between,
+    parameters the kernel does not read."""
+    if (type(ctx) is not NoGraph or X2.shape[0] > fmsa_hip.FEW_TOKENS
+            or not all(p.w.perm is None and fmsa_hip.lora_few_ok(X2, p.w.struct, p.A_param, p.B_param)
+                       and (d is None or isinstance(d, torch.nn.Identity) or not p.r) for p, d in zip(projs, dropouts))):
+        return None
+    il = _interleaved(projs, X2.dtype)
+    return fmsa_hip.lora_few(X2, [(p.w.struct_interleaved if il else p.w.struct, p.A_param, p.B_param, p.bias, p.s) for p in projs], mode)
 
 
 class _Proj:
@@ -353,6 +367,9 @@ def _linear_backward_dx(projs, dYs, Ts, Xds, M, K):
 # ----------------------------------------------------------------------------------------------
 def w_forward(ctx, X, p, dropout, dtype):
     X2 = _as2d(X, dtype)
+    few = _few_tokens(ctx, X2, [p], (dropout,))
+    if few is not None:
+        return few[0].view(*X.shape[:-1], p.w.N)
     p.pack()
     Xd = _apply_dropout(X2, dropout) if p.r else X2
     (Y,), (U,) = _linear_forward([p], X2, [Xd])
@@ -381,6 +398,9 @@ def qkv_forward(ctx, X, projs, dropouts, dtype, rope=None):
     """rope = (cos2d, sin2d, head_dim): Q and K leave rotated (rows of the [positions, >= head_dim / 2] tables are
     taken as token row % positions)."""
     X2 = _as2d(X, dtype)
+    few = _few_tokens(ctx, X2, projs, dropouts) if rope is None else None
+    if few is not None:
+        return tuple(y.view(*X.shape[:-1], p.w.N) for y, p in zip(few, projs))
     Xds = _dropped_inputs(X2, projs, dropouts)
     stack = _pack_group(projs, Xds, dtype)
     ctx.rope = None if rope is None else (rope[0], rope[1], rope[2], 0b011)
@@ -428,6 +448,10 @@ def qkv_backward(ctx, dQ, dK, dV):
 def mlp_forward(ctx, X, gate, up, down, dropouts, dtype):
     dropout_gate, dropout_up, dropout_down = dropouts
     X2 = _as2d(X, dtype)
+    if down.w.perm is None:  # (else gate and up are to leave in its column order)
+        h = _few_tokens(ctx, X2, (gate, up), (dropout_gate, dropout_up), fmsa_hip.FWD_SWIGLU)
+        if h is not None:
+            return w_forward(ctx, h, down, dropout_down, dtype).view(*X.shape[:-1], down.w.N)
     Xg, Xu = _dropped_inputs(X2, (gate, up), (dropout_gate, dropout_up))
     # act-order down projection: let gate / up write e, g, h in its kernel order, so that nothing between the two
     # GEMM stages is permuted and both SwiGLU epilogues stay fused (not with a dropout on h: its mask is tied to

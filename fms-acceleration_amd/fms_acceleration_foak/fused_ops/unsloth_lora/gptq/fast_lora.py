@@ -241,8 +241,8 @@ def apply_lora_mlp(self, X):
     gateQstate, gate_bias, gateA, gateB, gateS, dropout_gate = get_lora_parameters(self.gate_proj)
     upQState, up_bias, upA, upB, upS, dropout_up = get_lora_parameters(self.up_proj)
     downQState, down_bias, downA, downB, downS, dropout_down = get_lora_parameters(self.down_proj)
-    return LoRA_MLP.apply(
-        X,
+    return core.run(
+        LoRA_MLP, X,
         *unpack_gptqstate(gateQstate), gate_bias, gateA, gateB, gateS,
         *unpack_gptqstate(upQState), up_bias, upA, upB, upS,
         *unpack_gptqstate(downQState), down_bias, downA, downB, downS,
@@ -254,8 +254,8 @@ def apply_lora_qkv(self, X):
     Qqstate, Q_bias, QA, QB, QS, Qdropout = get_lora_parameters(self.q_proj)
     Kqstate, K_bias, KA, KB, KS, Kdropout = get_lora_parameters(self.k_proj)
     Vqstate, V_bias, VA, VB, VS, Vdropout = get_lora_parameters(self.v_proj)
-    return LoRA_QKV.apply(
-        X,
+    return core.run(
+        LoRA_QKV, X,
         *unpack_gptqstate(Qqstate), Q_bias, QA, QB, QS,
         *unpack_gptqstate(Kqstate), K_bias, KA, KB, KS,
         *unpack_gptqstate(Vqstate), V_bias, VA, VB, VS,
@@ -281,8 +281,8 @@ def apply_lora_qkv_rope(self, X, cos, sin):
     batch, seq_len = (X.shape[0], X.shape[1]) if X.dim() == 3 else (1, X.shape[0])
     cos2d, sin2d = rope_tables(cos, sin, batch, seq_len)
     head_dim = getattr(self, "head_dim", None) or self.config.head_dim
-    return LoRA_QKV_RoPE.apply(
-        X, cos2d, sin2d, head_dim,
+    return core.run(
+        LoRA_QKV_RoPE, X, cos2d, sin2d, head_dim,
         *unpack_gptqstate(Qqstate), Q_bias, QA, QB, QS,
         *unpack_gptqstate(Kqstate), K_bias, KA, KB, KS,
         *unpack_gptqstate(Vqstate), V_bias, VA, VB, VS,
@@ -292,10 +292,10 @@ def apply_lora_qkv_rope(self, X, cos, sin):
 
 def apply_lora_o(self, X):
     Oqstate, O_bias, OA, OB, OS, dropout = get_lora_parameters(self.o_proj)
-    return LoRA_W.apply(X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)
+    return core.run(LoRA_W, X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)
 
 
 def apply_lora_o_v2(self, X):
     """Patched directly on the output linear (`self` is the LoRA layer itself, :856-859)."""
     Oqstate, O_bias, OA, OB, OS, dropout = get_lora_parameters(self)
-    return LoRA_W.apply(X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)
+    return core.run(LoRA_W, X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)

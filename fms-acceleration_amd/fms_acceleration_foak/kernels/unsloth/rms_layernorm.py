@@ -6,6 +6,8 @@ import torch
 
 import fmsa_hip
 
+from ...autograd import run
+
 
 class Fast_RMS_Layernorm(torch.autograd.Function):
     @staticmethod
@@ -35,4 +37,4 @@ class Fast_RMS_Layernorm(torch.autograd.Function):
 def fast_rms_layernorm(layernorm, X, gemma=False):
     W = layernorm.weight
     eps = layernorm.variance_epsilon if hasattr(layernorm, "variance_epsilon") else layernorm.eps
-    return Fast_RMS_Layernorm.apply(X, W, eps, gemma)
+    return run(Fast_RMS_Layernorm, X, W, eps, gemma)

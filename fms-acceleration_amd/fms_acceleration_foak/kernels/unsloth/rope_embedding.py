@@ -11,6 +11,8 @@ import torch
 
 import fmsa_hip
 
+from ...autograd import run
+
 
 def _rows(t, batch, seq_len):
     """cos / sin as the [rows, head_dim] table the kernel indexes with (token row % rows):
@@ -76,6 +78,6 @@ def fast_rope_embedding(Q, K, cos, sin, position_ids=None, unsqueeze_dim=1):
             if done[1].untyped_storage().data_ptr() != K.untyped_storage().data_ptr():
                 raise RuntimeError("fast_rope_embedding: Q comes rotated from the fused projection, K does not")
             return Q, K
-    Q = Fast_RoPE_Embedding.apply(Q.transpose(1, 2), cos, sin).transpose(1, 2)
-    K = Fast_RoPE_Embedding.apply(K.transpose(1, 2), cos, sin).transpose(1, 2)
+    Q = run(Fast_RoPE_Embedding, Q.transpose(1, 2), cos, sin).transpose(1, 2)
+    K = run(Fast_RoPE_Embedding, K.transpose(1, 2), cos, sin).transpose(1, 2)
     return Q, K

@@ -43,6 +43,11 @@ EXPORTED_SYMBOLS = (
     "fmsa_gptq_lora_fwd",
     "fmsa_gptq_lora_fwd_workspace",
     "fmsa_gptq_lora_fwd_ws",
+    "fmsa_gptq_lora_fwd_is_few",
+    "fmsa_gptq_lora_fwd_few",
+    "fmsa_lora_few_is_few",
+    "fmsa_lora_few_workspace",
+    "fmsa_lora_few_fwd",
     "fmsa_gptq_lora_fwd_rope",
     "fmsa_gptq_lora_bwd_dx",
     "fmsa_gptq_lora_bwd_dx_workspace",
@@ -182,6 +187,21 @@ class FwdProj(Structure):
     ]
 
 
+class FewProj(Structure):
+    _fields_ = [
+        ("w", GptqWeight),
+        ("A", c_void_p),
+        ("B", c_void_p),
+        ("bias", c_void_p),
+        ("Y", c_void_p),
+        ("ldy", c_int64),
+        ("r", c_int32),
+        ("s", c_float),
+        ("param_dtype", c_int32),
+        ("reserved", c_int32),
+    ]
+
+
 class BwdProj(Structure):
     _fields_ = [
         ("w", GptqWeight),
@@ -204,7 +224,7 @@ class BwdProj(Structure):
 _lib = None
 
 
-ABI_VERSION = 10  # include/fmsa.h as this binding mirrors it (fmsa_abi_version of the library must agree)
+ABI_VERSION = 11  # include/fmsa.h as this binding mirrors it (fmsa_abi_version of the library must agree)
 
 
 def lib() -> ctypes.CDLL:
@@ -254,6 +274,13 @@ def lib() -> ctypes.CDLL:
     L.fmsa_gptq_lora_fwd_workspace.argtypes = [POINTER(FwdProj), c_int, c_int, c_int]
     L.fmsa_gptq_lora_fwd_ws.argtypes = [POINTER(FwdProj), c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p,
                                         c_size_t, c_void_p]
+    L.fmsa_gptq_lora_fwd_is_few.argtypes = [POINTER(FwdProj), c_int, c_int, c_int]
+    L.fmsa_gptq_lora_fwd_few.argtypes = L.fmsa_gptq_lora_fwd.argtypes
+    L.fmsa_lora_few_is_few.argtypes = [POINTER(FewProj), c_int, c_int, c_int]
+    L.fmsa_lora_few_workspace.restype = c_size_t
+    L.fmsa_lora_few_workspace.argtypes = [POINTER(FewProj), c_int, c_int]
+    L.fmsa_lora_few_fwd.argtypes = [POINTER(FewProj), c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p,
+                                    c_size_t, c_void_p]
     L.fmsa_gptq_lora_bwd_dx_workspace.restype = c_size_t
     L.fmsa_gptq_lora_bwd_dx_workspace.argtypes = [POINTER(BwdProj), c_int, c_int, c_int]
     L.fmsa_gptq_lora_bwd_dx_ws.argtypes = [POINTER(BwdProj), c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
@@ -520,7 +547,8 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None,
     Returns the list of outputs Y_p [M, N_p]; in SWIGLU mode returns (e, g, h).
     rope = (cos2d, sin2d, head_dim, proj_mask): LINEAR mode only; the projections whose bit is set in proj_mask
     leave with the rotary embedding applied (token row m takes row m % cos2d.shape[0] of the tables).
-    split=True lets the call cut tiles that do not fill the chip along K (another, still fixed, order of the fp32 sums)."""
+    split=True lets the call cut tiles that do not fill the chip along K, and take the kernel for few tokens (other, still
+    fixed, orders of the fp32 sums)."""
     M = x2d.shape[0]
     arr = (FwdProj * len(projs))()
     outs = []
@@ -546,18 +574,71 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None,
                lib().fmsa_gptq_lora_fwd_rope(arr, len(projs), _ptr(x2d), x2d.stride(0), M, ctypes.byref(desc),
                                              act_enum(x2d.dtype), _stream(x2d)))
         return outs
-    nbytes = lib().fmsa_gptq_lora_fwd_workspace(arr, len(projs), M, mode) if split else 0
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x2d.device) if nbytes else None
-    _check("fmsa_gptq_lora_fwd_ws",
-           lib().fmsa_gptq_lora_fwd_ws(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
-                                       0 if h is None else h.stride(0), act_enum(x2d.dtype), _ptr(ws), nbytes, _stream(x2d)))
+    if split and M <= FEW_MAX_TOKENS and lib().fmsa_gptq_lora_fwd_is_few(arr, len(projs), M, mode):
+        _check("fmsa_gptq_lora_fwd_few",
+               lib().fmsa_gptq_lora_fwd_few(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
+                                            0 if h is None else h.stride(0), act_enum(x2d.dtype), _stream(x2d)))
+    else:
+        nbytes = lib().fmsa_gptq_lora_fwd_workspace(arr, len(projs), M, mode) if split else 0
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x2d.device) if nbytes else None
+        _check("fmsa_gptq_lora_fwd_ws",
+               lib().fmsa_gptq_lora_fwd_ws(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
+                                           0 if h is None else h.stride(0), act_enum(x2d.dtype), _ptr(ws), nbytes, _stream(x2d)))
     if mode == FWD_SWIGLU:
         return outs[0], outs[1], h
     return outs
 
 
+FEW_MAX_TOKENS = 768  # FMSA_FEW_MAX_TOKENS
+FEW_TOKENS = 64  # up to here a pass without a graph goes straight from the adapters' parameters
+
+
+def lora_few_ok(x2d, w: GptqWeight, A, B) -> bool:
+    """Whether lora_few takes a projection (weight w, not act-order; adapter parameters A, B or None) as it is."""
+    if x2d.shape[0] > FEW_TOKENS or w.group_size % 64:
+        return False
+    if A is None:
+        return True
+    r = A.shape[0]
+    return (A.dtype == B.dtype and (A.dtype == torch.float32 or A.dtype == x2d.dtype) and A.is_cuda and B.is_cuda and r % 8 == 0
+            and 0 < r <= 128 and A.is_contiguous() and B.is_contiguous() and (A.data_ptr() | B.data_ptr()) % 16 == 0)
+
+
+def lora_few(x2d, projs, mode: int = FWD_LINEAR):
+    """projs: (GptqWeight, A, B, bias, s) with the adapter's own parameters (None: no adapter).  The outputs of
+    gptq_lora_fwd([...], split=True) on U = lora_down(x2d, A), to the last bit, from one launch for every U and one for every
+    output; in SWIGLU mode h alone.  Nothing is kept for a backward.  None where gptq_lora_fwd would not take the kernel for
+    few tokens."""
+    M, dev, dt = x2d.shape[0], x2d.device, x2d.dtype
+    arr = (FewProj * len(projs))()
+    for q, (w, A, B, bias, s) in zip(arr, projs):
+        q.w = w
+        q.ldy = w.N
+        if bias is not None:
+            q.bias = bias.data_ptr()
+        if A is not None:
+            assert A.shape[1] == w.K and B.shape == (w.N, A.shape[0])
+            q.A, q.B, q.r, q.s, q.param_dtype = A.data_ptr(), B.data_ptr(), A.shape[0], float(s), _DTYPE_ENUM[A.dtype]
+    L, n = lib(), len(projs)
+    if not L.fmsa_lora_few_is_few(arr, n, M, mode):
+        return None
+    if mode == FWD_SWIGLU:
+        outs = h = torch.empty((M, projs[0][0].N), dtype=dt, device=dev)
+    else:
+        h, outs = None, [torch.empty((M, p[0].N), dtype=dt, device=dev) for p in projs]
+        for q, y in zip(arr, outs):
+            q.Y = y.data_ptr()
+    nbytes = L.fmsa_lora_few_workspace(arr, n, M)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    _check("fmsa_lora_few_fwd",
+           L.fmsa_lora_few_fwd(arr, n, x2d.data_ptr(), x2d.stride(0), M, mode, _ptr(h), 0 if h is None else h.stride(0),
+                               act_enum(dt), _ptr(ws), nbytes, _stream(x2d)))
+    return outs
+
+
 def gptq_lora_fwd_splits(weights, M: int) -> bool:
-    """Whether gptq_lora_fwd(split=True) cuts the tiles of a LINEAR launch of these weights over M tokens."""
+    """Whether the 256-token tiles of a LINEAR launch of these weights over M tokens are cut (where the kernel for few tokens is
+    taken instead, they would be, unless the launch is very small)."""
     arr = (FwdProj * len(weights))()
     for i, w in enumerate(weights):
         arr[i].w = w

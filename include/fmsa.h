@@ -43,7 +43,7 @@ enum fmsa_dtype { FMSA_F16 = 0, FMSA_BF16 = 1, FMSA_F32 = 2 };
 /* Human-readable text for an error code (host pointer to a static string). */
 const char* fmsa_strerror(int code);
 
-/* ABI version; bumped on any change of a signature or struct layout (10 here).  A binding should refuse a library whose
+/* ABI version; bumped on any change of a signature or struct layout (11 here).  A binding should refuse a library whose
  * version is not the one it was written for. */
 int fmsa_abi_version(void);
 
@@ -262,6 +262,37 @@ int fmsa_gptq_lora_fwd(const fmsa_fwd_proj* projs /*host*/, int n_proj, const vo
 size_t fmsa_gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M, int mode);
 int fmsa_gptq_lora_fwd_ws(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M, int mode,
                           void* H, int64_t ldh, int act_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same forward for few tokens (any number is taken; fmsa_gptq_lora_fwd_is_few says where it pays, from shapes
+ * and formats alone): workgroups of 16 or 32 columns
+ * whose waves share K, one launch, no workspace.  Same operands and rounding points, another fixed order of the fp32 sums.
+ * Every group_size % 64 == 0, else FMSA_ERR_UNSUPPORTED. */
+#define FMSA_FEW_MAX_TOKENS 768 /* beyond, fmsa_gptq_lora_fwd_is_few always says no */
+int fmsa_gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M, int mode); /* 1: expected to be faster */
+int fmsa_gptq_lora_fwd_few(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M, int mode,
+                           void* H, int64_t ldh, int act_dtype, void* stream);
+
+/* The same again straight from the adapters' parameters, for a pass that keeps nothing for a backward: U = X A^T of all
+ * projections in one launch (fp32 sums of a few ranges of K in `workspace`, rounded to act_dtype once where the second
+ * launch adds them), Y in another; neither A nor B is packed.  fmsa_lora_few_workspace gives the bytes (16-byte aligned, no
+ * initialisation needed, calls that may overlap in time need separate ones).  X in the model's K order: weights that are not
+ * act-order.  In FMSA_FWD_SWIGLU mode Y may be NULL (only h leaves). */
+typedef struct fmsa_few_proj {
+  fmsa_gptq_weight w;
+  const void* A;       /* [r, K] lora_A.weight, NULL when r == 0 */
+  const void* B;       /* [N, r] lora_B.weight                   */
+  const void* bias;    /* [N] act_dtype or NULL                  */
+  void* Y;             /* [M, N] act_dtype                       */
+  int64_t ldy;
+  int32_t r;           /* 0, or r % 8 == 0, r <= 128             */
+  float s;
+  int32_t param_dtype; /* of A and B: FMSA_F32 or act_dtype      */
+  int32_t reserved;
+} fmsa_few_proj;
+int fmsa_lora_few_is_few(const fmsa_few_proj* projs /*host*/, int n_proj, int M, int mode); /* as fmsa_gptq_lora_fwd_is_few */
+size_t fmsa_lora_few_workspace(const fmsa_few_proj* projs /*host*/, int n_proj, int M);
+int fmsa_lora_few_fwd(const fmsa_few_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
+                      int64_t ldh, int act_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same forward (FMSA_FWD_LINEAR) with the rotary position embedding of the attention block applied in the
  * epilogue of the projections named by `proj_mask` (bit p = projection p; q and k of LoRA_QKV): replaces the

@@ -106,3 +106,21 @@ def test_rotation_is_decided_per_launch(monkeypatch, cut, rotating):
     outs, _ = core._linear_forward(projs, _meta(M, 256), [_meta(M, 256)] * 3, None, (table, table, 64, 0b011))
     assert len(outs) == 3 and launches == [("q", rotating[0]), ("k", rotating[1]), ("v", False)]
     assert len(passes) == 2 - sum(rotating)
+
+
+def _few(M, K, Ns, swiglu=False, **kw):
+    arr = (fmsa_hip.FwdProj * len(Ns))()
+    for q, N in zip(arr, Ns):
+        q.w = _struct(K, N, **kw)
+    return fmsa_hip.lib().fmsa_gptq_lora_fwd_is_few(arr, len(Ns), M, fmsa_hip.FWD_SWIGLU if swiglu else fmsa_hip.FWD_LINEAR) == 1
+
+
+def test_the_kernel_for_few_tokens_is_taken_where_it_is_faster():
+    for M in (1, 64):
+        assert _few(M, 14336, [4096]) and _few(M, 4096, [14336, 14336], swiglu=True) and _few(M, 8192, [28672], codebook=True)
+    assert _few(300, 4096, [4096]) and not _few(513, 4096, [4096])
+    assert _few(700, 2048, [2048]) and not _few(769, 2048, [2048])
+    assert _few(300, 2048, [4096, 4096], swiglu=True) and not _few(513, 2048, [4096, 4096], swiglu=True)
+    assert not _few(129, 4096, [14336, 14336], swiglu=True) and not _few(64, 4096, [4096], group=32)
+    assert not _few(700, 4096, [4096, 1024, 1024])
+    assert not _few(1, 256, [256, 64, 64]) and _few(1, 256, [256, 256], swiglu=True)
