@@ -6,7 +6,8 @@ hipcc cross-compiles for gfx950 without a GPU.  Each translation unit is compile
 in parallel and the objects are linked into ``lib/libfmsa_hip.so`` next to this file; the
 Python side loads that file with ctypes and never builds at import time.  The measurement probe
 (``csrc/probe.hip``, what ``bench.py --yardsticks`` times) is not part of the product: it becomes a
-library of its own, ``lib/libfmsa_probe.so``.
+library of its own, ``lib/libfmsa_probe.so``.  The extension that makes the operators' calls
+(``csrc/host_calls.cpp``, host code against torch's headers) becomes ``lib/_fmsa_calls.so``.
 """
 from __future__ import annotations
 
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -25,6 +27,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libfmsa_hip.so")
 SOURCES = ["api.hip", "dequant.hip", "gemm_fwd.hip", "gemm_few.hip", "gemm_bwd.hip", "gemm_bwd_t.hip", "lora_skinny.hip", "elementwise.hip", "nf4.hip", "norm_rope.hip"]
 PROBE_SOURCE = "probe.hip"
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libfmsa_probe.so")
+CALLS_SOURCE = "host_calls.cpp"
+CALLS_PATH = os.path.join(LIB_DIR, "_fmsa_calls.so")
 
 # -packed-fp32-ops is switched off on purpose: the packed fp32 VALU forms are not trusted on the
 # target machines, so fp32 math is emitted as scalar-per-lane instructions.
@@ -53,6 +57,18 @@ def _run(cmd):
     return out
 
 
+def _compile_calls(obj):
+    import torch.utils.cpp_extension as ext  # the headers and libraries of the torch that will load it
+
+    flags = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(ext.torch._C._GLIBCXX_USE_CXX11_ABI)}"]  # pylint: disable=protected-access
+    includes = [*ext.include_paths(), sysconfig.get_paths()["include"]]
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    _run(["g++", *flags, *(f"-I{d}" for d in includes), "-isystem", os.path.join(rocm, "include"), "-c",
+          os.path.join(CSRC, CALLS_SOURCE), "-o", obj])
+    return [f"-L{d}" for d in ext.library_paths()]
+
+
 def build(verbose: bool = False, extra_flags=()) -> str:
     """Compile every source unconditionally and link the library.  Returns its path."""
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -69,8 +85,11 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         return obj
 
     probe_obj = os.path.join(OBJ_DIR, PROBE_SOURCE.replace(".hip", ".o"))
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
+    calls_obj = os.path.join(OBJ_DIR, CALLS_SOURCE.replace(".cpp", ".o"))
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 2)) as pool:
+        calls = pool.submit(_compile_calls, calls_obj)
         list(pool.map(compile_one, list(zip(SOURCES, objs)) + [(PROBE_SOURCE, probe_obj)]))
+        torch_libs = calls.result()
     for path, members in ((LIB_PATH, objs), (PROBE_LIB_PATH, [probe_obj])):
         tmp = path + ".tmp"
         # --no-undefined: a kernel whose host stub was not emitted must fail the link, not the first call
@@ -78,6 +97,12 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         os.replace(tmp, path)
         if verbose:
             print("built", path)
+    tmp = CALLS_PATH + ".tmp"
+    _run(["g++", "-shared", "-o", tmp, calls_obj, f"-L{LIB_DIR}", "-lfmsa_hip", *torch_libs, "-lc10", "-lc10_hip", "-ltorch_cpu",
+          "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, CALLS_PATH)
+    if verbose:
+        print("built", CALLS_PATH)
     return LIB_PATH
 
 

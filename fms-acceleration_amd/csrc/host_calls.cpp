@@ -1,0 +1,620 @@
+// The tensor-level calls of the operators' hot path as a CPython extension: what fmsa_hip/__init__.py names lora_down,
+// gptq_lora_fwd, .. allocates the outputs and partial sums, fills the C-ABI structs and calls libfmsa_hip.so here.  A layer's
+// training pass makes 23 of these calls, and in Python (ctypes structs, torch.empty, attribute reads) they cost the host
+// 15 to 30 us each, which is more than the GPU spends on them up to a few hundred tokens.  Host code only; arguments are checked
+// as the C ABI checks them and a refusal raises the FmsaError that install() was given.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <algorithm>
+#include <vector>
+
+#include "../../include/fmsa.h"
+
+namespace {
+
+struct PyFailure {};  // a Python error is set
+
+PyObject* g_fmsa_error = nullptr;  // fmsa_hip.FmsaError(fn, code)
+
+void check(const char* fn, int code) {
+  if (code == FMSA_OK) return;
+  PyObject* err = PyObject_CallFunction(g_fmsa_error, "si", fn, code);
+  if (err) {
+    PyErr_SetObject(g_fmsa_error, err);
+    Py_DECREF(err);
+  }
+  throw PyFailure();
+}
+
+void need(bool ok, const char* what) {
+  if (ok) return;
+  PyErr_SetString(PyExc_AssertionError, what);
+  throw PyFailure();
+}
+
+const at::Tensor& tensor(PyObject* o) {
+  if (!o || !THPVariable_Check(o)) {
+    PyErr_SetString(PyExc_TypeError, "expected a tensor");
+    throw PyFailure();
+  }
+  return THPVariable_Unpack(o);
+}
+
+at::Tensor optional(PyObject* o) { return !o || o == Py_None ? at::Tensor() : tensor(o); }
+
+void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+int dtype_enum(at::ScalarType t) {
+  switch (t) {
+    case at::kHalf: return FMSA_F16;
+    case at::kBFloat16: return FMSA_BF16;
+    case at::kFloat: return FMSA_F32;
+    default: PyErr_SetString(PyExc_KeyError, "dtype must be float16, bfloat16 or float32"); throw PyFailure();
+  }
+}
+
+int act_enum(at::ScalarType t) {
+  if (t == at::kHalf) return FMSA_F16;
+  if (t == at::kBFloat16) return FMSA_BF16;
+  PyErr_Format(PyExc_TypeError, "activations must be float16 or bfloat16, got %s", c10::toString(t));
+  throw PyFailure();
+}
+
+void* stream(const at::Tensor& t) {
+  if (!t.is_cuda()) {
+    PyErr_SetString(PyExc_RuntimeError, "libfmsa_hip kernels need tensors on the GPU (there is no CPU implementation)");
+    throw PyFailure();
+  }
+  return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream();
+}
+
+// The call itself without the interpreter lock: a full launch queue blocks it.
+template <typename F> int unlocked(F&& f) {
+  PyThreadState* s = PyEval_SaveThread();
+  const int rc = f();
+  PyEval_RestoreThread(s);
+  return rc;
+}
+
+at::Tensor empty(std::initializer_list<int64_t> sizes, const at::Tensor& like) { return at::empty(sizes, like.options()); }
+at::Tensor empty(std::initializer_list<int64_t> sizes, const at::Tensor& like, at::ScalarType t) {
+  return at::empty(sizes, like.options().dtype(t));
+}
+at::Tensor workspace(size_t bytes, const at::Tensor& like) {
+  return at::empty({(int64_t)std::max<size_t>(bytes, 16)}, like.options().dtype(at::kByte));
+}
+
+// Owned reference released on every way out
+struct Ref {
+  PyObject* o;
+  explicit Ref(PyObject* p) : o(p) {
+    if (!p) throw PyFailure();
+  }
+  ~Ref() { Py_XDECREF(o); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  PyObject* release() {
+    PyObject* r = o;
+    o = nullptr;
+    return r;
+  }
+};
+
+PyObject* wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
+
+PyObject* wrap_list(const std::vector<at::Tensor>& ts) {
+  Ref list(PyList_New((Py_ssize_t)ts.size()));
+  for (size_t i = 0; i < ts.size(); ++i) PyList_SET_ITEM(list.o, (Py_ssize_t)i, wrap(ts[i]));
+  return list.release();
+}
+
+double number(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw PyFailure();
+  return v;
+}
+
+long integer(PyObject* o) {
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw PyFailure();
+  return v;
+}
+
+bool truth(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw PyFailure();
+  return v != 0;
+}
+
+at::ScalarType dtype_of(PyObject* o) {
+  if (!THPDtype_Check(o)) {
+    PyErr_SetString(PyExc_TypeError, "expected a dtype");
+    throw PyFailure();
+  }
+  return reinterpret_cast<THPDtype*>(o)->scalar_type;
+}
+
+fmsa_gptq_weight weight(PyObject* o) {  // the ctypes GptqWeight, whose memory is the C struct
+  Py_buffer b;
+  if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) throw PyFailure();
+  const bool ok = b.len == (Py_ssize_t)sizeof(fmsa_gptq_weight);
+  fmsa_gptq_weight w{};
+  if (ok) w = *static_cast<const fmsa_gptq_weight*>(b.buf);
+  PyBuffer_Release(&b);
+  need(ok, "w must be a GptqWeight");
+  return w;
+}
+
+struct Sequence {  // list or tuple
+  PyObject* fast;
+  explicit Sequence(PyObject* o) : fast(PySequence_Fast(o, "expected a sequence")) {
+    if (!fast) throw PyFailure();
+  }
+  ~Sequence() { Py_DECREF(fast); }
+  Sequence(const Sequence&) = delete;
+  Sequence& operator=(const Sequence&) = delete;
+  Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(fast); }
+  PyObject* operator[](Py_ssize_t i) const { return PySequence_Fast_GET_ITEM(fast, i); }
+};
+
+PyObject* key(const char* name) { return PyUnicode_InternFromString(name); }
+
+PyObject* item(PyObject* dict, PyObject* k, bool required = true) {  // borrowed; nullptr where absent
+  PyObject* v = PyDict_GetItemWithError(dict, k);
+  if (!v && (required || PyErr_Occurred())) {
+    if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, k);
+    throw PyFailure();
+  }
+  return v;
+}
+
+template <PyObject* (*F)(PyObject* const*, Py_ssize_t), int N>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != N) {
+    PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", N, n);
+    return nullptr;
+  }
+  try {
+    return F(args, n);
+  } catch (const PyFailure&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- rank-r products ----------------------------------------------------------------------------------------------------
+at::Tensor down_one(const at::Tensor& x, const at::Tensor& wd, at::Tensor out) {
+  const int64_t M = x.size(0), C = x.size(1), r = wd.size(0);
+  need(wd.size(1) == C && wd.is_contiguous() && wd.scalar_type() == x.scalar_type() && x.stride(1) == 1, "lora_down: x2d, wd");
+  if (!out.defined()) out = empty({M, r}, x);
+  need(out.dim() == 2 && out.size(0) == M && out.size(1) == r && out.stride(1) == 1 && out.scalar_type() == x.scalar_type(), "lora_down: out");
+  const int act = act_enum(x.scalar_type());
+  void* st = stream(out);
+  const size_t bytes = fmsa_lora_down_split_workspace((int)M, (int)C, (int)r);
+  const at::Tensor ws = bytes ? workspace(bytes, x) : at::Tensor();
+  check("fmsa_lora_down_split", unlocked([&] {
+          return fmsa_lora_down_split(ptr(x), x.stride(0), ptr(wd), (int)M, (int)C, (int)r, act, ptr(out), out.stride(0), ptr(ws),
+                                      ws.defined() ? ws.numel() : 0, st);
+        }));
+  return out;
+}
+
+PyObject* lora_down(PyObject* const* a, Py_ssize_t) { return wrap(down_one(tensor(a[0]), tensor(a[1]), optional(a[2]))); }
+
+PyObject* lora_down_batch(PyObject* const* a, Py_ssize_t) {  // jobs, most tokens
+  Sequence jobs(a[0]);
+  const Py_ssize_t n = jobs.size();
+  need(n > 0, "lora_down_batch: no jobs");
+  struct Job {
+    at::Tensor x, wd, out;
+  };
+  std::vector<Job> js;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    Sequence j(jobs[i]);
+    need(j.size() == 3, "lora_down_batch: (x2d, wd, out)");
+    js.push_back({tensor(j[0]), tensor(j[1]), optional(j[2])});
+  }
+  const int64_t M = js[0].x.size(0);
+  bool single = n < 2 || M > integer(a[1]);
+  for (const Job& j : js)
+    single = single || j.x.size(1) % 8 || (j.out.defined() && (reinterpret_cast<uintptr_t>(ptr(j.out)) % 8 || j.out.stride(0) % 4));
+  std::vector<at::Tensor> outs;
+  if (single) {
+    for (const Job& j : js) outs.push_back(down_one(j.x, j.wd, j.out));
+    return wrap_list(outs);
+  }
+  const at::Tensor& x0 = js[0].x;
+  const int act = act_enum(x0.scalar_type());
+  void* st = stream(x0);
+  for (Py_ssize_t i = 0; i < n; i += FMSA_LORA_DOWN_MAX_JOBS) {
+    const int m = (int)std::min<Py_ssize_t>(FMSA_LORA_DOWN_MAX_JOBS, n - i);
+    fmsa_lora_down_job arr[FMSA_LORA_DOWN_MAX_JOBS] = {};
+    for (int q = 0; q < m; ++q) {
+      Job& j = js[i + q];
+      const int64_t r = j.wd.size(0), C = j.wd.size(1);
+      need(j.x.size(0) == M && j.x.size(1) == C && j.wd.is_contiguous() && j.wd.scalar_type() == x0.scalar_type() &&
+               j.x.scalar_type() == x0.scalar_type() && j.x.stride(1) == 1, "lora_down_batch: x2d, wd");
+      if (!j.out.defined()) j.out = empty({M, r}, j.x);
+      need(j.out.dim() == 2 && j.out.size(0) == M && j.out.size(1) == r && j.out.stride(1) == 1 && j.out.scalar_type() == x0.scalar_type(),
+           "lora_down_batch: out");
+      arr[q].X = ptr(j.x);
+      arr[q].Wd = ptr(j.wd);
+      arr[q].out = ptr(j.out);
+      arr[q].ldx = j.x.stride(0);
+      arr[q].ldout = j.out.stride(0);
+      arr[q].C = (int)C;
+      arr[q].r = (int)r;
+      outs.push_back(j.out);
+    }
+    const at::Tensor ws = workspace(fmsa_lora_down_batch_workspace(arr, m, (int)M), x0);
+    check("fmsa_lora_down_batch",
+          unlocked([&] { return fmsa_lora_down_batch(arr, m, (int)M, act, ptr(ws), ws.numel(), st); }));
+  }
+  return wrap_list(outs);
+}
+
+PyObject* lora_grad_batch(PyObject* const* a, Py_ssize_t) {  // jobs, most of them a launch
+  Sequence jobs(a[0]);
+  const Py_ssize_t n = jobs.size();
+  const long most = integer(a[1]);
+  std::vector<at::Tensor> outs;
+  for (Py_ssize_t i = 0; i < n; i += most) {
+    const int m = (int)std::min<Py_ssize_t>(most, n - i);
+    std::vector<fmsa_lora_grad_job> arr(m);
+    at::Tensor r0;
+    int64_t M = 0;
+    for (int q = 0; q < m; ++q) {
+      Sequence j(jobs[i + q]);
+      need(j.size() == 5 || j.size() == 7, "lora_grad_batch: (L, R, scale, transpose_out, out_dtype[, Wt, T_out])");
+      const at::Tensor &L = tensor(j[0]), &R = tensor(j[1]);
+      const at::Tensor Wt = j.size() == 7 ? optional(j[5]) : at::Tensor(), T = j.size() == 7 ? optional(j[6]) : at::Tensor();
+      if (q == 0) {
+        M = L.size(0);
+        r0 = R;
+      }
+      const int64_t r = L.size(1), C = R.size(1);
+      need(L.size(0) == M && R.size(0) == M && L.stride(1) == 1 && R.stride(1) == 1, "lora_grad_batch: L, R");
+      need(L.scalar_type() == R.scalar_type() && R.scalar_type() == r0.scalar_type(), "lora_grad_batch: dtypes");
+      if (Wt.defined()) {
+        need(Wt.size(0) == r && Wt.size(1) == C && Wt.is_contiguous() && Wt.scalar_type() == R.scalar_type(), "lora_grad_batch: Wt");
+        need(T.defined() && T.size(0) == M && T.size(1) == r && T.stride(1) == 1 && T.scalar_type() == R.scalar_type(), "lora_grad_batch: T_out");
+      }
+      const bool tr = truth(j[3]);
+      const at::ScalarType od = dtype_of(j[4]);
+      at::Tensor out = tr ? empty({C, r}, R, od) : empty({r, C}, R, od);
+      arr[q] = {};
+      arr[q].L = ptr(L);
+      arr[q].R = ptr(R);
+      arr[q].out = ptr(out);
+      arr[q].ldl = L.stride(0);
+      arr[q].ldr = R.stride(0);
+      arr[q].C = (int)C;
+      arr[q].r = (int)r;
+      arr[q].scale = (float)number(j[2]);
+      arr[q].transpose_out = tr;
+      arr[q].out_dtype = dtype_enum(od);
+      arr[q].Wt = ptr(Wt);
+      arr[q].T = ptr(T);
+      arr[q].ldt = T.defined() ? T.stride(0) : 0;
+      outs.push_back(std::move(out));
+    }
+    const int act = act_enum(r0.scalar_type());
+    void* st = stream(r0);
+    const at::Tensor ws = workspace(fmsa_lora_grad_batch_workspace(arr.data(), m, (int)M), r0);
+    check("fmsa_lora_grad_batch",
+          unlocked([&] { return fmsa_lora_grad_batch(arr.data(), m, (int)M, act, ptr(ws), ws.numel(), st); }));
+  }
+  return wrap_list(outs);
+}
+
+PyObject* lora_pack_batch(PyObject* const* a, Py_ssize_t) {  // adapters, act_dtype, most of them a launch
+  Sequence adapters(a[0]);
+  const at::ScalarType act = dtype_of(a[1]);
+  const int act_e = act_enum(act);
+  const long most = integer(a[2]);
+  const Py_ssize_t n = adapters.size();
+  Ref list(PyList_New(n));
+  std::vector<fmsa_lora_pack_job> jobs(n);
+  std::vector<at::Tensor> keep;
+  void* st = nullptr;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    Sequence j(adapters[i]);
+    need(j.size() == 3, "lora_pack_batch: (A, B, A16_out)");
+    at::Tensor A = tensor(j[0]), B = tensor(j[1]), A16 = optional(j[2]);
+    if (!(A.is_cuda() && B.is_cuda())) {
+      PyErr_SetString(PyExc_RuntimeError, "fmsa_hip needs GPU tensors");
+      throw PyFailure();
+    }
+    if (A.scalar_type() != B.scalar_type()) B = B.detach().to(A.scalar_type());
+    if (!A.is_contiguous()) A = A.detach().contiguous();
+    if (!B.is_contiguous()) B = B.detach().contiguous();
+    const int64_t r = A.size(0), K = A.size(1), N = B.size(0);
+    if (A16.defined())
+      need(A16.dim() == 2 && A16.size(0) == r && A16.size(1) == K && A16.is_contiguous() && A16.scalar_type() == act, "lora_pack_batch: A16_out");
+    else
+      A16 = empty({r, K}, A, act);
+    at::Tensor At = empty({K, r}, A, act), B16 = empty({N, r}, A, act), Bt = empty({r, N}, A, act);
+    jobs[i] = {};
+    jobs[i].A = ptr(A);
+    jobs[i].B = ptr(B);
+    jobs[i].A16 = ptr(A16);
+    jobs[i].At16 = ptr(At);
+    jobs[i].B16 = ptr(B16);
+    jobs[i].Bt16 = ptr(Bt);
+    jobs[i].r = (int)r;
+    jobs[i].K = (int)K;
+    jobs[i].N = (int)N;
+    jobs[i].param_dtype = dtype_enum(A.scalar_type());
+    if (i == 0) st = stream(A);
+    keep.push_back(std::move(A));
+    keep.push_back(std::move(B));
+    Ref quad(PyTuple_New(4));
+    PyTuple_SET_ITEM(quad.o, 0, j[2] == Py_None ? wrap(std::move(A16)) : (Py_INCREF(j[2]), j[2]));
+    PyTuple_SET_ITEM(quad.o, 1, wrap(std::move(At)));
+    PyTuple_SET_ITEM(quad.o, 2, wrap(std::move(B16)));
+    PyTuple_SET_ITEM(quad.o, 3, wrap(std::move(Bt)));
+    PyList_SET_ITEM(list.o, i, quad.release());
+  }
+  for (Py_ssize_t i = 0; i < n; i += most)
+    check("fmsa_lora_pack_batch", unlocked([&] {
+            return fmsa_lora_pack_batch(jobs.data() + i, (int)std::min<Py_ssize_t>(most, n - i), act_e, st);
+          }));
+  return list.release();
+}
+
+// ---- fused GEMMs ----------------------------------------------------------------------------------------------------------
+PyObject* gptq_lora_fwd(PyObject* const* a, Py_ssize_t) {  // x2d, projs, mode, split
+  const at::Tensor& x = tensor(a[0]);
+  Sequence projs(a[1]);
+  const int mode = (int)integer(a[2]), n = (int)projs.size();
+  const bool split = truth(a[3]);
+  static PyObject *kw = key("w"), *kU = key("U"), *kB = key("B"), *kbias = key("bias"), *kr = key("r"), *ks = key("s");
+  need(n >= 1 && n <= 3 && x.dim() == 2, "gptq_lora_fwd: one to three projections of x2d [M, K]");
+  const int64_t M = x.size(0);
+  fmsa_fwd_proj arr[3] = {};
+  std::vector<at::Tensor> outs;
+  for (int i = 0; i < n; ++i) {
+    PyObject* p = projs[i];
+    need(PyDict_Check(p), "gptq_lora_fwd: projections are dicts");
+    fmsa_fwd_proj& q = arr[i];
+    q.w = weight(item(p, kw));
+    outs.push_back(empty({M, q.w.N}, x));
+    q.Y = ptr(outs[i]);
+    q.ldy = outs[i].stride(0);
+    q.r = (int)integer(item(p, kr));
+    PyObject* s = item(p, ks);
+    q.s = s == Py_None ? 0.f : (float)number(s);
+    if (q.r) {
+      const at::Tensor U = optional(item(p, kU, false)), B = optional(item(p, kB, false));
+      if (U.defined()) {
+        need(U.stride(1) == 1, "gptq_lora_fwd: U");
+        q.U = ptr(U);
+        q.ldu = U.stride(0);
+      }
+      q.B = ptr(B);
+    }
+    q.bias = ptr(optional(item(p, kbias, false)));
+  }
+  at::Tensor h;
+  if (mode == FMSA_FWD_SWIGLU) h = at::empty_like(outs[0]);
+  const int act = act_enum(x.scalar_type());
+  void* st = stream(x);
+  const int64_t ldh = h.defined() ? h.stride(0) : 0;
+  if (split && fmsa_gptq_lora_fwd_is_few(arr, n, (int)M, mode)) {
+    check("fmsa_gptq_lora_fwd_few",
+          unlocked([&] { return fmsa_gptq_lora_fwd_few(arr, n, ptr(x), x.stride(0), (int)M, mode, ptr(h), ldh, act, st); }));
+  } else {
+    const size_t bytes = split ? fmsa_gptq_lora_fwd_workspace(arr, n, (int)M, mode) : 0;
+    const at::Tensor ws = bytes ? workspace(bytes, x) : at::Tensor();
+    check("fmsa_gptq_lora_fwd_ws", unlocked([&] {
+            return fmsa_gptq_lora_fwd_ws(arr, n, ptr(x), x.stride(0), (int)M, mode, ptr(h), ldh, act, ptr(ws), bytes, st);
+          }));
+  }
+  if (mode == FMSA_FWD_SWIGLU) {
+    Ref t(PyTuple_New(3));
+    PyTuple_SET_ITEM(t.o, 0, wrap(outs[0]));
+    PyTuple_SET_ITEM(t.o, 1, wrap(outs[1]));
+    PyTuple_SET_ITEM(t.o, 2, wrap(h));
+    return t.release();
+  }
+  return wrap_list(outs);
+}
+
+PyObject* gptq_lora_bwd_dx(PyObject* const* a, Py_ssize_t) {  // projs, M, K, mode, e, g, split
+  Sequence projs(a[0]);
+  const int n = (int)projs.size(), M = (int)integer(a[1]), K = (int)integer(a[2]), mode = (int)integer(a[3]);
+  const at::Tensor e = optional(a[4]), g = optional(a[5]);
+  const bool split = truth(a[6]);
+  static PyObject *kw = key("w"), *knsz = key("nsz"), *kdY = key("dY"), *kT = key("T"), *kAt = key("At"), *kms = key("mask_src"), *kr = key("r"),
+                  *ks = key("s"), *kqt = key("qweight_t"), *ksf = key("scale_f32"), *knz = key("negzp_f16");
+  need(n >= 1 && n <= 3, "gptq_lora_bwd_dx: one to three projections");
+  fmsa_bwd_proj arr[3] = {};
+  at::Tensor ref;
+  for (int i = 0; i < n; ++i) {
+    PyObject* p = projs[i];
+    need(PyDict_Check(p), "gptq_lora_bwd_dx: projections are dicts");
+    fmsa_bwd_proj& q = arr[i];
+    const at::Tensor& dy = tensor(item(p, kdY));
+    if (i == 0) ref = dy;
+    need(dy.dim() == 2 && dy.stride(1) == 1, "gptq_lora_bwd_dx: dY");
+    q.w = weight(item(p, kw));
+    q.nsz = (const float*)ptr(optional(item(p, knsz)));
+    q.dY = ptr(dy);
+    q.lddy = dy.stride(0);
+    q.r = (int)integer(item(p, kr));
+    PyObject* s = item(p, ks);
+    q.s = s == Py_None ? 0.f : (float)number(s);
+    if (q.r) {
+      const at::Tensor T = optional(item(p, kT, false));
+      if (T.defined()) {
+        need(T.stride(1) == 1, "gptq_lora_bwd_dx: T");
+        q.T = ptr(T);
+        q.ldt = T.stride(0);
+      }
+      q.At = ptr(optional(item(p, kAt, false)));
+    }
+    const at::Tensor ms = optional(item(p, kms, false));
+    q.mask_src = ptr(ms);
+    q.ldmask = ms.defined() ? ms.stride(0) : 0;
+    q.qweight_t = (const int32_t*)ptr(optional(item(p, kqt, false)));
+    q.scale_f32 = (const float*)ptr(optional(item(p, ksf, false)));
+    q.negzp_f16 = static_cast<decltype(q.negzp_f16)>(ptr(optional(item(p, knz, false))));
+  }
+  const int act = act_enum(ref.scalar_type());
+  void* st = stream(ref);
+  const size_t bytes = split ? fmsa_gptq_lora_bwd_dx_workspace(arr, n, M, act) : 0;
+  const at::Tensor ws = bytes ? workspace(bytes, ref) : at::Tensor();
+  if (mode == FMSA_BWD_SWIGLU) {
+    need(e.defined() && g.defined(), "gptq_lora_bwd_dx: e, g");
+    at::Tensor h = at::empty_like(e);
+    check("fmsa_gptq_lora_bwd_dx_ws", unlocked([&] {
+            return fmsa_gptq_lora_bwd_dx_ws(arr, n, M, mode, nullptr, 0, ptr(e), ptr(g), ptr(h), e.stride(0), act, ptr(ws), bytes, st);
+          }));
+    return wrap(h);
+  }
+  at::Tensor dx = empty({M, K}, ref);
+  check("fmsa_gptq_lora_bwd_dx_ws", unlocked([&] {
+          return fmsa_gptq_lora_bwd_dx_ws(arr, n, M, mode, ptr(dx), dx.stride(0), nullptr, nullptr, nullptr, 0, act, ptr(ws), bytes, st);
+        }));
+  return wrap(dx);
+}
+
+PyObject* lora_few(PyObject* const* a, Py_ssize_t) {  // x2d, ((w, A, B, bias, s), ..), mode
+  const at::Tensor& x = tensor(a[0]);
+  Sequence projs(a[1]);
+  const int n = (int)projs.size(), mode = (int)integer(a[2]);
+  need(n >= 1 && n <= 3 && x.dim() == 2, "lora_few: one to three projections of x2d [M, K]");
+  const int M = (int)x.size(0);
+  fmsa_few_proj arr[3] = {};
+  for (int i = 0; i < n; ++i) {
+    Sequence p(projs[i]);
+    need(p.size() == 5, "lora_few: (w, A, B, bias, s)");
+    fmsa_few_proj& q = arr[i];
+    q.w = weight(p[0]);
+    q.ldy = q.w.N;
+    q.bias = ptr(optional(p[3]));
+    const at::Tensor A = optional(p[1]);
+    if (A.defined()) {
+      const at::Tensor& B = tensor(p[2]);
+      need(A.size(1) == q.w.K && B.size(0) == q.w.N && B.size(1) == A.size(0), "lora_few: A, B");
+      q.A = ptr(A);
+      q.B = ptr(B);
+      q.r = (int)A.size(0);
+      q.s = (float)number(p[4]);
+      q.param_dtype = dtype_enum(A.scalar_type());
+    }
+  }
+  if (!fmsa_lora_few_is_few(arr, n, M, mode)) Py_RETURN_NONE;
+  at::Tensor h;
+  std::vector<at::Tensor> outs;
+  if (mode == FMSA_FWD_SWIGLU)
+    h = empty({M, arr[0].w.N}, x);
+  else
+    for (int i = 0; i < n; ++i) {
+      outs.push_back(empty({M, arr[i].w.N}, x));
+      arr[i].Y = ptr(outs[i]);
+    }
+  const int act = act_enum(x.scalar_type());
+  void* st = stream(x);
+  const size_t bytes = fmsa_lora_few_workspace(arr, n, M);
+  const at::Tensor ws = bytes ? workspace(bytes, x) : at::Tensor();
+  check("fmsa_lora_few_fwd", unlocked([&] {
+          return fmsa_lora_few_fwd(arr, n, ptr(x), x.stride(0), M, mode, ptr(h), h.defined() ? h.stride(0) : 0, act, ptr(ws), bytes, st);
+        }));
+  return mode == FMSA_FWD_SWIGLU ? wrap(h) : wrap_list(outs);
+}
+
+// ---- norm and rotary embedding --------------------------------------------------------------------------------------------
+void on_gpu(bool ok) {
+  if (ok) return;
+  PyErr_SetString(PyExc_RuntimeError, "fmsa_hip needs GPU tensors");
+  throw PyFailure();
+}
+
+PyObject* rms_layernorm_fwd(PyObject* const* a, Py_ssize_t) {  // x2d, weight, eps, gemma
+  const at::Tensor &x = tensor(a[0]), &w = tensor(a[1]);
+  on_gpu(x.is_cuda() && w.is_cuda());
+  need(x.dim() == 2 && x.stride(1) == 1 && w.is_contiguous() && w.numel() == x.size(1), "rms_layernorm_fwd: x2d, weight");
+  const float eps = (float)number(a[2]);
+  const int gemma = truth(a[3]), M = (int)x.size(0), C = (int)x.size(1);
+  at::Tensor y = empty({M, C}, x), r = empty({M}, x, at::kFloat);
+  void* st = stream(x);
+  const int xd = dtype_enum(x.scalar_type()), wd = dtype_enum(w.scalar_type());
+  check("fmsa_rms_layernorm_fwd", unlocked([&] {
+          return fmsa_rms_layernorm_fwd(ptr(x), x.stride(0), ptr(w), M, C, eps, gemma, xd, wd, ptr(y), y.stride(0), (float*)ptr(r), st);
+        }));
+  Ref t(PyTuple_New(2));
+  PyTuple_SET_ITEM(t.o, 0, wrap(y));
+  PyTuple_SET_ITEM(t.o, 1, wrap(r));
+  return t.release();
+}
+
+PyObject* rms_layernorm_bwd(PyObject* const* a, Py_ssize_t) {  // dy2d, x2d, weight, r, gemma
+  const at::Tensor &dy = tensor(a[0]), &x = tensor(a[1]), &w = tensor(a[2]), &r = tensor(a[3]);
+  need(dy.dim() == 2 && dy.sizes() == x.sizes() && dy.stride(1) == 1 && x.stride(1) == 1 && dy.scalar_type() == x.scalar_type(), "rms_layernorm_bwd: dy2d, x2d");
+  const int gemma = truth(a[4]), M = (int)x.size(0), C = (int)x.size(1);
+  void* st = stream(x);
+  const int xd = dtype_enum(x.scalar_type()), wd = dtype_enum(w.scalar_type());
+  check("fmsa_rms_layernorm_bwd", unlocked([&] {
+          return fmsa_rms_layernorm_bwd(ptr(dy), dy.stride(0), ptr(x), x.stride(0), ptr(w), (const float*)ptr(r), M, C, gemma, xd, wd, st);
+        }));
+  Py_INCREF(a[0]);
+  return a[0];
+}
+
+PyObject* rope_embedding_(PyObject* const* a, Py_ssize_t) {  // q2d, cos2d, sin2d, n_heads, head_dim, backward
+  const at::Tensor &q = tensor(a[0]), &c = tensor(a[1]), &s = tensor(a[2]);
+  on_gpu(q.is_cuda() && c.is_cuda() && s.is_cuda());
+  need(q.stride(1) == 1 && c.stride(1) == 1 && c.strides() == s.strides() && c.scalar_type() == s.scalar_type(), "rope_embedding_: q2d, cos2d, sin2d");
+  const int heads = (int)integer(a[3]), hd = (int)integer(a[4]), bwd = truth(a[5]);
+  void* st = stream(q);
+  const int qd = dtype_enum(q.scalar_type()), cd = dtype_enum(c.scalar_type());
+  check("fmsa_rope_embedding", unlocked([&] {
+          return fmsa_rope_embedding(ptr(q), q.stride(0), ptr(c), ptr(s), c.stride(0), (int)q.size(0), heads, hd, (int)c.size(0), bwd, qd, cd, st);
+        }));
+  Py_INCREF(a[0]);
+  return a[0];
+}
+
+PyObject* rope_embedding_strided(PyObject* const* a, Py_ssize_t) {  // q4d, cos2d, sin2d, backward
+  const at::Tensor &q = tensor(a[0]), &c = tensor(a[1]), &s = tensor(a[2]);
+  on_gpu(q.is_cuda() && c.is_cuda() && s.is_cuda());
+  need(q.dim() == 4 && q.stride(3) == 1 && c.stride(1) == 1 && c.strides() == s.strides() && c.scalar_type() == s.scalar_type(),
+       "rope_embedding_strided: q4d, cos2d, sin2d");
+  const int bwd = truth(a[3]), b = (int)q.size(0), t = (int)q.size(1), h = (int)q.size(2), d = (int)q.size(3);
+  at::Tensor out = empty({(int64_t)b * t, (int64_t)h * d}, q);
+  void* st = stream(q);
+  const int qd = dtype_enum(q.scalar_type()), cd = dtype_enum(c.scalar_type());
+  check("fmsa_rope_embedding_strided", unlocked([&] {
+          return fmsa_rope_embedding_strided(ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(out), ptr(c), ptr(s), c.stride(0), b, t, h, d,
+                                             (int)c.size(0), bwd, qd, cd, st);
+        }));
+  return wrap(out);
+}
+
+PyObject* install(PyObject* const* a, Py_ssize_t) {  // FmsaError
+  Py_INCREF(a[0]);
+  Py_XDECREF(g_fmsa_error);
+  g_fmsa_error = a[0];
+  return PyLong_FromLong(fmsa_abi_version());
+}
+
+#define ENTRY(name, n) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, n>)), METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {ENTRY(lora_down, 3),           ENTRY(lora_down_batch, 2),   ENTRY(lora_grad_batch, 2),
+                           ENTRY(lora_pack_batch, 3),     ENTRY(gptq_lora_fwd, 4),     ENTRY(gptq_lora_bwd_dx, 7),
+                           ENTRY(lora_few, 3),            ENTRY(rms_layernorm_fwd, 4), ENTRY(rms_layernorm_bwd, 5),
+                           ENTRY(rope_embedding_, 6),     ENTRY(rope_embedding_strided, 4), ENTRY(install, 1),
+                           {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fmsa_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__fmsa_calls() { return PyModule_Create(&g_module); }

@@ -1,4 +1,7 @@
-"""Running the autograd functions of the fused operators by themselves where no graph is built."""
+"""Running the autograd functions of the fused operators: by themselves where no graph is built, and their backward under
+the autocast state of their forward."""
+import functools
+
 import torch
 
 
@@ -19,3 +22,18 @@ def no_graph() -> bool:
 def run(function, *args):
     """function.apply(*args); without the node where nothing could follow from it."""
     return function.forward(NoGraph(), *args) if no_graph() else function.apply(*args)
+
+
+def bwd_as_fwd(backward):
+    """torch.amp.custom_bwd, whose autocast context costs the host 15 us a node, entered only where it would change
+    something: where the state the backward meets is not the one its forward (torch.amp.custom_fwd) ran under."""
+    entered = torch.amp.custom_bwd(backward, device_type="cuda")
+
+    @functools.wraps(backward)
+    def run_backward(ctx, *grads):
+        on = torch.is_autocast_enabled("cuda")
+        if on == ctx._fwd_used_autocast and (not on or torch.get_autocast_dtype("cuda") == ctx._dtype):  # pylint: disable=protected-access
+            return backward(ctx, *grads)
+        return entered(ctx, *grads)
+
+    return run_backward

@@ -23,6 +23,7 @@ import torch
 import fmsa_hip
 from fmsa_hip.nf4_prepared import prepare as _prepare
 
+from ....autograd import bwd_as_fwd
 from .. import fused_core as core
 from ..fused_core import _act_dtype, _Proj
 from ..utils import get_lora_parameters
@@ -42,7 +43,7 @@ class LoRA_W(torch.autograd.Function):
         return core.w_forward(ctx, X, _proj(W, W_quant, bias, A, B, S, dtype), dropout_O, dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dY):
         dX, dA, dB = core.w_backward(ctx, dY)
         return dX, None, None, None, dA, dB, None, None
@@ -62,7 +63,7 @@ class LoRA_QKV(torch.autograd.Function):
         return core.qkv_forward(ctx, X, projs, (dropout_Q, dropout_K, dropout_V), dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dQ, dK, dV):
         dX, grads = core.qkv_backward(ctx, dQ, dK, dV)
         n3 = (None,) * 3
@@ -91,7 +92,7 @@ class LoRA_QKV_RoPE(torch.autograd.Function):
         return core.qkv_forward(ctx, X, projs, (dropout_Q, dropout_K, dropout_V), dtype, rope=(cos, sin, int(head_dim)))
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dQ, dK, dV):
         dX, grads = core.qkv_backward(ctx, dQ, dK, dV)
         n3 = (None,) * 3
@@ -131,7 +132,7 @@ class LoRA_MLP(torch.autograd.Function):
         return core.mlp_forward(ctx, X, gate, up, down, (dropout_gate, dropout_up, dropout_down), dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dY):
         dX, (dAg, dBg), (dAu, dBu), (dAd, dBd) = core.mlp_backward(ctx, dY)
         n3 = (None,) * 3

@@ -36,6 +36,7 @@ import torch
 
 from fmsa_hip.gptq_prepared import prepare as _prepare  # per-weight C-ABI view, cached on the qweight tensor
 
+from ....autograd import bwd_as_fwd
 from .. import fused_core as core
 from ..fused_core import _act_dtype, _Proj
 from ..utils import active_adapter_parts, member
@@ -123,7 +124,7 @@ class LoRA_W(torch.autograd.Function):
         return core.w_forward(ctx, X, p, dropout_O, dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dY):
         dX, dA, dB = core.w_backward(ctx, dY)
         return (dX, None, None, None, None, None, None, dA, dB, None, None)
@@ -151,7 +152,7 @@ class LoRA_QKV(torch.autograd.Function):
         return core.qkv_forward(ctx, X, projs, (dropout_Q, dropout_K, dropout_V), dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dQ, dK, dV):
         dX, grads = core.qkv_backward(ctx, dQ, dK, dV)
         n6 = (None,) * 6
@@ -188,7 +189,7 @@ class LoRA_QKV_RoPE(torch.autograd.Function):
         return core.qkv_forward(ctx, X, projs, (dropout_Q, dropout_K, dropout_V), dtype, rope=(cos, sin, int(head_dim)))
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dQ, dK, dV):
         dX, grads = core.qkv_backward(ctx, dQ, dK, dV)
         n6 = (None,) * 6
@@ -221,7 +222,7 @@ class LoRA_MLP(torch.autograd.Function):
         return core.mlp_forward(ctx, X, gate, up, down, (dropout_gate, dropout_up, dropout_down), dtype)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
+    @bwd_as_fwd
     def backward(ctx, dY):
         dX, (dAg, dBg), (dAu, dBu), (dAd, dBd) = core.mlp_backward(ctx, dY)
         n6 = (None,) * 6

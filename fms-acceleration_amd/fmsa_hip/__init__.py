@@ -1,12 +1,14 @@
-"""ctypes binding of libfmsa_hip.so (C ABI declared in include/fmsa.h).
+"""Binding of libfmsa_hip.so (C ABI declared in include/fmsa.h): the calls of the operators' hot path through the extension
+built from csrc/host_calls.cpp, everything else through ctypes.
 
-The library is built in-tree by ``build_hip.py`` and loaded from ``../lib``.  Nothing here falls
+Both are built in-tree by ``build_hip.py`` and loaded from ``../lib``.  Nothing here falls
 back to another implementation: if the library is missing, or a call returns an error code, a
 RuntimeError is raised.  torch is used only for device memory (tensors) and the current stream.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import POINTER, Structure, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from typing import Optional, Sequence
@@ -15,6 +17,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libfmsa_hip.so")
+CALLS_PATH = os.path.join(os.path.dirname(_HERE), "lib", "_fmsa_calls.so")
 
 F16, BF16, F32 = 0, 1, 2
 FWD_LINEAR, FWD_SWIGLU = 0, 1
@@ -327,13 +330,32 @@ class FmsaError(RuntimeError):
         self.code = code
 
 
+_native = None
+
+
+def native():
+    """The extension of csrc/host_calls.cpp; raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(f"{CALLS_PATH} is missing: build it with `python fms-acceleration_amd/build_hip.py`")
+        spec = importlib.util.spec_from_file_location("_fmsa_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        if module.install(FmsaError) != ABI_VERSION:
+            raise RuntimeError(f"{CALLS_PATH} was built against another library than {LIB_PATH}: rebuild both")
+        _native = module
+    return _native
+
+
 def _check(fn: str, code: int):
     if code != 0:
         raise FmsaError(fn, code)
 
 
-# A small launch costs the host as much as the GPU, so pointers and streams go to ctypes as plain integers (it makes its own
-# c_void_p from the argument types) and the stream is asked for by its raw handle, without a Stream object per launch.
+# Pointers and streams go to ctypes as plain integers (it makes its own c_void_p from the argument types) and the stream is
+# asked for by its raw handle, without a Stream object per launch.
 def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -421,18 +443,7 @@ def permute_cols(x2d, perm, gather: bool):
 
 def lora_down(x2d, wd, out=None):
     """out [M, r] = x2d [M, C] @ wd [r, C]^T.  `out` may be a column slice of a wider buffer."""
-    M, C = x2d.shape
-    r = wd.shape[0]
-    assert wd.shape[1] == C and wd.is_contiguous() and wd.dtype == x2d.dtype and x2d.stride(1) == 1
-    if out is None:
-        out = x2d.new_empty((M, r))
-    assert out.shape == (M, r) and out.stride(1) == 1 and out.dtype == x2d.dtype
-    nbytes = lib().fmsa_lora_down_split_workspace(M, C, r)
-    ws = _workspace(nbytes, x2d.device) if nbytes else None
-    _check("fmsa_lora_down_split",
-           lib().fmsa_lora_down_split(_ptr(x2d), x2d.stride(0), _ptr(wd), M, C, r, act_enum(x2d.dtype), _ptr(out), out.stride(0),
-                                      _ptr(ws), 0 if ws is None else ws.numel(), _stream(out)))
-    return out
+    return (_native or native()).lora_down(x2d, wd, out)
 
 
 LORA_DOWN_MAX_JOBS = 3
@@ -442,28 +453,7 @@ LORA_DOWN_BATCH_TOKENS = 2047  # from 2048 tokens on a product fills the chip by
 def lora_down_batch(jobs):
     """jobs: (x2d, wd, out or None) triples over the same M tokens; the list of lora_down(x2d, wd, out).  With few tokens
     one launch (and one of column sums) per LORA_DOWN_MAX_JOBS of them, single calls otherwise."""
-    M = jobs[0][0].shape[0]
-    if len(jobs) < 2 or M > LORA_DOWN_BATCH_TOKENS or any(
-            x.shape[1] % 8 or (o is not None and (o.data_ptr() % 8 or o.stride(0) % 4)) for x, _, o in jobs):
-        return [lora_down(x, wd, out=o) for x, wd, o in jobs]
-    outs = []
-    for i in range(0, len(jobs), LORA_DOWN_MAX_JOBS):
-        chunk = jobs[i : i + LORA_DOWN_MAX_JOBS]
-        arr = (LoraDownJob * len(chunk))()
-        for q, (x, wd, out) in enumerate(chunk):
-            r, C = wd.shape
-            assert x.shape == (M, C) and wd.is_contiguous() and wd.dtype == x.dtype == chunk[0][0].dtype and x.stride(1) == 1
-            if out is None:
-                out = x.new_empty((M, r))
-            assert out.shape == (M, r) and out.stride(1) == 1 and out.dtype == x.dtype
-            outs.append(out)
-            arr[q] = LoraDownJob(_ptr(x), _ptr(wd), _ptr(out), x.stride(0), out.stride(0), C, r)
-        x0 = chunk[0][0]
-        nbytes = lib().fmsa_lora_down_batch_workspace(arr, len(chunk), M)
-        ws = _workspace(nbytes, x0.device)
-        _check("fmsa_lora_down_batch",
-               lib().fmsa_lora_down_batch(arr, len(chunk), M, act_enum(x0.dtype), _ptr(ws), ws.numel(), _stream(x0)))
-    return outs
+    return (_native or native()).lora_down_batch(jobs, LORA_DOWN_BATCH_TOKENS)
 
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
@@ -517,29 +507,7 @@ def lora_grad_batch(jobs):
     the list of scale * L^T @ R, each as lora_grad would give it, from one launch of each pass per
     LORA_GRAD_MAX_JOBS jobs.  A job with Wt [r, C] and T_out [M, r] (may be a column slice) also gets
     T_out = R @ Wt^T from the same pass over R (all ranks of such a call <= LORA_GRAD_T_MAX_RANK)."""
-    outs = []
-    for i in range(0, len(jobs), LORA_GRAD_MAX_JOBS):
-        chunk = jobs[i : i + LORA_GRAD_MAX_JOBS]
-        M = chunk[0][0].shape[0]
-        arr = (LoraGradJob * len(chunk))()
-        for q, job in enumerate(chunk):
-            L, R, scale, tr, out_dtype = job[:5]
-            Wt, T_out = job[5:7] if len(job) > 5 else (None, None)
-            r, C = L.shape[1], R.shape[1]
-            assert L.shape[0] == M and R.shape[0] == M and L.stride(1) == 1 and R.stride(1) == 1
-            assert L.dtype == R.dtype == chunk[0][1].dtype
-            if Wt is not None:
-                assert Wt.shape == (r, C) and Wt.is_contiguous() and Wt.dtype == R.dtype
-                assert T_out.shape == (M, r) and T_out.stride(1) == 1 and T_out.dtype == R.dtype
-            out = torch.empty((C, r) if tr else (r, C), dtype=out_dtype, device=R.device)
-            outs.append(out)
-            arr[q] = LoraGradJob(_ptr(L), _ptr(R), _ptr(out), L.stride(0), R.stride(0), C, r, float(scale), int(tr),
-                                 _DTYPE_ENUM[out_dtype], 0, _ptr(Wt), _ptr(T_out), 0 if T_out is None else T_out.stride(0))
-        R0 = chunk[0][1]
-        ws = _workspace(lib().fmsa_lora_grad_batch_workspace(arr, len(chunk), M), R0.device)
-        _check("fmsa_lora_grad_batch",
-               lib().fmsa_lora_grad_batch(arr, len(chunk), M, act_enum(R0.dtype), _ptr(ws), ws.numel(), _stream(R0)))
-    return outs
+    return (_native or native()).lora_grad_batch(jobs, LORA_GRAD_MAX_JOBS)
 
 
 def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None, split: bool = False):
@@ -549,6 +517,13 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None,
     leave with the rotary embedding applied (token row m takes row m % cos2d.shape[0] of the tables).
     split=True lets the call cut tiles that do not fill the chip along K, and take the kernel for few tokens (other, still
     fixed, orders of the fp32 sums)."""
+    if rope is None:
+        return (_native or native()).gptq_lora_fwd(x2d, projs, mode, split)
+    cos2d, sin2d, head_dim, proj_mask = rope
+    assert mode == FWD_LINEAR and cos2d.shape == sin2d.shape and cos2d.dtype == sin2d.dtype
+    assert cos2d.stride(1) == 1 and sin2d.stride(1) == 1 and cos2d.stride(0) == sin2d.stride(0) and cos2d.is_cuda
+    if cos2d.dim() != 2 or cos2d.shape[1] < int(head_dim) // 2:
+        raise ValueError("cos / sin must be [positions, >= head_dim / 2]")
     M = x2d.shape[0]
     arr = (FwdProj * len(projs))()
     outs = []
@@ -560,36 +535,13 @@ def gptq_lora_fwd(x2d, projs: Sequence[dict], mode: int = FWD_LINEAR, rope=None,
         assert U is None or U.stride(1) == 1
         arr[i] = FwdProj(w, _ptr(U), 0 if U is None else U.stride(0), _ptr(p.get("B")) if p["r"] else None,
                          _ptr(p.get("bias")), _ptr(y), y.stride(0), int(p["r"]), float(p["s"] or 0.0))
-    h = None
-    if mode == FWD_SWIGLU:
-        h = torch.empty_like(outs[0])
-    if rope is not None:
-        cos2d, sin2d, head_dim, proj_mask = rope
-        assert mode == FWD_LINEAR and cos2d.shape == sin2d.shape and cos2d.dtype == sin2d.dtype
-        assert cos2d.stride(1) == 1 and sin2d.stride(1) == 1 and cos2d.stride(0) == sin2d.stride(0) and cos2d.is_cuda
-        if cos2d.dim() != 2 or cos2d.shape[1] < int(head_dim) // 2:
-            raise ValueError("cos / sin must be [positions, >= head_dim / 2]")
-        desc = Rope(_ptr(cos2d), _ptr(sin2d), cos2d.stride(0), cos2d.shape[0], int(head_dim), _DTYPE_ENUM[cos2d.dtype], int(proj_mask))
-        _check("fmsa_gptq_lora_fwd_rope",
-               lib().fmsa_gptq_lora_fwd_rope(arr, len(projs), _ptr(x2d), x2d.stride(0), M, ctypes.byref(desc),
-                                             act_enum(x2d.dtype), _stream(x2d)))
-        return outs
-    if split and M <= FEW_MAX_TOKENS and lib().fmsa_gptq_lora_fwd_is_few(arr, len(projs), M, mode):
-        _check("fmsa_gptq_lora_fwd_few",
-               lib().fmsa_gptq_lora_fwd_few(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
-                                            0 if h is None else h.stride(0), act_enum(x2d.dtype), _stream(x2d)))
-    else:
-        nbytes = lib().fmsa_gptq_lora_fwd_workspace(arr, len(projs), M, mode) if split else 0
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=x2d.device) if nbytes else None
-        _check("fmsa_gptq_lora_fwd_ws",
-               lib().fmsa_gptq_lora_fwd_ws(arr, len(projs), _ptr(x2d), x2d.stride(0), M, mode, _ptr(h),
-                                           0 if h is None else h.stride(0), act_enum(x2d.dtype), _ptr(ws), nbytes, _stream(x2d)))
-    if mode == FWD_SWIGLU:
-        return outs[0], outs[1], h
+    desc = Rope(_ptr(cos2d), _ptr(sin2d), cos2d.stride(0), cos2d.shape[0], int(head_dim), _DTYPE_ENUM[cos2d.dtype], int(proj_mask))
+    _check("fmsa_gptq_lora_fwd_rope",
+           lib().fmsa_gptq_lora_fwd_rope(arr, len(projs), _ptr(x2d), x2d.stride(0), M, ctypes.byref(desc),
+                                         act_enum(x2d.dtype), _stream(x2d)))
     return outs
 
 
-FEW_MAX_TOKENS = 768  # FMSA_FEW_MAX_TOKENS
 FEW_TOKENS = 64  # up to here a pass without a graph goes straight from the adapters' parameters
 
 
@@ -609,31 +561,7 @@ def lora_few(x2d, projs, mode: int = FWD_LINEAR):
     gptq_lora_fwd([...], split=True) on U = lora_down(x2d, A), to the last bit, from one launch for every U and one for every
     output; in SWIGLU mode h alone.  Nothing is kept for a backward.  None where gptq_lora_fwd would not take the kernel for
     few tokens."""
-    M, dev, dt = x2d.shape[0], x2d.device, x2d.dtype
-    arr = (FewProj * len(projs))()
-    for q, (w, A, B, bias, s) in zip(arr, projs):
-        q.w = w
-        q.ldy = w.N
-        if bias is not None:
-            q.bias = bias.data_ptr()
-        if A is not None:
-            assert A.shape[1] == w.K and B.shape == (w.N, A.shape[0])
-            q.A, q.B, q.r, q.s, q.param_dtype = A.data_ptr(), B.data_ptr(), A.shape[0], float(s), _DTYPE_ENUM[A.dtype]
-    L, n = lib(), len(projs)
-    if not L.fmsa_lora_few_is_few(arr, n, M, mode):
-        return None
-    if mode == FWD_SWIGLU:
-        outs = h = torch.empty((M, projs[0][0].N), dtype=dt, device=dev)
-    else:
-        h, outs = None, [torch.empty((M, p[0].N), dtype=dt, device=dev) for p in projs]
-        for q, y in zip(arr, outs):
-            q.Y = y.data_ptr()
-    nbytes = L.fmsa_lora_few_workspace(arr, n, M)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
-    _check("fmsa_lora_few_fwd",
-           L.fmsa_lora_few_fwd(arr, n, x2d.data_ptr(), x2d.stride(0), M, mode, _ptr(h), 0 if h is None else h.stride(0),
-                               act_enum(dt), _ptr(ws), nbytes, _stream(x2d)))
-    return outs
+    return (_native or native()).lora_few(x2d, projs, mode)
 
 
 def gptq_lora_fwd_splits(weights, M: int) -> bool:
@@ -651,31 +579,7 @@ def gptq_lora_bwd_dx(projs: Sequence[dict], M: int, K: int, mode: int = BWD_LINE
     g <- d_e and returns h.
     split=True lets a call on the twins cut tiles that do not fill the chip along the contraction (another, still fixed,
     order of the fp32 sums: the checkpoint layout's results, which run whole, then differ in their last bits)."""
-    arr = (BwdProj * len(projs))()
-    ref = projs[0]["dY"]
-    for i, p in enumerate(projs):
-        dy = p["dY"]
-        assert dy.stride(1) == 1
-        ms = p.get("mask_src")
-        T = p.get("T") if p["r"] else None
-        assert T is None or T.stride(1) == 1
-        arr[i] = BwdProj(p["w"], _ptr(p["nsz"]), _ptr(dy), dy.stride(0), _ptr(T), 0 if T is None else T.stride(0),
-                         _ptr(p.get("At")) if p["r"] else None, _ptr(ms), 0 if ms is None else ms.stride(0),
-                         int(p["r"]), float(p["s"] or 0.0), _ptr(p.get("qweight_t")), _ptr(p.get("scale_f32")),
-                         _ptr(p.get("negzp_f16")))
-    nbytes = lib().fmsa_gptq_lora_bwd_dx_workspace(arr, len(projs), M, act_enum(ref.dtype)) if split else 0
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=ref.device) if nbytes else None
-    if mode == BWD_SWIGLU:
-        h = torch.empty_like(e)
-        _check("fmsa_gptq_lora_bwd_dx_ws",
-               lib().fmsa_gptq_lora_bwd_dx_ws(arr, len(projs), M, mode, None, 0, _ptr(e), _ptr(g), _ptr(h), e.stride(0),
-                                              act_enum(ref.dtype), _ptr(ws), nbytes, _stream(ref)))
-        return h
-    dx = torch.empty((M, K), dtype=ref.dtype, device=ref.device)
-    _check("fmsa_gptq_lora_bwd_dx_ws",
-           lib().fmsa_gptq_lora_bwd_dx_ws(arr, len(projs), M, mode, _ptr(dx), dx.stride(0), None, None, None, 0,
-                                          act_enum(ref.dtype), _ptr(ws), nbytes, _stream(ref)))
-    return dx
+    return (_native or native()).gptq_lora_bwd_dx(projs, M, K, mode, e, g, split)
 
 
 def dx_twin_enabled() -> bool:
@@ -769,33 +673,7 @@ def lora_pack_batch(adapters, act_dtype):
     parameters).  Returns one (A16 [r, K], At16 [K, r], B16 [N, r], Bt16 [r, N]) per adapter in `act_dtype`,
     from one launch per LORA_PACK_MAX_JOBS adapters.  `A16_out` (contiguous [r, K]) lets the caller place A16
     inside a larger stacked matrix."""
-    outs, jobs = [], []
-    for A, B, A16_out in adapters:
-        if not (A.is_cuda and B.is_cuda):
-            raise RuntimeError("fmsa_hip needs GPU tensors")
-        if A.dtype != B.dtype:
-            B = B.detach().to(A.dtype)
-        A = A if A.is_contiguous() else A.detach().contiguous()
-        B = B if B.is_contiguous() else B.detach().contiguous()
-        r, K = A.shape
-        N = B.shape[0]
-        # an allocation each: four cost the host less than one and its four views
-        dev = A.device
-        if A16_out is None:
-            A16_out = torch.empty((r, K), dtype=act_dtype, device=dev)
-        else:
-            assert A16_out.shape == (r, K) and A16_out.is_contiguous() and A16_out.dtype == act_dtype
-        At16 = torch.empty((K, r), dtype=act_dtype, device=dev)
-        B16 = torch.empty((N, r), dtype=act_dtype, device=dev)
-        Bt16 = torch.empty((r, N), dtype=act_dtype, device=dev)
-        outs.append((A16_out, At16, B16, Bt16))
-        jobs.append((A, B, LoraPackJob(_ptr(A), _ptr(B), _ptr(A16_out), _ptr(At16), _ptr(B16), _ptr(Bt16), r, K, N,
-                                       _DTYPE_ENUM[A.dtype])))
-    for i in range(0, len(jobs), LORA_PACK_MAX_JOBS):
-        chunk = jobs[i : i + LORA_PACK_MAX_JOBS]
-        arr = (LoraPackJob * len(chunk))(*[j for _, _, j in chunk])
-        _check("fmsa_lora_pack_batch", lib().fmsa_lora_pack_batch(arr, len(chunk), act_enum(act_dtype), _stream(chunk[0][0])))
-    return outs
+    return (_native or native()).lora_pack_batch(adapters, act_dtype, LORA_PACK_MAX_JOBS)
 
 
 def lora_pack(A, B, act_dtype, A16_out=None):
@@ -805,26 +683,12 @@ def lora_pack(A, B, act_dtype, A16_out=None):
 
 def rms_layernorm_fwd(x2d, weight, eps: float, gemma: bool = False):
     """(Y [M, C] in x2d's dtype, r [M] fp32 = 1 / rms) of an RMS layer norm over the rows of x2d."""
-    if not (x2d.is_cuda and weight.is_cuda):
-        raise RuntimeError("fmsa_hip needs GPU tensors")
-    M, C = x2d.shape
-    assert x2d.stride(1) == 1 and weight.is_contiguous() and weight.numel() == C
-    y = torch.empty((M, C), dtype=x2d.dtype, device=x2d.device)
-    r = torch.empty(M, dtype=torch.float32, device=x2d.device)
-    _check("fmsa_rms_layernorm_fwd",
-           lib().fmsa_rms_layernorm_fwd(_ptr(x2d), x2d.stride(0), _ptr(weight), M, C, float(eps), int(gemma), _DTYPE_ENUM[x2d.dtype],
-                                        _DTYPE_ENUM[weight.dtype], _ptr(y), y.stride(0), _ptr(r), _stream(x2d)))
-    return y, r
+    return (_native or native()).rms_layernorm_fwd(x2d, weight, eps, gemma)
 
 
 def rms_layernorm_bwd(dy2d, x2d, weight, r, gemma: bool = False):
     """Overwrites dy2d with dX and returns it."""
-    M, C = x2d.shape
-    assert dy2d.shape == (M, C) and dy2d.stride(1) == 1 and x2d.stride(1) == 1 and dy2d.dtype == x2d.dtype
-    _check("fmsa_rms_layernorm_bwd",
-           lib().fmsa_rms_layernorm_bwd(_ptr(dy2d), dy2d.stride(0), _ptr(x2d), x2d.stride(0), _ptr(weight), _ptr(r), M, C, int(gemma),
-                                        _DTYPE_ENUM[x2d.dtype], _DTYPE_ENUM[weight.dtype], _stream(x2d)))
-    return dy2d
+    return (_native or native()).rms_layernorm_bwd(dy2d, x2d, weight, r, gemma)
 
 
 def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bool = False, strided: bool = False):
@@ -833,14 +697,7 @@ def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bo
     if strided:
         assert q2d.shape[2:] == (n_heads, head_dim)
         return rope_embedding_strided(q2d, cos2d, sin2d, backward)
-    if not (q2d.is_cuda and cos2d.is_cuda and sin2d.is_cuda):
-        raise RuntimeError("fmsa_hip needs GPU tensors")
-    assert q2d.stride(1) == 1 and cos2d.stride(1) == 1 and cos2d.stride() == sin2d.stride() and cos2d.dtype == sin2d.dtype
-    _check("fmsa_rope_embedding",
-           lib().fmsa_rope_embedding(_ptr(q2d), q2d.stride(0), _ptr(cos2d), _ptr(sin2d), cos2d.stride(0), q2d.shape[0], n_heads,
-                                     head_dim, cos2d.shape[0], int(backward), _DTYPE_ENUM[q2d.dtype], _DTYPE_ENUM[cos2d.dtype],
-                                     _stream(q2d)))
-    return q2d
+    return (_native or native()).rope_embedding_(q2d, cos2d, sin2d, n_heads, head_dim, backward)
 
 
 def rope_strided_ok(q4d, cos2d, sin2d) -> bool:
@@ -854,16 +711,7 @@ def rope_strided_ok(q4d, cos2d, sin2d) -> bool:
 def rope_embedding_strided(q4d, cos2d, sin2d, backward: bool = False):
     """The rotation of q4d [batch, seq, heads, head_dim], any strides (see rope_strided_ok), as contiguous rows
     [batch * seq, heads * head_dim]; row m uses row m % cos2d.shape[0] of cos / sin.  q4d is left alone."""
-    if not (q4d.is_cuda and cos2d.is_cuda and sin2d.is_cuda):
-        raise RuntimeError("fmsa_hip needs GPU tensors")
-    b, t, h, d = q4d.shape
-    assert q4d.stride(3) == 1 and cos2d.stride(1) == 1 and cos2d.stride() == sin2d.stride() and cos2d.dtype == sin2d.dtype
-    out = q4d.new_empty((b * t, h * d))
-    _check("fmsa_rope_embedding_strided",
-           lib().fmsa_rope_embedding_strided(_ptr(q4d), q4d.stride(0), q4d.stride(1), q4d.stride(2), _ptr(out), _ptr(cos2d), _ptr(sin2d),
-                                             cos2d.stride(0), b, t, h, d, cos2d.shape[0], int(backward), _DTYPE_ENUM[q4d.dtype],
-                                             _DTYPE_ENUM[cos2d.dtype], _stream(q4d)))
-    return out
+    return (_native or native()).rope_embedding_strided(q4d, cos2d, sin2d, backward)
 
 
 def cross_entropy_fwd(logits2d, labels):

@@ -18,23 +18,43 @@ def _no_further(few, whole, ref):
     assert err <= 1.02 * base, (float(err), float(base))
 
 
-def _packed(monkeypatch, x, projs, mode):
-    """gptq_lora_fwd on the kernel for few tokens whatever the rule says of the shape."""
+def _packed(x, projs, mode):
+    """What gptq_lora_fwd returns, on the kernel for few tokens whatever the rule says of the shape."""
     import fmsa_hip
 
-    L = fmsa_hip.lib()
-    with monkeypatch.context() as m:
-        m.setattr(L, "fmsa_gptq_lora_fwd_is_few", lambda *a: 1)
-        return fmsa_hip.gptq_lora_fwd(x, projs, mode, split=True)
+    arr, outs = (fmsa_hip.FwdProj * len(projs))(), []
+    for q, p in zip(arr, projs):
+        y = x.new_empty((x.shape[0], p["w"].N))
+        outs.append(y)
+        q.w, q.Y, q.ldy, q.bias = p["w"], y.data_ptr(), y.stride(0), None if p["bias"] is None else p["bias"].data_ptr()
+        if p["r"]:
+            q.U, q.ldu, q.B, q.r, q.s = p["U"].data_ptr(), p["U"].stride(0), p["B"].data_ptr(), p["r"], p["s"]
+    h = torch.empty_like(outs[0]) if mode == fmsa_hip.FWD_SWIGLU else None
+    rc = fmsa_hip.lib().fmsa_gptq_lora_fwd_few(arr, len(projs), x.data_ptr(), x.stride(0), x.shape[0], mode,
+                                               None if h is None else h.data_ptr(), 0 if h is None else h.stride(0),
+                                               fmsa_hip.act_enum(x.dtype), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    return outs if h is None else [*outs, h]
 
 
-def _direct(monkeypatch, x, few, mode):
+def _direct(x, few, mode):
+    """lora_few, whatever the rule says of the shape."""
     import fmsa_hip
 
-    L = fmsa_hip.lib()
-    with monkeypatch.context() as m:
-        m.setattr(L, "fmsa_lora_few_is_few", lambda *a: 1)
-        return fmsa_hip.lora_few(x, few, mode)
+    L, arr, outs = fmsa_hip.lib(), (fmsa_hip.FewProj * len(few))(), []
+    for q, (w, A, B, bias, s) in zip(arr, few):
+        y = x.new_empty((x.shape[0], w.N))
+        outs.append(y)
+        q.w, q.Y, q.ldy, q.bias = w, y.data_ptr(), y.stride(0), None if bias is None else bias.data_ptr()
+        if A is not None:
+            q.A, q.B, q.r, q.s, q.param_dtype = A.data_ptr(), B.data_ptr(), A.shape[0], s, fmsa_hip.F32
+    h = torch.empty_like(outs[0]) if mode == fmsa_hip.FWD_SWIGLU else None
+    ws = torch.empty(max(16, L.fmsa_lora_few_workspace(arr, len(few), x.shape[0])), dtype=torch.uint8, device="cuda")
+    rc = L.fmsa_lora_few_fwd(arr, len(few), x.data_ptr(), x.stride(0), x.shape[0], mode, None if h is None else h.data_ptr(),
+                             0 if h is None else h.stride(0), fmsa_hip.act_enum(x.dtype), ws.data_ptr(), ws.numel(),
+                             torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    return outs if h is None else h
 
 
 def _weights(K, Ns, fmt, gs):
@@ -72,7 +92,7 @@ def _weights(K, Ns, fmt, gs):
     (130, 544, [96, 96], True, "gptq", 64, True, 72),
     (200, 1024, [64], False, "nf4", 64, False, 16),
 ])
-def test_few_tokens(monkeypatch, M, K, Ns, swiglu, fmt, gs, bias, r, dtype):
+def test_few_tokens(M, K, Ns, swiglu, fmt, gs, bias, r, dtype):
     import fmsa_hip
 
     if fmt == "interleaved" and dtype != torch.float16:
@@ -95,13 +115,13 @@ def test_few_tokens(monkeypatch, M, K, Ns, swiglu, fmt, gs, bias, r, dtype):
             ref = ref + s * (x.float() @ A.to(dtype).float().t()) @ B.to(dtype).float().t()
         refs.append(ref if b is None else ref + b.float())
     whole = fmsa_hip.gptq_lora_fwd(x, projs, mode)
-    packed = _packed(monkeypatch, x, projs, mode)
-    direct = _direct(monkeypatch, x, few, mode)
+    packed = _packed(x, projs, mode)
+    direct = _direct(x, few, mode)
     if swiglu:
         refs = refs + [torch.nn.functional.silu(refs[0]) * refs[1]]
     for a, b, ref in zip(packed, whole, refs):
         _no_further(a, b, ref)
-    for a, b in zip(packed, _packed(monkeypatch, x, projs, mode)):
+    for a, b in zip(packed, _packed(x, projs, mode)):
         assert torch.equal(a, b)
     # U of one projection is one lora_down; of several, what their stacked adapters give, whose ranges may be others
     for a, b, ref in zip([direct] if swiglu else direct, packed[2:] if swiglu else packed, refs[2:] if swiglu else refs):

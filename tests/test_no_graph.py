@@ -1,7 +1,8 @@
-"""When the fused operators run without an autograd node: host-side rule, no GPU."""
+"""When the fused operators run without an autograd node, and the autocast state their backward runs under."""
+import pytest
 import torch
 
-from fms_acceleration_foak.autograd import no_graph, run
+from fms_acceleration_foak.autograd import bwd_as_fwd, no_graph, run
 
 
 class _Double(torch.autograd.Function):
@@ -30,3 +31,39 @@ def test_a_node_where_something_can_follow():
         assert seen == [False]
     with torch.inference_mode():
         assert no_graph()
+
+
+@pytest.mark.gpu
+def test_backward_meets_the_autocast_state_of_its_forward():
+    seen = []
+
+    class F(torch.autograd.Function):
+        @staticmethod
+        @torch.amp.custom_fwd(device_type="cuda")
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        @bwd_as_fwd
+        def backward(ctx, dy):
+            seen.append((torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")))
+            return dy
+
+    def state(dtype):
+        return torch.autocast("cuda", dtype=dtype, enabled=dtype is not None)
+
+    off = torch.get_autocast_dtype("cuda")
+    for fwd in (None, torch.float16, torch.bfloat16):
+        for bwd in (None, torch.float16, torch.bfloat16):
+            x = torch.ones(2, device="cuda", requires_grad=True)
+            with state(fwd):
+                y = F.apply(x)
+            with state(bwd):
+                y.backward(torch.ones(2, device="cuda"))
+            assert seen.pop()[0] is (fwd is not None)
+            if fwd is not None:
+                with state(bwd):
+                    ctx = type("Ctx", (), {"_fwd_used_autocast": True, "_dtype": fwd})()
+                    F.backward(ctx, torch.ones(2, device="cuda"))
+                assert seen.pop() == (True, fwd)
+    assert torch.get_autocast_dtype("cuda") == off
