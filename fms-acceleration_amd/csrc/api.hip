@@ -52,10 +52,12 @@ int launch_ce_fwd(const void* logits, int64_t ld, const int64_t* labels, int M, 
                   hipStream_t st);
 int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse, const int64_t* labels, int M,
                   int V, int dtype, int vec, hipStream_t st);
-int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
-                       int dtype, float* losses, float* lse, hipStream_t st);
-int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse,
-                       const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st);
+int ce_rows_parts(int rows, int V);
+int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int64_t label_seq, int n_seq, int seq_in,
+                       int seq_out, int V, int dtype, int parts, float* partial, float* losses, float* lse, int64_t* targets, float* sum,
+                       float* count, int mean, hipStream_t st);
+int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* count,
+                       const float* lse, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st);
 int launch_ce_fused(void* logits, int64_t ld, const int64_t* labels, int M, int V, int dtype, int vec, int64_t ignore_index,
                     const float* scale, float smoothing, float* losses, hipStream_t st);
 int launch_nf4_dequant(const fmsa_nf4_weight* w, int out_dtype, void* out, hipStream_t st);
@@ -702,7 +704,8 @@ int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* l
                                 int dtype, float* losses, float* logsumexp, void* stream) {
   if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
   if (!losses || !logsumexp) return FMSA_ERR_NULL;
-  return launch_ce_rows_fwd(logits, nullptr, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
+  return launch_ce_rows_fwd(logits, nullptr, ld, labels, seq_out, n_seq, seq_in, seq_out, V, dtype, 1, nullptr, losses, logsumexp,
+                            nullptr, nullptr, nullptr, 0, (hipStream_t)stream);
 }
 
 int fmsa_cross_entropy_rows_fwd_keep(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in,
@@ -710,7 +713,8 @@ int fmsa_cross_entropy_rows_fwd_keep(const void* logits, void* kept, int64_t ld,
   if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
   if (!kept || !losses || !logsumexp) return FMSA_ERR_NULL;
   if ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(kept)) & 15u) return FMSA_ERR_ALIGN;
-  return launch_ce_rows_fwd(logits, kept, ld, labels, n_seq, seq_in, seq_out, V, dtype, losses, logsumexp, (hipStream_t)stream);
+  return launch_ce_rows_fwd(logits, kept, ld, labels, seq_out, n_seq, seq_in, seq_out, V, dtype, 1, nullptr, losses, logsumexp,
+                            nullptr, nullptr, nullptr, 0, (hipStream_t)stream);
 }
 
 int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride,
@@ -720,7 +724,35 @@ int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, cons
   if (!grad || !dloss || !logsumexp) return FMSA_ERR_NULL;
   if (dloss_stride < 0) return FMSA_ERR_SHAPE;
   if (reinterpret_cast<uintptr_t>(grad) & 1u) return FMSA_ERR_ALIGN;
-  return launch_ce_rows_bwd(logits, grad, ld, dloss, dloss_stride, logsumexp, labels, n_seq, seq_in, seq_out, V, dtype,
+  return launch_ce_rows_bwd(logits, grad, ld, dloss, dloss_stride, nullptr, logsumexp, labels, n_seq, seq_in, seq_out, V, dtype,
+                            (hipStream_t)stream);
+}
+
+size_t fmsa_causal_lm_loss_workspace(int n_seq, int seq_out, int V) {
+  if (n_seq <= 0 || seq_out <= 0 || V <= 0 || (int64_t)n_seq * seq_out > 0x7fffffff) return 0;
+  const int rows = n_seq * seq_out;
+  return (size_t)2 * ce_rows_parts(rows, V) * rows * sizeof(float);
+}
+
+int fmsa_causal_lm_loss_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int64_t label_stride, int n_seq, int seq_in,
+                            int seq_out, int V, int dtype, int mean, float* loss, float* count, float* logsumexp, int64_t* targets,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = check_ce_rows(logits, ld, labels, n_seq, seq_in, seq_out, V, dtype)) return rc;
+  if (!loss || !count || !logsumexp) return FMSA_ERR_NULL;
+  if (label_stride < 0) return FMSA_ERR_SHAPE;
+  if (kept && ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(kept)) & 15u)) return FMSA_ERR_ALIGN;
+  if (!workspace || workspace_bytes < fmsa_causal_lm_loss_workspace(n_seq, seq_out, V)) return FMSA_ERR_WORKSPACE;
+  if (!aligned16(workspace)) return FMSA_ERR_ALIGN;
+  return launch_ce_rows_fwd(logits, kept, ld, labels, label_stride, n_seq, seq_in, seq_out, V, dtype, ce_rows_parts(n_seq * seq_out, V),
+                            (float*)workspace, nullptr, logsumexp, targets, loss, count, mean != 0, (hipStream_t)stream);
+}
+
+int fmsa_causal_lm_loss_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, const float* count, const float* logsumexp,
+                            const int64_t* targets, int n_seq, int seq_in, int seq_out, int V, int dtype, void* stream) {
+  if (int rc = check_ce_rows(logits, ld, targets, n_seq, seq_in, seq_out, V, dtype)) return rc;
+  if (!grad || !dloss || !count || !logsumexp) return FMSA_ERR_NULL;
+  if (reinterpret_cast<uintptr_t>(grad) & 1u) return FMSA_ERR_ALIGN;
+  return launch_ce_rows_bwd(logits, grad, ld, dloss, 0, count, logsumexp, targets, n_seq, seq_in, seq_out, V, dtype,
                             (hipStream_t)stream);
 }
 

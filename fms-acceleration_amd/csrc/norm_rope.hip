@@ -4,6 +4,8 @@
 // twice (statistics, then output), the second time out of cache.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 // eight consecutive elements of a row as fp32, for the three storage types (tag = fmsa_dtype)
@@ -519,13 +521,15 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(void* __restrict__ logits, 
 
 
 // The causal-LM loss straight on the model's 16-bit logits [sequences, seq_in, V]: rows 0 .. seq_out - 1 of every sequence
-// count (seq_out = seq_in - 1 where the labels are shifted against the logits).  Forward: one read of the logits.
-// Backward: one read, and one write of a gradient of its own, whole: the rows past seq_out and the rows without a label are
-// written as zeros and not read.  Both are bound by HBM.  The widening copy to fp32, the copy that drops every sequence's
-// last row, the pass over the fp32 gradient and its narrowing and padding copies took 1040 us at 1024 x 128256 bf16 (4.2 GB
-// of traffic); the two kernels move 0.55 - 0.79 GB, and 0.18 - 0.26 GB more where the forward keeps the live rows for the
-// backward (KEEP), so that the caller may overwrite the logits in between (loss and gradient of 1024 x 128256, three rows in
-// ten without a label: 159 us a pass where the backward reads the caller's logits, 204 us with the rows kept).
+// count (seq_out = seq_in - 1 where the labels are shifted against the logits).  Forward: one read of the logits, by `parts`
+// workgroups a row; their (max, sum) pairs, the labels, the losses, their sum and the mean meet in a second launch of one
+// workgroup.  Backward: one read, and one write of a gradient of its own, whole: the rows past seq_out and the rows without a
+// label are written as zeros and not read.  Bound by HBM: 0.37 GB forward where the live rows are kept for the backward (KEEP:
+// the caller may overwrite the logits in between) and 0.45 GB backward at 1024 x 128256, three rows in ten without a label,
+// at 5.3 TB/s: 70 us (94 with one workgroup a row) and 83 us; the second launch takes 5 us in the place of eight of torch's
+// (the labels' copy, two counts, sum, quotient, their backward: 29 us).  The logits' loads of KEEP are non-temporal, so
+// that the copy, which the backward reads, and not they stay in the memory-side cache (a pass 184 -> 171 us); non-temporal
+// stores of the gradient and rows taken in the order opposite to the forward's change nothing on top.
 // Rows are walked in 16-byte chunks from the first aligned element on (V need not be a multiple of 8, so every row of a
 // contiguous matrix may begin elsewhere), with four chunks per thread in flight; the ends are element accesses.
 struct RowSpan {
@@ -541,39 +545,53 @@ FMSA_DEVI RowSpan row_span(const uint16_t* x, int V, bool vec) {
 }
 FMSA_DEVI int64_t logits_row(int row, int seq_in, int seq_out) { return (int64_t)(row / seq_out) * seq_in + row % seq_out; }
 
-// KEEP: the live rows also go to `kept`, laid out and aligned (modulo 16) as the logits
+struct CeRowsArgs {
+  const uint16_t* logits;
+  uint16_t* kept;  // KEEP: the live rows, laid out and aligned (modulo 16) as the logits
+  int64_t ld;
+  const int64_t* labels;  // row t of sequence q: labels[q * label_seq + t]
+  int64_t label_seq;
+  int seq_in, seq_out, V, rows, parts;
+  float *pm, *ps;  // [parts][rows]: running maximum and sum of exp(. - maximum) of a part
+  float *losses, *lse;
+  int64_t* targets;  // contiguous labels for the backward, or nullptr
+  float *sum, *count;  // sum of the losses (mean != 0: over the number of labels that are not -100) and that number, or nullptr
+  int mean;
+};
+FMSA_DEVI int64_t row_label(const CeRowsArgs& a, int row) { return a.labels[(row / a.seq_out) * a.label_seq + row % a.seq_out]; }
+
+// blockIdx.x: row; blockIdx.y: part of the row's chunks (the unaligned ends go with the first and last).  Several parts a row
+// where the rows alone leave CUs without work: 1022 rows in 2 parts.
 template <int D, bool KEEP>
-__global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __restrict__ logits, uint16_t* __restrict__ kept, int64_t ld,
-                                                          const int64_t* __restrict__ labels, int seq_in, int seq_out, int V,
-                                                          float* __restrict__ losses, float* __restrict__ lse_out) {
+__global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const CeRowsArgs a) {
   __shared__ float red_m[256], red_s[256];
-  const int row = blockIdx.x, tid = threadIdx.x;
-  const int64_t label = labels[row];
-  if (label < 0 || label >= V) {  // ignored (or a caller error, treated as such): uniform over the workgroup
-    if (tid == 0) losses[row] = lse_out[row] = 0.f;
-    return;
-  }
-  const int64_t row0 = logits_row(row, seq_in, seq_out) * ld;
-  const uint16_t* x = logits + row0;
+  const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x, V = a.V;
+  const int64_t label = row_label(a, row);
+  if (label < 0 || label >= V) return;  // ignored (or a caller error, treated as such): uniform over the workgroup
+  const int64_t row0 = logits_row(row, a.seq_in, a.seq_out) * a.ld;
+  const uint16_t* x = a.logits + row0;
   const RowSpan sp = row_span(x, V, true);
   float m = -INFINITY, s = 0.f;
   auto element = [&](int c) {
     online_add(m, s, load1<D>(x, c));
-    if constexpr (KEEP) kept[row0 + c] = x[c];
+    if constexpr (KEEP) a.kept[row0 + c] = x[c];
   };
-  for (int c = tid; c < sp.head; c += 256) element(c);
-  for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) element(c);
+  if (part == 0)
+    for (int c = tid; c < sp.head; c += 256) element(c);
+  if (part == a.parts - 1)
+    for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) element(c);
   const u32x4* xv = reinterpret_cast<const u32x4*>(x + sp.head);
-  for (int i = tid; i < sp.n_vec; i += 1024) {
+  const int v_begin = (int)((int64_t)sp.n_vec * part / a.parts), v_end = (int)((int64_t)sp.n_vec * (part + 1) / a.parts);
+  for (int i = v_begin + tid; i < v_end; i += 1024) {
     u32x4 w[4];
     float v[4][8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) w[u] = xv[min(i + 256 * u, sp.n_vec - 1)];
+    for (int u = 0; u < 4; ++u) w[u] = KEEP ? __builtin_nontemporal_load(xv + min(i + 256 * u, v_end - 1)) : xv[min(i + 256 * u, v_end - 1)];
     if constexpr (KEEP) {
-      u32x4* kv = reinterpret_cast<u32x4*>(kept + row0 + sp.head);
+      u32x4* kv = reinterpret_cast<u32x4*>(a.kept + row0 + sp.head);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (i + 256 * u < sp.n_vec) kv[i + 256 * u] = w[u];
+        if (i + 256 * u < v_end) kv[i + 256 * u] = w[u];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) Vec8<D>::unpack(w[u], v[u]);
@@ -593,7 +611,7 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __rest
       float acc = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc += __builtin_amdgcn_exp2f((v[u][k] - mn) * kLog2e);
-      s += i + 256 * u < sp.n_vec ? acc : 0.f;
+      s += i + 256 * u < v_end ? acc : 0.f;
     }
     m = mn;
   }
@@ -610,9 +628,54 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const uint16_t* __rest
     __syncthreads();
   }
   if (tid == 0) {
-    const float lse = red_m[0] + __builtin_amdgcn_logf(red_s[0]) * kLn2;
-    lse_out[row] = lse;
-    losses[row] = lse - load1<D>(x, label);
+    a.pm[(size_t)part * a.rows + row] = red_m[0];
+    a.ps[(size_t)part * a.rows + row] = red_s[0];
+  }
+}
+
+// One workgroup: logsumexp and loss of every row (parts in index order), the contiguous copy of the labels, sum and count.
+// (pm, ps may be the lse and losses of a call with one part: a thread reads its row's before it writes them.)
+template <int D>
+__global__ __launch_bounds__(1024) void ce_rows_finish_kernel(const CeRowsArgs a) {
+  __shared__ float red[1024];
+  __shared__ int red_n[1024];
+  const int tid = threadIdx.x;
+  float sum = 0.f;
+  int n = 0;
+  for (int row = tid; row < a.rows; row += 1024) {
+    const int64_t label = row_label(a, row);
+    if (a.targets) a.targets[row] = label;
+    n += label != -100;
+    float lse = 0.f, loss = 0.f;
+    if (label >= 0 && label < a.V) {
+      float m = a.pm[row], s = a.ps[row];
+      for (int part = 1; part < a.parts; ++part) {
+        const float m2 = a.pm[(size_t)part * a.rows + row], s2 = a.ps[(size_t)part * a.rows + row];
+        const float mn = fmaxf(m, m2);
+        s = merge_term(m, s, mn) + merge_term(m2, s2, mn);
+        m = mn;
+      }
+      lse = m + __builtin_amdgcn_logf(s) * kLn2;
+      loss = lse - load1<D>(a.logits + logits_row(row, a.seq_in, a.seq_out) * a.ld, label);
+    }
+    a.lse[row] = lse;
+    if (a.losses) a.losses[row] = loss;
+    sum += loss;
+  }
+  if (!a.sum) return;
+  red[tid] = sum;
+  red_n[tid] = n;
+  __syncthreads();
+  for (int o = 512; o > 0; o >>= 1) {
+    if (tid < o) {
+      red[tid] += red[tid + o];
+      red_n[tid] += red_n[tid + o];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    *a.count = a.mean ? (float)red_n[0] : 1.0f;
+    *a.sum = a.mean ? red[0] / (float)red_n[0] : red[0];
   }
 }
 
@@ -621,7 +684,7 @@ constexpr int CE_CHUNKS = 4;  // 16-byte chunks per thread of the backward
 // grad has the logits' shape, row stride and alignment modulo 16 (vec; otherwise element accesses)
 template <int D>
 __global__ __launch_bounds__(256) void ce_rows_bwd_kernel(const uint16_t* __restrict__ logits, uint16_t* __restrict__ grad, int64_t ld,
-                                                          const float* __restrict__ dloss, int64_t dloss_stride,
+                                                          const float* __restrict__ dloss, int64_t dloss_stride, const float* __restrict__ count,
                                                           const float* __restrict__ lse, const int64_t* __restrict__ labels, int seq_in,
                                                           int seq_out, int V, int vec) {
   const int seq = blockIdx.x / seq_in, t = blockIdx.x % seq_in;
@@ -630,7 +693,8 @@ __global__ __launch_bounds__(256) void ce_rows_bwd_kernel(const uint16_t* __rest
   const int row = seq * seq_out + t;
   const int64_t label = t < seq_out ? labels[row] : -100;
   const bool live = label >= 0 && label < V;  // uniform over the workgroup
-  const float dl = live ? dloss[(int64_t)row * dloss_stride] : 0.f;
+  float dl = live ? dloss[(int64_t)row * dloss_stride] : 0.f;
+  if (live && count) dl /= *count;
   const float l = live ? lse[row] : 0.f;
   const RowSpan sp = row_span(x, V, vec != 0);
   auto element = [&](int c) {
@@ -800,25 +864,46 @@ int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_st
   return FMSA_OK;
 }
 
-int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
-                       int dtype, float* losses, float* lse, hipStream_t st) {
-  const dim3 grid(n_seq * seq_out), block(256);
-  const uint16_t* x = (const uint16_t*)logits;
-  uint16_t* k = (uint16_t*)kept;
-#define ROWS_FWD(D, KEEP) hipLaunchKernelGGL((ce_rows_fwd_kernel<D, KEEP>), grid, block, 0, st, x, k, ld, labels, seq_in, seq_out, V, losses, lse)
-  if (dtype == FMSA_BF16) {
-    if (k) ROWS_FWD(FMSA_BF16, true);
-    else ROWS_FWD(FMSA_BF16, false);
-  } else {
-    if (k) ROWS_FWD(FMSA_F16, true);
-    else ROWS_FWD(FMSA_F16, false);
-  }
+int ce_rows_parts(int rows, int V) { return std::max(1, std::min(2048 / rows, V / 8192)); }
+
+// parts = 1: the losses and lse of the rows serve as the parts' pairs; otherwise `partial` [2][parts][rows]
+int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int64_t label_seq, int n_seq, int seq_in,
+                       int seq_out, int V, int dtype, int parts, float* partial, float* losses, float* lse, int64_t* targets, float* sum,
+                       float* count, int mean, hipStream_t st) {
+  CeRowsArgs a{};
+  a.logits = (const uint16_t*)logits;
+  a.kept = (uint16_t*)kept;
+  a.ld = ld;
+  a.labels = labels;
+  a.label_seq = label_seq;
+  a.seq_in = seq_in;
+  a.seq_out = seq_out;
+  a.V = V;
+  a.rows = n_seq * seq_out;
+  a.parts = parts;
+  a.pm = partial ? partial : lse;
+  a.ps = partial ? partial + (size_t)parts * a.rows : losses;
+  a.losses = losses;
+  a.lse = lse;
+  a.targets = targets;
+  a.sum = sum;
+  a.count = count;
+  a.mean = mean;
+  const dim3 grid(a.rows, parts), block(256);
+#define ROWS_FWD(D)                                                                          \
+  do {                                                                                       \
+    if (kept) hipLaunchKernelGGL((ce_rows_fwd_kernel<D, true>), grid, block, 0, st, a);       \
+    else hipLaunchKernelGGL((ce_rows_fwd_kernel<D, false>), grid, block, 0, st, a);           \
+    hipLaunchKernelGGL((ce_rows_finish_kernel<D>), dim3(1), dim3(1024), 0, st, a);            \
+  } while (0)
+  if (dtype == FMSA_BF16) ROWS_FWD(FMSA_BF16);
+  else ROWS_FWD(FMSA_F16);
 #undef ROWS_FWD
   FMSA_CHECK_LAUNCH();
   return FMSA_OK;
 }
 
-int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* lse,
+int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, int64_t dloss_stride, const float* count, const float* lse,
                        const int64_t* labels, int n_seq, int seq_in, int seq_out, int V, int dtype, hipStream_t st) {
   const int per_block = 256 * CE_CHUNKS * 8;
   const dim3 grid(n_seq * seq_in, (V + per_block - 1) / per_block), block(256);
@@ -826,9 +911,9 @@ int launch_ce_rows_bwd(const void* logits, void* grad, int64_t ld, const float* 
   uint16_t* g = (uint16_t*)grad;
   const int vec = ((reinterpret_cast<uintptr_t>(x) ^ reinterpret_cast<uintptr_t>(g)) & 15) == 0;
   if (dtype == FMSA_BF16)
-    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_BF16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, lse, labels, seq_in, seq_out, V, vec);
+    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_BF16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, count, lse, labels, seq_in, seq_out, V, vec);
   else
-    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_F16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, lse, labels, seq_in, seq_out, V, vec);
+    hipLaunchKernelGGL((ce_rows_bwd_kernel<FMSA_F16>), grid, block, 0, st, x, g, ld, dloss, dloss_stride, count, lse, labels, seq_in, seq_out, V, vec);
   FMSA_CHECK_LAUNCH();
   return FMSA_OK;
 }

@@ -9,6 +9,8 @@ import torch
 
 import fmsa_hip
 
+from ...autograd import run
+
 
 class Fast_CrossEntropyLoss(torch.autograd.Function):
     @staticmethod
@@ -28,24 +30,22 @@ class Fast_CrossEntropyLoss(torch.autograd.Function):
 
 
 class Fast_CausalLMLossRows(torch.autograd.Function):
-    """Losses of rows 0 .. seq_out - 1 of every sequence, read from the 16-bit logits where they are; the gradient is a
-    tensor of its own, so the logits stay as the caller sees them.  keep (a backward may follow): the forward leaves the
-    rows it read in a copy for the backward, so the caller may overwrite the logits before it, as with the fp32 copy of
-    the general way."""
+    """Sum (mean: over the labels that are not -100) of the losses of rows 0 .. seq_out - 1 of every sequence, read from the
+    16-bit logits where they are; the gradient is a tensor of its own, so the logits stay as the caller sees them.  keep (a
+    backward may follow): the forward leaves the rows it read and their labels in copies for the backward, so the caller may
+    overwrite both before it, as with the fp32 copy of the general way."""
 
     @staticmethod
-    def forward(ctx, logits, labels, seq_out, keep):
-        if not keep:
-            return fmsa_hip.cross_entropy_rows_fwd(logits, labels, seq_out)[0]
-        losses, logsumexp, kept = fmsa_hip.cross_entropy_rows_fwd_keep(logits, labels, seq_out)
-        ctx.save_for_backward(kept, logsumexp, labels)
-        ctx.seq_out = seq_out
-        return losses
+    def forward(ctx, logits, labels, label_stride, seq_out, mean, keep):
+        loss, saved = fmsa_hip.causal_lm_loss_fwd(logits, labels, label_stride, seq_out, mean, keep)
+        if keep:
+            ctx.save_for_backward(*saved)
+            ctx.seq_out = seq_out
+        return loss
 
     @staticmethod
-    def backward(ctx, dlosses):
-        kept, logsumexp, labels = ctx.saved_tensors
-        return fmsa_hip.cross_entropy_rows_bwd(kept, dlosses.float(), logsumexp, labels, ctx.seq_out), None, None, None
+    def backward(ctx, dloss):
+        return fmsa_hip.causal_lm_loss_bwd(*ctx.saved_tensors, dloss.float(), ctx.seq_out), None, None, None, None, None
 
 
 def _rows_in_place(logits, labels, vocab_size, shifted):
@@ -82,11 +82,18 @@ def FastForCausalLMLoss(logits, labels, vocab_size: int, num_items_in_batch: int
     if ignore_index == -100 and _rows_in_place(logits, labels if shift_labels is None else shift_labels, vocab_size, shift_labels is not None):
         # the fp32 copy, the shifted copy and their gradients' copies cost five times the two kernels
         seq_out = logits.shape[1] - (shift_labels is None)
-        target = labels[:, 1:] if shift_labels is None else shift_labels
-        target = target.to(device=logits.device, dtype=torch.int64).reshape(-1).contiguous()  # a row of a strided view stays strided
-        loss = Fast_CausalLMLossRows.apply(logits, target, seq_out, torch.is_grad_enabled() and logits.requires_grad)
-        n_items = num_items_in_batch if num_items_in_batch is not None else torch.count_nonzero(target != -100)
-        return loss.sum() / n_items
+        target = labels if shift_labels is None else shift_labels
+        target = target.to(device=logits.device, dtype=torch.int64)
+        if target.shape != logits.shape[:2] or target.stride(1) != 1:
+            target = target.reshape(logits.shape[:2]).contiguous()
+            if target.stride(1) != 1:  # (a single row of a strided view counts as contiguous)
+                target = target.clone(memory_format=torch.contiguous_format)
+        stride = target.stride(0)
+        if shift_labels is None:
+            target = target[:, 1:]  # the kernel reads the labels where they are, one token on
+        loss = run(Fast_CausalLMLossRows, logits, target, stride, seq_out, num_items_in_batch is None,
+                   torch.is_grad_enabled() and logits.requires_grad)
+        return loss if num_items_in_batch is None else loss / num_items_in_batch
     logits = logits.float()
     if shift_labels is None:
         labels = labels.to(logits.device)

@@ -73,6 +73,9 @@ EXPORTED_SYMBOLS = (
     "fmsa_cross_entropy_rows_fwd",
     "fmsa_cross_entropy_rows_fwd_keep",
     "fmsa_cross_entropy_rows_bwd",
+    "fmsa_causal_lm_loss_workspace",
+    "fmsa_causal_lm_loss_fwd",
+    "fmsa_causal_lm_loss_bwd",
     "fmsa_cross_entropy_fused",
 )
 
@@ -316,6 +319,12 @@ def lib() -> ctypes.CDLL:
                                                    c_void_p, c_void_p]
     L.fmsa_cross_entropy_rows_bwd.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                               c_int, c_void_p]
+    L.fmsa_causal_lm_loss_workspace.restype = c_size_t
+    L.fmsa_causal_lm_loss_workspace.argtypes = [c_int, c_int, c_int]
+    L.fmsa_causal_lm_loss_fwd.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                                          c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]
+    L.fmsa_causal_lm_loss_bwd.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                          c_int, c_void_p]
     L.fmsa_cross_entropy_fused.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_int64, c_void_p, c_float, c_void_p, c_void_p]
     for name in EXPORTED_SYMBOLS:
         getattr(L, name)  # AttributeError here means the library is stale: rebuild it
@@ -751,22 +760,6 @@ def cross_entropy_rows_fwd(logits3d, labels, seq_out: int):
     return losses, lse
 
 
-def cross_entropy_rows_fwd_keep(logits3d, labels, seq_out: int):
-    """(losses, logsumexp, kept): cross_entropy_rows_fwd that leaves the rows with a label in a tensor of its own too, for a
-    backward that must not depend on what the caller does to the logits in the meantime."""
-    n_seq, seq_in, V = logits3d.shape
-    rows = n_seq * seq_out
-    assert logits3d.is_contiguous() and labels.dtype == torch.int64 and labels.is_contiguous() and labels.numel() == rows
-    losses = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
-    lse = torch.empty(rows, dtype=torch.float32, device=logits3d.device)
-    offset = logits3d.data_ptr() % 16 // logits3d.element_size()  # a row begins where it does in the logits, modulo 16 bytes
-    kept = logits3d.new_empty(offset + logits3d.numel())[offset:].view(logits3d.shape)
-    _check("fmsa_cross_entropy_rows_fwd_keep",
-           lib().fmsa_cross_entropy_rows_fwd_keep(_ptr(logits3d), _ptr(kept), V, _ptr(labels), n_seq, seq_in, seq_out, V,
-                                                  act_enum(logits3d.dtype), _ptr(losses), _ptr(lse), _stream(logits3d)))
-    return losses, lse, kept
-
-
 def cross_entropy_rows_bwd(logits3d, dlosses, lse, labels, seq_out: int):
     """Gradient of cross_entropy_rows_fwd's losses, a tensor of its own; dlosses fp32 (any stride, 0 included)."""
     n_seq, seq_in, V = logits3d.shape
@@ -775,6 +768,42 @@ def cross_entropy_rows_bwd(logits3d, dlosses, lse, labels, seq_out: int):
     _check("fmsa_cross_entropy_rows_bwd",
            lib().fmsa_cross_entropy_rows_bwd(_ptr(logits3d), _ptr(grad), V, _ptr(dlosses), dlosses.stride(0), _ptr(lse), _ptr(labels),
                                              n_seq, seq_in, seq_out, V, act_enum(logits3d.dtype), _stream(logits3d)))
+    return grad
+
+
+def causal_lm_loss_fwd(logits3d, labels, label_stride: int, seq_out: int, mean: bool, keep: bool):
+    """(loss, saved): the sum (mean: over the labels that are not -100) of cross_entropy_rows_fwd's losses of contiguous 16-bit
+    logits [n_seq, seq_in, V], a scalar; label of row t of sequence q: element q * label_stride + t of the int64 `labels`.
+    saved, with keep: what causal_lm_loss_bwd takes, none of it the caller's (the rows with a label are copied, so that the
+    logits may be overwritten before the backward)."""
+    n_seq, seq_in, V = logits3d.shape
+    rows, dev = n_seq * seq_out, logits3d.device
+    assert logits3d.is_contiguous() and labels.dtype == torch.int64 and labels.is_cuda
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    count = torch.empty((), dtype=torch.float32, device=dev)
+    lse = torch.empty(rows, dtype=torch.float32, device=dev)
+    targets = kept = None
+    if keep:
+        targets = torch.empty(rows, dtype=torch.int64, device=dev)
+        offset = logits3d.data_ptr() % 16 // logits3d.element_size()  # a row begins where it does in the logits, modulo 16 bytes
+        kept = logits3d.new_empty(offset + logits3d.numel())[offset:].view(logits3d.shape)
+    nbytes = lib().fmsa_causal_lm_loss_workspace(n_seq, seq_out, V)
+    ws = _workspace(nbytes, dev)
+    _check("fmsa_causal_lm_loss_fwd",
+           lib().fmsa_causal_lm_loss_fwd(_ptr(logits3d), _ptr(kept), V, _ptr(labels), int(label_stride), n_seq, seq_in, seq_out, V,
+                                         act_enum(logits3d.dtype), int(mean), _ptr(loss), _ptr(count), _ptr(lse), _ptr(targets), _ptr(ws),
+                                         ws.numel(), _stream(logits3d)))
+    return loss, (kept, lse, targets, count) if keep else None
+
+
+def causal_lm_loss_bwd(kept, lse, targets, count, dloss, seq_out: int):
+    """Gradient of causal_lm_loss_fwd's logits, a tensor of its own; dloss an fp32 scalar on the GPU."""
+    n_seq, seq_in, V = kept.shape
+    assert dloss.dtype == torch.float32 and dloss.numel() == 1 and dloss.is_cuda
+    grad = torch.empty_like(kept)
+    _check("fmsa_causal_lm_loss_bwd",
+           lib().fmsa_causal_lm_loss_bwd(_ptr(kept), _ptr(grad), V, _ptr(dloss), _ptr(count), _ptr(lse), _ptr(targets), n_seq, seq_in, seq_out,
+                                         V, act_enum(kept.dtype), _stream(kept)))
     return grad
 
 

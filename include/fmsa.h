@@ -478,6 +478,19 @@ int fmsa_cross_entropy_rows_bwd(const void* logits, void* grad, int64_t ld, cons
                                 const float* logsumexp, const int64_t* labels, int n_seq, int seq_in, int seq_out, int V,
                                 int dtype, void* stream);
 
+/* The loss itself, for a caller that wants one number: the sum of those rows' losses (mean != 0: over the number of labels
+ * that are not -100, a NaN where there is none) in `loss`, and in `count` what the backward divides by (1 where mean == 0).
+ * Label of row t of sequence q: labels[q * label_stride + t], so that shifted labels are a pointer into the unshifted ones.
+ * kept (may be NULL) as above; logsumexp [n_seq * seq_out] and targets (a contiguous copy of the labels, may be NULL) serve
+ * the backward, which divides dloss[0] by count[0]. */
+size_t fmsa_causal_lm_loss_workspace(int n_seq, int seq_out, int V);
+int fmsa_causal_lm_loss_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int64_t label_stride, int n_seq,
+                            int seq_in, int seq_out, int V, int dtype, int mean, float* loss, float* count, float* logsumexp,
+                            int64_t* targets, void* workspace, size_t workspace_bytes, void* stream);
+int fmsa_causal_lm_loss_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, const float* count,
+                            const float* logsumexp, const int64_t* targets, int n_seq, int seq_in, int seq_out, int V, int dtype,
+                            void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Loss and logits gradient in one launch, for a loss head that consumes its logits chunk by chunk
  * (fused_ops/liger_ce/cross_entropy.py:33-186, called from

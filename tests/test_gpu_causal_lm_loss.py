@@ -117,3 +117,35 @@ def test_logits_overwritten_before_the_backward(b, s, V, offset, shifted, dtype)
     assert torch.equal(*grads) and bool((grads[0] != 0).any())
     with torch.no_grad():  # nothing is kept where no backward can follow
         assert torch.equal(FastForCausalLMLoss(store[offset:].view(b, s, V), labels, V, **kw), loss)
+
+
+@pytest.mark.parametrize("rows,V", [(1, 16384), (3, 24579), (1500, 8192), (40, 16390)])
+@pytest.mark.parametrize("mean", [True, False])
+def test_parts_of_a_row_and_the_sum(rows, V, mean):
+    """Rows cut into parts (chunks that do not divide evenly, ends on the first and last), more rows than the second launch has
+    threads, labels read in place through their stride: against fp64."""
+    import fmsa_hip
+
+    x = randn((1, rows + 1, V), V, torch.bfloat16, scale=2.0).cuda()
+    store = torch.randint(0, V, (2, 2 * rows + 2), generator=torch.Generator().manual_seed(rows)).cuda()
+    labels = store[:1, : rows + 1]
+    labels[0, 1::5] = -100
+    if rows > 2:
+        labels[0, 3] = V + 5  # no row of the loss, but counted as a label
+    loss, (kept, lse, targets, count) = fmsa_hip.causal_lm_loss_fwd(x, labels[:, 1:], labels.stride(0), rows, mean, True)
+    want = labels[0, 1:].clone()
+    live = (want >= 0) & (want < V)
+    exact = x[0, :rows].double()
+    total = (exact.logsumexp(-1) - exact.gather(1, want.clamp(0, V - 1)[:, None])[:, 0])[live].sum()
+    n = int((want != -100).sum()) if mean else 1
+    assert torch.equal(targets, want) and count.item() == n
+    # fp32: a sum of V exponentials each good to 1e-6, then a sum of the rows
+    assert (n == 0 and loss.isnan()) or abs(loss.item() - total.item() / n) <= 1e-5 * max(1.0, abs(total.item() / n))
+    labels.fill_(0)
+    x.fill_(0)
+    grad = fmsa_hip.causal_lm_loss_bwd(kept, lse, targets, count, torch.tensor(3.0, device="cuda"), rows)
+    p = exact.softmax(-1)
+    p[torch.arange(rows, device="cuda")[live], want[live]] -= 1.0
+    ref = torch.where(live[:, None], p * (3.0 / max(n, 1)), torch.zeros_like(p))
+    assert bool((grad[0, rows] == 0).all())
+    assert bool(((grad[0, :rows].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-9).all())
