@@ -123,7 +123,7 @@ struct LoraDownJobDev {
 };
 struct LoraDownArgs {
   LoraDownJobDev j[FMSA_LORA_DOWN_MAX_JOBS];
-  int M;
+  int M, r_max;
 };
 FMSA_DEVI LoraDownJobDev select_down_job(const LoraDownArgs& a, int q) { return q == 0 ? a.j[0] : (q == 1 ? a.j[1] : a.j[2]); }
 
@@ -133,6 +133,122 @@ __global__ __launch_bounds__(64 * NW) void lora_down_batch_kernel(const LoraDown
   if ((int)blockIdx.y >= J.n_split) return;
   lora_down_tile<T, RT, MTL, NW>(J.X, J.ldx, J.Wd, a.M, J.C, J.r, J.out, J.ldo, J.partial, J.n_split);
 }
+
+// ---- lora_down, a few hundred tokens ---------------------------------------------------------------------
+// Between the few tokens of a generation step and the thousands that fill the chip by themselves, the fragment kernel above is
+// bound by the address path of its loads: a fragment's four rows in every four lanes go one by one, 16 bytes per clock and CU,
+// and every 16 tokens read all of Wd that way.  Here a workgroup owns 64 tokens and 64 ranks at most; its four waves take the
+// 64-wide chunks of the columns in turn, each through LDS of its own (no barrier: direct loads of 8 rows x 128 bytes, slot s
+// of row i holding the 16 bytes s ^ ((i >> 1) & 7), two chunks in flight), and their sums meet in LDS in wave order.  Columns are
+// split over workgroups as in the kernels around it; ranks above 64 are further workgroups.
+constexpr int LM_NW = 4, LM_MT = 4;  // waves; 16-token tiles
+constexpr int lm_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }  // s_waitcnt operand: vmcnt(n) only, n < 64
+
+template <typename T, int RT>
+__global__ __launch_bounds__(64 * LM_NW) void lora_down_mid_kernel(const LoraDownArgs a) {
+  // one array per buffer, so that the compiler's wait counts tell reads of one from loads in flight into the other
+  __shared__ __attribute__((aligned(1024))) uint16_t b0[LM_NW * (LM_MT + RT) * 1024];
+  __shared__ __attribute__((aligned(1024))) uint16_t b1[LM_NW * (LM_MT + RT) * 1024];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, kq = lane >> 4;
+  const int rank_blocks = (a.r_max + 63) / 64;
+  const LoraDownJobDev J = select_down_job(a, blockIdx.z / rank_blocks);
+  const int r0 = 64 * (blockIdx.z % rank_blocks);
+  if ((int)blockIdx.y >= J.n_split || r0 >= J.r) return;
+  const int m0 = blockIdx.x * (16 * LM_MT), C = J.C;
+  const int rows = min(16 * LM_MT, a.M - m0), ranks = min(64, J.r - r0);
+  const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(J.X + (size_t)m0 * J.ldx, (size_t)rows * J.ldx * 2);
+  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(J.Wd + (size_t)r0 * C, (size_t)ranks * C * 2);
+  // the lane's 16 bytes of row 8 i + (lane >> 3): chunk piece (lane & 7) ^ ((row >> 1) & 7); rows 16 apart share it
+  uint32_t x_off[2], w_off[2], piece[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    piece[i] = 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    x_off[i] = (uint32_t)((row * J.ldx + piece[i]) * 2);
+    w_off[i] = (uint32_t)((row * (int64_t)C + piece[i]) * 2);
+  }
+  const uint32_t x_tile = (uint32_t)(16 * J.ldx * 2), w_tile = (uint32_t)(16 * (int64_t)C * 2);
+  uint32_t frag[2];  // the lane's fragment of a tile's 32-wide half t
+#pragma unroll
+  for (int t = 0; t < 2; ++t) frag[t] = (uint32_t)(c * 128 + 16 * ((4 * t + kq) ^ ((c >> 1) & 7)));
+  const int n_chunks = (C + 63) / 64, n_slices = J.n_split * LM_NW, slice = blockIdx.y * LM_NW + wave;
+  const int n_it = (n_chunks + n_slices - 1) / n_slices;
+  f32x4 acc[LM_MT][RT];
+#pragma unroll
+  for (int u = 0; u < LM_MT; ++u)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // columns past C (and chunks past the wave's last) are out of range by their lane offsets: zeros, and no traffic
+  auto load = [&](int it, uint16_t* buf) {
+    const int col = 64 * (slice + n_slices * it);
+    char* dst = reinterpret_cast<char*>(buf) + wave * ((LM_MT + RT) * 2048);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t dead = col + (int)piece[i] < C ? 0u : 0x80000000u;
+#pragma unroll
+      for (int u = 0; u < LM_MT; ++u)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (__attribute__((address_space(3))) void*)(dst + u * 2048 + i * 1024), 16,
+                                                 (x_off[i] + u * x_tile) | dead, (uint32_t)col * 2, 0, 2);
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (__attribute__((address_space(3))) void*)(dst + (LM_MT + t) * 2048 + i * 1024), 16,
+                                                 (w_off[i] + t * w_tile) | dead, (uint32_t)col * 2, 0, 0);
+    }
+  };
+  auto multiply = [&](const uint16_t* buf) {
+    __builtin_amdgcn_s_waitcnt(lm_vmcnt(2 * (LM_MT + RT)));  // the other buffer's loads are younger
+    __builtin_amdgcn_sched_barrier(0);
+    const char* src = reinterpret_cast<const char*>(buf) + wave * ((LM_MT + RT) * 2048);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4 xf[LM_MT];
+#pragma unroll
+      for (int u = 0; u < LM_MT; ++u) xf[u] = *reinterpret_cast<const u32x4*>(src + u * 2048 + frag[h]);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const u32x4 wf = *reinterpret_cast<const u32x4*>(src + (LM_MT + t) * 2048 + frag[h]);
+#pragma unroll
+        for (int u = 0; u < LM_MT; ++u) acc[u][t] = mfma16<T>(xf[u], wf, acc[u][t]);  // D[i = token][j = rank]
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the fragments have arrived before the buffer is loaded again
+  };
+  load(0, b0);
+  load(1, b1);
+  for (int it = 0; it < n_it; it += 2) {
+    multiply(b0);
+    load(it + 2, b0);
+    multiply(b1);
+    load(it + 3, b1);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the surplus direct loads, every wave's
+  __syncthreads();
+  float(*red)[LM_MT][RT][64][4] = reinterpret_cast<float(*)[LM_MT][RT][64][4]>(b0);
+#pragma unroll
+  for (int u = 0; u < LM_MT; ++u)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) *reinterpret_cast<f32x4*>(red[wave][u][t][lane]) = acc[u][t];
+  __syncthreads();
+  // wave = token tile: lane holds D[4 kq + i][c] of every rank tile
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    f32x4 v = *reinterpret_cast<const f32x4*>(red[0][wave][t][lane]);
+#pragma unroll
+    for (int w = 1; w < LM_NW; ++w) v += *reinterpret_cast<const f32x4*>(red[w][wave][t][lane]);
+    const int j = r0 + 16 * t + c;
+    if (j >= J.r) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + 16 * wave + 4 * kq + i;
+      if (m >= a.M) continue;
+      if (J.partial)
+        J.partial[((size_t)blockIdx.y * a.M + m) * J.r + j] = v[i];
+      else
+        J.out[(size_t)m * J.ldo + j] = pack1<T>(v[i]);
+    }
+  }
+}
+static_assert(LM_MT == LM_NW, "one token tile of the sums per wave");
 
 // ---- lora_down, staged ----------------------------------------------------------------------------
 // The same product for the large-M case, with X going through LDS: a direct load of one wave moves a
@@ -501,6 +617,7 @@ __global__ __launch_bounds__(256) void lora_down_reduce_kernel(const float* __re
 template <typename T>
 __global__ __launch_bounds__(256) void lora_down_reduce_batch_kernel(const LoraDownArgs a) {
   const LoraDownJobDev J = select_down_job(a, blockIdx.y);
+  if (!J.partial) return;  // rounded by the first launch
   lora_down_reduce<T>(J.partial, J.n_split, a.M, J.r, J.out, J.ldo);
 }
 
@@ -523,7 +640,7 @@ struct LoraGradJobDev {
   const uint16_t* L;
   const uint16_t* R;
   void* out;
-  float* partial;  // [splits][r][C] of this job
+  float* partial;  // [splits][r][C] of this job, or [splits][C][r] where the output is transposed
   int64_t ldl, ldr;
   int C, r, splits, rows_per_split;
   int block_start;   // first workgroup of the job in pass 1
@@ -715,30 +832,32 @@ __global__ __launch_bounds__(512) void lora_grad_partial_kernel(const LoraGradAr
     __syncthreads();
   }
   if (n_tiles > 0) flush_t(n_tiles - 1);
-  // lane holds D[c = 4*kg + i][j = l16]: four consecutive columns -> one 16-byte store
+  // lane holds D[c = 4*kg + i][j = l16]: four consecutive columns -> one 16-byte store, or, for a transposed output, its
+  // rank of four columns (16 lanes: 64 bytes of a column's row of ranks)
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
     const int c = c0 + 32 * wave + 16 * g + 4 * kg;
-    if (c >= C) continue;
+    if (c >= C) continue;  // C % 8 == 0: the four columns are inside
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       const int j = 16 * t + l16;
       if (j >= r) continue;
-      float* dst = partial + ((size_t)split * r + j) * C + c;
-      if (c + 4 <= C) {
-        *reinterpret_cast<f32x4*>(dst) = acc[g][t];
+      if (J.transpose_out) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) partial[((size_t)split * C + c + i) * r + j] = acc[g][t][i];
       } else {
-        for (int i = 0; i < 4; ++i)
-          if (c + i < C) dst[i] = acc[g][t][i];
+        *reinterpret_cast<f32x4*>(partial + ((size_t)split * r + j) * C + c) = acc[g][t];
       }
     }
   }
 }
 
+// Four elements of the output per thread, in the output's order (which the partial sums are in too: the transposed outputs
+// were written 4 bytes at a time, r elements apart, 10.5 us where the sums of q, k, v at rank 64 and 1100 tokens now take 6).
 __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGradArgs a) {
   const LoraGradJobDev J = select_job<true>(a, blockIdx.x);
   const int r = J.r, C = J.C;
-  const int nb_grad = (r * C + 255) / 256;
+  const int nb_grad = (r * C / 4 + 255) / 256;
   const int lb = blockIdx.x - J.rblock_start;
   if (lb >= nb_grad) {  // the job's T: column blocks added in index order, one rounding; four ranks per thread
     const int64_t ti = ((int64_t)(lb - nb_grad) * 256 + threadIdx.x) * 4;
@@ -765,27 +884,40 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGradArg
     *reinterpret_cast<u32x2*>(J.T + (size_t)m * J.ldt + j) = pk;
     return;
   }
-  const int idx = lb * 256 + threadIdx.x;  // over r*C, c fastest
+  const int idx = 4 * (lb * 256 + threadIdx.x);
   if (idx >= r * C) return;
-  const int j = idx / C, c = idx % C;
-  const float* src = J.partial + (size_t)j * C + c;
+  const float* src = J.partial + idx;
   const size_t step = (size_t)r * C;
-  float v = 0.f;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
   int sp = 0;
   for (; sp + 8 <= J.splits; sp += 8) {  // eight loads in flight, summed in index order
-    float p[8];
+    f32x4 p[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) p[k] = src[(size_t)(sp + k) * step];
+    for (int k = 0; k < 8; ++k) p[k] = *reinterpret_cast<const f32x4*>(src + (size_t)(sp + k) * step);
 #pragma unroll
     for (int k = 0; k < 8; ++k) v += p[k];
   }
-  for (; sp < J.splits; ++sp) v += src[(size_t)sp * step];
+#pragma unroll 4
+  for (; sp < J.splits; ++sp) v += *reinterpret_cast<const f32x4*>(src + (size_t)sp * step);
   v *= J.scale;
-  const size_t o = J.transpose_out ? ((size_t)c * r + j) : (size_t)idx;
-  if (J.out_dtype == FMSA_F32)
-    reinterpret_cast<float*>(J.out)[o] = v;
-  else
-    reinterpret_cast<uint16_t*>(J.out)[o] = J.out_dtype == FMSA_BF16 ? pack1<bf16_t>(v) : pack1<f16_t>(v);
+  const bool aligned = reinterpret_cast<uintptr_t>(J.out) % 16 == 0;
+  if (J.out_dtype == FMSA_F32) {
+    float* out = reinterpret_cast<float*>(J.out) + idx;
+    if (aligned) {
+      *reinterpret_cast<f32x4*>(out) = v;
+    } else {
+      for (int i = 0; i < 4; ++i) out[i] = v[i];
+    }
+  } else {
+    uint16_t* out = reinterpret_cast<uint16_t*>(J.out) + idx;
+    const u32x2 o = J.out_dtype == FMSA_BF16 ? u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])}
+                                             : u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
+    if (aligned) {
+      *reinterpret_cast<u32x2*>(out) = o;
+    } else {
+      for (int i = 0; i < 4; ++i) out[i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
+    }
+  }
 }
 
 }  // namespace
@@ -872,6 +1004,59 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
   return FMSA_OK;
 }
 
+// Whether products over M tokens and `columns` columns in all take the kernel of 64-token workgroups (us before / with it):
+// below 2048 tokens from the traffic on that the fragment kernel's loads are bound by, X and the re-reads of Wd (rank 64: 4096
+// columns at 512 tokens, 21 MB, 7.5 / 10.1, q, k, v at 512, 31 MB, 12.0 / 10.6, gate and up of 14336 at 1100, 317 MB, 39.6 / 21.6;
+// rank 32: 4096 at 512, 13 MB, 7.4 / 8.1, at 1100, 27 MB, 9.9 / 8.4; rank 16: 2048 at 2047, 17 MB, 6.6 / 6.0) and always above
+// rank 64, whose eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48).
+// From 2048 tokens on above rank 16 (rank 32: 4096 at 8192 tokens 17.9 / 16.6; rank 64: 2048 at 2048 15.4 / 9.3, 4096 at 8192
+// 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99);
+// rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them and
+// short ones of many (14336 at 3217: 25.8 / 19.6; 4096 at 16384: 39 / 26).
+static bool down_is_mid(int M, int r_max, int64_t columns) {
+  if (M <= 64) return false;  // few tokens: the ranges of the products straight from the parameters are the fragment kernel's
+  if (M >= 2048) {
+    const bool many = M >= 16384, wide = columns >= 8192;
+    if (columns < 2048) return false;
+    return r_max > 16 ? !(many && wide && r_max > 32) : (many ? !wide : (wide && M < 4096));
+  }
+  const int64_t bytes = (int64_t)((M + 15) / 16) * (16 + std::max(16, r_max)) * columns * 2;
+  return r_max > 64 || bytes >= (r_max > 32 ? 22000000 : 14000000);
+}
+// column ranges: two chunks of 64 columns a wave at least, and no more workgroups than run at once (one per CU, two up to rank 16)
+static int down_mid_split(int M, int C, int r_max, int blocks_per_row) {
+  const int blocks = ((M + 16 * LM_MT - 1) / (16 * LM_MT)) * blocks_per_row, slots = r_max <= 16 ? 512 : 256;
+  return std::max(1, std::min(slots / blocks, ((C + 63) / 64) / (2 * LM_NW)));
+}
+static int rank_blocks(int r) { return (r + 63) / 64; }
+
+static int launch_down_mid(LoraDownArgs& a, int n_jobs, int act_dtype, hipStream_t st) {
+  int split_max = 1, r_max = 0;
+  bool sums = false;
+  for (int q = 0; q < n_jobs; ++q) {
+    if (a.j[q].n_split == 1) a.j[q].partial = nullptr;
+    sums = sums || a.j[q].partial;
+    split_max = std::max(split_max, a.j[q].n_split);
+    r_max = std::max(r_max, a.j[q].r);
+  }
+  a.r_max = r_max;
+  const dim3 grid((a.M + 16 * LM_MT - 1) / (16 * LM_MT), split_max, n_jobs * rank_blocks(r_max)), block(64 * LM_NW);
+  const dim3 rgrid((unsigned)(((int64_t)a.M * (r_max / 4) + 255) / 256), n_jobs);
+  const int rt = (std::min(r_max, 64) + 15) / 16;
+#define MID(TT)                                                                                       \
+  do {                                                                                                \
+    if (rt <= 1) hipLaunchKernelGGL((lora_down_mid_kernel<TT, 1>), grid, block, 0, st, a);             \
+    else if (rt == 2) hipLaunchKernelGGL((lora_down_mid_kernel<TT, 2>), grid, block, 0, st, a);        \
+    else hipLaunchKernelGGL((lora_down_mid_kernel<TT, 4>), grid, block, 0, st, a);                     \
+    if (sums) hipLaunchKernelGGL((lora_down_reduce_batch_kernel<TT>), rgrid, dim3(256), 0, st, a);     \
+  } while (0)
+  if (act_dtype == FMSA_BF16) MID(bf16_t);
+  else MID(f16_t);
+#undef MID
+  FMSA_CHECK_LAUNCH();
+  return FMSA_OK;
+}
+
 int launch_lora_down(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
                      int64_t ldo, hipStream_t st) {
   return launch_lora_down_plain(X, ldx, Wd, M, C, r, act_dtype, out, ldo, nullptr, 1, st);
@@ -910,6 +1095,10 @@ DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
 }  // namespace
 
 size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
+  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C)) {
+    const int n = down_mid_split(M, C, r, rank_blocks(r));
+    return n > 1 ? (size_t)n * M * r * sizeof(float) : 0;
+  }
   const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
   const int ranks = d.g == 1 ? r : std::min(r, 64);
   return d.g && d.n_split > 1 ? (size_t)d.n_split * (size_t)M * (size_t)ranks * sizeof(float) : 0;
@@ -918,8 +1107,14 @@ size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
 // The split kernel where it pays and the caller brought the partial-sum buffer (or none is needed); launch_lora_down otherwise.
 int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
                         int64_t ldo, void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st) {
-  const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
   const size_t need = lora_down_workspace(M, C, r, few_tokens);
+  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C) && (!need || (workspace && workspace_bytes >= need && (uintptr_t)out % 8 == 0 && ldo % 4 == 0))) {
+    LoraDownArgs a{};
+    a.M = M;
+    a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
+    return launch_down_mid(a, 1, act_dtype, st);
+  }
+  const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
   const bool out_ok = ((uintptr_t)out % 8 == 0) && ldo % 4 == 0;  // the reduce pass stores four ranks at a time
   if (!d.g || (need && (!workspace || workspace_bytes < need || !out_ok)))
     return launch_lora_down(X, ldx, Wd, M, C, r, act_dtype, out, ldo, st);
@@ -973,16 +1168,8 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
 }
 
 // One launch for up to FMSA_LORA_DOWN_MAX_JOBS products over the same tokens, for few tokens (the rule of the g = 1 split).
-// Token tiles of 16 per workgroup.  Every workgroup reads its columns of all r rows of Wd out of L2, which at rank 64 is four
-// times what it reads of X: two tiles halve that.  Three launches at 1100 tokens, rank 64 (q k v; gate, up of 14336 columns;
-// 4096 columns): 34.4 us each on average with one tile, 23.3 with two, 20.4 with four (which leaves a quarter of the token blocks
-// to split for).  The line at 1024 tokens: two tiles against one, ranks 24 to 64, take 0.58 - 0.98 of the time from 1536 tokens
-// on for q k v and gate, up of hidden 1024 to 8192; at 1024 - 1280 tokens 0.71 - 0.92 from hidden 4096 on and 0.97 - 1.07
-// below; at 64 tokens 1.03 - 1.20 (28672 columns 0.9), where the narrow projections run out of workgroups.  Rank 16 and
-// below reads less of Wd than of X.
-static int down_batch_tiles(int M, int r_max) { return M >= 1024 && r_max > 16 && r_max <= 64 ? 2 : 1; }
-static int down_batch_split(int M, int C, int n_jobs, int mtl) {
-  const int n_tb = (M + 16 * mtl - 1) / (16 * mtl);
+static int down_batch_split(int M, int C, int n_jobs) {
+  const int n_tb = (M + 15) / 16;
   return std::max(1, std::min(512 / (n_tb * n_jobs), C / 512));
 }
 static int max_rank(const fmsa_lora_down_job* jobs, int n_jobs) {
@@ -993,22 +1180,32 @@ static int max_rank(const fmsa_lora_down_job* jobs, int n_jobs) {
 
 // Column ranges of lora_down (one job) and of the batched launch over few tokens
 int lora_down_few_splits(int M, int C, int r, int n_jobs) {
-  if (n_jobs > 1) return down_batch_split(M, C, n_jobs, 1);
+  if (n_jobs > 1) return down_batch_split(M, C, n_jobs);
   const DownSplit d = lora_down_split_shape(M, C, r, true);
   return d.g == 1 ? d.n_split : 1;
 }
 
+static int64_t all_columns(const fmsa_lora_down_job* jobs, int n_jobs) {
+  int64_t c = 0;
+  for (int q = 0; q < n_jobs; ++q) c += jobs[q].C;
+  return c;
+}
+static int down_batch_split_any(const fmsa_lora_down_job* jobs, int q, int n_jobs, int M) {
+  const int r_max = max_rank(jobs, n_jobs);
+  return down_is_mid(M, r_max, all_columns(jobs, n_jobs)) ? down_mid_split(M, jobs[q].C, r_max, n_jobs * rank_blocks(r_max))
+                               : down_batch_split(M, jobs[q].C, n_jobs);
+}
+
 size_t lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
-  const int mtl = down_batch_tiles(M, max_rank(jobs, n_jobs));
   size_t bytes = 0;
-  for (int q = 0; q < n_jobs; ++q) bytes += (size_t)down_batch_split(M, jobs[q].C, n_jobs, mtl) * M * jobs[q].r * sizeof(float);
+  for (int q = 0; q < n_jobs; ++q) bytes += (size_t)down_batch_split_any(jobs, q, n_jobs, M) * M * jobs[q].r * sizeof(float);
   return bytes;
 }
 
 int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, int act_dtype, void* workspace, hipStream_t st) {
   LoraDownArgs a{};
   a.M = M;
-  const int r_max = max_rank(jobs, n_jobs), mtl = down_batch_tiles(M, r_max);
+  const int r_max = max_rank(jobs, n_jobs);
   int split_max = 1;
   float* p = (float*)workspace;
   for (int q = 0; q < n_jobs; ++q) {
@@ -1021,23 +1218,22 @@ int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, in
     d.ldo = s.ldout;
     d.C = s.C;
     d.r = s.r;
-    d.n_split = down_batch_split(M, s.C, n_jobs, mtl);
+    d.n_split = down_batch_split_any(jobs, q, n_jobs, M);
     d.partial = p;
     p += (size_t)d.n_split * M * s.r;
     split_max = std::max(split_max, d.n_split);
   }
+  if (down_is_mid(M, r_max, all_columns(jobs, n_jobs))) return launch_down_mid(a, n_jobs, act_dtype, st);
   constexpr int NW = 8;
-  const dim3 grid((M + 16 * mtl - 1) / (16 * mtl), split_max, n_jobs), block(64 * NW);
+  const dim3 grid((M + 15) / 16, split_max, n_jobs), block(64 * NW);
   const dim3 rgrid((unsigned)(((int64_t)M * (r_max / 4) + 255) / 256), n_jobs);
   const int rt = (r_max + 15) / 16;
 #define BATCH(TT)                                                                                            \
   do {                                                                                                       \
     if (rt <= 1) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 1, 1, NW>), grid, block, 0, st, a);              \
-    else if (rt <= 2 && mtl == 2) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 2, 2, NW>), grid, block, 0, st, a);  \
     else if (rt <= 2) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 2, 1, NW>), grid, block, 0, st, a);         \
-    else if (rt <= 4 && mtl == 2) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 4, 2, NW>), grid, block, 0, st, a);  \
     else if (rt <= 4) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 4, 1, NW>), grid, block, 0, st, a);         \
-    else hipLaunchKernelGGL((lora_down_batch_kernel<TT, 8, 1, NW>), grid, block, 0, st, a);                      \
+    else hipLaunchKernelGGL((lora_down_batch_kernel<TT, 8, 1, NW>), grid, block, 0, st, a); /* up to 64 tokens */ \
     hipLaunchKernelGGL((lora_down_reduce_batch_kernel<TT>), rgrid, dim3(256), 0, st, a);                      \
   } while (0)
   if (act_dtype == FMSA_BF16) BATCH(bf16_t);
@@ -1092,7 +1288,7 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
     d.out_dtype = s.out_dtype;
     d.scale = s.scale;
     blocks += ((s.C + tc - 1) / tc) * d.splits;
-    rblocks += (s.r * s.C + 255) / 256;
+    rblocks += (s.r * s.C / 4 + 255) / 256;
     ws_off += job_partial_bytes(s, M);
     if (s.Wt) {
       d.Wt = (const uint16_t*)s.Wt;
