@@ -758,7 +758,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
 
   if constexpr (SPLIT) {
     if (work.range >= 0) {
-      split_store(acc, a.partial, work.cut, work.range, a.n_ranges);
+      split_store(acc, a.partial, work.cut, work.range, a.n_ranges, rows_valid);
       return;
     }
   }
@@ -957,21 +957,24 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   (void)active;
 }
 
-// Second launch of a split call: workgroup = token tile mt (32 rows) of a cut tile; lane, column and register layout of
-// the kernel above, outputs as 8-byte stores (a row segment of 64 bytes is completed by four of them in L2).
-template <typename T>
+// Second launch of a split call: workgroup = token tile mt (32 rows) of a cut tile and, linear, one column tile of its waves
+// (SwiGLU needs both, its e and its g); lane, column and register layout of the kernel above, outputs as 8-byte stores (a row
+// segment of 64 bytes is completed by four of them in L2).  A chain of memory latencies: with the ranges asked for four at a
+// time (split_tiles.h) the four of a layer at 700 tokens take 49 us instead of 55 (SwiGLU 14336 columns, rank 64: 14.0 -> 11.1).
+template <typename T, bool SWIGLU>
 __global__ __launch_bounds__(256) void gptq_lora_fwd_finish_kernel(const FwdArgs a) {
-  const int cut = blockIdx.x / MT, mt = blockIdx.x % MT;
+  constexpr int NJ = SWIGLU ? 1 : NT;  // workgroups a token tile
+  const int cut = blockIdx.x / (MT * NJ), mt = blockIdx.x / NJ % MT, j = blockIdx.x % NJ;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
   int bm, bn;
   fwd_tile(a, a.n_whole + cut, bm, bn);
   const int m = bm * BM + 32 * mt + l32;
   if (bm * BM + 32 * mt >= a.M) return;  // the whole workgroup
-  f32x4 acc[NT][4];
-  split_load(acc, a.partial, cut, mt, a.n_ranges);
+  f32x4 acc[SWIGLU ? NT : 1][4];
+  split_load<NT>(acc[0], a.partial, cut, mt, j, a.n_ranges);
+  if constexpr (SWIGLU) split_load<NT>(acc[1], a.partial, cut, mt, 1, a.n_ranges);
   if (m >= a.M) return;
-  const bool swiglu = a.mode == FMSA_FWD_SWIGLU;
-  const int p = swiglu ? 0 : (bn >= a.nblk_start[2] ? 2 : (bn >= a.nblk_start[1] ? 1 : 0));
+  const int p = SWIGLU ? 0 : (bn >= a.nblk_start[2] ? 2 : (bn >= a.nblk_start[1] ? 1 : 0));
   auto biased = [&](const FwdProjDev& P, const f32x4& v, int col) {
     f32x4 o = v;
     if (P.bias) {
@@ -980,7 +983,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_finish_kernel(const FwdArgs
     }
     return u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
   };
-  if (swiglu) {
+  if constexpr (SWIGLU) {
     const int col0 = bn * 128 + 32 * wave + 4 * half;
     if (bn * 128 + 32 * wave >= a.p[0].N) return;  // N % 32 == 0: a column tile is wholly inside or outside
 #pragma unroll
@@ -1000,15 +1003,12 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_finish_kernel(const FwdArgs
     }
   } else {
     const FwdProjDev P = select_proj(a, p);
+    const int col0 = (bn - a.nblk_start[p]) * 256 + 64 * wave + 32 * j;
+    if (col0 >= P.N) return;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int col0 = (bn - a.nblk_start[p]) * 256 + 64 * wave + 32 * j;
-      if (col0 >= P.N) continue;
-#pragma unroll
-      for (int i0 = 0; i0 < 4; ++i0) {
-        const int col = col0 + 8 * i0 + 4 * half;
-        *reinterpret_cast<u32x2*>(P.Y + (size_t)m * P.ldy + col) = biased(P, acc[j][i0], col);
-      }
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = col0 + 8 * i0 + 4 * half;
+      *reinterpret_cast<u32x2*>(P.Y + (size_t)m * P.ldy + col) = biased(P, acc[0][i0], col);
     }
   }
 }
@@ -1136,9 +1136,15 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
     else SPLIT_K(f16_t, 0, false);
 #undef SPLIT_K
     FMSA_CHECK_LAUNCH();
-    const dim3 fgrid(plan.n_split * MT);
-    if (act_dtype == FMSA_BF16) hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<bf16_t>), fgrid, block, 0, st, a);
-    else hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<f16_t>), fgrid, block, 0, st, a);
+    const bool swiglu = mode == FMSA_FWD_SWIGLU;
+    const dim3 fgrid(plan.n_split * MT * (swiglu ? 1 : NT));
+    if (act_dtype == FMSA_BF16) {
+      if (swiglu) hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<bf16_t, true>), fgrid, block, 0, st, a);
+      else hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<bf16_t, false>), fgrid, block, 0, st, a);
+    } else {
+      if (swiglu) hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<f16_t, true>), fgrid, block, 0, st, a);
+      else hipLaunchKernelGGL((gptq_lora_fwd_finish_kernel<f16_t, false>), fgrid, block, 0, st, a);
+    }
     FMSA_CHECK_LAUNCH();
     return FMSA_OK;
   }

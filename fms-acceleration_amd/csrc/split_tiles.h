@@ -67,34 +67,48 @@ FMSA_DEVI SplitWork split_work(int n_whole, int n_split, int s) {
   return {n_whole + u / s, u % s, u / s};
 }
 
-// One range's sums: quad (mt * NT + j) * 4 + i0 of lane l of wave w at [range][w][quad][l]
+// One range's sums: quad (mt * NT + j) * 4 + i0 of lane l of wave w at [range][w][quad][l].  Token tiles past the last row are
+// not read by the second launch and not written (700 tokens, two of 24: the four GEMMs of a layer 338 -> 331 us).
 template <int MT, int NT>
-FMSA_DEVI void split_store(const f32x16 (&acc)[MT][NT], float* partial, int cut, int range, int s) {
+FMSA_DEVI void split_store(const f32x16 (&acc)[MT][NT], float* partial, int cut, int range, int s, int rows) {
   static_assert(MT * NT * 4 == SPLIT_QUADS, "a wave's accumulators");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   f32x4* dst = reinterpret_cast<f32x4*>(partial + (size_t)(cut * s + range) * (SPLIT_TILE_BYTES / 4)) + (size_t)wave * SPLIT_QUADS * 64 + lane;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  static_for<0, MT>([&](auto mt_c) {
+    constexpr int mt = decltype(mt_c)::value;
+    if (32 * mt >= rows) return;
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int i0 = 0; i0 < 4; ++i0)
         dst[((mt * NT + j) * 4 + i0) * 64] =
             f32x4{acc[mt][j][4 * i0], acc[mt][j][4 * i0 + 1], acc[mt][j][4 * i0 + 2], acc[mt][j][4 * i0 + 3]};
+  });
 }
 
-// The sums of token tile mt of a cut tile, all ranges in index order: register layout of the GEMM's accumulators
+// The sums of column tile j of token tile mt of a cut tile, all ranges in index order: register layout of the GEMM's accumulators.
+// Four ranges are asked for at once: a second launch is a chain of memory latencies.
 template <int NT>
-FMSA_DEVI void split_load(f32x4 (&acc)[NT][4], const float* partial, int cut, int mt, int s) {
+FMSA_DEVI void split_load(f32x4 (&acc)[4], const float* partial, int cut, int mt, int j, int s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const f32x4* src = reinterpret_cast<const f32x4*>(partial + (size_t)cut * s * (SPLIT_TILE_BYTES / 4)) +
-                     ((size_t)wave * SPLIT_QUADS + mt * NT * 4) * 64 + lane;
+                     ((size_t)wave * SPLIT_QUADS + (mt * NT + j) * 4) * 64 + lane;
+  for (int r0 = 0; r0 < s; r0 += 4) {
+    f32x4 v[4][4];
 #pragma unroll
-  for (int q = 0; q < NT * 4; ++q) acc[q >> 2][q & 3] = src[q * 64];
-#pragma unroll 4
-  for (int rg = 1; rg < s; ++rg)
+    for (int r = 0; r < 4; ++r) {
+      if (r0 + r < s) {
 #pragma unroll
-    for (int q = 0; q < NT * 4; ++q) acc[q >> 2][q & 3] += src[(size_t)rg * (SPLIT_TILE_BYTES / 16) + q * 64];
+        for (int q = 0; q < 4; ++q) v[r][q] = src[(size_t)(r0 + r) * (SPLIT_TILE_BYTES / 16) + q * 64];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (r0 + r >= s) break;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = r0 + r == 0 ? v[r][q] : acc[q] + v[r][q];
+    }
+  }
 }
 
 }  // namespace
