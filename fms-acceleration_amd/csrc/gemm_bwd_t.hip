@@ -109,7 +109,10 @@ FMSA_DEVI void swiglu_bwd_pair(uint32_t ev, uint32_t gv, uint32_t bv, uint32_t l
                 unpack_hi<T>(tp) * se1 * (1.0f + e1 * (1.0f - se1)));
 }
 
-// CODEBOOK: W = code[q] * block_scale[group, n] instead of the affine scale * q + (-scale * zero).
+// CODEBOOK: W = code[q] * block_scale[group, n] instead of the affine scale * q + (-scale * zero), the codes from a table in
+// LDS, two per 8-byte read.  One ds_bpermute per code had the LDS pipe as its limit (26 instructions a step next to the 16
+// MFMAs, now 18): 16384 tokens, 28672 -> 4096 (gate and up) 3741 -> 2951 us, SwiGLU 4096 -> 14336 2222 -> 1797, at the affine
+// kernel's rate (1300 and 1070 TFLOP/s).
 // SPLIT: the tiles that do not fill a round of the chip are cut along the contraction (split_tiles.h).
 template <typename T, bool NTAIL, int MODE, bool CODEBOOK, bool PK16 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs a) {
@@ -121,7 +124,8 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
   // per buffer 4 KB: scales [8][64] fp32 | offsets [8][64] fp32 (PK16: fp16 scales [8][64] | fp16 offsets [8][64], 2 KB used)
   __shared__ __attribute__((aligned(1024))) uint32_t tb0[1024];
   __shared__ __attribute__((aligned(1024))) uint32_t tb1[1024];
-  __shared__ __attribute__((aligned(16))) uint16_t ep_planes[2 * EP_ROWS * EP_STRIDE];
+  // CODEBOOK: the pair table until the epilogue (the strictest alignment puts it at LDS address 0: no base to add to a lookup)
+  __shared__ alignas(CODEBOOK ? 2048 : 16) uint16_t ep_planes[2 * EP_ROWS * EP_STRIDE];
   auto dy_buf = [&](auto b_c) -> char* { return reinterpret_cast<char*>(decltype(b_c)::value == 0 ? dy0 : dy1); };
   auto tb_buf = [&](auto b_c) -> char* { return reinterpret_cast<char*>(decltype(b_c)::value == 0 ? tb0 : tb1); };
 
@@ -232,8 +236,6 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
     const uint32_t q_step_bytes = (uint32_t)K * 8;    // two packed rows per 16-wide step
     const uint32_t q_stage_bytes = (uint32_t)K * 32;  // eight packed rows per stage
     const uint32_t q_last = (uint32_t)((N >> 3) - 2) * K * 4;
-    const float lut = CODEBOOK ? P.code[lane & 15] : 0.f;
-
     uint32_t qw[2][NT][4];
     u32x4 xf[2][MT], wf[2][NT];
 
@@ -318,44 +320,31 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
         }
       }
     };
-    // ---- code book, two phases so that no gather is waited for right after its issue.  Phase a: fragment reads,
-    // the block scales of the step, and the 16 gathers from the lane-resident table (ds_bpermute; the codes of
-    // elements 2b / 2b+1 of a word in gath[j][b] / [4 + b]); phase b: code * block scale in fp32, one rounding.
-    uint32_t gath[NT][8];
-    u32x4 bsv[2];
-    auto prefetch_a = [&](auto sb_c, auto t_c, auto par_c) {
-      constexpr int SB = decltype(sb_c)::value;
-      constexpr int t = decltype(t_c)::value;
-      constexpr int par = decltype(par_c)::value;
-      const char* lt = tb_buf(sb_c);
-      const char* lr = dy_buf(sb_c) + dy_r[t];
-      bsv[0] = *reinterpret_cast<const u32x4*>(lt + tb_r + t * TB_STEP);
-      bsv[1] = *reinterpret_cast<const u32x4*>(lt + tb_r + t * TB_STEP + 16);
+    // ---- code book: a lookup brings the codes of a byte's two nibbles (elements 0, 2 | 4, 6 | 1, 3 | 5, 7 of a word) from the
+    // pair table [byte][32 copies]: lane l32 reads copy l32, so no two lanes of a half wave meet in a bank whatever the codes
+    // are, and the address is one byte permute (byte << 8 | 8 * l32).  Then code * block scale in fp32, one rounding.
+    const char* const pairs = reinterpret_cast<const char*>(ep_planes);
+    const uint32_t pair_lane = (uint32_t)(8 * l32);
+    auto look_up = [&](uint32_t w, auto byte_c) -> u32x2 {
+      return *reinterpret_cast<const u32x2*>(pairs + __builtin_amdgcn_perm(w, pair_lane, 0x0C0C0400u + 256 * decltype(byte_c)::value));
+    };
+    // fragment register `reg` of a word: v = {byte 0, byte 2, byte 1, byte 3}
+    auto scaled = [&](const u32x2 (&v)[4], const u32x4 (&bs)[2], auto reg_c) -> uint32_t {
+      constexpr int reg = decltype(reg_c)::value;
+      return pack2<T>(__uint_as_float(v[2 * (reg >> 1)][reg & 1]) * __uint_as_float(bs[reg >> 1][2 * (reg & 1)]),
+                      __uint_as_float(v[2 * (reg >> 1) + 1][reg & 1]) * __uint_as_float(bs[reg >> 1][2 * (reg & 1) + 1]));
+    };
+    // the very first step of a projection
+    auto prefetch_codebook = [&]() {
+      const u32x4 bs[2] = {*reinterpret_cast<const u32x4*>(tb_buf(I0{}) + tb_r), *reinterpret_cast<const u32x4*>(tb_buf(I0{}) + tb_r + 16)};
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) xf[par][mt] = *reinterpret_cast<const u32x4*>(lr + mt * 32 * BK * 2);
-      const int li = (int)__float_as_uint(lut);
+      for (int mt = 0; mt < MT; ++mt) xf[0][mt] = *reinterpret_cast<const u32x4*>(dy_buf(I0{}) + dy_r[0] + mt * 32 * BK * 2);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const uint32_t w = qw[SB][j][t];
-        // byte planes of table addresses (4 * code): a0 = elements 0, 4, 1, 5, a1 = elements 2, 6, 3, 7; fragment
-        // register b takes bytes b >> 1 and (b >> 1) + 2 of plane b & 1
-        const uint32_t a0 = opaque((w << 2) & 0x3C3C3C3Cu), a1 = opaque((w >> 2) & 0x3C3C3C3Cu);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const uint32_t pl = (b & 1) ? a1 : a0;
-          gath[j][b] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((pl >> (8 * (b >> 1))) & 0xffu), li);
-          gath[j][4 + b] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((pl >> (8 * ((b >> 1) + 2))) & 0xffu), li);
-        }
+        const uint32_t w = qw[0][j][0];
+        const u32x2 v[4] = {look_up(w, I0{}), look_up(w, I2{}), look_up(w, I1{}), look_up(w, I3{})};
+        static_for<0, 4>([&](auto r_c) { wf[0][j][decltype(r_c)::value] = scaled(v, bs, r_c); });
       }
-    };
-    auto prefetch_b = [&](auto par_c) {
-      constexpr int par = decltype(par_c)::value;
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          wf[par][j][b] = pack2<T>(__uint_as_float(gath[j][b]) * __uint_as_float(bsv[b >> 1][2 * (b & 1)]),
-                                   __uint_as_float(gath[j][4 + b]) * __uint_as_float(bsv[b >> 1][2 * (b & 1) + 1]));
     };
     using WithVmem = std::integral_constant<bool, true>;
     using NoVmem = std::integral_constant<bool, false>;
@@ -430,9 +419,8 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
         fence();
       });
     };
-    // The code-book step slot by slot.  The LDS pipe carries 26 instructions per step here (8 fragment reads, 2 table
-    // reads, 16 gathers) next to the other waves' share, so they are spread as evenly as the dependencies allow: the
-    // gathers of a fragment register's two weights go out first, its product follows about four MFMAs later.
+    // The code-book step slot by slot: the block scales and the 8 lookups lead, a fragment register's product follows its
+    // lookups about four MFMAs later.
     auto step_codebook = [&](auto nb_c, auto nt_c, auto nx_c, auto cur_c, auto vmem_c, int st_next, auto lb_c) {
       constexpr int SB = decltype(nb_c)::value;
       constexpr int t = decltype(nt_c)::value;
@@ -441,110 +429,50 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
       constexpr bool with_vmem = decltype(vmem_c)::value;
       const char* lt = tb_buf(nb_c);
       const char* lr = dy_buf(nb_c) + dy_r[t];
-      const int li = (int)__float_as_uint(lut);
       auto mfma_slot = [&](int slot) { acc[slot >> 1][slot & 1] = mfma32<T>(wf[cur][slot & 1], xf[cur][slot >> 1], acc[slot >> 1][slot & 1]); };
       auto frag = [&](int mt) { xf[par][mt] = *reinterpret_cast<const u32x4*>(lr + mt * 32 * BK * 2); };
       auto fence = [&]() { __builtin_amdgcn_sched_barrier(0); };
       auto dma = [&](auto idx_c) {
         if constexpr (with_vmem) load_piece(st_next, lb_c, idx_c);
       };
-      uint32_t ad[NT][2];  // byte planes of table addresses (4 * code): [tile][0] elements 0, 4, 1, 5; [1] elements 2, 6, 3, 7
-      uint32_t ga[NT][8];  // code of element 2b in [b], of element 2b + 1 in [4 + b]
       u32x4 bs[2];
-      // the two gathers of fragment register `reg` of tile `j`
-      auto gather2 = [&](auto j_c, auto reg_c) {
-        constexpr int j = decltype(j_c)::value;
-        constexpr int reg = decltype(reg_c)::value;
-        ga[j][reg] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((ad[j][reg & 1] >> (8 * (reg >> 1))) & 0xffu), li);
-        ga[j][4 + reg] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((ad[j][reg & 1] >> (8 * ((reg >> 1) + 2))) & 0xffu), li);
-      };
-      auto piece = [&](auto j_c, auto reg_c) {
-        constexpr int j = decltype(j_c)::value;
-        constexpr int reg = decltype(reg_c)::value;
-        wf[par][j][reg] = pack2<T>(__uint_as_float(ga[j][reg]) * __uint_as_float(bs[reg >> 1][2 * (reg & 1)]),
-                                   __uint_as_float(ga[j][4 + reg]) * __uint_as_float(bs[reg >> 1][2 * (reg & 1) + 1]));
-      };
-      using J0 = std::integral_constant<int, 0>;
-      using J1 = std::integral_constant<int, 1>;
+      u32x2 v[NT][4];
       mfma_slot(0);
       bs[0] = *reinterpret_cast<const u32x4*>(lt + tb_r + t * TB_STEP);
-      bs[1] = *reinterpret_cast<const u32x4*>(lt + tb_r + t * TB_STEP + 16);
-      ad[0][0] = opaque((qw[SB][0][t] << 2) & 0x3C3C3C3Cu);
-      ad[0][1] = opaque((qw[SB][0][t] >> 2) & 0x3C3C3C3Cu);
-      gather2(J0{}, I0{});
+      v[0][0] = look_up(qw[SB][0][t], I0{});
+      v[0][1] = look_up(qw[SB][0][t], I2{});
       dma(std::integral_constant<int, 0>{});
       fence();
       mfma_slot(1);
-      ad[1][0] = opaque((qw[SB][1][t] << 2) & 0x3C3C3C3Cu);
-      ad[1][1] = opaque((qw[SB][1][t] >> 2) & 0x3C3C3C3Cu);
-      gather2(J1{}, I0{});
+      v[1][0] = look_up(qw[SB][1][t], I0{});
+      v[1][1] = look_up(qw[SB][1][t], I2{});
       dma(std::integral_constant<int, 1>{});
       fence();
       mfma_slot(2);
-      gather2(J0{}, I1{});
+      bs[1] = *reinterpret_cast<const u32x4*>(lt + tb_r + t * TB_STEP + 16);
+      v[0][2] = look_up(qw[SB][0][t], I1{});
+      v[0][3] = look_up(qw[SB][0][t], I3{});
       dma(std::integral_constant<int, 2>{});
       fence();
       mfma_slot(3);
-      gather2(J1{}, I1{});
+      v[1][2] = look_up(qw[SB][1][t], I1{});
+      v[1][3] = look_up(qw[SB][1][t], I3{});
       dma(std::integral_constant<int, 3>{});
       fence();
-      mfma_slot(4);
-      frag(0);
-      frag(1);
-      dma(std::integral_constant<int, 4>{});
-      fence();
-      mfma_slot(5);
-      frag(2);
-      gather2(J0{}, I2{});
-      piece(J0{}, I0{});
-      dma(std::integral_constant<int, 5>{});
-      fence();
-      mfma_slot(6);
-      frag(3);
-      gather2(J1{}, I2{});
-      piece(J1{}, I0{});
-      dma(std::integral_constant<int, 6>{});
-      fence();
-      mfma_slot(7);
-      frag(4);
-      piece(J0{}, I1{});
-      dma(std::integral_constant<int, 7>{});
-      fence();
-      mfma_slot(8);
-      frag(5);
-      gather2(J0{}, I3{});
-      piece(J1{}, I1{});
-      dma(std::integral_constant<int, 8>{});
-      fence();
-      mfma_slot(9);
-      frag(6);
-      gather2(J1{}, I3{});
-      dma(std::integral_constant<int, 9>{});
-      fence();
-      mfma_slot(10);
-      frag(7);
-      piece(J0{}, I2{});
-      dma(std::integral_constant<int, 10>{});
-      fence();
-      mfma_slot(11);
-      piece(J1{}, I2{});
-      dma(std::integral_constant<int, 11>{});
-      fence();
-      mfma_slot(12);
-      dma(std::integral_constant<int, 12>{});
-      dma(std::integral_constant<int, 13>{});
-      fence();
-      mfma_slot(13);
-      dma(std::integral_constant<int, 14>{});
-      dma(std::integral_constant<int, 15>{});
-      fence();
-      mfma_slot(14);
-      piece(J0{}, I3{});
-      dma(std::integral_constant<int, 16>{});
-      fence();
-      mfma_slot(15);
-      piece(J1{}, I3{});
-      fence();
+      static_for<0, 12>([&](auto u_c) {
+        constexpr int u = decltype(u_c)::value;  // slots 4 .. 15
+        mfma_slot(4 + u);
+        if constexpr (u < 8) frag(u);
+        // products, tile 0 and 1 in turn
+        if constexpr (u >= 1 && u < 9) {
+          constexpr int j = (u - 1) & 1, reg = (u - 1) >> 1;
+          wf[par][j][reg] = scaled(v[j], bs, std::integral_constant<int, reg>{});
+        }
+        if constexpr (u < 8) dma(std::integral_constant<int, 9 + u>{});   // the 8 weight words
+        if constexpr (u >= 8) dma(std::integral_constant<int, u - 4>{});  // dY loads 4-7
+        if constexpr (u == 8) dma(std::integral_constant<int, 8>{});      // the tables
+        fence();
+      });
     };
     auto step = [&](auto nb_c, auto nt_c, auto nx_c, auto cur_c, auto vmem_c, int st_next, auto lb_c) {
       if constexpr (CODEBOOK) {
@@ -572,12 +500,21 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
 
     __syncthreads();  // the previous projection's last LDS reads are done
     load_stage(st0, I0{});
+    if constexpr (CODEBOOK) {
+      // pair table: entry 16 hi + lo = (code[lo], code[hi]); thread (lo = tid >> 4, copies 2 * (tid & 15), + 1), all hi
+      const uint32_t lo = __float_as_uint(P.code[tid >> 4]);
+      u32x4* dst = reinterpret_cast<u32x4*>(ep_planes) + tid;
+#pragma unroll
+      for (int hi = 0; hi < 16; ++hi) {
+        const uint32_t up = __float_as_uint(P.code[hi]);
+        dst[256 * hi] = u32x4{lo, up, lo, up};
+      }
+    }
     __builtin_amdgcn_s_waitcnt(WAIT_VM0);
     __syncthreads();
     load_stage(min(st0 + 1, st_end - 1), I1{});
     if constexpr (CODEBOOK) {
-      prefetch_a(I0{}, I0{}, I0{});
-      prefetch_b(I0{});
+      prefetch_codebook();
     } else {
       prefetch(I0{}, I0{}, I0{});
     }
@@ -977,9 +914,10 @@ static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M, int 
   const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;
   const bool swiglu = mode == FMSA_BWD_SWIGLU;
   // measured per whole round, over 1 to 6 of them: 11 to 13 % of its time, 15 to 16 % with the SwiGLU epilogue; from a code
-  // book, where the gathers hide some of it, 6 to 9 and 12 to 15 %
-  const float whole_slow = codebook ? (swiglu ? 0.15f : 0.09f) : (swiglu ? 0.16f : 0.13f);
-  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), whole_slow, codebook ? 1.7f : 1.4f,
+  // book without the epilogue 6 to 9 % (28672 -> 4096 at three rounds and 96 or 128 tiles: cutting them takes 1.9 and 0.9 % off
+  // the whole MLP step; SwiGLU 4096 -> 14336 at two rounds and 48 tiles: cutting them adds 1.2 %)
+  const float whole_slow = swiglu ? 0.16f : (codebook ? 0.09f : 0.13f);
+  return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), whole_slow,
                     swiglu ? 0.12f : 0.f);
 }
 

@@ -212,6 +212,35 @@ def test_gemm_operands_are_the_dequantised_weight_bit_for_bit(blocksize, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Ns,K", [((96, 160), 320), ((32, 64, 32), 64), ((2080, 1056), 256)])  # tails of a stage; the last one is cut
+def test_input_gradient_with_a_code_book_per_projection(Ns, K, dtype):
+    """The twin's kernel looks codes up in a table that it lays out per projection: one-hot gradients, each token for one column
+    of one projection, read every projection's operand back bit for bit, each under its own code book (unsorted, with a
+    negative zero and values near the ends of the range)."""
+    import fmsa_hip
+
+    g = torch.Generator().manual_seed(3)
+    projs, wants, keeps = [], [], []
+    M = sum(Ns)
+    row = 0
+    for i, N in enumerate(Ns):
+        _, keep, q = _prepared(N, K, 21 + i)
+        book = torch.randn(16, generator=g) * torch.tensor([1.0, 1e-3, 200.0, 1.0] * 4)
+        book[i] = -0.0
+        code = book.cuda()
+        w = fmsa_hip.make_codebook_weight(keep[0], code, keep[1], 64)
+        dy = torch.zeros(M, N, dtype=dtype, device="cuda")
+        dy[row : row + N] = torch.eye(N, dtype=dtype, device="cuda")
+        row += N
+        projs.append({"w": w, "nsz": None, "dY": dy, "T": None, "At": None, "mask_src": None, "r": 0, "s": 0.0,
+                      "qweight_t": fmsa_hip.gptq_transpose(keep[0])})
+        wants.append(onf4.dequant(q, _NAME[dtype], code=book.numpy()))  # [N, K]
+        keeps.append((keep, code))
+    dx = fmsa_hip.gptq_lora_bwd_dx(projs, M, K)
+    assert torch.equal(dx.cpu(), torch.cat(wants) + 0.0)  # a sum with zeros: no negative zero is left
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N,r,blocksize", [(200, 256, 96, 16, 64), (512, 1024, 512, 8, 64), (64, 1056, 288, 32, 32), (300, 512, 256, 16, 128),
                                                (1, 64, 32, 8, 64), (257, 1344, 608, 24, 64), (31, 96, 1184, 40, 32), (513, 640, 160, 8, 128),
                                                (100, 1152, 896, 16, 64), (7, 2048, 96, 64, 64)])
