@@ -82,11 +82,11 @@ FMSA_DEVI void fwd_tile(const FwdArgs& a, int pid, int& bm, int& bn) {
 }
 
 // GPS = scale groups per 64-wide K stage: 1 for group_size % 64 == 0, 2 / 4 for group sizes 32 / 16.
-// CODEBOOK (1, 2): the nibbles index a 16-entry table and one fp32 scale per (group, column) multiplies the
-// entry (W = code[q] * block_scale); 0: the affine GPTQ form W = scale * (q - zero).  1 gathers code[q] from the
-// lanes of the wave (one ds_bpermute per weight) and multiplies; 2 (GPS == 1) multiplies the 16 entries by the lane's
-// block scale once per stage and column, keeps the 16 rounded products as two byte planes in registers, and looks the
-// weights up with byte permutes: the same products, no gather on the LDS pipe that the X fragments keep busy.
+// CODEBOOK: the nibbles index a 16-entry table and one fp32 scale per (group, column) multiplies the entry
+// (W = code[q] * block_scale) instead of the affine GPTQ form W = scale * (q - zero); the codes come from a table of pairs in
+// LDS, two per 8-byte read, which leaves the LDS pipe the room that one ds_bpermute per code did not and takes 40 vector
+// instructions a step less than 16 rounded products per block kept in registers and looked up with byte permutes did: 16384
+// tokens, 4096 -> 14336 with the SwiGLU and 14336 -> 4096 together 5100 -> 4757 us (1213 TFLOP/s; affine 1264).
 // ROPE (1: cos / sin tables in the activation type, 2: in fp32; 0: none): the Q / K projections of an attention block
 // leave the kernel with the rotary embedding applied
 // (kernels/unsloth/rope_embedding.py:36-65 of the reference: (q1, q2) <- (q1 cos - q2 sin, q2 cos + q1 sin) on the two
@@ -97,15 +97,20 @@ FMSA_DEVI void fwd_tile(const FwdArgs& a, int pid, int& bm, int& bn) {
 // in 15 instead of 22 instructions per word.
 // SPLIT: the tiles that do not fill a round of the chip are cut along K (split_tiles.h); a template parameter, because the
 // flavours without it are scheduled instruction by instruction.
-template <typename T, int GPS, bool KTAIL, int CODEBOOK, int ROPE = 0, bool PK16 = false, bool SPLIT = false>
+template <typename T, int GPS, bool KTAIL, bool CODEBOOK, int ROPE = 0, bool PK16 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
-  static_assert(!PK16 || (std::is_same<T, f16_t>::value && CODEBOOK == 0 && GPS == 1 && ROPE == 0), "packed half unpack");
+  static_assert(!PK16 || (std::is_same<T, f16_t>::value && !CODEBOOK && GPS == 1 && ROPE == 0), "packed half unpack");
   // two separate arrays (not one 2-D array): every access names its buffer statically, which is
   // what lets the compiler see that fragment reads of one buffer do not depend on the direct loads
   // in flight into the other
   __shared__ __attribute__((aligned(1024))) uint16_t lds0[BM * BK];
   __shared__ __attribute__((aligned(1024))) uint16_t lds1[BM * BK];
-  __shared__ __attribute__((aligned(16))) uint16_t ep_planes[3 * EP_ROWS * EP_STRIDE_S];  // >= EP_ROWS * EP_STRIDE_L
+  // CODEBOOK: the pair table until the epilogue, the adapter's staged operands behind it (the strictest alignment puts the
+  // array at LDS address 0: no base to add to a lookup)
+  constexpr int PAIR_BYTES = CODEBOOK ? 256 * 32 * 8 : 0;
+  constexpr int LORA_BYTES = (16 + 4 * NT) * 1024;
+  __shared__ alignas(CODEBOOK ? 2048 : 16) uint16_t ep_planes[CODEBOOK ? (PAIR_BYTES + LORA_BYTES) / 2 : 3 * EP_ROWS * EP_STRIDE_S];  // >= EP_ROWS * EP_STRIDE_L
+  static_assert(sizeof(ep_planes) >= 3 * EP_ROWS * EP_STRIDE_S * 2, "the SwiGLU planes must fit");
   static_assert(3 * EP_STRIDE_S >= EP_STRIDE_L, "the linear plane must fit");
   auto lds_buf = [&](auto b_c) -> char* {
     constexpr int b = decltype(b_c)::value;
@@ -148,7 +153,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   const char* scbase[NT];
   const char* zbase[NT];
   int Np[NT], zshift[NT], gs[NT];
-  float zoff[NT], lut[NT];  // lut: this lane's entry of the projection's code book (lanes 0..15 serve as the table)
+  float zoff[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const FwdProjDev P = select_proj(a, pj[j]);
@@ -160,26 +165,29 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     gs[j] = __builtin_amdgcn_readfirstlane(P.group_size);
     qbase[j] = reinterpret_cast<const char*>(P.qweight);
     scbase[j] = CODEBOOK ? reinterpret_cast<const char*>(P.block_scale) : reinterpret_cast<const char*>(P.scales);
-    lut[j] = CODEBOOK == 1 ? P.code[lane & 15] : 0.f;
     zbase[j] = reinterpret_cast<const char*>(P.qzeros);
     zshift[j] = 4 * (col & 7);
     zoff[j] = (float)P.zero_offset;
   }
 
-  // table flavour: the code book as wave-uniform values (the launcher takes this flavour only when the projections of
-  // the launch share one code book), and per column tile the byte planes of the current stage's 16 rounded products:
-  // byte e of tlo[set][j][d] / thi[set][j][d] = low / high byte of entry 4 d + e.  Two sets: while the stage in slot SB
-  // looks its weights up in set SB, the steps of that stage build set SB ^ 1 for the next one, a quarter per step, so
-  // the 80 instructions of a table pair sit between MFMAs like the rest.  That needs the block scale one stage earlier
-  // than the weights: load_stage(st) fetches the scale of stage st + 1.
-  float cd[16];
-  uint32_t tlo[NBUF][NT][4], thi[NBUF][NT][4];
-  int gshift[NT];  // log2 of the block size (the launcher takes this flavour for powers of two only)
-  if constexpr (CODEBOOK == 2) {
+  // code book: entry [16 hi + lo][copy] = (code[lo], code[hi]) as fp32, 32 copies of 8 bytes; lane l32 reads copy l32, so no two
+  // lanes of a half wave meet in a bank whatever the codes are, and the address is one byte permute (byte << 8 | 8 * copy).
+  // Copies 16-31 hold the second column tile's book; where the two differ (SwiGLU) a tile has 16 copies.
+  uint32_t pair_lane[NT];
+  if constexpr (CODEBOOK) {
+    const float* c0 = select_proj(a, pj[0]).code;
+    const float* c1 = select_proj(a, pj[1]).code;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) cd[i] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(a.p[0].code[i])));
+    for (int j = 0; j < NT; ++j) pair_lane[j] = c0 == c1 ? (uint32_t)(8 * l32) : (uint32_t)(8 * (l32 & 15) + 128 * j);
+    // thread: entry lo = tid >> 4, copies 2 * (tid & 15) and the next, all hi
+    const float* c = (tid & 15) < 8 ? c0 : c1;
+    const uint32_t lo = __float_as_uint(c[tid >> 4]);
+    u32x4* dst = reinterpret_cast<u32x4*>(ep_planes) + tid;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) gshift[j] = 31 - __builtin_clz(gs[j]);
+    for (int hi = 0; hi < 16; ++hi) {
+      const uint32_t up = __float_as_uint(c[hi]);
+      dst[256 * hi] = u32x4{lo, up, lo, up};
+    }
   }
 
   const int K = a.K;
@@ -296,10 +304,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
           gu = (ku < K ? ku : st * BK) / gs[j];
         }
         gu = __builtin_amdgcn_readfirstlane(gu);  // uniform; keeps the scalar offsets out of vector registers
-        if constexpr (CODEBOOK == 2) {
-          const int g1 = __builtin_amdgcn_readfirstlane(min(((st + 1) * BK) >> gshift[j], n_groups_j[j] - 1));
-          zw_raw[SB ^ 1][j][u] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], (uint32_t)g1 * Np[j] * 4, 0);
-        } else if constexpr (CODEBOOK == 1) {
+        if constexpr (CODEBOOK) {
           zw_raw[SB][j][u] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], (uint32_t)gu * Np[j] * 4, 0);
         } else {
           sc_raw[SB][j][u] = __builtin_amdgcn_raw_buffer_load_b16(sc_rsrc[j], sc_off[j], (uint32_t)gu * Np[j] * 2, 0);
@@ -321,9 +326,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     for (int j = 0; j < NT; ++j) {
 #pragma unroll
       for (int u = 0; u < GPS; ++u) {
-        if constexpr (CODEBOOK == 2) {
-          // (the tables are built step by step in prefetch)
-        } else if constexpr (CODEBOOK == 1) {
+        if constexpr (CODEBOOK) {
           sf[j][u] = __uint_as_float(zw_raw[SB][j][u]);
         } else if constexpr (PK16) {
           sp16[j] = (uint32_t)sc_raw[SB][j][u] * 0x00010001u;
@@ -344,19 +347,13 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   // into the other half of xf / wf.  The stage barrier sits after step 2, so step 3 can already
   // fetch step 0 of the next stage from the next LDS buffer.
   u32x4 xf[2][MT], wf[2][NT];
-  // entries 4 d .. 4 d + 3 of table set SET from the block scales in raw slot SET: the products rounded to the storage
-  // type in pairs, then the two byte planes
-  auto build_table_part = [&](auto set_c, auto d_c) {
-    constexpr int SET = decltype(set_c)::value;
-    constexpr int d = decltype(d_c)::value;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const float sc = __uint_as_float(zw_raw[SET][j][0]);
-      const uint32_t p0 = pack2<T>(cd[4 * d] * sc, cd[4 * d + 1] * sc), p1 = pack2<T>(cd[4 * d + 2] * sc, cd[4 * d + 3] * sc);
-      tlo[SET][j][d] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
-      thi[SET][j][d] = __builtin_amdgcn_perm(p1, p0, 0x07050301u);
-    }
+  const char* const pairs = reinterpret_cast<const char*>(ep_planes);
+  // the codes of a word's byte: elements 2 byte, 2 byte + 1 = fragment register `byte`
+  auto look_up = [&](uint32_t w, int j, auto byte_c) -> u32x2 {
+    return *reinterpret_cast<const u32x2*>(pairs + __builtin_amdgcn_perm(w, pair_lane[j], 0x0C0C0400u + 256 * decltype(byte_c)::value));
   };
+  // code * block scale in fp32, one rounding
+  auto scaled = [&](const u32x2& v, float sc) -> uint32_t { return pack2<T>(__uint_as_float(v[0]) * sc, __uint_as_float(v[1]) * sc); };
   auto prefetch = [&](auto sb_c, auto t_c, auto par_c) {
     constexpr int SB = decltype(sb_c)::value;
     constexpr int t = decltype(t_c)::value;
@@ -366,23 +363,11 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     for (int mt = 0; mt < MT; ++mt) xf[par][mt] = *reinterpret_cast<const u32x4*>(lr + mt * 32 * BK * 2);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      if constexpr (CODEBOOK == 2) {
-        // nibble 2b / 2b + 1 of the word (weights k = 2b, 2b + 1 of the step) sit in byte b: per byte plane two
-        // permutes over entries 0-7 and 8-15 with the nibble's low three bits, a third picks by its top bit
-        const uint32_t w = qw[SB][j][t];
-        const uint32_t se = w & 0x07070707u, so = (w >> 4) & 0x07070707u;
-        const uint32_t pe = ((w >> 1) & 0x04040404u) | 0x03020100u, po = ((w >> 5) & 0x04040404u) | 0x03020100u;
-        const uint32_t loe = __builtin_amdgcn_perm(__builtin_amdgcn_perm(tlo[SB][j][3], tlo[SB][j][2], se), __builtin_amdgcn_perm(tlo[SB][j][1], tlo[SB][j][0], se), pe);
-        const uint32_t hie = __builtin_amdgcn_perm(__builtin_amdgcn_perm(thi[SB][j][3], thi[SB][j][2], se), __builtin_amdgcn_perm(thi[SB][j][1], thi[SB][j][0], se), pe);
-        const uint32_t loo = __builtin_amdgcn_perm(__builtin_amdgcn_perm(tlo[SB][j][3], tlo[SB][j][2], so), __builtin_amdgcn_perm(tlo[SB][j][1], tlo[SB][j][0], so), po);
-        const uint32_t hio = __builtin_amdgcn_perm(__builtin_amdgcn_perm(thi[SB][j][3], thi[SB][j][2], so), __builtin_amdgcn_perm(thi[SB][j][1], thi[SB][j][0], so), po);
-        // 16-bit values of weights (0, 2), (4, 6) and (1, 3), (5, 7), then the pairs (k, k + 1) the fragment holds
-        const uint32_t e01 = __builtin_amdgcn_perm(hie, loe, 0x05010400u), e23 = __builtin_amdgcn_perm(hie, loe, 0x07030602u);
-        const uint32_t o01 = __builtin_amdgcn_perm(hio, loo, 0x05010400u), o23 = __builtin_amdgcn_perm(hio, loo, 0x07030602u);
-        wf[par][j][0] = __builtin_amdgcn_perm(o01, e01, 0x05040100u);
-        wf[par][j][1] = __builtin_amdgcn_perm(o01, e01, 0x07060302u);
-        wf[par][j][2] = __builtin_amdgcn_perm(o23, e23, 0x05040100u);
-        wf[par][j][3] = __builtin_amdgcn_perm(o23, e23, 0x07060302u);
+      if constexpr (CODEBOOK) {
+        u32x2 v[4];
+        static_for<0, 4>([&](auto r_c) { v[decltype(r_c)::value] = look_up(qw[SB][j][t], j, r_c); });
+#pragma unroll
+        for (int r = 0; r < 4; ++r) wf[par][j][r] = scaled(v[r], sf[j][t * GPS / 4]);
       } else if constexpr (PK16) {
         static_for<0, 4>([&](auto r_c) {
           constexpr int r = decltype(r_c)::value;
@@ -392,55 +377,11 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
         wf[par][j] = dequant8<T>(qw[SB][j][t], sf[j][t * GPS / 4], sf16[j][t * GPS / 4], nsz[j][t * GPS / 4]);
       }
     }
-    if constexpr (CODEBOOK == 2) build_table_part(std::integral_constant<int, SB ^ 1>{}, t_c);
-  };
-  // Code-book flavour in two phases, so that a step's first 8 MFMAs cover the table gathers and its
-  // last 8 the arithmetic on what they returned.  Phase a: the 8 X fragments and the 16 gathers
-  // (ds_bpermute from the lane-resident table; element 2b / 2b+1 of a word in gath[j][b] / [4 + b]).
-  uint32_t gath[NT][8];
-  auto prefetch_a = [&](auto sb_c, auto t_c, auto par_c) {
-    constexpr int SB = decltype(sb_c)::value;
-    constexpr int t = decltype(t_c)::value;
-    constexpr int par = decltype(par_c)::value;
-    const char* lr = lds_buf(sb_c) + lds_r_off[t];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xf[par][mt] = *reinterpret_cast<const u32x4*>(lr + mt * 32 * BK * 2);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const uint32_t w = qw[SB][j][t];
-      const uint32_t e = opaque((w << 2) & 0x3C3C3C3Cu);  // byte b: 4 * nibble 2b (a lane's byte address)
-      const uint32_t o = opaque((w >> 2) & 0x3C3C3C3Cu);  // byte b: 4 * nibble 2b+1
-      const int li = (int)__float_as_uint(lut[j]);
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        gath[j][b] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((e >> (8 * b)) & 0xffu), li);
-        gath[j][4 + b] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((o >> (8 * b)) & 0xffu), li);
-      }
-    }
-  };
-  // phase b: code * block scale in fp32, one rounding
-  auto prefetch_b = [&](auto t_c, auto par_c) {
-    constexpr int t = decltype(t_c)::value;
-    constexpr int par = decltype(par_c)::value;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const float sc = sf[j][t * GPS / 4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) wf[par][j][b] = pack2<T>(__uint_as_float(gath[j][b]) * sc, __uint_as_float(gath[j][4 + b]) * sc);
-    }
   };
   auto mfma_step = [&](auto par_c) {
     constexpr int par = decltype(par_c)::value;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[mt][j] = mfma32<T>(wf[par][j], xf[par][mt], acc[mt][j]);
-  };
-  auto mfma_half = [&](auto par_c, auto h_c) {
-    constexpr int par = decltype(par_c)::value;
-    constexpr int h = decltype(h_c)::value;
-#pragma unroll
-    for (int mt = h * (MT / 2); mt < (h + 1) * (MT / 2); ++mt)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[mt][j] = mfma32<T>(wf[par][j], xf[par][mt], acc[mt][j]);
   };
@@ -453,8 +394,8 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, CODEBOOK == 2 ? 5 : 3, 0);
-      if ((i & 1) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      if (CODEBOOK || (i & 1) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       if (with_vmem) {
         if (i < 6)
           __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
@@ -463,33 +404,6 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // nothing from the next step (or the stage hand-over) moves up
-  };
-  // code-book halves: (a) 8 MFMAs with the address arithmetic (3 VALU) and 3 LDS-pipe instructions
-  // each (8 fragment reads + 16 gathers); (b) 8 MFMAs with the 24 multiplies / conversions and, in the
-  // last step of a stage, the global loads of a later stage
-  auto interleave_a = [&]() {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-      __builtin_amdgcn_sched_group_barrier(0x080, 3, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto interleave_b = [&](auto with_vmem_c) {
-    constexpr bool with_vmem = decltype(with_vmem_c)::value;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-      if (with_vmem) {
-        if (i < 2)
-          __builtin_amdgcn_sched_group_barrier(0x020, 3, 0);
-        else
-          __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
   };
   using WithVmem = std::integral_constant<bool, true>;
   using NoVmem = std::integral_constant<bool, false>;
@@ -508,29 +422,21 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   // one 16-wide K step: the MFMAs of parity `cur` while fragments and weights of (buffer nb, step nt)
   // are produced into parity `nx`
   auto step = [&](auto nb_c, auto nt_c, auto nx_c, auto cur_c, auto vmem_c) {
-    if constexpr (CODEBOOK == 1) {
-      prefetch_a(nb_c, nt_c, nx_c);
-      mfma_half(cur_c, I0{});
-      interleave_a();
-      prefetch_b(nt_c, nx_c);
-      mfma_half(cur_c, I1{});
-      interleave_b(vmem_c);
-    } else {
-      prefetch(nb_c, nt_c, nx_c);
-      mfma_step(cur_c);
-      interleave(vmem_c);
-    }
+    prefetch(nb_c, nt_c, nx_c);
+    mfma_step(cur_c);
+    interleave(vmem_c);
   };
-  // The affine step (one scale group per stage) written slot by slot, as the input-gradient kernel on the transposed
+  // The step with one scale group per stage written slot by slot, as the input-gradient kernel on the transposed
   // twin does: the 16 MFMAs of parity `cur`, behind each one its share of the work that produces step (nb, nt) into
   // parity `nx` -- a fragment read behind the first eight, one unpacked fragment register (2 conversions, 2
   // multiply-adds, 1 packed conversion) behind every even one -- and, in the last step of a stage, the 20 loads of
   // stage `st_next` into buffer / slot `lb`.  A scheduling fence closes every slot: the order below is the schedule
   // (about 1 % faster than what the group-barrier matcher makes of the same step; the fragment reads spread over the
-  // odd slots instead measured no gain).
-  constexpr bool HAND = CODEBOOK == 0 && GPS == 1;
-  // load number `idx` of stage `st` into slot SB (GPS == 1, affine): 0-7 the X tile (direct loads), 8-15 the weight
-  // words (idx - 8 = 4 j + t), 16-17 scale and zero word of column tile 0, 18-19 of column tile 1
+  // odd slots instead measured no gain).  From a code book the 8 lookups lead, two behind each of the first four, the fragment
+  // reads follow, and a register's product comes about four MFMAs after its lookup.
+  constexpr bool HAND = GPS == 1;
+  // load number `idx` of stage `st` into slot SB (GPS == 1): 0-7 the X tile (direct loads), 8-15 the weight words
+  // (idx - 8 = 4 j + t), 16-17 scale and zero word of column tile 0, 18-19 of column tile 1 (code book: 16, 18 the block scale)
   auto load_piece = [&](int st, auto sb_c, auto idx_c) {
     constexpr int SB = decltype(sb_c)::value;
     constexpr int idx = decltype(idx_c)::value;
@@ -549,9 +455,10 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       constexpr int j = (idx - 16) >> 1;
       const int gu = __builtin_amdgcn_readfirstlane(min(g_ld[j], n_groups_j[j] - 1));
       if constexpr (((idx - 16) & 1) == 0) {
-        sc_raw[SB][j][0] = __builtin_amdgcn_raw_buffer_load_b16(sc_rsrc[j], sc_off[j], (uint32_t)gu * Np[j] * 2, 0);
+        if constexpr (CODEBOOK) zw_raw[SB][j][0] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], (uint32_t)gu * Np[j] * 4, 0);
+        else sc_raw[SB][j][0] = __builtin_amdgcn_raw_buffer_load_b16(sc_rsrc[j], sc_off[j], (uint32_t)gu * Np[j] * 2, 0);
       } else {
-        zw_raw[SB][j][0] = __builtin_amdgcn_raw_buffer_load_b32(z_rsrc[j], z_off[j], (uint32_t)gu * (Np[j] >> 3) * 4, 0);
+        if constexpr (!CODEBOOK) zw_raw[SB][j][0] = __builtin_amdgcn_raw_buffer_load_b32(z_rsrc[j], z_off[j], (uint32_t)gu * (Np[j] >> 3) * 4, 0);
         k_in_g[j] += BK;  // uniform scalar bookkeeping, no division
         const bool wrap = k_in_g[j] >= gs[j];
         k_in_g[j] -= wrap ? gs[j] : 0;
@@ -559,7 +466,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       }
     }
   };
-  auto step_affine = [&](auto nb_c, auto nt_c, auto nx_c, auto cur_c, auto vmem_c, int st_next, auto lb_c) {
+  auto step_hand = [&](auto nb_c, auto nt_c, auto nx_c, auto cur_c, auto vmem_c, int st_next, auto lb_c) {
     constexpr int SB = decltype(nb_c)::value;
     constexpr int t = decltype(nt_c)::value;
     constexpr int par = decltype(nx_c)::value;
@@ -603,6 +510,27 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
       }
       wf[par][j][reg] = pack2<T>(__builtin_fmaf(sf[j][0], b0, nsz[j][0]), __builtin_fmaf(sf16[j][0], b1, nsz[j][0]));
     };
+    if constexpr (CODEBOOK) {
+      u32x2 v[NT][4];
+      static_for<0, 16>([&](auto u_c) {
+        constexpr int u = decltype(u_c)::value;
+        mfma_slot(u);
+        if constexpr (u < 4) {
+          constexpr int j = u & 1, b = 2 * (u >> 1);
+          v[j][b] = look_up(qw[SB][j][t], j, std::integral_constant<int, b>{});
+          v[j][b + 1] = look_up(qw[SB][j][t], j, std::integral_constant<int, b + 1>{});
+        }
+        if constexpr (u >= 4 && u < 12) frag(u - 4);
+        if constexpr (u >= 5 && u < 13) {
+          constexpr int j = (u - 5) & 1, reg = (u - 5) >> 1;
+          wf[par][j][reg] = scaled(v[j][reg], sf[j][0]);
+        }
+        dma(std::integral_constant<int, u>{});
+        if constexpr (u >= 12) dma(std::integral_constant<int, 4 + u>{});
+        fence();
+      });
+      return;
+    }
     static_for<0, 16>([&](auto u_c) {
       constexpr int u = decltype(u_c)::value;
       mfma_slot(u);
@@ -619,9 +547,9 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     constexpr int SB = decltype(sb_c)::value;
     using S1 = std::integral_constant<int, SB ^ 1>;
     if constexpr (HAND) {
-      step_affine(sb_c, I1{}, I1{}, I0{}, NoVmem{}, 0, sb_c);
-      step_affine(sb_c, I2{}, I0{}, I1{}, NoVmem{}, 0, sb_c);
-      step_affine(sb_c, I3{}, I1{}, I0{}, NoVmem{}, 0, sb_c);
+      step_hand(sb_c, I1{}, I1{}, I0{}, NoVmem{}, 0, sb_c);
+      step_hand(sb_c, I2{}, I0{}, I1{}, NoVmem{}, 0, sb_c);
+      step_hand(sb_c, I3{}, I1{}, I0{}, NoVmem{}, 0, sb_c);
     } else {
       step(sb_c, I1{}, I1{}, I0{}, NoVmem{});
       step(sb_c, I2{}, I0{}, I1{}, NoVmem{});
@@ -631,7 +559,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
     commit_stage(S1{});
     __syncthreads();
     if constexpr (HAND) {
-      step_affine(S1{}, I0{}, I0{}, I1{}, WithVmem{}, min(s + 2, st_end - 1), sb_c);
+      step_hand(S1{}, I0{}, I0{}, I1{}, WithVmem{}, min(s + 2, st_end - 1), sb_c);
     } else {
       load_stage(min(s + 2, st_end - 1), sb_c);
       step(S1{}, I0{}, I0{}, I1{}, WithVmem{});
@@ -643,8 +571,8 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
   // KB (8u + mt): rows 32mt..32mt+31 of U of the tile's u-th projection, 16 B per (row, rank half) at slot
   // 2 * row + half.  KB (16 + NT * wave + j): the same for the wave's 32 rows of B of column tile j.
   // Ranks past r and rows past M / N arrive as zeros through the range check.
-  char* const lora_lds = reinterpret_cast<char*>(ep_planes);
-  static_assert(sizeof(ep_planes) >= (16 + 4 * NT) * 1024, "LoRA operands must fit into the epilogue planes");
+  char* const lora_lds = reinterpret_cast<char*>(ep_planes) + PAIR_BYTES;
+  static_assert(sizeof(ep_planes) >= PAIR_BYTES + LORA_BYTES, "LoRA operands must fit into the epilogue planes");
   const bool lora_any = (a.p[0].r | a.p[1].r | a.p[2].r) != 0;
   if (lora_any) {
     const int prow = lane >> 1, phalf = lane & 1;
@@ -666,30 +594,12 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_kernel(const FwdArgs a) {
                                                16, (uint32_t)(((col0[j] + prow) * rp + 8 * phalf) * 2) | dead, 0, 0, 0);
     }
   }
-  if constexpr (CODEBOOK == 2) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int g0 = __builtin_amdgcn_readfirstlane((st0 * BK) >> gshift[j]);
-      zw_raw[0][j][0] = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc[j], sc_off[j], SPLIT ? (uint32_t)g0 * Np[j] * 4 : 0u, 0);
-    }
-  }
   load_stage(st0, I0{});
   __builtin_amdgcn_s_waitcnt(WAIT_VM0);
   commit_stage(I0{});
-  if constexpr (CODEBOOK == 2) {  // the first stage's tables, all at once
-    build_table_part(I0{}, I0{});
-    build_table_part(I0{}, I1{});
-    build_table_part(I0{}, I2{});
-    build_table_part(I0{}, I3{});
-  }
   __syncthreads();
   load_stage(min(st0 + 1, st_end - 1), I1{});
-  if constexpr (CODEBOOK == 1) {
-    prefetch_a(I0{}, I0{}, I0{});
-    prefetch_b(I0{}, I0{});
-  } else {
-    prefetch(I0{}, I0{}, I0{});
-  }
+  prefetch(I0{}, I0{}, I0{});
 
   // whole pairs in a single-exit loop (slots 0, 1), then the odd stage
   const int s_full = st0 + ((st_end - st0) & ~1);
@@ -1015,8 +925,7 @@ __global__ __launch_bounds__(256) void gptq_lora_fwd_finish_kernel(const FwdArgs
 
 }  // namespace
 
-// The cut of a launch.  Flavours that are compiled with it: one scale group per stage, no rotary epilogue, and not the
-// gathering code-book unpack.
+// The cut of a launch.  Flavours that are compiled with it: one scale group per stage, no rotary epilogue.
 static SplitPlan fwd_split(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
   int nb = 0;
   bool ok = true;
@@ -1024,7 +933,6 @@ static SplitPlan fwd_split(const fmsa_fwd_proj* projs, int n_proj, int M, int mo
     const fmsa_gptq_weight& w = projs[p].w;
     nb += (w.N + 255) / 256;
     ok = ok && w.group_size % 64 == 0;
-    if (w.format == FMSA_WEIGHT_CODEBOOK) ok = ok && w.code == projs[0].w.code && (w.group_size & (w.group_size - 1)) == 0;
   }
   if (mode == FMSA_FWD_SWIGLU) nb = (projs[0].w.N + 127) / 128;
   const int tiles = ((M + BM - 1) / BM) * nb;
@@ -1116,24 +1024,20 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
   }
   const bool ktail = (a.K % BK) != 0;
   const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;  // api.hip: all projections of a launch share the format
-  // table flavour: one code book for the launch, one block per 64-wide stage
   // packed-half unpack: fp16 activations and interleaved words (api.hip: then every projection is affine, interleaved, with
   // group_size % 64 == 0, and there is no rotary epilogue)
   const bool pk16 = act_dtype == FMSA_F16 && !codebook && projs[0].w.nibble_order == 1;
-  bool table = codebook && gps == 1;
-  for (int p = 0; p < n_proj; ++p)
-    table = table && projs[p].w.code == projs[0].w.code && (projs[p].w.group_size & (projs[p].w.group_size - 1)) == 0;
   if (plan.s > 1) {
 #define SPLIT_K(TT, CB, PK)                                                                                         \
   do {                                                                                                              \
     if (ktail) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, true, CB, 0, PK, true>), grid, block, 0, st, a);      \
     else hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, false, CB, 0, PK, true>), grid, block, 0, st, a);           \
   } while (0)
-    if (pk16) SPLIT_K(f16_t, 0, true);
-    else if (codebook && act_dtype == FMSA_BF16) SPLIT_K(bf16_t, 2, false);
-    else if (codebook) SPLIT_K(f16_t, 2, false);
-    else if (act_dtype == FMSA_BF16) SPLIT_K(bf16_t, 0, false);
-    else SPLIT_K(f16_t, 0, false);
+    if (pk16) SPLIT_K(f16_t, false, true);
+    else if (codebook && act_dtype == FMSA_BF16) SPLIT_K(bf16_t, true, false);
+    else if (codebook) SPLIT_K(f16_t, true, false);
+    else if (act_dtype == FMSA_BF16) SPLIT_K(bf16_t, false, false);
+    else SPLIT_K(f16_t, false, false);
 #undef SPLIT_K
     FMSA_CHECK_LAUNCH();
     const bool swiglu = mode == FMSA_FWD_SWIGLU;
@@ -1158,11 +1062,8 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
   } while (0)
 #define LAUNCH2(TT, KT)          \
   do {                           \
-    if (table && rope && rope->dtype == FMSA_F32) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, false, 2, 2>), grid, block, 0, st, a); \
-    else if (table && rope) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, false, 2, 1>), grid, block, 0, st, a); \
-    else if (table) hipLaunchKernelGGL((gptq_lora_fwd_kernel<TT, 1, KT, 2>), grid, block, 0, st, a); \
-    else if (codebook) LAUNCH3(TT, KT, 1); \
-    else LAUNCH3(TT, KT, 0); \
+    if (codebook) LAUNCH3(TT, KT, true); \
+    else LAUNCH3(TT, KT, false); \
   } while (0)
 #define LAUNCH(TT)            \
   do {                        \
@@ -1170,8 +1071,8 @@ int launch_gptq_lora_fwd(const fmsa_fwd_proj* projs, int n_proj, const void* X, 
     else LAUNCH2(TT, false);  \
   } while (0)
   if (pk16) {
-    if (ktail) hipLaunchKernelGGL((gptq_lora_fwd_kernel<f16_t, 1, true, 0, 0, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((gptq_lora_fwd_kernel<f16_t, 1, false, 0, 0, true>), grid, block, 0, st, a);
+    if (ktail) hipLaunchKernelGGL((gptq_lora_fwd_kernel<f16_t, 1, true, false, 0, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((gptq_lora_fwd_kernel<f16_t, 1, false, false, 0, true>), grid, block, 0, st, a);
   } else if (act_dtype == FMSA_BF16) {
     LAUNCH(bf16_t);
   } else {

@@ -212,6 +212,32 @@ def test_gemm_operands_are_the_dequantised_weight_bit_for_bit(blocksize, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Ns,K,blocksize,swiglu", [
+    ((96, 160), 320, 64, False), ((96, 96), 320, 64, True),
+    ((160, 32, 96), 352, 32, False), ((64, 64), 352, 32, True),  # two blocks a stage, tail of K
+    ((512, 512), 2176, 64, True), ((512, 288), 2176, 128, False),  # cut along K
+])
+def test_forward_with_a_code_book_per_projection(Ns, K, blocksize, swiglu, dtype):
+    """The forward looks codes up in a table that holds the books of a workgroup's two column tiles: one-hot tokens read every
+    projection's operand back bit for bit, each under its own code book, gate and up of a SwiGLU launch included."""
+    import fmsa_hip
+
+    g = torch.Generator().manual_seed(4)
+    projs, wants, keeps = [], [], []
+    for i, N in enumerate(Ns):
+        _, keep, q = _prepared(N, K, 41 + i, blocksize)
+        book = torch.randn(16, generator=g) * torch.tensor([1.0, 1e-3, 200.0, 1.0] * 4)
+        code = book.cuda()
+        projs.append({"w": fmsa_hip.make_codebook_weight(keep[0], code, keep[1], blocksize), "U": None, "B": None, "bias": None, "r": 0, "s": 0.0})
+        wants.append(onf4.dequant(q, _NAME[dtype], code=book.numpy()).t().contiguous())  # [K, N]
+        keeps.append((keep, code))
+    eye = torch.eye(K, dtype=dtype, device="cuda")
+    out = fmsa_hip.gptq_lora_fwd(eye, projs, fmsa_hip.FWD_SWIGLU if swiglu else fmsa_hip.FWD_LINEAR, split=K > 2048)
+    for y, want in zip(out[:2] if swiglu else out, wants):
+        assert torch.equal(y.cpu(), want + 0.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Ns,K", [((96, 160), 320), ((32, 64, 32), 64), ((2080, 1056), 256)])  # tails of a stage; the last one is cut
 def test_input_gradient_with_a_code_book_per_projection(Ns, K, dtype):
     """The twin's kernel looks codes up in a table that it lays out per projection: one-hot gradients, each token for one column
