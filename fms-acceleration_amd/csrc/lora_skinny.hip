@@ -1011,14 +1011,15 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
 // rank 64, whose eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48).
 // From 2048 tokens on above rank 16 (rank 32: 4096 at 8192 tokens 17.9 / 16.6; rank 64: 2048 at 2048 15.4 / 9.3, 4096 at 8192
 // 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99);
-// rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them and
-// short ones of many (14336 at 3217: 25.8 / 19.6; 4096 at 16384: 39 / 26).
+// rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them
+// (14336 at 3217: 25.8 / 19.6; short ones of many, 4096 at 16384: 39 / 26, would need a buffer that the size query does not ask
+// for there).
 static bool down_is_mid(int M, int r_max, int64_t columns) {
   if (M <= 64) return false;  // few tokens: the ranges of the products straight from the parameters are the fragment kernel's
   if (M >= 2048) {
     const bool many = M >= 16384, wide = columns >= 8192;
     if (columns < 2048) return false;
-    return r_max > 16 ? !(many && wide && r_max > 32) : (many ? !wide : (wide && M < 4096));
+    return r_max > 16 ? !(many && wide && r_max > 32) : (wide && M < 4096);
   }
   const int64_t bytes = (int64_t)((M + 15) / 16) * (16 + std::max(16, r_max)) * columns * 2;
   return r_max > 64 || bytes >= (r_max > 32 ? 22000000 : 14000000);
@@ -1094,26 +1095,36 @@ DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
 }
 }  // namespace
 
-size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
-  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C)) {
-    const int n = down_mid_split(M, C, r, rank_blocks(r));
-    return n > 1 ? (size_t)n * M * r * sizeof(float) : 0;
-  }
+static size_t down_mid_bytes(int M, int C, int r) {
+  const int n = down_mid_split(M, C, r, rank_blocks(r));
+  return n > 1 ? (size_t)n * M * r * sizeof(float) : 0;
+}
+
+static size_t down_split_bytes(int M, int C, int r, bool few_tokens) {
   const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
   const int ranks = d.g == 1 ? r : std::min(r, 64);
   return d.g && d.n_split > 1 ? (size_t)d.n_split * (size_t)M * (size_t)ranks * sizeof(float) : 0;
 }
 
+// Enough for either kernel, so that the answer for a shape does not depend on which of them is the faster one today.
+size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
+  const bool mid = (few_tokens || M >= 2048) && down_is_mid(M, r, C);
+  return std::max(mid ? down_mid_bytes(M, C, r) : 0, down_split_bytes(M, C, r, few_tokens));
+}
+
 // The split kernel where it pays and the caller brought the partial-sum buffer (or none is needed); launch_lora_down otherwise.
 int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
                         int64_t ldo, void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st) {
-  const size_t need = lora_down_workspace(M, C, r, few_tokens);
-  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C) && (!need || (workspace && workspace_bytes >= need && (uintptr_t)out % 8 == 0 && ldo % 4 == 0))) {
-    LoraDownArgs a{};
-    a.M = M;
-    a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
-    return launch_down_mid(a, 1, act_dtype, st);
+  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C)) {
+    const size_t mid = down_mid_bytes(M, C, r);
+    if (!mid || (workspace && workspace_bytes >= mid && (uintptr_t)out % 8 == 0 && ldo % 4 == 0)) {
+      LoraDownArgs a{};
+      a.M = M;
+      a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
+      return launch_down_mid(a, 1, act_dtype, st);
+    }
   }
+  const size_t need = down_split_bytes(M, C, r, few_tokens);
   const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
   const bool out_ok = ((uintptr_t)out % 8 == 0) && ldo % 4 == 0;  // the reduce pass stores four ranks at a time
   if (!d.g || (need && (!workspace || workspace_bytes < need || !out_ok)))
