@@ -43,8 +43,8 @@ int launch_rms_fwd(const void* X, int64_t ldx, const void* W, int M, int C, floa
                    int64_t ldy, float* r, hipStream_t st);
 int launch_rms_bwd(void* dY, int64_t lddy, const void* X, int64_t ldx, const void* W, const float* r, int M, int C, int gemma,
                    int x_dtype, int w_dtype, hipStream_t st);
-int launch_rope(void* Q, int64_t ldq, const void* cosp, const void* sinp, int64_t ldcs, int M, int n_heads, int head_dim, int cs_rows,
-                int backward, int q_dtype, int cs_dtype, hipStream_t st);
+int launch_rope(void* Q, int64_t ldq, int n_heads, void* K, int64_t ldk, int k_heads, const void* cosp, const void* sinp, int64_t ldcs,
+                int M, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype, hipStream_t st);
 int launch_rope_strided(const void* src, int64_t s_batch, int64_t s_tok, int64_t s_head, void* dst, const void* cosp, const void* sinp,
                         int64_t ldcs, int batch, int seq, int n_heads, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype,
                         hipStream_t st);
@@ -646,15 +646,27 @@ int fmsa_rms_layernorm_bwd(void* dY, int64_t lddy, const void* X, int64_t ldx, c
   return launch_rms_bwd(dY, lddy, X, ldx, W, r, M, C, gemma, x_dtype, w_dtype, (hipStream_t)stream);
 }
 
+static int rope_embedding(void* Q, int64_t ldq, int n_heads, void* K, int64_t ldk, int k_heads, const void* cos, const void* sin,
+                          int64_t ldcs, int M, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype, void* stream) {
+  if (!Q || !cos || !sin || (k_heads && !K)) return FMSA_ERR_NULL;
+  if (M <= 0 || n_heads <= 0 || k_heads < 0 || head_dim <= 0 || head_dim % 16 != 0 || cs_rows <= 0) return FMSA_ERR_SHAPE;
+  if (ldq < (int64_t)n_heads * head_dim || (k_heads && ldk < (int64_t)k_heads * head_dim) || ldcs < head_dim / 2) return FMSA_ERR_SHAPE;
+  if (!is_float_dtype(q_dtype) || !is_float_dtype(cs_dtype)) return FMSA_ERR_DTYPE;
+  if (!aligned_rows(Q, ldq, q_dtype) || (k_heads && !aligned_rows(K, ldk, q_dtype)) || !aligned_rows(cos, ldcs, cs_dtype) ||
+      !aligned_rows(sin, ldcs, cs_dtype))
+    return FMSA_ERR_ALIGN;
+  return launch_rope(Q, ldq, n_heads, K, ldk, k_heads, cos, sin, ldcs, M, head_dim, cs_rows, backward, q_dtype, cs_dtype, (hipStream_t)stream);
+}
+
 int fmsa_rope_embedding(void* Q, int64_t ldq, const void* cos, const void* sin, int64_t ldcs, int M, int n_heads,
                         int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype, void* stream) {
-  if (!Q || !cos || !sin) return FMSA_ERR_NULL;
-  if (M <= 0 || n_heads <= 0 || head_dim <= 0 || head_dim % 16 != 0 || cs_rows <= 0) return FMSA_ERR_SHAPE;
-  if (ldq < (int64_t)n_heads * head_dim || ldcs < head_dim / 2) return FMSA_ERR_SHAPE;
-  if (!is_float_dtype(q_dtype) || !is_float_dtype(cs_dtype)) return FMSA_ERR_DTYPE;
-  if (!aligned_rows(Q, ldq, q_dtype) || !aligned_rows(cos, ldcs, cs_dtype) || !aligned_rows(sin, ldcs, cs_dtype))
-    return FMSA_ERR_ALIGN;
-  return launch_rope(Q, ldq, cos, sin, ldcs, M, n_heads, head_dim, cs_rows, backward, q_dtype, cs_dtype, (hipStream_t)stream);
+  return rope_embedding(Q, ldq, n_heads, nullptr, 0, 0, cos, sin, ldcs, M, head_dim, cs_rows, backward, q_dtype, cs_dtype, stream);
+}
+
+int fmsa_rope_embedding_pair(void* Q, int64_t ldq, int n_heads, void* K, int64_t ldk, int k_heads, const void* cos, const void* sin,
+                             int64_t ldcs, int M, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype, void* stream) {
+  if (k_heads <= 0) return FMSA_ERR_SHAPE;
+  return rope_embedding(Q, ldq, n_heads, K, ldk, k_heads, cos, sin, ldcs, M, head_dim, cs_rows, backward, q_dtype, cs_dtype, stream);
 }
 
 int fmsa_rope_embedding_strided(const void* src, int64_t stride_batch, int64_t stride_token, int64_t stride_head, void* dst,

@@ -584,6 +584,23 @@ PyObject* rope_embedding_(PyObject* const* a, Py_ssize_t) {  // q2d, cos2d, sin2
   return a[0];
 }
 
+PyObject* rope_embedding_pair_(PyObject* const* a, Py_ssize_t) {  // q2d, k2d, cos2d, sin2d, head_dim
+  const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &c = tensor(a[2]), &s = tensor(a[3]);
+  on_gpu(q.is_cuda() && k.is_cuda() && c.is_cuda() && s.is_cuda());
+  const int hd = (int)integer(a[4]);
+  need(q.dim() == 2 && k.dim() == 2 && q.size(0) == k.size(0) && q.stride(1) == 1 && k.stride(1) == 1 && q.scalar_type() == k.scalar_type() &&
+           q.device() == k.device() && hd > 0 && q.size(1) % hd == 0 && k.size(1) % hd == 0,
+       "rope_embedding_pair_: q2d, k2d");
+  need(c.stride(1) == 1 && c.strides() == s.strides() && c.scalar_type() == s.scalar_type(), "rope_embedding_pair_: cos2d, sin2d");
+  void* st = stream(q);
+  const int qd = dtype_enum(q.scalar_type()), cd = dtype_enum(c.scalar_type());
+  check("fmsa_rope_embedding_pair", unlocked([&] {
+          return fmsa_rope_embedding_pair(ptr(q), q.stride(0), (int)(q.size(1) / hd), ptr(k), k.stride(0), (int)(k.size(1) / hd), ptr(c), ptr(s),
+                                          c.stride(0), (int)q.size(0), hd, (int)c.size(0), 0, qd, cd, st);
+        }));
+  Py_RETURN_NONE;
+}
+
 PyObject* rope_embedding_strided(PyObject* const* a, Py_ssize_t) {  // q4d, cos2d, sin2d, backward
   const at::Tensor &q = tensor(a[0]), &c = tensor(a[1]), &s = tensor(a[2]);
   on_gpu(q.is_cuda() && c.is_cuda() && s.is_cuda());
@@ -611,7 +628,8 @@ PyObject* install(PyObject* const* a, Py_ssize_t) {  // FmsaError
 PyMethodDef g_methods[] = {ENTRY(lora_down, 3),           ENTRY(lora_down_batch, 2),   ENTRY(lora_grad_batch, 2),
                            ENTRY(lora_pack_batch, 3),     ENTRY(gptq_lora_fwd, 4),     ENTRY(gptq_lora_bwd_dx, 7),
                            ENTRY(lora_few, 3),            ENTRY(rms_layernorm_fwd, 4), ENTRY(rms_layernorm_bwd, 5),
-                           ENTRY(rope_embedding_, 6),     ENTRY(rope_embedding_strided, 4), ENTRY(install, 1),
+                           ENTRY(rope_embedding_, 6),     ENTRY(rope_embedding_pair_, 5),
+                           ENTRY(rope_embedding_strided, 4), ENTRY(install, 1),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fmsa_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -251,18 +251,26 @@ __global__ __launch_bounds__(256) void rms_bwd_reg_kernel(void* __restrict__ dY,
 
 // In place: (q1, q2) <- (q1 cos - q2 sin, q2 cos + q1 sin) on the two halves of every head, sin
 // negated for the backward pass (rope_embedding.py:36-65).  One thread = 8 + 8 elements; the
-// position of row m is m % cs_rows.  fp32 arithmetic, one rounding to Q's type.
+// position of row m is m % cs_rows.  fp32 arithmetic, one rounding to Q's type.  Heads from n_heads on are K's, k_heads of
+// them (0: none): a few tokens' rotation is a launch and little else, so Q and K of one call share it where no graph is
+// built (a layer's decode step of one token 152 -> 145 us, most of it the second call on the host).
 template <int QD, int CD>
-__global__ __launch_bounds__(256) void rope_kernel(void* __restrict__ Q, int64_t ldq, const void* __restrict__ cosp,
-                                                   const void* __restrict__ sinp, int64_t ldcs, int M, int n_heads, int head_dim,
-                                                   int cs_rows, float sin_sign) {
+__global__ __launch_bounds__(256) void rope_kernel(void* __restrict__ Q, int64_t ldq, void* __restrict__ K, int64_t ldk,
+                                                   const void* __restrict__ cosp, const void* __restrict__ sinp, int64_t ldcs, int M,
+                                                   int n_heads, int k_heads, int head_dim, int cs_rows, float sin_sign) {
   const int chunks = head_dim / 16;  // 8-element chunks in half a head
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t per_row = (int64_t)n_heads * chunks;
+  const int64_t per_row = (int64_t)(n_heads + k_heads) * chunks;
   if (idx >= (int64_t)M * per_row) return;
   const int row = (int)(idx / per_row);
   const int rem = (int)(idx % per_row);
-  const int head = rem / chunks, ch = rem % chunks;
+  int head = rem / chunks;
+  const int ch = rem % chunks;
+  if (head >= n_heads) {
+    head -= n_heads;
+    Q = K;
+    ldq = ldk;
+  }
   const int64_t cso = (int64_t)(row % cs_rows) * ldcs + 8 * ch;
   const int64_t q1o = (int64_t)row * ldq + (int64_t)head * head_dim + 8 * ch;
   const int64_t q2o = q1o + head_dim / 2;
@@ -388,13 +396,14 @@ int launch_rope_strided(const void* src, int64_t s_batch, int64_t s_tok, int64_t
   return FMSA_OK;
 }
 
-int launch_rope(void* Q, int64_t ldq, const void* cosp, const void* sinp, int64_t ldcs, int M, int n_heads, int head_dim, int cs_rows,
-                int backward, int q_dtype, int cs_dtype, hipStream_t st) {
-  const int64_t n = (int64_t)M * n_heads * (head_dim / 16);
+int launch_rope(void* Q, int64_t ldq, int n_heads, void* K, int64_t ldk, int k_heads, const void* cosp, const void* sinp, int64_t ldcs,
+                int M, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype, hipStream_t st) {
+  const int64_t n = (int64_t)M * (n_heads + k_heads) * (head_dim / 16);
   dim3 grid((unsigned)((n + 255) / 256)), block(256);
   const float sign = backward ? -1.0f : 1.0f;
   FMSA_DISPATCH_DTYPE(q_dtype, QD, FMSA_DISPATCH_DTYPE(cs_dtype, CD, {
-    hipLaunchKernelGGL((rope_kernel<QD, CD>), grid, block, 0, st, Q, ldq, cosp, sinp, ldcs, M, n_heads, head_dim, cs_rows, sign);
+    hipLaunchKernelGGL((rope_kernel<QD, CD>), grid, block, 0, st, Q, ldq, K, ldk, cosp, sinp, ldcs, M, n_heads, k_heads, head_dim,
+                       cs_rows, sign);
   }))
   FMSA_CHECK_LAUNCH();
   return FMSA_OK;

@@ -11,7 +11,7 @@ import torch
 
 import fmsa_hip
 
-from ...autograd import run
+from ...autograd import no_graph, run
 
 
 def _rows(t, batch, seq_len):
@@ -78,6 +78,16 @@ def fast_rope_embedding(Q, K, cos, sin, position_ids=None, unsqueeze_dim=1):
             if done[1].untyped_storage().data_ptr() != K.untyped_storage().data_ptr():
                 raise RuntimeError("fast_rope_embedding: Q comes rotated from the fused projection, K does not")
             return Q, K
+    if no_graph():
+        q, k = Q.transpose(1, 2), K.transpose(1, 2)
+        if (q.is_contiguous() and k.is_contiguous() and q.dtype == k.dtype and q.device == k.device and q.dim() == k.dim() == 4
+                and q.shape[:2] == k.shape[:2] and q.shape[3] == k.shape[3] and q.numel() and k.numel()
+                and q.untyped_storage().data_ptr() != k.untyped_storage().data_ptr()):
+            # one launch for both; no memory of theirs is shared, so their order does not matter
+            batch, seq_len, _, head_dim = q.shape
+            fmsa_hip.rope_embedding_pair_(q.view(batch * seq_len, -1), k.view(batch * seq_len, -1), _rows(cos, batch, seq_len),
+                                          _rows(sin, batch, seq_len), head_dim)
+            return q.transpose(1, 2), k.transpose(1, 2)
     Q = run(Fast_RoPE_Embedding, Q.transpose(1, 2), cos, sin).transpose(1, 2)
     K = run(Fast_RoPE_Embedding, K.transpose(1, 2), cos, sin).transpose(1, 2)
     return Q, K

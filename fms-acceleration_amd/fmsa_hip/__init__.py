@@ -67,6 +67,7 @@ EXPORTED_SYMBOLS = (
     "fmsa_rms_layernorm_fwd",
     "fmsa_rms_layernorm_bwd",
     "fmsa_rope_embedding",
+    "fmsa_rope_embedding_pair",
     "fmsa_rope_embedding_strided",
     "fmsa_cross_entropy_fwd",
     "fmsa_cross_entropy_bwd",
@@ -310,6 +311,8 @@ def lib() -> ctypes.CDLL:
                                          c_int, c_void_p]
     L.fmsa_rope_embedding.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int,
                                       c_int, c_void_p]
+    L.fmsa_rope_embedding_pair.argtypes = [c_void_p, c_int64, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                           c_int, c_int, c_int, c_int, c_void_p]
     L.fmsa_rope_embedding_strided.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                               c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]
     L.fmsa_cross_entropy_fwd.argtypes = [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]
@@ -707,6 +710,11 @@ def rope_embedding_(q2d, cos2d, sin2d, n_heads: int, head_dim: int, backward: bo
         assert q2d.shape[2:] == (n_heads, head_dim)
         return rope_embedding_strided(q2d, cos2d, sin2d, backward)
     return (_native or native()).rope_embedding_(q2d, cos2d, sin2d, n_heads, head_dim, backward)
+
+
+def rope_embedding_pair_(q2d, k2d, cos2d, sin2d, head_dim: int):
+    """rope_embedding_ of q2d [M, n_heads * head_dim] and k2d [M, k_heads * head_dim], which do not overlap, in one launch."""
+    return (_native or native()).rope_embedding_pair_(q2d, k2d, cos2d, sin2d, head_dim)
 
 
 def rope_strided_ok(q4d, cos2d, sin2d) -> bool:

@@ -440,6 +440,10 @@ int fmsa_rms_layernorm_bwd(void* dY, int64_t lddy, const void* X, int64_t ldx, c
 int fmsa_rope_embedding(void* Q, int64_t ldq, const void* cos, const void* sin, int64_t ldcs, int M,
                         int n_heads, int head_dim, int cs_rows, int backward, int q_dtype, int cs_dtype,
                         void* stream);
+/* The same in one launch for Q [M, n_heads * head_dim] and K [M, k_heads * head_dim] of one type, which do not overlap. */
+int fmsa_rope_embedding_pair(void* Q, int64_t ldq, int n_heads, void* K, int64_t ldk, int k_heads, const void* cos,
+                             const void* sin, int64_t ldcs, int M, int head_dim, int cs_rows, int backward, int q_dtype,
+                             int cs_dtype, void* stream);
 /* The same rotation out of src [batch, seq, n_heads, head_dim] of any element strides (last dimension contiguous, the others
  * multiples of 16 bytes) into dst, contiguous rows [batch * seq, n_heads * head_dim]; src is left alone. */
 int fmsa_rope_embedding_strided(const void* src, int64_t stride_batch, int64_t stride_token, int64_t stride_head, void* dst,
