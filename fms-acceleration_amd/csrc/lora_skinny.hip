@@ -1115,19 +1115,17 @@ size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
 // The split kernel where it pays and the caller brought the partial-sum buffer (or none is needed); launch_lora_down otherwise.
 int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C, int r, int act_dtype, void* out,
                         int64_t ldo, void* workspace, size_t workspace_bytes, bool few_tokens, hipStream_t st) {
-  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C)) {
-    const size_t mid = down_mid_bytes(M, C, r);
-    if (!mid || (workspace && workspace_bytes >= mid && (uintptr_t)out % 8 == 0 && ldo % 4 == 0)) {
-      LoraDownArgs a{};
-      a.M = M;
-      a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
-      return launch_down_mid(a, 1, act_dtype, st);
-    }
+  const size_t need = lora_down_workspace(M, C, r, few_tokens);
+  // a buffer smaller than the query's answer is as good as none; the reduce pass stores four ranks at a time
+  const bool sums = workspace && workspace_bytes >= need && (uintptr_t)out % 8 == 0 && ldo % 4 == 0;
+  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C) && (sums || !down_mid_bytes(M, C, r))) {
+    LoraDownArgs a{};
+    a.M = M;
+    a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
+    return launch_down_mid(a, 1, act_dtype, st);
   }
-  const size_t need = down_split_bytes(M, C, r, few_tokens);
   const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
-  const bool out_ok = ((uintptr_t)out % 8 == 0) && ldo % 4 == 0;  // the reduce pass stores four ranks at a time
-  if (!d.g || (need && (!workspace || workspace_bytes < need || !out_ok)))
+  if (!d.g || (down_split_bytes(M, C, r, few_tokens) && !sums))
     return launch_lora_down(X, ldx, Wd, M, C, r, act_dtype, out, ldo, st);
   auto reduce = [&]() -> int {
     const int64_t quads = (int64_t)M * (r / 4);
