@@ -13,10 +13,13 @@ class NoGraph:
 
 
 def no_graph() -> bool:
-    """Whether a call can run its forward by itself, without an autograd node: no gradients are recorded, and neither
-    forward-mode AD nor a functorch transform (which would ask the autograd function for its rules) is active."""
+    """Whether a call can run its forward by itself, without an autograd node: no gradients are recorded, neither
+    forward-mode AD nor a functorch transform (which would ask the autograd function for its rules) is active, and
+    torch.jit is not tracing (the kernels are no torch operators: a graph that does not hold the autograd function holds
+    the allocation of its outputs and nothing that fills them)."""
     return (not torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0  # pylint: disable=protected-access
-            and not torch._C._are_functorch_transforms_active())  # pylint: disable=protected-access
+            and not torch._C._are_functorch_transforms_active()  # pylint: disable=protected-access
+            and torch._C._get_tracing_state() is None)  # pylint: disable=protected-access
 
 
 def run(function, *args):

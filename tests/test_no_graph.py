@@ -33,6 +33,62 @@ def test_a_node_where_something_can_follow():
         assert no_graph()
 
 
+class _Opaque(torch.autograd.Function):
+    """Fills its output behind torch's back, as the kernels do."""
+
+    @staticmethod
+    def forward(ctx, x):
+        y = torch.empty_like(x)
+        y.numpy()[...] = 3.0 * x.numpy()
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        return 3 * dy
+
+
+def _traced(f, *args):
+    """f under no_grad as torch.jit.trace records it, run on inputs of its own."""
+    with torch.no_grad():
+        return torch.jit.trace(f, tuple(torch.zeros_like(a) for a in args), check_trace=False)(*args)
+
+
+def test_a_trace_holds_the_autograd_function():
+    x = torch.arange(6.0).view(2, 3)
+    assert torch.equal(_traced(lambda t: run(_Opaque, t), x), 3 * x)
+
+
+def test_traces_of_the_norm_and_the_rotation(monkeypatch):
+    """The operators that need no GPU to be entered, over stand-ins for their kernels."""
+    import fmsa_hip
+    from fms_acceleration_foak.kernels.unsloth import fast_rms_layernorm, fast_rope_embedding
+
+    def norm(x, w, eps, gemma=False):
+        y = torch.empty_like(x)
+        y.numpy()[...] = 2.0 * x.numpy()
+        return y, torch.empty(x.shape[0])
+
+    def rotate(q, cos, sin, n_heads, head_dim, backward=False, strided=False):
+        q.numpy()[...] *= -1.0
+        return q
+
+    def rotate_pair(q, k, cos, sin, head_dim):
+        rotate(q, cos, sin, 0, head_dim)
+        rotate(k, cos, sin, 0, head_dim)
+
+    monkeypatch.setattr(fmsa_hip, "rms_layernorm_fwd", norm)
+    monkeypatch.setattr(fmsa_hip, "rope_embedding_", rotate)
+    monkeypatch.setattr(fmsa_hip, "rope_embedding_pair_", rotate_pair)
+    layer = torch.nn.Module()
+    layer.weight, layer.variance_epsilon = torch.nn.Parameter(torch.ones(8), requires_grad=False), 1e-5
+    x = torch.randn(4, 8)
+    assert torch.equal(_traced(lambda t: fast_rms_layernorm(layer, t), x), 2 * x)
+    q, k, cos = torch.randn(1, 5, 4, 16), torch.randn(1, 5, 2, 16), torch.ones(5, 16)
+    rotated = _traced(lambda a, b: fast_rope_embedding(a.clone().transpose(1, 2), b.clone().transpose(1, 2), cos, cos), q, k)
+    for got, want in zip(rotated, (q, k)):
+        assert torch.equal(got, -want.transpose(1, 2))
+
+
 @pytest.mark.gpu
 def test_backward_meets_the_autocast_state_of_its_forward():
     seen = []
