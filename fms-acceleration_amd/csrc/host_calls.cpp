@@ -192,6 +192,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // ---- rank-r products ----------------------------------------------------------------------------------------------------
 at::Tensor down_one(const at::Tensor& x, const at::Tensor& wd, at::Tensor out) {
+  need(x.dim() == 2, "lora_down: x2d");
   const int64_t M = x.size(0), C = x.size(1), r = wd.size(0);
   need(wd.size(1) == C && wd.is_contiguous() && wd.scalar_type() == x.scalar_type() && x.stride(1) == 1, "lora_down: x2d, wd");
   if (!out.defined()) out = empty({M, r}, x);
@@ -231,6 +232,7 @@ PyObject* lora_down_batch(PyObject* const* a, Py_ssize_t) {  // jobs, most token
     for (const Job& j : js) outs.push_back(down_one(j.x, j.wd, j.out));
     return wrap_list(outs);
   }
+  for (const Job& j : js) need(j.x.dim() == 2 && j.wd.dim() == 2, "lora_down_batch: x2d, wd");
   const at::Tensor& x0 = js[0].x;
   const int act = act_enum(x0.scalar_type());
   void* st = stream(x0);
@@ -284,8 +286,8 @@ PyObject* lora_grad_batch(PyObject* const* a, Py_ssize_t) {  // jobs, most of th
       need(L.size(0) == M && R.size(0) == M && L.stride(1) == 1 && R.stride(1) == 1, "lora_grad_batch: L, R");
       need(L.scalar_type() == R.scalar_type() && R.scalar_type() == r0.scalar_type(), "lora_grad_batch: dtypes");
       if (Wt.defined()) {
-        need(Wt.size(0) == r && Wt.size(1) == C && Wt.is_contiguous() && Wt.scalar_type() == R.scalar_type(), "lora_grad_batch: Wt");
-        need(T.defined() && T.size(0) == M && T.size(1) == r && T.stride(1) == 1 && T.scalar_type() == R.scalar_type(), "lora_grad_batch: T_out");
+        need(Wt.dim() == 2 && Wt.size(0) == r && Wt.size(1) == C && Wt.is_contiguous() && Wt.scalar_type() == R.scalar_type(), "lora_grad_batch: Wt");
+        need(T.defined() && T.dim() == 2 && T.size(0) == M && T.size(1) == r && T.stride(1) == 1 && T.scalar_type() == R.scalar_type(), "lora_grad_batch: T_out");
       }
       const bool tr = truth(j[3]);
       const at::ScalarType od = dtype_of(j[4]);
@@ -329,6 +331,7 @@ PyObject* lora_pack_batch(PyObject* const* a, Py_ssize_t) {  // adapters, act_dt
     Sequence j(adapters[i]);
     need(j.size() == 3, "lora_pack_batch: (A, B, A16_out)");
     at::Tensor A = tensor(j[0]), B = tensor(j[1]), A16 = optional(j[2]);
+    need(A.dim() == 2, "lora_pack_batch: A");
     if (!(A.is_cuda() && B.is_cuda())) {
       PyErr_SetString(PyExc_RuntimeError, "fmsa_hip needs GPU tensors");
       throw PyFailure();
