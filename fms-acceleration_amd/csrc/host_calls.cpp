@@ -75,6 +75,12 @@ void* stream(const at::Tensor& t) {
   return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream();
 }
 
+void on_gpu(bool ok) {
+  if (ok) return;
+  PyErr_SetString(PyExc_RuntimeError, "fmsa_hip needs GPU tensors");
+  throw PyFailure();
+}
+
 // The call itself without the interpreter lock: a full launch queue blocks it.
 template <typename F> int unlocked(F&& f) {
   PyThreadState* s = PyEval_SaveThread();
@@ -494,20 +500,27 @@ PyObject* lora_few(PyObject* const* a, Py_ssize_t) {  // x2d, ((w, A, B, bias, s
   const at::Tensor& x = tensor(a[0]);
   Sequence projs(a[1]);
   const int n = (int)projs.size(), mode = (int)integer(a[2]);
-  need(n >= 1 && n <= 3 && x.dim() == 2, "lora_few: one to three projections of x2d [M, K]");
+  need(n >= 1 && n <= 3 && x.dim() == 2 && x.stride(1) == 1, "lora_few: one to three projections of x2d [M, K]");
   const int M = (int)x.size(0);
+  bool adapters_on_gpu = true;
   fmsa_few_proj arr[3] = {};
   for (int i = 0; i < n; ++i) {
     Sequence p(projs[i]);
     need(p.size() == 5, "lora_few: (w, A, B, bias, s)");
     fmsa_few_proj& q = arr[i];
     q.w = weight(p[0]);
+    need(x.size(1) == q.w.K, "lora_few: x2d, w");
     q.ldy = q.w.N;
-    q.bias = ptr(optional(p[3]));
+    const at::Tensor bias = optional(p[3]);
+    need(!bias.defined() || (bias.numel() == q.w.N && bias.is_contiguous() && bias.scalar_type() == x.scalar_type()), "lora_few: bias");
+    q.bias = ptr(bias);
     const at::Tensor A = optional(p[1]);
     if (A.defined()) {
       const at::Tensor& B = tensor(p[2]);
-      need(A.size(1) == q.w.K && B.size(0) == q.w.N && B.size(1) == A.size(0), "lora_few: A, B");
+      need(A.dim() == 2 && B.dim() == 2 && A.size(1) == q.w.K && B.size(0) == q.w.N && B.size(1) == A.size(0) && A.is_contiguous() &&
+               B.is_contiguous() && A.scalar_type() == B.scalar_type(),
+           "lora_few: A, B");
+      adapters_on_gpu = adapters_on_gpu && A.is_cuda() && B.is_cuda();
       q.A = ptr(A);
       q.B = ptr(B);
       q.r = (int)A.size(0);
@@ -516,6 +529,7 @@ PyObject* lora_few(PyObject* const* a, Py_ssize_t) {  // x2d, ((w, A, B, bias, s
     }
   }
   if (!fmsa_lora_few_is_few(arr, n, M, mode)) Py_RETURN_NONE;
+  on_gpu(adapters_on_gpu);
   at::Tensor h;
   std::vector<at::Tensor> outs;
   if (mode == FMSA_FWD_SWIGLU)
@@ -536,12 +550,6 @@ PyObject* lora_few(PyObject* const* a, Py_ssize_t) {  // x2d, ((w, A, B, bias, s
 }
 
 // ---- norm and rotary embedding --------------------------------------------------------------------------------------------
-void on_gpu(bool ok) {
-  if (ok) return;
-  PyErr_SetString(PyExc_RuntimeError, "fmsa_hip needs GPU tensors");
-  throw PyFailure();
-}
-
 PyObject* rms_layernorm_fwd(PyObject* const* a, Py_ssize_t) {  // x2d, weight, eps, gemma
   const at::Tensor &x = tensor(a[0]), &w = tensor(a[1]);
   on_gpu(x.is_cuda() && w.is_cuda());

@@ -28,3 +28,28 @@ def _grad(Wt, T):
 def test_operands_that_are_no_matrices(call):
     with pytest.raises(AssertionError):
         call()
+
+
+def _few(x=None, A=None, B=None, bias=None, K=4096, N=4096):
+    """lora_few on a weight that is described only: nothing is read before the refusal."""
+    w = fmsa_hip.GptqWeight(0x1000, 0x1000, 0x1000, None, K, N, 128, 0, fmsa_hip.WEIGHT_AFFINE, 0, None, None)
+    x = _t(4, K) if x is None else x
+    A, B = torch.zeros(16, K) if A is None else A, torch.zeros(N, 16) if B is None else B
+    return fmsa_hip.lora_few(x, [(w, A, B, bias, 2.0)])
+
+
+@pytest.mark.parametrize("kw", [
+    {"x": _t(4, 2048)}, {"x": _t(4, 8192)[:, ::2]},
+    {"A": torch.zeros(16, 4096, dtype=torch.bfloat16)}, {"B": torch.zeros(4096, 16, dtype=torch.bfloat16)},
+    {"A": torch.zeros(4096, 16).t()}, {"B": torch.zeros(16, 4096).t()}, {"A": torch.zeros(16, 4096, 1)}, {"B": torch.zeros(4096, 16, 1)},
+    {"bias": torch.zeros(4096)}, {"bias": _t(4095)}, {"bias": _t(8192)[::2]},
+], ids=["columns of x", "stride of x", "type of A", "type of B", "order of A", "order of B", "A", "B", "type of bias", "length of bias",
+        "stride of bias"])
+def test_lora_few_takes_what_its_kernels_read(kw):
+    with pytest.raises(AssertionError):
+        _few(**kw)
+
+
+def test_lora_few_gets_as_far_as_the_gpu():
+    with pytest.raises(RuntimeError, match="GPU"):
+        _few(bias=_t(4096))
