@@ -632,7 +632,7 @@ PyObject* install(PyObject* const* a, Py_ssize_t) {  // FmsaError
   Py_INCREF(a[0]);
   Py_XDECREF(g_fmsa_error);
   g_fmsa_error = a[0];
-  return PyLong_FromLong(fmsa_abi_version());
+  return PyLong_FromLong(FMSA_ABI_VERSION);  // of the structs that were compiled in, whatever library is loaded
 }
 
 #define ENTRY(name, n) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, n>)), METH_FASTCALL, nullptr}

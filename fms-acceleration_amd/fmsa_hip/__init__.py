@@ -356,7 +356,7 @@ def native():
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
         if module.install(FmsaError) != ABI_VERSION:
-            raise RuntimeError(f"{CALLS_PATH} was built against another library than {LIB_PATH}: rebuild both")
+            raise RuntimeError(f"{CALLS_PATH} was built for another ABI version than {ABI_VERSION}, that of {LIB_PATH}: rebuild both")
         _native = module
     return _native
 

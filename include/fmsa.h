@@ -43,8 +43,9 @@ enum fmsa_dtype { FMSA_F16 = 0, FMSA_BF16 = 1, FMSA_F32 = 2 };
 /* Human-readable text for an error code (host pointer to a static string). */
 const char* fmsa_strerror(int code);
 
-/* ABI version; bumped on any change of a signature or struct layout (11 here).  A binding should refuse a library whose
- * version is not the one it was written for. */
+/* ABI version; bumped on any change of a signature or struct layout.  A binding should refuse a library whose version
+ * (fmsa_abi_version) is not the one it was written for, or, in C, compiled against (FMSA_ABI_VERSION). */
+#define FMSA_ABI_VERSION 11
 int fmsa_abi_version(void);
 
 /* ------------------------------------------------------------------------------------------

@@ -27,6 +27,14 @@ def test_header_and_library_agree():
     assert lib.fmsa_strerror(0) == b"ok" and b"NULL" in lib.fmsa_strerror(-1)
 
 
+def test_the_extension_tells_the_version_of_its_own_header():
+    """What it reports is compiled in with its struct layouts; the library's answer says nothing about them."""
+    header = open(os.path.join(ROOT, "include", "fmsa.h")).read()
+    assert int(re.search(r"#define FMSA_ABI_VERSION (\d+)", header).group(1)) == fmsa_hip.ABI_VERSION
+    assert fmsa_hip.native().install(fmsa_hip.FmsaError) == fmsa_hip.ABI_VERSION
+    assert b"fmsa_abi_version" not in open(fmsa_hip.CALLS_PATH, "rb").read()
+
+
 def test_probe_is_a_library_of_its_own():
     """The MFMA-loop probe of `bench.py --yardsticks` is measurement support: the product library does not export it;
     its own library does, and checks its arguments before any HIP call."""
