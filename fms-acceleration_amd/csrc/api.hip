@@ -755,8 +755,10 @@ int fmsa_causal_lm_loss_fwd(const void* logits, void* kept, int64_t ld, const in
   if (kept && ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(kept)) & 15u)) return FMSA_ERR_ALIGN;
   if (!workspace || workspace_bytes < fmsa_causal_lm_loss_workspace(n_seq, seq_out, V)) return FMSA_ERR_WORKSPACE;
   if (!aligned16(workspace)) return FMSA_ERR_ALIGN;
-  return launch_ce_rows_fwd(logits, kept, ld, labels, label_stride, n_seq, seq_in, seq_out, V, dtype, ce_rows_parts(n_seq * seq_out, V),
-                            (float*)workspace, nullptr, logsumexp, targets, loss, count, mean != 0, (hipStream_t)stream);
+  const int parts = ce_rows_parts(n_seq * seq_out, V);
+  float* const sums = (float*)workspace;  // the parts' pairs, or the losses of whole rows
+  return launch_ce_rows_fwd(logits, kept, ld, labels, label_stride, n_seq, seq_in, seq_out, V, dtype, parts, parts > 1 ? sums : nullptr,
+                            parts > 1 ? nullptr : sums, logsumexp, targets, loss, count, mean != 0, (hipStream_t)stream);
 }
 
 int fmsa_causal_lm_loss_bwd(const void* logits, void* grad, int64_t ld, const float* dloss, const float* count, const float* logsumexp,

@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(void* __restrict__ logits, 
 
 // The causal-LM loss straight on the model's 16-bit logits [sequences, seq_in, V]: rows 0 .. seq_out - 1 of every sequence
 // count (seq_out = seq_in - 1 where the labels are shifted against the logits).  Forward: one read of the logits, by `parts`
-// workgroups a row; their (max, sum) pairs, the labels, the losses, their sum and the mean meet in a second launch of one
+// workgroups a row; their (max, sum) pairs, and of every call the losses, their sum and the mean, meet in a second launch of one
 // workgroup.  Backward: one read, and one write of a gradient of its own, whole: the rows past seq_out and the rows without a
 // label are written as zeros and not read.  Bound by HBM: 0.37 GB forward where the live rows are kept for the backward (KEEP:
 // the caller may overwrite the logits in between) and 0.45 GB backward at 1024 x 128256, three rows in ten without a label,
@@ -561,8 +561,8 @@ struct CeRowsArgs {
   const int64_t* labels;  // row t of sequence q: labels[q * label_seq + t]
   int64_t label_seq;
   int seq_in, seq_out, V, rows, parts;
-  float *pm, *ps;  // [parts][rows]: running maximum and sum of exp(. - maximum) of a part
-  float *losses, *lse;
+  float *pm, *ps;  // parts > 1: [parts][rows], running maximum and sum of exp(. - maximum) of a part
+  float *losses, *lse;  // losses: of whole rows (parts == 1)
   int64_t* targets;  // contiguous labels for the backward, or nullptr
   float *sum, *count;  // sum of the losses (mean != 0: over the number of labels that are not -100) and that number, or nullptr
   int mean;
@@ -576,7 +576,11 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const CeRowsArgs a) {
   __shared__ float red_m[256], red_s[256];
   const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x, V = a.V;
   const int64_t label = row_label(a, row);
-  if (label < 0 || label >= V) return;  // ignored (or a caller error, treated as such): uniform over the workgroup
+  if (a.parts == 1 && a.targets && tid == 0) a.targets[row] = label;
+  if (label < 0 || label >= V) {  // ignored (or a caller error, treated as such): uniform over the workgroup
+    if (a.parts == 1 && tid == 0) a.losses[row] = a.lse[row] = 0.f;
+    return;
+  }
   const int64_t row0 = logits_row(row, a.seq_in, a.seq_out) * a.ld;
   const uint16_t* x = a.logits + row0;
   const RowSpan sp = row_span(x, V, true);
@@ -590,7 +594,11 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const CeRowsArgs a) {
   if (part == a.parts - 1)
     for (int c = sp.head + 8 * sp.n_vec + tid; c < V; c += 256) element(c);
   const u32x4* xv = reinterpret_cast<const u32x4*>(x + sp.head);
-  const int v_begin = (int)((int64_t)sp.n_vec * part / a.parts), v_end = (int)((int64_t)sp.n_vec * (part + 1) / a.parts);
+  int v_begin = 0, v_end = sp.n_vec;
+  if (a.parts > 1) {  // (the quotients cost a workgroup of 1024 logits a tenth of its time)
+    v_begin = (int)((int64_t)sp.n_vec * part / a.parts);
+    v_end = (int)((int64_t)sp.n_vec * (part + 1) / a.parts);
+  }
   for (int i = v_begin + tid; i < v_end; i += 1024) {
     u32x4 w[4];
     float v[4][8];
@@ -637,13 +645,21 @@ __global__ __launch_bounds__(256) void ce_rows_fwd_kernel(const CeRowsArgs a) {
     __syncthreads();
   }
   if (tid == 0) {
-    a.pm[(size_t)part * a.rows + row] = red_m[0];
-    a.ps[(size_t)part * a.rows + row] = red_s[0];
+    if (a.parts == 1) {
+      const float lse = red_m[0] + __builtin_amdgcn_logf(red_s[0]) * kLn2;
+      a.lse[row] = lse;
+      a.losses[row] = lse - load1<D>(x, label);
+    } else {
+      a.pm[(size_t)part * a.rows + row] = red_m[0];
+      a.ps[(size_t)part * a.rows + row] = red_s[0];
+    }
   }
 }
 
-// One workgroup: logsumexp and loss of every row (parts in index order), the contiguous copy of the labels, sum and count.
-// (pm, ps may be the lse and losses of a call with one part: a thread reads its row's before it writes them.)
+// One workgroup: sum and count, and where rows came in parts (1024 of them at most, a thread's one) first their logsumexp and
+// loss, parts in index order, and the contiguous copy of the labels.  Whole rows are finished by their own workgroups: a turn of
+// this loop is a chain of memory latencies, 3 us, and 128 turns took 8 x 16383 rows of 1024 logits from 258 to 631 us; with
+// eight rows' losses and labels in flight a turn, and nothing else to do, 257.
 template <int D>
 __global__ __launch_bounds__(1024) void ce_rows_finish_kernel(const CeRowsArgs a) {
   __shared__ float red[1024];
@@ -651,27 +667,44 @@ __global__ __launch_bounds__(1024) void ce_rows_finish_kernel(const CeRowsArgs a
   const int tid = threadIdx.x;
   float sum = 0.f;
   int n = 0;
-  for (int row = tid; row < a.rows; row += 1024) {
-    const int64_t label = row_label(a, row);
-    if (a.targets) a.targets[row] = label;
-    n += label != -100;
-    float lse = 0.f, loss = 0.f;
-    if (label >= 0 && label < a.V) {
-      float m = a.pm[row], s = a.ps[row];
-      for (int part = 1; part < a.parts; ++part) {
-        const float m2 = a.pm[(size_t)part * a.rows + row], s2 = a.ps[(size_t)part * a.rows + row];
-        const float mn = fmaxf(m, m2);
-        s = merge_term(m, s, mn) + merge_term(m2, s2, mn);
-        m = mn;
+  if (a.parts == 1) {
+    for (int row0 = tid; row0 < a.rows; row0 += 8 * 1024) {
+      float loss[8];
+      int64_t label[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int row = min(row0 + 1024 * u, a.rows - 1);
+        loss[u] = a.losses[row];
+        label[u] = row_label(a, row);
       }
-      lse = m + __builtin_amdgcn_logf(s) * kLn2;
-      loss = lse - load1<D>(a.logits + logits_row(row, a.seq_in, a.seq_out) * a.ld, label);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (row0 + 1024 * u < a.rows) {
+          sum += loss[u];
+          n += label[u] != -100;
+        }
     }
-    a.lse[row] = lse;
-    if (a.losses) a.losses[row] = loss;
-    sum += loss;
+  } else {
+    for (int row = tid; row < a.rows; row += 1024) {
+      const int64_t label = row_label(a, row);
+      if (a.targets) a.targets[row] = label;
+      n += label != -100;
+      float lse = 0.f, loss = 0.f;
+      if (label >= 0 && label < a.V) {
+        float m = a.pm[row], s = a.ps[row];
+        for (int part = 1; part < a.parts; ++part) {
+          const float m2 = a.pm[(size_t)part * a.rows + row], s2 = a.ps[(size_t)part * a.rows + row];
+          const float mn = fmaxf(m, m2);
+          s = merge_term(m, s, mn) + merge_term(m2, s2, mn);
+          m = mn;
+        }
+        lse = m + __builtin_amdgcn_logf(s) * kLn2;
+        loss = lse - load1<D>(a.logits + logits_row(row, a.seq_in, a.seq_out) * a.ld, label);
+      }
+      a.lse[row] = lse;
+      sum += loss;
+    }
   }
-  if (!a.sum) return;
   red[tid] = sum;
   red_n[tid] = n;
   __syncthreads();
@@ -875,7 +908,8 @@ int launch_ce_bwd(void* logits, int64_t ld, const float* dloss, int64_t dloss_st
 
 int ce_rows_parts(int rows, int V) { return std::max(1, std::min(2048 / rows, V / 8192)); }
 
-// parts = 1: the losses and lse of the rows serve as the parts' pairs; otherwise `partial` [2][parts][rows]
+// parts > 1: `partial` [2][parts][rows], no losses of the rows.  parts == 1: losses [rows].  sum may be nullptr then: the losses are
+// the result.
 int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t* labels, int64_t label_seq, int n_seq, int seq_in,
                        int seq_out, int V, int dtype, int parts, float* partial, float* losses, float* lse, int64_t* targets, float* sum,
                        float* count, int mean, hipStream_t st) {
@@ -890,8 +924,8 @@ int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t
   a.V = V;
   a.rows = n_seq * seq_out;
   a.parts = parts;
-  a.pm = partial ? partial : lse;
-  a.ps = partial ? partial + (size_t)parts * a.rows : losses;
+  a.pm = partial;
+  a.ps = partial ? partial + (size_t)parts * a.rows : nullptr;
   a.losses = losses;
   a.lse = lse;
   a.targets = targets;
@@ -903,7 +937,7 @@ int launch_ce_rows_fwd(const void* logits, void* kept, int64_t ld, const int64_t
   do {                                                                                       \
     if (kept) hipLaunchKernelGGL((ce_rows_fwd_kernel<D, true>), grid, block, 0, st, a);       \
     else hipLaunchKernelGGL((ce_rows_fwd_kernel<D, false>), grid, block, 0, st, a);           \
-    hipLaunchKernelGGL((ce_rows_finish_kernel<D>), dim3(1), dim3(1024), 0, st, a);            \
+    if (sum) hipLaunchKernelGGL((ce_rows_finish_kernel<D>), dim3(1), dim3(1024), 0, st, a);   \
   } while (0)
   if (dtype == FMSA_BF16) ROWS_FWD(FMSA_BF16);
   else ROWS_FWD(FMSA_F16);

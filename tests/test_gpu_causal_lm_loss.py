@@ -149,3 +149,21 @@ def test_parts_of_a_row_and_the_sum(rows, V, mean):
     ref = torch.where(live[:, None], p * (3.0 / max(n, 1)), torch.zeros_like(p))
     assert bool((grad[0, rows] == 0).all())
     assert bool(((grad[0, :rows].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-9).all())
+
+
+@pytest.mark.parametrize("rows", [8191, 8193])
+def test_sum_of_more_rows_than_one_turn(rows):
+    """Whole rows, whose losses the second launch takes 8192 a turn."""
+    test_parts_of_a_row_and_the_sum(rows, 40, True)
+
+
+def test_rows_by_themselves_are_those_of_the_sum():
+    """cross_entropy_rows_fwd has no second launch; its losses add up to the call that has."""
+    import fmsa_hip
+
+    x, labels = randn((3, 41, 520), 5, torch.float16).cuda(), torch.randint(0, 520, (3, 41), generator=torch.Generator().manual_seed(6)).cuda()
+    labels[1] = -100
+    losses, lse = fmsa_hip.cross_entropy_rows_fwd(x, labels[:, 1:].reshape(-1).contiguous(), 40)
+    loss, (_, lse2, _, count) = fmsa_hip.causal_lm_loss_fwd(x, labels[:, 1:], labels.stride(0), 40, False, True)
+    assert torch.equal(lse, lse2) and bool((losses[40:80] == 0).all()) and count.item() == 1
+    assert abs(losses.double().sum().item() - loss.item()) <= 120 * 2.0 ** -24 * losses.double().abs().sum().item()
