@@ -317,7 +317,12 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
 
   // turn `it` of the wave: chunk wave + NW * it
   const int n_it = (n_chunks + NW - 1) / NW;
-  static_for<0, DEPTH>([&](auto d_c) { load(wave + NW * decltype(d_c)::value, d_c); });
+  static_for<0, DEPTH>([&](auto d_c) {
+    load(wave + NW * decltype(d_c)::value, d_c);
+    // the counted wait for a chunk takes the loads of the younger ones to be younger: nothing but this keeps the compiler, which
+    // knows the buffers for separate arrays, from issuing them first
+    __builtin_amdgcn_sched_barrier(0);
+  });
   for (int it = 0; it < n_it; it += DEPTH)
     static_for<0, DEPTH>([&](auto d_c) {
       constexpr int d = decltype(d_c)::value;

@@ -214,6 +214,7 @@ __global__ __launch_bounds__(64 * LM_NW) void lora_down_mid_kernel(const LoraDow
     __builtin_amdgcn_sched_barrier(0);  // the fragments have arrived before the buffer is loaded again
   };
   load(0, b0);
+  __builtin_amdgcn_sched_barrier(0);  // the counted wait takes b1's loads to be younger, and the compiler knows of no order between them
   load(1, b1);
   for (int it = 0; it < n_it; it += 2) {
     multiply(b0);
