@@ -917,8 +917,12 @@ static SplitPlan bwd_t_split(const fmsa_bwd_proj* projs, int n_proj, int M, int 
   // book without the epilogue 6 to 9 % (28672 -> 4096 at three rounds and 96 or 128 tiles: cutting them takes 1.9 and 0.9 % off
   // the whole MLP step; SwiGLU 4096 -> 14336 at two rounds and 48 tiles: cutting them adds 1.2 %)
   const float whole_slow = swiglu ? 0.16f : (codebook ? 0.09f : 0.13f);
+  // a launch from a code book takes longer to start than its stages (34 us for 16 of them, 52 for 32), and is cut where that
+  // pays: 1024 -> 4096 at 64 tokens 34 -> 19 us, 2048 -> 4096 at 700 52 -> 36, 2048 -> 2048 at 2048 53 -> 41; SwiGLU 4096 -> 14336
+  // at 512 tokens, 112 tiles, stays whole (101 us, cut 111)
+  const float start_us = codebook ? 5.0f : -3.0f;
   return plan_split(((M + BM - 1) / BM) * ((projs[0].w.K + 255) / 256), bwd_t_stages(projs, n_proj), whole_slow,
-                    swiglu ? 0.12f : 0.f);
+                    swiglu ? 0.12f : 0.f, start_us);
 }
 
 size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M) {

@@ -28,19 +28,22 @@ struct SplitPlan {
 };
 
 // A stage of 64 contraction elements takes a tile about 1.4 us where the chip is not full, from a code book too; the split
-// costs the second launch and the start-up of its ranges (8 us), the sums' way to memory and back (about 4 TB/s) and, where the second launch does more than round and store, `finish_us` per tile.
+// costs the second launch and the start-up of its ranges (8 us), the sums' way to memory and back (about 4 TB/s) and, where the
+// second launch does more than round and store, `finish_us` per tile.  Without whole rounds a launch is held against the split
+// with `start_us` beside its stages.
 // Behind whole rounds less of the tiles' time is there to be won: they start as CUs come free (10 % off).  And the whole
 // tiles of a cut launch run on the flavour that can cut, which takes `whole_slow` of their time more than the one that
 // cannot: with whole rounds enough in front, that is more than the cut gives (SwiGLU backward 4096 -> 14336, 6107 tokens,
 // five rounds and 64 tiles: 696 us whole, 766 us cut; at 256 tokens, 56 tiles: 96 and 63 us).
-inline SplitPlan plan_split(int tiles, int n_stages, float whole_slow, float finish_us = 0.f) {
+inline SplitPlan plan_split(int tiles, int n_stages, float whole_slow, float finish_us = 0.f, float start_us = -3.0f) {
   constexpr float stage_us = 1.4f;
   const int rest = tiles % SPLIT_CUS, rounds = tiles / SPLIT_CUS;
   SplitPlan p{tiles, 0, 1, (rounds + (rest > 0)) * n_stages * stage_us + 8.0f};
   if (rest == 0) return p;
   const float range_us = 2.0f * SPLIT_TILE_BYTES / 4.0e6f;
   const float fixed_us = 8.0f + rest * finish_us + whole_slow * rounds * n_stages * stage_us;
-  float best = n_stages * stage_us * (tiles > rest ? 0.9f : 1.0f) - 3.0f;  // not for a gain that the noise of a launch would hide
+  // not for a gain that the noise of a launch would hide
+  float best = rounds > 0 ? 0.9f * n_stages * stage_us - 3.0f : n_stages * stage_us + start_us;
   int s_best = 1;
   for (int s = 2; s <= SPLIT_CUS / rest && 2 * s <= n_stages; ++s) {
     const float us = n_stages * stage_us / s + fixed_us + rest * s * range_us;

@@ -88,6 +88,12 @@ def test_tiles_are_cut_where_that_pays():
     assert not _cut_bwd(7131, 8192, [8192, 1024, 1024])            # three rounds and 128 tiles: 941 / 986
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 4096, 1024), (256, 4096, 1024), (1024, 1024, 1024), (700, 4096, 2048), (2048, 2048, 2048)])
+def test_short_contractions_from_a_code_book_are_cut(M, K, N):
+    """16 and 32 stages on 16 to 64 tiles: whole they take 34 and 52 us, cut 18 to 42."""
+    assert _cut_bwd(M, K, [N], codebook=True)
+
+
 @pytest.mark.parametrize("cut,rotating", [((), (True, True)), (("k",), (True, False)), (("q",), (False, True)), (("q", "k"), (False, False))])
 def test_rotation_is_decided_per_launch(monkeypatch, cut, rotating):
     """Projections that walk K in orders of their own are launched one by one: each is asked whether its launch is cut."""
