@@ -740,7 +740,11 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const BwdTArgs a) {
   constexpr bool swiglu = MODE == FMSA_BWD_SWIGLU;
-  const int cut = blockIdx.x / (MT * NT), mt = blockIdx.x / NT % MT, j = blockIdx.x % NT;
+  // The two column tiles share the 128-byte lines of what is read and written row by row, so their workgroups are MT = 8 ids
+  // apart, on one XCD; token tile 0 of consecutive cuts goes to different ones.  (On two XCDs the SwiGLU's six arrays moved half
+  // a line at a time: 4096 -> 14336, 64 / 256 tokens, 45 / 70 us a call, and 39 / 61 this way; 4096 of 2048 at 512 41 and 36.)
+  static_assert(MT == 8 && NT == 2, "workgroups go to the XCDs by id % 8");
+  const int cut = blockIdx.x / (MT * NT), mt = (blockIdx.x + cut) % MT, j = blockIdx.x / MT % NT;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
   int bm, bk;
   bwd_tile(a, a.n_whole + cut, bm, bk);
