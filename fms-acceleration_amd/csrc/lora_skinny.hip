@@ -648,6 +648,7 @@ struct LoraGradJobDev {
   int rblock_start;  // ... in pass 2
   int transpose_out, out_dtype;
   float scale;
+  int per_thread;  // elements of the output that a thread of pass 2 adds: 4 or 1
   // optional second product of the same pass over R: T[M, r] = R * Wt^T (see below)
   const uint16_t* Wt;  // [r, C]
   float* tpart;        // [column blocks][M][r]
@@ -853,12 +854,54 @@ __global__ __launch_bounds__(512) void lora_grad_partial_kernel(const LoraGradAr
   }
 }
 
-// Four elements of the output per thread, in the output's order (which the partial sums are in too: the transposed outputs
-// were written 4 bytes at a time, r elements apart, 10.5 us where the sums of q, k, v at rank 64 and 1100 tokens now take 6).
+// The sums of a job's splits, in the output's order (which the partial sums are in too), V elements a thread: four, whose loads
+// are whole lines (the transposed outputs were written 4 bytes at a time, r elements apart, 10.5 us where the sums of q, k, v at
+// rank 64 and 1100 tokens take 6), or one, of straight outputs in launches that four leave short of workgroups (below).
+template <int V> FMSA_DEVI void grad_reduce(const LoraGradJobDev& J, int idx) {
+  using fv = std::conditional_t<V == 4, f32x4, float>;
+  const float* src = J.partial + idx;
+  const size_t step = (size_t)J.r * J.C;
+  fv v{};
+  int sp = 0;
+  for (; sp + 8 <= J.splits; sp += 8) {  // eight loads in flight, summed in index order
+    fv p[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) p[k] = *reinterpret_cast<const fv*>(src + (size_t)(sp + k) * step);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += p[k];
+  }
+#pragma unroll 4
+  for (; sp < J.splits; ++sp) v += *reinterpret_cast<const fv*>(src + (size_t)sp * step);
+  v *= J.scale;
+  if constexpr (V == 1) {
+    if (J.out_dtype == FMSA_F32) reinterpret_cast<float*>(J.out)[idx] = v;
+    else reinterpret_cast<uint16_t*>(J.out)[idx] = J.out_dtype == FMSA_BF16 ? pack1<bf16_t>(v) : pack1<f16_t>(v);
+  } else {
+    const bool aligned = reinterpret_cast<uintptr_t>(J.out) % 16 == 0;
+    if (J.out_dtype == FMSA_F32) {
+      float* out = reinterpret_cast<float*>(J.out) + idx;
+      if (aligned) {
+        *reinterpret_cast<f32x4*>(out) = v;
+      } else {
+        for (int i = 0; i < 4; ++i) out[i] = v[i];
+      }
+    } else {
+      uint16_t* out = reinterpret_cast<uint16_t*>(J.out) + idx;
+      const u32x2 o = J.out_dtype == FMSA_BF16 ? u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])}
+                                               : u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
+      if (aligned) {
+        *reinterpret_cast<u32x2*>(out) = o;
+      } else {
+        for (int i = 0; i < 4; ++i) out[i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
+      }
+    }
+  }
+}
+
 __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGradArgs a) {
   const LoraGradJobDev J = select_job<true>(a, blockIdx.x);
   const int r = J.r, C = J.C;
-  const int nb_grad = (r * C / 4 + 255) / 256;
+  const int nb_grad = (r * C / J.per_thread + 255) / 256;
   const int lb = blockIdx.x - J.rblock_start;
   if (lb >= nb_grad) {  // the job's T: column blocks added in index order, one rounding; four ranks per thread
     const int64_t ti = ((int64_t)(lb - nb_grad) * 256 + threadIdx.x) * 4;
@@ -885,39 +928,11 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGradArg
     *reinterpret_cast<u32x2*>(J.T + (size_t)m * J.ldt + j) = pk;
     return;
   }
-  const int idx = 4 * (lb * 256 + threadIdx.x);
-  if (idx >= r * C) return;
-  const float* src = J.partial + idx;
-  const size_t step = (size_t)r * C;
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  int sp = 0;
-  for (; sp + 8 <= J.splits; sp += 8) {  // eight loads in flight, summed in index order
-    f32x4 p[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) p[k] = *reinterpret_cast<const f32x4*>(src + (size_t)(sp + k) * step);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v += p[k];
-  }
-#pragma unroll 4
-  for (; sp < J.splits; ++sp) v += *reinterpret_cast<const f32x4*>(src + (size_t)sp * step);
-  v *= J.scale;
-  const bool aligned = reinterpret_cast<uintptr_t>(J.out) % 16 == 0;
-  if (J.out_dtype == FMSA_F32) {
-    float* out = reinterpret_cast<float*>(J.out) + idx;
-    if (aligned) {
-      *reinterpret_cast<f32x4*>(out) = v;
-    } else {
-      for (int i = 0; i < 4; ++i) out[i] = v[i];
-    }
-  } else {
-    uint16_t* out = reinterpret_cast<uint16_t*>(J.out) + idx;
-    const u32x2 o = J.out_dtype == FMSA_BF16 ? u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])}
-                                             : u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
-    if (aligned) {
-      *reinterpret_cast<u32x2*>(out) = o;
-    } else {
-      for (int i = 0; i < 4; ++i) out[i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
-    }
+  const int at = lb * 256 + threadIdx.x;
+  if (J.per_thread == 4) {
+    if (4 * at < r * C) grad_reduce<4>(J, 4 * at);
+  } else if (at < r * C) {
+    grad_reduce<1>(J, at);
   }
 }
 
@@ -1274,7 +1289,11 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
   a.M = M;
   a.act_dtype = act_dtype;
   bool any_t = false;
-  for (int q = 0; q < n_jobs; ++q) any_t = any_t || jobs[q].Wt != nullptr;
+  int64_t elements = 0;
+  for (int q = 0; q < n_jobs; ++q) {
+    any_t = any_t || jobs[q].Wt != nullptr;
+    elements += (int64_t)jobs[q].r * jobs[q].C;
+  }
   const int tc = LG_TC_T;
   int blocks = 0, rblocks = 0, r_max = 0;
   size_t ws_off = 0;
@@ -1298,7 +1317,12 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
     d.out_dtype = s.out_dtype;
     d.scale = s.scale;
     blocks += ((s.C + tc - 1) / tc) * d.splits;
-    rblocks += (s.r * s.C / 4 + 255) / 256;
+    // one element a thread: straight sums over several splits, in launches of fewer than 1024 workgroups with four (us with four /
+    // one; single outputs: 4096 of rank 64 at 3217 tokens 25.2 / 22.8, 14336 of rank 32 at 8192 50.6 / 46.9, of rank 64 at 1100
+    // 25.3 / 23.7, of rank 128 at 3217, 1792 workgroups, 58.8 / 60.4; q, k, v of rank 128 at 2048, 2304, 54 / 58; 14336 of rank 128
+    // at 300 tokens, one split, 23.7 / 27.3)
+    d.per_thread = !s.transpose_out && d.splits > 1 && elements < 1024 * 1024 ? 1 : 4;
+    rblocks += (s.r * s.C / d.per_thread + 255) / 256;
     ws_off += job_partial_bytes(s, M);
     if (s.Wt) {
       d.Wt = (const uint16_t*)s.Wt;
