@@ -84,14 +84,16 @@ FMSA_DEVI float load_param_rt(const void* p, int64_t i, int dtype) {
   return dtype == FMSA_BF16 ? load_param<bf16_t>(p, i) : load_param<f16_t>(p, i);
 }
 
-// A workgroup takes a tile of 4096 elements (1024 up to rank 16, whose copies are small and a matter of latency) of one matrix
-// (A [r, K] or B [N, r]), as many ranks wide as there are (a power of two from 8 to 64), in 4-element pieces: the rounded copy leaves row by row as it came, the transposed copy through LDS, so
-// that both are written in whole lines.  (One thread per element wrote the transposed copies 2 bytes at a time, r or N elements
-// apart; q, k, v / the MLP's three of 4096 and 14336: 5.0 / 9.6 -> 3.7 / 4.5 us at rank 32, 9.0 / 21 -> 4.1 / 5.8 at rank 64.)
+// A workgroup takes a tile of 4096 elements (1024 up to rank 16 and of matrices up to 128 Ki elements, which are a matter of
+// latency: 2048 x 2048 of rank 32 4.2 us with the large tile, 3.6 with the small one) of one matrix
+// (A [r, K] or B [N, r]), as many ranks wide as there are (a power of two from 8 to 64), in 4-element pieces: the rounded copy
+// leaves row by row as it came, the transposed copy through LDS, so that both are written in whole lines.  (One thread per
+// element wrote the transposed copies 2 bytes at a time, r or N elements apart; q, k, v / the MLP's three of 4096 and 14336: 5.0 /
+// 9.6 -> 3.7 / 4.5 us at rank 32, 9.0 / 21 -> 4.1 / 5.8 at rank 64.)
 __host__ __device__ inline int pack_log2_ranks(int r) { return r > 32 ? 6 : (r > 16 ? 5 : (r > 8 ? 4 : 3)); }
-__host__ __device__ inline int pack_log2_tile(int r) { return r > 16 ? 12 : 10; }
+__host__ __device__ inline int pack_log2_tile(int r, int n) { return r > 16 && (int64_t)r * n > (1 << 17) ? 12 : 10; }
 __host__ __device__ inline int pack_tiles(int r, int n) {  // of a matrix of r ranks and n columns (A) or rows (B)
-  const int lr = pack_log2_ranks(r), ln = pack_log2_tile(r) - lr;
+  const int lr = pack_log2_ranks(r), ln = pack_log2_tile(r, n) - lr;
   return ((r + (1 << lr) - 1) >> lr) * ((n + (1 << ln) - 1) >> ln);
 }
 template <typename T>
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(256) void lora_pack_kernel(const LoraPackArgs a) {
   const bool is_a = t < n_a;
   if (!is_a) t -= n_a;
   const int rows = is_a ? J.r : J.N, cols = is_a ? J.K : J.r;
-  const int log_tile = pack_log2_tile(J.r), log_rows = is_a ? lr : log_tile - lr, log_cols = log_tile - log_rows;
+  const int log_tile = pack_log2_tile(J.r, is_a ? J.K : J.N), log_rows = is_a ? lr : log_tile - lr, log_cols = log_tile - log_rows;
   const int rank0 = (t % rt) << lr, other0 = (t / rt) << (log_tile - lr);
   const int row0 = is_a ? rank0 : other0, col0 = is_a ? other0 : rank0;
   const int stride = (1 << log_cols) + 2;
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(256) void lora_pack_kernel(const LoraPackArgs a) {
   uint16_t* copy = reinterpret_cast<uint16_t*>(is_a ? J.A16 : J.B16);
   uint16_t* turned = reinterpret_cast<uint16_t*>(is_a ? J.At16 : J.Bt16);
   // parameters may be views into a flat buffer and begin anywhere; ranks, K and N of the fused operators are multiples of 8
-  const bool wide = rows % 4 == 0 && cols % 4 == 0 && J.param_dtype == FMSA_F32 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
+  const bool f32 = J.param_dtype == FMSA_F32, wide = cols % 4 == 0 && reinterpret_cast<uintptr_t>(src) % (f32 ? 16 : 8) == 0;
   const bool wide_copy = cols % 4 == 0 && reinterpret_cast<uintptr_t>(copy) % 8 == 0;
   const bool wide_turned = rows % 4 == 0 && reinterpret_cast<uintptr_t>(turned) % 8 == 0;
 #pragma unroll 4
@@ -129,8 +131,14 @@ __global__ __launch_bounds__(256) void lora_pack_kernel(const LoraPackArgs a) {
     const int64_t at = (int64_t)(row0 + rr) * cols + col0 + piece;
     const int n = min(4, cols - (col0 + piece));
     f32x4 f = {0.f, 0.f, 0.f, 0.f};
-    if (wide) {
+    if (wide && f32) {
       f = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(src) + at);
+    } else if (wide) {
+      const u32x2 w = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(src) + at);
+      if (J.param_dtype == FMSA_BF16)
+        f = f32x4{unpack_lo<bf16_t>(w[0]), unpack_hi<bf16_t>(w[0]), unpack_lo<bf16_t>(w[1]), unpack_hi<bf16_t>(w[1])};
+      else
+        f = f32x4{unpack_lo<f16_t>(w[0]), unpack_hi<f16_t>(w[0]), unpack_lo<f16_t>(w[1]), unpack_hi<f16_t>(w[1])};
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)

@@ -38,3 +38,10 @@ def test_gradients_of_both_orders(M, C, r, out_dtype):
     out = store[1:].view(C, r)
     fmsa_hip.lora_grad_static(L, R, 0.5, True, out)
     assert torch.equal(out, turned)
+
+
+@pytest.mark.parametrize("param", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,K,N,offset", [(32, 4096, 4104, 0), (24, 1024, 5464, 4), (64, 2056, 2048, 2), (40, 36, 12, 0)])
+def test_pack_on_both_sides_of_the_tile_rule(r, K, N, offset, param):
+    """Matrices of up to 128 Ki elements and more in one call, rows that are no whole tiles, parameters read 8 and 2 bytes at a time."""
+    test_pack(r, K, N, offset, param, torch.bfloat16)
