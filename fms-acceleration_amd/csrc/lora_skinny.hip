@@ -1023,22 +1023,25 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
 // Whether products over M tokens and `columns` columns in all take the kernel of 64-token workgroups (us before / with it):
 // below 2048 tokens from the traffic on that the fragment kernel's loads are bound by, X and the re-reads of Wd (rank 64: 4096
 // columns at 512 tokens, 21 MB, 7.5 / 10.1, q, k, v at 512, 31 MB, 12.0 / 10.6, gate and up of 14336 at 1100, 317 MB, 39.6 / 21.6;
-// rank 32: 4096 at 512, 13 MB, 7.4 / 8.1, at 1100, 27 MB, 9.9 / 8.4; rank 16: 2048 at 2047, 17 MB, 6.6 / 6.0) and always above
+// rank 32: 4096 at 512, 13 MB, 7.4 / 8.1, at 1100, 27 MB, 9.9 / 8.4; rank 16: 2048 at 2047, 17 MB, 6.6 / 6.0; rank 8, half of whose
+// tile the fragment kernel does not read: 8192 at 700, 23 MB, 8.1 / 9.1, q, k, v of 8192 and 1024 at 512, 21 MB, 9.8 / 10.6, 14336 at
+// 512, 29 MB, 10.4 / 8.7, q, k, v at 1536, 38 MB, 14.4 / 11.4) and always above
 // rank 64, whose eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48).
 // From 2048 tokens on above rank 16 (rank 32: 4096 at 8192 tokens 17.9 / 16.6; rank 64: 2048 at 2048 15.4 / 9.3, 4096 at 8192
-// 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99);
+// 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99, 28672
+// at 8192: 97 / 103);
 // rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them
 // (14336 at 3217: 25.8 / 19.6; short ones of many, 4096 at 16384: 39 / 26, would need a buffer that the size query does not ask
 // for there).
 static bool down_is_mid(int M, int r_max, int64_t columns) {
   if (M <= 64) return false;  // few tokens: the ranges of the products straight from the parameters are the fragment kernel's
   if (M >= 2048) {
-    const bool many = M >= 16384, wide = columns >= 8192;
+    const bool many = M >= 16384 || M * columns >= 200000000, wide = columns >= 8192;
     if (columns < 2048) return false;
     return r_max > 16 ? !(many && wide && r_max > 32) : (wide && M < 4096);
   }
   const int64_t bytes = (int64_t)((M + 15) / 16) * (16 + std::max(16, r_max)) * columns * 2;
-  return r_max > 64 || bytes >= (r_max > 32 ? 22000000 : 14000000);
+  return r_max > 64 || bytes >= (r_max > 32 ? 22000000 : (r_max > 8 ? 14000000 : 28000000));
 }
 // column ranges: two chunks of 64 columns a wave at least, and no more workgroups than run at once (one per CU, two up to rank 16)
 static int down_mid_split(int M, int C, int r_max, int blocks_per_row) {
