@@ -1029,14 +1029,14 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
 // rank 64, whose eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48).
 // From 2048 tokens on above rank 16 (rank 32: 4096 at 8192 tokens 17.9 / 16.6; rank 64: 2048 at 2048 15.4 / 9.3, 4096 at 8192
 // 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99, 28672
-// at 8192: 97 / 103);
+// at 8192: 97 / 103; rank 128 there 194 / 174);
 // rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them
 // (14336 at 3217: 25.8 / 19.6; short ones of many, 4096 at 16384: 39 / 26, would need a buffer that the size query does not ask
 // for there).
 static bool down_is_mid(int M, int r_max, int64_t columns) {
   if (M <= 64) return false;  // few tokens: the ranges of the products straight from the parameters are the fragment kernel's
   if (M >= 2048) {
-    const bool many = M >= 16384 || M * columns >= 200000000, wide = columns >= 8192;
+    const bool wide = columns >= 8192, many = M >= 16384 || (r_max <= 64 && M * columns >= 200000000);
     if (columns < 2048) return false;
     return r_max > 16 ? !(many && wide && r_max > 32) : (wide && M < 4096);
   }
