@@ -89,6 +89,26 @@ def test_traces_of_the_norm_and_the_rotation(monkeypatch):
         assert torch.equal(got, -want.transpose(1, 2))
 
 
+def test_one_launch_for_both_only_without_shared_storage(monkeypatch):
+    """Two rotations of one memory have an order; two workgroups of one launch have none."""
+    import fmsa_hip
+    from fms_acceleration_foak.kernels.unsloth import fast_rope_embedding
+
+    calls = []
+    monkeypatch.setattr(fmsa_hip, "rope_embedding_", lambda q, *a, **k: calls.append(q.data_ptr()) or q)
+    monkeypatch.setattr(fmsa_hip, "rope_embedding_pair_", lambda q, k, *a: calls.append("pair"))
+    base, cos = torch.randn(192), torch.ones(2, 16)
+    q = base[:128].view(1, 2, 4, 16).transpose(1, 2)
+    with torch.no_grad():
+        for k in (q, base[64:128].view(1, 2, 2, 16).transpose(1, 2), base[128:].view(1, 2, 2, 16).transpose(1, 2)):
+            calls.clear()
+            fast_rope_embedding(q, k, cos, cos)
+            assert calls == [q.data_ptr(), k.data_ptr()]
+        calls.clear()
+        fast_rope_embedding(q, q.clone(memory_format=torch.preserve_format), cos, cos)
+        assert calls == ["pair"]
+
+
 @pytest.mark.gpu
 def test_backward_meets_the_autocast_state_of_its_forward():
     seen = []
