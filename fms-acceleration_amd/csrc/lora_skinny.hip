@@ -1105,9 +1105,7 @@ DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
     return {1, n_tb, n_split};
   }
   if (rt < 2 && M >= 16384) return {0, 0, 0};  // rank 16 and below with a workgroup per CU anyway: the 32-token kernels do as well
-  // up to rank 16 64 tokens per workgroup; 48 / 64: 128 (32 takes the kernel of 64-token workgroups above; what is worked out here
-  // for it goes into the size query, whose answers stay)
-  const int g = rt <= 2 ? 2 : 4;
+  const int g = rt <= 2 ? 2 : 4;  // rank 32: 64 tokens per workgroup; 48 / 64: 128
   const int n_tb = (M + 32 * g - 1) / (32 * g);
   const int n_chunks = (C + 511) / 512;
   int n_split = (256 + n_tb - 1) / n_tb;                 // a workgroup per CU at least
@@ -1146,7 +1144,7 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
     return launch_down_mid(a, 1, act_dtype, st);
   }
   const DownSplit d = lora_down_split_shape(M, C, r, few_tokens);
-  if (!d.g || (d.g == 2 && r > 16) || (down_split_bytes(M, C, r, few_tokens) && !sums))
+  if (!d.g || (down_split_bytes(M, C, r, few_tokens) && !sums))
     return launch_lora_down(X, ldx, Wd, M, C, r, act_dtype, out, ldo, st);
   auto reduce = [&]() -> int {
     const int64_t quads = (int64_t)M * (r / 4);
@@ -1182,6 +1180,7 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
 #define SPLIT_DISPATCH(TT)                            \
   switch (rt) {                                       \
     case 1: SPLIT_LAUNCH(TT, 1, 2); break;            \
+    case 2: SPLIT_LAUNCH(TT, 2, 2); break;            \
     default: SPLIT_LAUNCH(TT, 4, 4); break;           \
   }
   if (act_dtype == FMSA_BF16) {
