@@ -31,6 +31,20 @@ def test_single(M, C, r, dtype):
     assert torch.equal(out, fmsa_hip.lora_down(x, wd))
 
 
+@pytest.mark.parametrize("M,C,r", [(700, 5120, 64), (1100, 14336, 16), (3217, 8256, 16), (2050, 2112, 32), (600, 1088, 128)])
+def test_rows_of_whole_lines_and_others(M, C, r):
+    """Rows on 128-byte lines are read past the caches, others through them: the same sums."""
+    import fmsa_hip
+
+    x, wd = randn((M, C), 1, torch.bfloat16).cuda(), randn((r, C), 2, torch.bfloat16, 0.05).cuda()
+    out = fmsa_hip.lora_down(x, wd)
+    assert _within(out, x, wd, torch.bfloat16)
+    for start, ld in ((0, C + 64), (32, C + 64), (0, C + 40)):  # whole lines; half a line on; rows between lines
+        view = torch.empty(M * ld + start, dtype=torch.bfloat16, device="cuda").as_strided((M, C), (ld, 1), start)
+        view.copy_(x)
+        assert torch.equal(fmsa_hip.lora_down(view, wd), out)
+
+
 @pytest.mark.parametrize("M,shapes", [(300, [(4096, 64), (1024, 64), (1024, 64)]), (512, [(96, 128), (520, 8)]),
                                       (1100, [(14336, 64), (64, 16), (4096, 72)])])
 def test_batch(M, shapes):
