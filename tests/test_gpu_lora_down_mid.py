@@ -17,6 +17,7 @@ def _within(out, x, wd, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,C,r", [(65, 64, 72), (128, 1032, 128), (129, 200, 80),      # fewer chunks than waves, ragged ends
+                                   (300, 520, 128), (128, 1056, 128), (513, 3104, 64),  # a last range of one chunk, of fewer than the others
                                    (700, 4160, 64), (1100, 14336, 16), (1999, 4104, 24),
                                    (2048, 2048, 32), (2050, 8200, 8), (3001, 2056, 120)])
 def test_single(M, C, r, dtype):
