@@ -1023,29 +1023,63 @@ static int launch_lora_down_plain(const void* X, int64_t ldx, const void* Wd, in
   return FMSA_OK;
 }
 
-// Whether products over M tokens and `columns` columns in all take the kernel of 64-token workgroups (us before / with it):
-// below 2048 tokens from the traffic on that the fragment kernel's loads are bound by, X and the re-reads of Wd (rank 64: 4096
-// columns at 512 tokens, 21 MB, 7.5 / 10.1, q, k, v at 512, 31 MB, 12.0 / 10.6, gate and up of 14336 at 1100, 317 MB, 39.6 / 21.6;
-// rank 32: 4096 at 512, 13 MB, 7.4 / 8.1, at 1100, 27 MB, 9.9 / 8.4; rank 16: 2048 at 2047, 17 MB, 6.6 / 6.0; rank 8, half of whose
-// tile the fragment kernel does not read: 8192 at 700, 23 MB, 8.1 / 9.1, q, k, v of 8192 and 1024 at 512, 21 MB, 9.8 / 10.6, 14336 at
-// 512, 29 MB, 10.4 / 8.7, q, k, v at 1536, 38 MB, 14.4 / 11.4) and always above
-// rank 64, whose eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48).
-// From 2048 tokens on above rank 16 (rank 32: 4096 at 8192 tokens 17.9 / 16.6; rank 64: 2048 at 2048 15.4 / 9.3, 4096 at 8192
-// 25.7 / 20.2; rank 128: 14336 at 4096 75 / 47) but for the longest rows of the most tokens (rank 64, 14336 at 16384: 94 / 99, 28672
-// at 8192: 97 / 103; rank 128 there 194 / 174);
-// rank 16 and below takes the kernels of 32 to 64 tokens (4096 at 8192: 14.5 / 15.3) but for long rows of few of them
-// (14336 at 3217: 25.8 / 19.6; short ones of many, 4096 at 16384: 39 / 26, would need a buffer that the size query does not ask
-// for there).
-static bool down_is_mid(int M, int r_max, int64_t columns) {
+// Whether products over M tokens take the kernel of 64-token workgroups: `columns` in all, of one product (`single`) or of a batch;
+// `lines`: every product's columns are whole 128-byte lines, and so, as a rule, its rows (the size query knows no strides).  us with
+// the other kernels / with it, over 5100 forms of one product and 1900 of batches:
+//
+// Below 2048 tokens from the traffic on that the fragment kernel's loads are bound by, X and the re-reads of Wd.
+//   rank 8, half of whose tile the fragment kernel does not read: 22 MB up to 8192 columns (4096 at 1300 tokens, 21 MB, 7.8 / 8.6;
+//     5120 at 1536, 31 MB, 9.5 / 8.2), 52 MB above (8192 at 1300, 43 MB, 11.1 / 11.8; 14336 at 1100, 63 MB, 13.8 / 12.0), a batch
+//     35 MB (q, k, v of 4096 and 1024 at 1300, 32 MB, 9.8 / 10.8, at 1536, 38 MB, 14.7 / 11.4); 14 MB where rows are no whole lines,
+//     which the fragment kernel reads worst (8224 at 900, 30 MB, 11.0 / 7.3)
+//   rank 16: 15 MB (4096 at 900, 15 MB, 8.0 / 8.6; 8192 at 512, 17 MB, 8.9 / 7.0)
+//   rank 32: 18 MB, a batch 14 (11008 at 256, 17 MB, 9.0 / 9.9; 4096 at 1100, 27 MB, 10.4 / 9.0; q, k, v at 512, rank 24, 16 MB, 10.1 /
+//     9.3)
+//   rank 64: 22 MB (1100 tokens of 2048, 23 MB, 10.0 / 9.2), 33 where rows are no whole lines (5472 twice at 200, 26 MB, 8.7 / 9.8),
+//     34 for a product of up to 512 tokens, whose column ranges fill the chip evenly (8192 at 384, 31 MB, 10.2 / 11.4; 11008 at 320,
+//     35 MB, 13.3 / 11.9)
+//   rank 96: 24 MB, a batch 18 (1056 at 1300, 19 MB, 8.3 / 9.2; q, k, v at 256, 22 MB, 13.9 / 10.6)
+//   above, always: its eight rank tiles are one long chain there (1024 columns at 65 tokens 8.8 / 7.7, gate and up at 2047 131 / 48)
+//
+// From 2048 tokens and columns on (below, 1024 columns at 3000 tokens 7.5 / 9.9) against the staged kernels of 64 tokens up to rank
+// 32 and 128 above, whose workgroups run one to a CU and are at their best where their ranges make one even round.
+//   up to rank 16: long rows of less than 4096 tokens, where they need a second round (14336 at 3217 26 / 20, 28672 at 2500 42 / 29;
+//     one round: 14336 at 4095 23 / 28, 8192 at 2048 10.1 / 10.6), and a good part of it where rows are no whole lines (10976 at 2300,
+//     288 workgroups, 17.5 / 15.5, at 2800, 264, 15.2 / 16.1)
+//   rank 32: all (2048 at 8192 11.0 / 10.4, 14336 at 3217 31 / 21) but 8192 at 16384, one round, 51 / 55
+//   rank 64: all (4096 at 8192 25 / 20, 28672 at 7000 115 / 93) but long rows where the others have one round (28672 at 8192 95 / 98)
+//     and the longest of the most tokens (14336 at 16384 94 / 102, 11008 at 16383 92 / 78)
+//   rank 32 and 64, rows that are no whole lines: up to 140 M elements (7200 at 12000 68 / 39, at 20000 87 / 98; 10976 at 16384 63 / 71),
+//     but not the 8192 columns and a few that leave most waves a step of nothing (8224 at 3500 tokens, rank 32, 18 / 22, at 7000, rank
+//     64, 36 / 43)
+//   above: all (14336 at 4096 81 / 46, 28672 at 8192 194 / 165) but the longest of the most tokens (14336 at 16383 186 / 197)
+// Short rows of many tokens at rank 16 and below (4096 at 16384: 39 / 26) would need a buffer that the size query does not ask for.
+static int staged_workgroups(int M, int64_t columns, int r);
+static bool down_is_mid(int M, int r_max, int64_t columns, bool lines, bool single) {
   if (M <= 64) return false;  // few tokens: the ranges of the products straight from the parameters are the fragment kernel's
   if (M >= 2048) {
-    const bool wide = columns >= 8192, many = M >= 16384 || (r_max <= 64 && M * columns >= 200000000);
     if (columns < 2048) return false;
-    return r_max > 16 ? !(many && wide && r_max > 32) : (wide && M < 4096);
+    const bool wide = columns >= 8192, many = M > 127 * 128;
+    const int64_t elements = M * columns;
+    if (r_max <= 16) return wide && M < 4096 && (lines || columns >= 9216) && staged_workgroups(M, columns, r_max) > (lines ? 256 : 280);
+    if (lines) {
+      if (r_max <= 32) return !(many && wide && columns < 11008);
+      if (many && columns >= 12800) return false;
+      return r_max > 64 || elements < 200000000 || staged_workgroups(M, columns, r_max) != 256;
+    }
+    if (r_max > 64) return !(many && columns >= 9216);
+    return elements < 140000000 && !(wide && columns < 9216 && M < 9000 && (r_max <= 32 || M >= 5000));
   }
   const int64_t bytes = (int64_t)((M + 15) / 16) * (16 + std::max(16, r_max)) * columns * 2;
-  return r_max > 64 || bytes >= (r_max > 32 ? 22000000 : (r_max > 8 ? 14000000 : 28000000));
+  if (r_max > 96) return true;
+  if (r_max > 64) return bytes >= (single ? 24000000 : 18000000);
+  if (r_max > 32) return bytes >= (single && M <= 512 ? 34000000 : (lines ? 22000000 : 33000000));
+  if (r_max > 16) return bytes >= (single ? 18000000 : 14000000);
+  if (r_max > 8) return bytes >= 15000000;
+  if (!lines) return bytes >= 14000000;
+  return bytes >= (!single ? 35000000 : (columns < 8192 ? 22000000 : 52000000));
 }
+static bool down_is_mid(int M, int C, int r) { return down_is_mid(M, r, C, C % 64 == 0, true); }
 // column ranges: a step of two chunks of 64 columns a wave, the last range shorter (rounded down, 1056 columns took every wave two
 // steps; rank 128 at 128 tokens 9.7 -> 8.7 us), and no more workgroups than run at once (one per CU, two up to rank 16)
 static int down_mid_split(int M, int C, int r_max, int blocks_per_row) {
@@ -1125,6 +1159,11 @@ DownSplit lora_down_split_shape(int M, int C, int r, bool few_tokens) {
 }
 }  // namespace
 
+static int staged_workgroups(int M, int64_t columns, int r) {
+  const DownSplit d = lora_down_split_shape(M, (int)columns, r, true);
+  return d.n_tb * d.n_split;
+}
+
 static size_t down_mid_bytes(int M, int C, int r) {
   const int n = down_mid_split(M, C, r, rank_blocks(r));
   return n > 1 ? (size_t)n * M * r * sizeof(float) : 0;
@@ -1138,7 +1177,7 @@ static size_t down_split_bytes(int M, int C, int r, bool few_tokens) {
 
 // Enough for either kernel, so that the answer for a shape does not depend on which of them is the faster one today.
 size_t lora_down_workspace(int M, int C, int r, bool few_tokens) {
-  const bool mid = (few_tokens || M >= 2048) && down_is_mid(M, r, C);
+  const bool mid = (few_tokens || M >= 2048) && down_is_mid(M, C, r);
   return std::max(mid ? down_mid_bytes(M, C, r) : 0, down_split_bytes(M, C, r, few_tokens));
 }
 
@@ -1148,7 +1187,7 @@ int launch_lora_down_ws(const void* X, int64_t ldx, const void* Wd, int M, int C
   const size_t need = lora_down_workspace(M, C, r, few_tokens);
   // a buffer smaller than the query's answer is as good as none; the reduce pass stores four ranks at a time
   const bool sums = workspace && workspace_bytes >= need && (uintptr_t)out % 8 == 0 && ldo % 4 == 0;
-  if ((few_tokens || M >= 2048) && down_is_mid(M, r, C) && (sums || !down_mid_bytes(M, C, r))) {
+  if ((few_tokens || M >= 2048) && down_is_mid(M, C, r) && (sums || !down_mid_bytes(M, C, r))) {
     LoraDownArgs a{};
     a.M = M;
     a.j[0] = {(const uint16_t*)X, (const uint16_t*)Wd, (uint16_t*)out, (float*)workspace, ldx, ldo, C, r, down_mid_split(M, C, r, rank_blocks(r))};
@@ -1224,15 +1263,19 @@ int lora_down_few_splits(int M, int C, int r, int n_jobs) {
   return d.g == 1 ? d.n_split : 1;
 }
 
-static int64_t all_columns(const fmsa_lora_down_job* jobs, int n_jobs) {
-  int64_t c = 0;
-  for (int q = 0; q < n_jobs; ++q) c += jobs[q].C;
-  return c;
+static bool down_batch_is_mid(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
+  int64_t columns = 0;
+  bool lines = true;
+  for (int q = 0; q < n_jobs; ++q) {
+    columns += jobs[q].C;
+    lines = lines && jobs[q].C % 64 == 0;
+  }
+  return down_is_mid(M, max_rank(jobs, n_jobs), columns, lines, n_jobs == 1);
 }
 static int down_batch_split_any(const fmsa_lora_down_job* jobs, int q, int n_jobs, int M) {
   const int r_max = max_rank(jobs, n_jobs);
-  return down_is_mid(M, r_max, all_columns(jobs, n_jobs)) ? down_mid_split(M, jobs[q].C, r_max, n_jobs * rank_blocks(r_max))
-                               : down_batch_split(M, jobs[q].C, n_jobs);
+  return down_batch_is_mid(jobs, n_jobs, M) ? down_mid_split(M, jobs[q].C, r_max, n_jobs * rank_blocks(r_max))
+                                            : down_batch_split(M, jobs[q].C, n_jobs);
 }
 
 size_t lora_down_batch_workspace(const fmsa_lora_down_job* jobs, int n_jobs, int M) {
@@ -1262,7 +1305,7 @@ int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, in
     p += (size_t)d.n_split * M * s.r;
     split_max = std::max(split_max, d.n_split);
   }
-  if (down_is_mid(M, r_max, all_columns(jobs, n_jobs))) return launch_down_mid(a, n_jobs, act_dtype, st);
+  if (down_batch_is_mid(jobs, n_jobs, M)) return launch_down_mid(a, n_jobs, act_dtype, st);
   constexpr int NW = 8;
   const dim3 grid((M + 15) / 16, split_max, n_jobs), block(64 * NW);
   const dim3 rgrid((unsigned)(((int64_t)M * (r_max / 4) + 255) / 256), n_jobs);
@@ -1272,7 +1315,7 @@ int launch_lora_down_batch(const fmsa_lora_down_job* jobs, int n_jobs, int M, in
     if (rt <= 1) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 1, 1, NW>), grid, block, 0, st, a);              \
     else if (rt <= 2) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 2, 1, NW>), grid, block, 0, st, a);         \
     else if (rt <= 4) hipLaunchKernelGGL((lora_down_batch_kernel<TT, 4, 1, NW>), grid, block, 0, st, a);         \
-    else hipLaunchKernelGGL((lora_down_batch_kernel<TT, 8, 1, NW>), grid, block, 0, st, a); /* up to 64 tokens */ \
+    else hipLaunchKernelGGL((lora_down_batch_kernel<TT, 8, 1, NW>), grid, block, 0, st, a);                      \
     hipLaunchKernelGGL((lora_down_reduce_batch_kernel<TT>), rgrid, dim3(256), 0, st, a);                      \
   } while (0)
   if (act_dtype == FMSA_BF16) BATCH(bf16_t);

@@ -55,6 +55,14 @@ def test_columns_are_split_where_the_second_launch_pays(M, C, r, split):
     assert (fmsa_hip.lib().fmsa_lora_down_split_workspace(M, C, r) > 0) == split
 
 
+@pytest.mark.parametrize("M,C,r,ranges", [(3217, 14336, 16, 10), (4095, 14336, 16, 4), (2048, 8192, 8, 8), (2100, 28672, 16, 15),
+                                          (1100, 8192, 8, 7), (1100, 14336, 8, 28)])
+def test_which_products_64_token_workgroups_take(M, C, r, ranges):
+    """By the ranges of their buffer: theirs where the staged kernels need a second round of workgroups or the fragment kernel
+    is bound by its loads (26 / 20, 23 / 28, 10.6 / 11.4, 24 / 17, 10.1 / 11.4, 14.6 / 11 us without / with)."""
+    assert fmsa_hip.lib().fmsa_lora_down_split_workspace(M, C, r) == ranges * M * r * 4
+
+
 def _struct(K, N, codebook=False, group=128):
     return fmsa_hip.GptqWeight(0x1000, None if codebook else 0x2000, None if codebook else 0x3000, None, K, N, 64 if codebook else group, 0,
                                fmsa_hip.WEIGHT_CODEBOOK if codebook else fmsa_hip.WEIGHT_AFFINE, 0, 0x7000 if codebook else None,
