@@ -733,18 +733,18 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_kernel(const BwdTArgs 
   }
 }
 
-// Second launch of a split call: workgroup = token tile mt (32 rows) and column tile j of the waves of a cut tile; lane, column
+// Second launch of a split call: workgroup = token tile mt (32 rows) and NJ column tiles of the waves of a cut tile; lane, column
 // and register layout and the rounding points of the kernel above, outputs as 8-byte stores.  One column tile instead of both
 // in a workgroup: twice the waves in flight and half the registers (4096 -> 2048, 300 tokens: 27.6 -> 22.1 us for the layer's
 // six; at 80 cut tiles of rank 64 the sums' bytes bound it either way, 27 us).
-template <typename T, int MODE>
+template <typename T, int MODE, int NJ>
 __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const BwdTArgs a) {
   constexpr bool swiglu = MODE == FMSA_BWD_SWIGLU;
   // The two column tiles share the 128-byte lines of what is read and written row by row, so their workgroups are MT = 8 ids
   // apart, on one XCD; token tile 0 of consecutive cuts goes to different ones.  (On two XCDs the SwiGLU's six arrays moved half
   // a line at a time: 4096 -> 14336, 64 / 256 tokens, 45 / 70 us a call, and 39 / 61 this way; 4096 of 2048 at 512 41 and 36.)
-  static_assert(MT == 8 && NT == 2, "workgroups go to the XCDs by id % 8");
-  const int cut = blockIdx.x / (MT * NT), mt = (blockIdx.x + cut) % MT, j = blockIdx.x / MT % NT;
+  static_assert(MT == 8 && NT == 2 && (NJ == 1 || NJ == 2), "workgroups go to the XCDs by id % 8");
+  const int cut = blockIdx.x / (MT * (NT / NJ)), mt = (blockIdx.x + cut) % MT, jt = NJ == 1 ? blockIdx.x / MT % NT : 0;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
   int bm, bk;
   bwd_tile(a, a.n_whole + cut, bm, bk);
@@ -757,76 +757,96 @@ __global__ __launch_bounds__(256) void gptq_lora_bwd_dx_t_finish_kernel(const Bw
   bool any_lora = false;
   for (int p = 0; p < a.n_proj; ++p) any_lora = any_lora || select_proj(a, p).r > 0;
   const bool has_mask = a.mask_src != nullptr && any_lora;
-  const int col0 = bk * 256 + 64 * wave + 32 * j;
-  u32x2 mask[4];
+  const int col0 = bk * 256 + 64 * wave + 32 * jt;
+  u32x2 mask[NJ][4];
+  f32x4 acc[NJ][4];
 #pragma unroll
-  for (int i0 = 0; i0 < 4; ++i0) {
-    const int col = col0 + 8 * i0 + 4 * half;
-    mask[i0] = u32x2{0u, 0u};
-    if (has_mask && m_ok && col < a.K) mask[i0] = *reinterpret_cast<const u32x2*>(a.mask_src + (size_t)m * a.ldmask + col);
+  for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = col0 + 32 * j + 8 * i0 + 4 * half;
+      mask[j][i0] = u32x2{0u, 0u};
+      if (has_mask && m_ok && col < a.K) mask[j][i0] = *reinterpret_cast<const u32x2*>(a.mask_src + (size_t)m * a.ldmask + col);
+    }
+    split_load<NT>(acc[j], a.partial, cut, mt, jt + j, a.n_ranges);
   }
-  f32x4 acc[4];
-  split_load<NT>(acc, a.partial, cut, mt, j, a.n_ranges);
-  f32x16 lora;
+  f32x16 lora[NJ];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) lora[i] = 0.f;
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lora[j][i] = 0.f;
   for (int p = 0; p < a.n_proj; ++p) {
     const BwdTProjDev P = select_proj(a, p);
     if (P.r <= 0) continue;
-    f32x16 tmp;
+    f32x16 tmp[NJ];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) tmp[i] = 0.f;
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tmp[j][i] = 0.f;
     for (int j0 = 0; j0 < P.r; j0 += 64) {
-      u32x4 tf[4], af[4];
+      u32x4 tf[4], af[4][NJ];
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         const int ko = j0 + 16 * st + 8 * half;
         tf[st] = u32x4{0u, 0u, 0u, 0u};
         if (m_ok && ko < P.r) tf[st] = *reinterpret_cast<const u32x4*>(P.T + (size_t)m * P.ldt + ko);
-        af[st] = u32x4{0u, 0u, 0u, 0u};
-        if (col0 < a.K && ko < P.r) af[st] = *reinterpret_cast<const u32x4*>(P.At + (size_t)(col0 + l32) * P.r + ko);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int col = col0 + 32 * j;
+          af[st][j] = u32x4{0u, 0u, 0u, 0u};
+          if (col < a.K && ko < P.r) af[st][j] = *reinterpret_cast<const u32x4*>(P.At + (size_t)(col + l32) * P.r + ko);
+        }
       }
 #pragma unroll
       for (int st = 0; st < 4; ++st)
-        if (j0 + 16 * st < P.r) tmp = mfma32<T>(af[st], tf[st], tmp);
+        if (j0 + 16 * st < P.r) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) tmp[j] = mfma32<T>(af[st][j], tf[st], tmp[j]);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) lora[i] += P.s * tmp[i];
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lora[j][i] += P.s * tmp[j][i];
   }
-  if (!m_ok || col0 >= a.K) return;
+  if (!m_ok) return;
 #pragma unroll
-  for (int i0 = 0; i0 < 4; ++i0) {
-    const int col = col0 + 8 * i0 + 4 * half;
-    const u32x2 bv = {pack2<T>(acc[i0][0], acc[i0][1]), pack2<T>(acc[i0][2], acc[i0][3])};
-    const u32x2 mv = mask[i0];
-    u32x2 lv = {0u, 0u};
-    if (any_lora) lv = u32x2{pack2<T>(lora[4 * i0], lora[4 * i0 + 1]), pack2<T>(lora[4 * i0 + 2], lora[4 * i0 + 3])};
-    if constexpr (swiglu) {
-      const size_t o = (size_t)m * a.ldeg + col;
-      const u32x2 ev = *reinterpret_cast<const u32x2*>(a.e + o), gv = *reinterpret_cast<const u32x2*>(a.g + o);
-      u32x2 hv, dgv, dev;
+  for (int j = 0; j < NJ; ++j) {
+    if (col0 + 32 * j >= a.K) continue;
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        uint32_t h, dg, de;
-        swiglu_bwd_pair<T>(ev[w], gv[w], bv[w], lv[w], mv[w], has_mask, h, dg, de);
-        hv[w] = h;
-        dgv[w] = dg;
-        dev[w] = de;
-      }
-      *reinterpret_cast<u32x2*>(a.h + o) = hv;
-      *reinterpret_cast<u32x2*>(a.e + o) = dgv;
-      *reinterpret_cast<u32x2*>(a.g + o) = dev;
-    } else {
-      u32x2 ov = bv;
-      if (any_lora) {
+    for (int i0 = 0; i0 < 4; ++i0) {
+      const int col = col0 + 32 * j + 8 * i0 + 4 * half;
+      const u32x2 bv = {pack2<T>(acc[j][i0][0], acc[j][i0][1]), pack2<T>(acc[j][i0][2], acc[j][i0][3])};
+      const u32x2 mv = mask[j][i0];
+      u32x2 lv = {0u, 0u};
+      if (any_lora) lv = u32x2{pack2<T>(lora[j][4 * i0], lora[j][4 * i0 + 1]), pack2<T>(lora[j][4 * i0 + 2], lora[j][4 * i0 + 3])};
+      if constexpr (swiglu) {
+        const size_t o = (size_t)m * a.ldeg + col;
+        const u32x2 ev = *reinterpret_cast<const u32x2*>(a.e + o), gv = *reinterpret_cast<const u32x2*>(a.g + o);
+        u32x2 hv, dgv, dev;
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
-          const float l0 = (!has_mask || (mv[w] & 0x7fffu)) ? unpack_lo<T>(lv[w]) : 0.f;
-          const float l1 = (!has_mask || ((mv[w] >> 16) & 0x7fffu)) ? unpack_hi<T>(lv[w]) : 0.f;
-          ov[w] = pack2<T>(unpack_lo<T>(bv[w]) + l0, unpack_hi<T>(bv[w]) + l1);
+          uint32_t h, dg, de;
+          swiglu_bwd_pair<T>(ev[w], gv[w], bv[w], lv[w], mv[w], has_mask, h, dg, de);
+          hv[w] = h;
+          dgv[w] = dg;
+          dev[w] = de;
         }
+        *reinterpret_cast<u32x2*>(a.h + o) = hv;
+        *reinterpret_cast<u32x2*>(a.e + o) = dgv;
+        *reinterpret_cast<u32x2*>(a.g + o) = dev;
+      } else {
+        u32x2 ov = bv;
+        if (any_lora) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const float l0 = (!has_mask || (mv[w] & 0x7fffu)) ? unpack_lo<T>(lv[w]) : 0.f;
+            const float l1 = (!has_mask || ((mv[w] >> 16) & 0x7fffu)) ? unpack_hi<T>(lv[w]) : 0.f;
+            ov[w] = pack2<T>(unpack_lo<T>(bv[w]) + l0, unpack_hi<T>(bv[w]) + l1);
+          }
+        }
+        *reinterpret_cast<u32x2*>(a.dX + (size_t)m * a.lddx + col) = ov;
       }
-      *reinterpret_cast<u32x2*>(a.dX + (size_t)m * a.lddx + col) = ov;
     }
   }
 }
@@ -1028,11 +1048,18 @@ int launch_gptq_lora_bwd_dx_t(const fmsa_bwd_proj* projs, int n_proj, int M, int
 #undef LAUNCH_S
   FMSA_CHECK_LAUNCH();
   if (plan.s > 1) {
-    const dim3 fgrid(plan.n_split * MT * NT);
-#define FINISH(TT)                                                                                                            \
-  do {                                                                                                                        \
-    if (mode == FMSA_BWD_SWIGLU) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_SWIGLU>), fgrid, block, 0, st, a); \
-    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_LINEAR>), fgrid, block, 0, st, a);                  \
+    // Many ranks are another chain of reads, of T by every column tile: both in a workgroup where ranks add up to 128 and the
+    // workgroups still are two to a CU, or many (one / both, us a call: q, k, v of rank 64 at 2048 tokens, K 4096, 128 tiles, 126.5 /
+    // 123.0, K 2048, 64 tiles, 56.0 / 52.1, rank 128 69 / 61; 2560 tokens, K 2048, 80 tiles, 80.3 / 80.4, K 3072, 72, 1.05 of the time)
+    int ranks = 0;
+    for (int p = 0; p < n_proj; ++p) ranks += projs[p].r;
+    const bool both = mode != FMSA_BWD_SWIGLU && ranks >= 128 && (plan.n_split == 64 || plan.n_split > 96);
+    const dim3 fgrid(plan.n_split * MT * (both ? 1 : NT));
+#define FINISH(TT)                                                                                                                     \
+  do {                                                                                                                                 \
+    if (mode == FMSA_BWD_SWIGLU) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_SWIGLU, 1>), fgrid, block, 0, st, a); \
+    else if (both) hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_LINEAR, 2>), fgrid, block, 0, st, a);              \
+    else hipLaunchKernelGGL((gptq_lora_bwd_dx_t_finish_kernel<TT, FMSA_BWD_LINEAR, 1>), fgrid, block, 0, st, a);                        \
   } while (0)
     if (act_dtype == FMSA_BF16) FINISH(bf16_t);
     else FINISH(f16_t);

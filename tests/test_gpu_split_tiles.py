@@ -161,6 +161,8 @@ def _bwd_projs(M, K, Ns, r, s, dtype, mask, base, blocksize=64):
     (300, 1152, [1024, 256, 1056], 24, True, True),  # ranges that begin and end inside a projection; N ends in half a stage
     (300, 1152, [1024, 256, 1056], 64, False, True),
     (65, 288, [2048], 0, False, True),               # no adapter
+    (2000, 2016, [2048, 512, 288], 64, True, True),  # 64 cut tiles and 192 ranks, 104 and 128: both column tiles in a workgroup
+    (2000, 3296, [4096], 128, False, True),          # of the second launch
     (513, 14336, [2048], 24, True, False),           # 168 tiles: too many to cut
     (1030, 14336, [2048], 24, True, False),          # 280 tiles: the whole round would cost more than the 24 give
     (8300, 2048, [2048], 24, True, True),            # 264 tiles: one whole round, 8 cut
