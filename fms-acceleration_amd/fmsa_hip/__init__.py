@@ -756,7 +756,8 @@ def cross_entropy_bwd_(logits2d, dlosses, lse, labels):
 
 def cross_entropy_rows_fwd(logits3d, labels, seq_out: int):
     """(losses, logsumexp), fp32 [n_seq * seq_out], of rows 0 .. seq_out - 1 of every sequence of contiguous 16-bit logits
-    [n_seq, seq_in, V]; labels int64 [n_seq * seq_out], -100 ignored."""
+    [n_seq, seq_in, V]; labels int64 [n_seq * seq_out], -100 ignored.  For callers that want them by rows: the loss operator
+    takes causal_lm_loss_fwd, which sums them on the way."""
     n_seq, seq_in, V = logits3d.shape
     rows = n_seq * seq_out
     assert logits3d.is_contiguous() and labels.dtype == torch.int64 and labels.is_contiguous() and labels.numel() == rows

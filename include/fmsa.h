@@ -470,7 +470,8 @@ int fmsa_cross_entropy_bwd(void* logits, int64_t ld, const float* dloss, int64_t
  * sequence count: seq_out = seq_in - 1 with labels [n_seq, seq_out] shifted by one token is the causal-LM loss
  * (kernels/unsloth/cross_entropy_loss.py:302-327) without a copy of the logits.  losses, logsumexp: [n_seq * seq_out].
  * The backward writes a gradient of its own, all of [n_seq, seq_in, V] (row stride ld; rows past seq_out and rows without
- * a label are zeros), and leaves the logits alone. */
+ * a label are zeros), and leaves the logits alone.  For callers that want the rows' losses; the loss as one number is
+ * fmsa_causal_lm_loss_fwd below, on the same kernels. */
 int fmsa_cross_entropy_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int n_seq, int seq_in, int seq_out,
                                 int V, int dtype, float* losses, float* logsumexp, void* stream);
 /* The same forward, leaving the rows that have a label in `kept` as well (the logits' layout and row stride, and their
