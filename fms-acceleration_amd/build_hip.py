@@ -24,7 +24,10 @@ OBJ_DIR = os.path.join(CSRC, "build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libfmsa_hip.so")
 
-SOURCES = ["api.hip", "dequant.hip", "gemm_fwd.hip", "gemm_few.hip", "gemm_bwd.hip", "gemm_bwd_t.hip", "lora_skinny.hip", "elementwise.hip", "nf4.hip", "norm_rope.hip"]
+SOURCES = ["api.hip", "dequant.hip", "gemm_fwd.hip", "gemm_few.hip", "gemm_bwd.hip", "gemm_bwd_t.hip", "lora_skinny.hip", "elementwise.hip", "nf4.hip", "norm_rope.hip", "tile_plan.hip"]
+# one source, a translation unit a tile height (the kernels of the low tiles take the longest to compile)
+HEIGHT_SOURCES = ["gemm_bwd_t_low.hip", "gemm_fwd_low.hip"]
+HEIGHTS = (4, 5, 6, 7)
 PROBE_SOURCE = "probe.hip"
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libfmsa_probe.so")
 CALLS_SOURCE = "host_calls.cpp"
@@ -74,11 +77,13 @@ def build(verbose: bool = False, extra_flags=()) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     hipcc = _hipcc()
-    objs = [os.path.join(OBJ_DIR, s.replace(".hip", ".o")) for s in SOURCES]
+    units = [(s, os.path.join(OBJ_DIR, s.replace(".hip", f"_{h}.o")), [f"-DFMSA_TILE_HEIGHT={h}"]) for s in HEIGHT_SOURCES for h in HEIGHTS]
+    units += [(s, os.path.join(OBJ_DIR, s.replace(".hip", ".o")), []) for s in SOURCES]
+    objs = [obj for _, obj, _ in units]
 
-    def compile_one(pair):
-        src, obj = pair
-        cmd = [hipcc, *HIPCC_FLAGS, *extra_flags, "-c", os.path.join(CSRC, src), "-o", obj]
+    def compile_one(unit):
+        src, obj, defines = unit
+        cmd = [hipcc, *HIPCC_FLAGS, *extra_flags, *defines, "-c", os.path.join(CSRC, src), "-o", obj]
         out = _run(cmd)
         if verbose and out.strip():
             print(out)
@@ -86,9 +91,9 @@ def build(verbose: bool = False, extra_flags=()) -> str:
 
     probe_obj = os.path.join(OBJ_DIR, PROBE_SOURCE.replace(".hip", ".o"))
     calls_obj = os.path.join(OBJ_DIR, CALLS_SOURCE.replace(".cpp", ".o"))
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 2)) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
         calls = pool.submit(_compile_calls, calls_obj)
-        list(pool.map(compile_one, list(zip(SOURCES, objs)) + [(PROBE_SOURCE, probe_obj)]))
+        list(pool.map(compile_one, units + [(PROBE_SOURCE, probe_obj, [])]))
         torch_libs = calls.result()
     for path, members in ((LIB_PATH, objs), (PROBE_LIB_PATH, [probe_obj])):
         tmp = path + ".tmp"

@@ -1,6 +1,7 @@
 // extern "C" entry points: argument validation (no HIP call before it passes) and dispatch to
 // the launchers in the kernel translation units.
 #include "common.h"
+#include "tile_plan.h"
 
 #include <atomic>
 
@@ -27,6 +28,7 @@ size_t lora_few_workspace(const fmsa_few_proj* projs, int n_proj, int M);
 int launch_lora_few(const fmsa_few_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H, int64_t ldh,
                     int act_dtype, void* workspace, hipStream_t st);
 size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode);
+bool gptq_lora_fwd_rope_pays(const fmsa_fwd_proj* projs, int n_proj, int M);
 size_t gptq_lora_bwd_dx_t_workspace(const fmsa_bwd_proj* projs, int n_proj, int M);
 int launch_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e,
                             void* g, void* h_out, int64_t ldeg, int act_dtype, hipStream_t st);
@@ -386,6 +388,20 @@ int fmsa_gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int
   return gptq_lora_fwd_is_few(projs, n_proj, M, mode) ? 1 : 0;
 }
 
+int fmsa_gptq_lora_fwd_tile(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return 32 * plan_fwd(projs, n_proj, M, mode).mt;
+}
+
+int fmsa_gptq_lora_fwd_rope_pays(const fmsa_fwd_proj* projs, int n_proj, int M) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return gptq_lora_fwd_rope_pays(projs, n_proj, M) ? 1 : 0;
+}
+
 int fmsa_gptq_lora_fwd_few(const fmsa_fwd_proj* projs, int n_proj, const void* X, int64_t ldx, int M, int mode, void* H,
                            int64_t ldh, int act_dtype, void* stream) {
   if (int rc = check_fwd(projs, n_proj, X, ldx, M, mode, H, ldh, act_dtype)) return rc;
@@ -480,6 +496,13 @@ size_t fmsa_gptq_lora_bwd_dx_workspace(const fmsa_bwd_proj* projs, int n_proj, i
   for (int p = 0; p < n_proj; ++p)
     if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
   return bwd_dx_twin_flavour(projs, n_proj, act_dtype) ? gptq_lora_bwd_dx_t_workspace(projs, n_proj, M) : 0;
+}
+
+int fmsa_gptq_lora_bwd_dx_tile(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, int act_dtype) {
+  if (!projs || n_proj < 1 || n_proj > 3 || M <= 0) return 0;
+  for (int p = 0; p < n_proj; ++p)
+    if (projs[p].w.K <= 0 || projs[p].w.N <= 0 || projs[p].w.group_size <= 0) return 0;
+  return bwd_dx_twin_flavour(projs, n_proj, act_dtype) ? 32 * plan_bwd_t(projs, n_proj, M, mode).mt : 256;
 }
 
 int fmsa_gptq_lora_bwd_dx_ws(const fmsa_bwd_proj* projs, int n_proj, int M, int mode, void* dX, int64_t lddx, void* e, void* g,

@@ -52,6 +52,9 @@ EXPORTED_SYMBOLS = (
     "fmsa_lora_few_workspace",
     "fmsa_lora_few_fwd",
     "fmsa_gptq_lora_fwd_rope",
+    "fmsa_gptq_lora_fwd_rope_pays",
+    "fmsa_gptq_lora_fwd_tile",
+    "fmsa_gptq_lora_bwd_dx_tile",
     "fmsa_gptq_lora_bwd_dx",
     "fmsa_gptq_lora_bwd_dx_workspace",
     "fmsa_gptq_lora_bwd_dx_ws",
@@ -282,6 +285,9 @@ def lib() -> ctypes.CDLL:
     L.fmsa_gptq_lora_fwd_ws.argtypes = [POINTER(FwdProj), c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p,
                                         c_size_t, c_void_p]
     L.fmsa_gptq_lora_fwd_is_few.argtypes = [POINTER(FwdProj), c_int, c_int, c_int]
+    L.fmsa_gptq_lora_fwd_rope_pays.argtypes = [POINTER(FwdProj), c_int, c_int]
+    L.fmsa_gptq_lora_fwd_tile.argtypes = [POINTER(FwdProj), c_int, c_int, c_int]
+    L.fmsa_gptq_lora_bwd_dx_tile.argtypes = [POINTER(BwdProj), c_int, c_int, c_int, c_int]
     L.fmsa_gptq_lora_fwd_few.argtypes = L.fmsa_gptq_lora_fwd.argtypes
     L.fmsa_lora_few_is_few.argtypes = [POINTER(FewProj), c_int, c_int, c_int]
     L.fmsa_lora_few_workspace.restype = c_size_t
@@ -577,12 +583,12 @@ def lora_few(x2d, projs, mode: int = FWD_LINEAR):
 
 
 def gptq_lora_fwd_splits(weights, M: int) -> bool:
-    """Whether the 256-token tiles of a LINEAR launch of these weights over M tokens are cut (where the kernel for few tokens is
-    taken instead, they would be, unless the launch is very small)."""
+    """Whether a LINEAR launch of these weights over M tokens, and a rotating pass over its outputs, is expected to be faster than
+    the launch that rotates in its epilogue: its tiles are cut, or lower than the rotating ones and enough is won that way."""
     arr = (FwdProj * len(weights))()
     for i, w in enumerate(weights):
         arr[i].w = w
-    return lib().fmsa_gptq_lora_fwd_workspace(arr, len(weights), M, FWD_LINEAR) > 0
+    return not lib().fmsa_gptq_lora_fwd_rope_pays(arr, len(weights), M)
 
 
 def gptq_lora_bwd_dx(projs: Sequence[dict], M: int, K: int, mode: int = BWD_LINEAR, e=None, g=None, split: bool = False):

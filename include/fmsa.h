@@ -258,9 +258,11 @@ int fmsa_gptq_lora_fwd(const fmsa_fwd_proj* projs /*host*/, int n_proj, const vo
 /* The same forward with a partial-sum buffer at hand: where the tiles do not fill the chip (few tokens, few columns, or
  * the rest of a launch), they are cut along K over the idle CUs; the ranges' fp32 sums are added in index order, so the
  * result does not depend on scheduling.  fmsa_gptq_lora_fwd_workspace gives the bytes (0: nothing is cut); with a smaller
- * or no workspace the call runs as fmsa_gptq_lora_fwd does.  16-byte aligned; calls that may overlap in time need separate
+ * or no workspace the call runs as fmsa_gptq_lora_fwd does.  (A tile has 256 tokens, or 128, 160, 192 or 224 where that fills the
+ * chip better; its height changes no bit.)  16-byte aligned; calls that may overlap in time need separate
  * workspaces. */
 size_t fmsa_gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M, int mode);
+int fmsa_gptq_lora_fwd_tile(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M, int mode); /* tokens of a tile of such a call */
 int fmsa_gptq_lora_fwd_ws(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M, int mode,
                           void* H, int64_t ldh, int act_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
@@ -316,6 +318,9 @@ typedef struct fmsa_rope {
 } fmsa_rope;
 int fmsa_gptq_lora_fwd_rope(const fmsa_fwd_proj* projs /*host*/, int n_proj, const void* X, int64_t ldx, int M,
                             const fmsa_rope* rope /*host*/, int act_dtype, void* stream);
+/* 1: fmsa_gptq_lora_fwd_rope over these projections is expected to take less time than fmsa_gptq_lora_fwd_ws and a rotating pass
+ * over what it wrote (tiles of fewer tokens and cut ones have no rotating flavours). */
+int fmsa_gptq_lora_fwd_rope_pays(const fmsa_fwd_proj* projs /*host*/, int n_proj, int M);
 
 /* ------------------------------------------------------------------------------------------
  * Fused input-gradient:
@@ -375,6 +380,7 @@ int fmsa_gptq_lora_bwd_dx(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M
 /* The same with a partial-sum buffer (see fmsa_gptq_lora_fwd_ws); calls that run on the transposed twin use it.  The bytes
  * are those of the mode that needs more. */
 size_t fmsa_gptq_lora_bwd_dx_workspace(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int act_dtype);
+int fmsa_gptq_lora_bwd_dx_tile(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int mode, int act_dtype); /* tokens of a tile */
 int fmsa_gptq_lora_bwd_dx_ws(const fmsa_bwd_proj* projs /*host*/, int n_proj, int M, int mode, void* dX, int64_t lddx,
                              void* e, void* g, void* h_out, int64_t ldeg, int act_dtype, void* workspace,
                              size_t workspace_bytes, void* stream);
