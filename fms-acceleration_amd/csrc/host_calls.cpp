@@ -13,6 +13,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "../../include/fmsa.h"
@@ -549,6 +550,384 @@ PyObject* lora_few(PyObject* const* a, Py_ssize_t) {  // x2d, ((w, A, B, bias, s
   return mode == FMSA_FWD_SWIGLU ? wrap(h) : wrap_list(outs);
 }
 
+// ---- adapted projections, read from their modules ---------------------------------------------------------------------------
+// What get_lora_parameters, prepare and lora_few_ok of the Python side find, in a third of their time: a pass over a layer without a
+// graph asks for seven projections, 50 of its 140 us on the host.  Nothing here raises and nothing is decided that they would decide
+// otherwise: whatever is not the ordinary case (`false`, None) is left to them.
+struct Obj {  // owned reference or null
+  PyObject* o;
+  explicit Obj(PyObject* p = nullptr) : o(p) {}
+  Obj(Obj&& other) noexcept : o(other.o) { other.o = nullptr; }
+  Obj& operator=(Obj&& other) noexcept {
+    std::swap(o, other.o);
+    return *this;
+  }
+  ~Obj() { Py_XDECREF(o); }
+  Obj(const Obj&) = delete;
+  Obj& operator=(const Obj&) = delete;
+  explicit operator bool() const { return o != nullptr; }
+};
+
+Obj borrowed(PyObject* o) {
+  Py_XINCREF(o);
+  return Obj(o);
+}
+
+PyObject *g_identity = nullptr, *g_module_dict = nullptr, *g_parameter = nullptr;  // torch.nn.Identity, ModuleDict, Parameter
+
+Obj attribute(PyObject* o, PyObject* name) {
+  Obj v(PyObject_GetAttr(o, name));
+  if (!v) PyErr_Clear();
+  return v;
+}
+
+Obj item_of(PyObject* container, PyObject* k) {
+  Obj v(PyDict_CheckExact(container) ? (Py_XINCREF(PyDict_GetItemWithError(container, k)), PyDict_GetItemWithError(container, k))
+                                     : PyObject_GetItem(container, k));
+  if (!v) PyErr_Clear();
+  return v;
+}
+
+// utils.member: the dictionary `kind` of a module first, then getattr
+Obj member(PyObject* module, PyObject* kind, PyObject* name) {
+  PyObject** own = _PyObject_GetDictPtr(module);
+  if (own && *own && PyDict_CheckExact(*own) && !PyDict_GetItemWithError(*own, name)) {
+    PyObject* held = PyDict_GetItemWithError(*own, kind);
+    if (held && held != Py_None) {
+      const int has = PySequence_Contains(held, name);
+      if (has > 0) return item_of(held, name);
+      if (has < 0) PyErr_Clear();
+    }
+  }
+  PyErr_Clear();
+  return attribute(module, name);
+}
+
+// getattr(module, name, None) of what modules keep as a buffer, a parameter or an attribute
+Obj held(PyObject* module, PyObject* name) {
+  static PyObject *buffers = key("_buffers"), *parameters = key("_parameters");
+  if (!_PyType_Lookup(Py_TYPE(module), name))
+    for (PyObject* kind : {buffers, parameters}) {
+      PyObject** own = _PyObject_GetDictPtr(module);
+      if (!own || !*own || !PyDict_CheckExact(*own) || PyDict_GetItemWithError(*own, name)) break;
+      PyObject* in = PyDict_GetItemWithError(*own, kind);
+      if (in && PyDict_CheckExact(in) && PyDict_GetItemWithError(in, name)) return item_of(in, name);
+    }
+  PyErr_Clear();
+  Obj v = attribute(module, name);
+  return v ? std::move(v) : borrowed(Py_None);
+}
+
+// container[active] of a ModuleDict, or of whatever stands in for one
+Obj active_of(PyObject* container, PyObject* active) {
+  static PyObject* modules = key("_modules");
+  if (reinterpret_cast<PyObject*>(Py_TYPE(container)) == g_module_dict) {
+    PyObject** own = _PyObject_GetDictPtr(container);
+    PyObject* in = own && *own ? PyDict_GetItemWithError(*own, modules) : nullptr;
+    if (in && PyDict_CheckExact(in)) return item_of(in, active);
+  }
+  return item_of(container, active);
+}
+
+// what was set on a tensor (borrowed); none of the names is one of the class
+PyObject* mark(PyObject* t, PyObject* name) {
+  PyObject** own = _PyObject_GetDictPtr(t);
+  PyObject* v = own && *own ? PyDict_GetItemWithError(*own, name) : nullptr;
+  PyErr_Clear();
+  return v;
+}
+
+bool plain(PyObject* o) { return o && THPVariable_CheckExact(o) && !THPVariable_Unpack(o).is_inference(); }
+
+bool equals(PyObject* number, int64_t v) {
+  const long long n = PyLong_Check(number) ? PyLong_AsLongLong(number) : -1;
+  if (n == -1 && PyErr_Occurred()) PyErr_Clear();
+  return PyLong_Check(number) && n == v;
+}
+
+// ... or a parameter of a class that stands for its data as torch.nn.Parameter does (bitsandbytes' Params4bit)
+bool plain_weight(PyObject* o) {
+  static PyObject* function = key("__torch_function__");
+  if (plain(o)) return true;
+  if (!o || !THPVariable_Check(o) || THPVariable_Unpack(o).is_inference()) return false;
+  PyTypeObject* parameter = reinterpret_cast<PyTypeObject*>(g_parameter);
+  return PyType_IsSubtype(Py_TYPE(o), parameter) && _PyType_Lookup(Py_TYPE(o), function) == _PyType_Lookup(parameter, function);
+}
+
+int64_t address(const at::Tensor& t) { return reinterpret_cast<int64_t>(t.data_ptr()); }
+
+// gptq_prepared.prepare's cached weight where its key still holds (borrowed; null: ask there)
+PyObject* prepared_gptq(PyObject* qweight, PyObject* scales, PyObject* qzeros, PyObject* g_idx) {
+  static PyObject *kprep = key("_fmsa_prepared"), *koff = key("offset");
+  if (!plain(qweight) || !plain(scales) || !plain(qzeros) || !plain(g_idx)) return nullptr;
+  PyObject* cached = mark(qweight, kprep);
+  if (!cached || !PyTuple_CheckExact(cached) || PyTuple_GET_SIZE(cached) != 2) return nullptr;
+  PyObject* k = PyTuple_GET_ITEM(cached, 0);
+  if (!PyTuple_CheckExact(k) || PyTuple_GET_SIZE(k) != 9) return nullptr;
+  PyObject* off = mark(qzeros, koff);
+  const long offset = off && off != Py_None ? (PyLong_CheckExact(off) ? PyLong_AsLong(off) : -1) : 0;
+  const at::Tensor &q = THPVariable_Unpack(qweight), &s = THPVariable_Unpack(scales), &z = THPVariable_Unpack(qzeros), &g = THPVariable_Unpack(g_idx);
+  const int64_t now[9] = {address(q), address(s), address(z), address(g), (int64_t)g._version(), (int64_t)q._version(), (int64_t)s._version(),
+                          (int64_t)z._version(), offset};
+  for (int i = 0; i < 9; ++i)
+    if (!equals(PyTuple_GET_ITEM(k, i), now[i])) return nullptr;
+  return PyTuple_GET_ITEM(cached, 1);
+}
+
+// nf4_prepared.prepare's, likewise
+PyObject* prepared_nf4(PyObject* W, PyObject* state) {
+  static PyObject *kprep = key("_fmsa_prepared"), *kabsmax = key("absmax"), *koff = key("offset"), *kshape = key("shape"), *kblock = key("blocksize");
+  if (!plain_weight(W)) return nullptr;
+  PyObject* cached = mark(W, kprep);
+  if (!cached || !PyTuple_CheckExact(cached) || PyTuple_GET_SIZE(cached) != 2) return nullptr;
+  PyObject* k = PyTuple_GET_ITEM(cached, 0);
+  if (!PyTuple_CheckExact(k) || PyTuple_GET_SIZE(k) != 7) return nullptr;
+  const Obj absmax = attribute(state, kabsmax), off = attribute(state, koff), shape = attribute(state, kshape), block = attribute(state, kblock);
+  if (!absmax || !plain(absmax.o) || !off || !plain(off.o) || !shape || !block) return nullptr;
+  PyObject* ok = PyTuple_GET_ITEM(k, 4);
+  const at::Tensor &w = THPVariable_Unpack(W), &a = THPVariable_Unpack(absmax.o), &o = THPVariable_Unpack(off.o);
+  // W.data, whose version counter is its own, for a parameter
+  const int64_t version = Py_TYPE(W) == reinterpret_cast<PyTypeObject*>(THPVariableClass) ? (int64_t)w._version() : 0;
+  if (!equals(PyTuple_GET_ITEM(k, 0), address(w)) || !equals(PyTuple_GET_ITEM(k, 1), version) || !equals(PyTuple_GET_ITEM(k, 2), address(a)) ||
+      !equals(PyTuple_GET_ITEM(k, 3), (int64_t)a._version()) || !PyTuple_CheckExact(ok) || PyTuple_GET_SIZE(ok) != 2 ||
+      !equals(PyTuple_GET_ITEM(ok, 0), address(o)) || !equals(PyTuple_GET_ITEM(ok, 1), (int64_t)o._version()) || !PyLong_Check(block.o) ||
+      PyObject_RichCompareBool(PyTuple_GET_ITEM(k, 6), block.o, Py_EQ) != 1)
+    return nullptr;
+  PyObject* kept = PyTuple_GET_ITEM(k, 5);
+  const bool same = PyTuple_Check(shape.o) && PyTuple_Check(kept) && PyObject_RichCompareBool(kept, shape.o, Py_EQ) == 1;
+  PyErr_Clear();
+  return same ? PyTuple_GET_ITEM(cached, 1) : nullptr;
+}
+
+struct Adapted {  // an adapted projection whose adapter is active
+  Obj parts[5];   // GPTQ: qweight, scales, qzeros, g_idx, bits; NF4: W, quant state
+  Obj bias, A, B, scaling, dropout;
+};
+
+bool read_adapted(PyObject* proj, bool nf4, Adapted& p) {
+  static PyObject *kmod = key("_modules"), *kbuf = key("_buffers"), *kpar = key("_parameters"), *kbase = key("base_layer"),
+                  *kdisable = key("disable_adapters"), *kmerged = key("merged"), *kactives = key("active_adapters"), *kactive = key("active_adapter"),
+                  *kA = key("lora_A"), *kB = key("lora_B"), *kdrop = key("lora_dropout"), *kweight = key("weight"), *kscaling = key("scaling"),
+                  *kbias = key("bias"), *knz = key("_fmsa_nonzero"), *kmodule = key("__module__"), *kbits = key("bits"), *kstate = key("quant_state");
+  static PyObject* kq[4] = {key("qweight"), key("scales"), key("qzeros"), key("g_idx")};
+  const Obj disabled = attribute(proj, kdisable), merged = attribute(proj, kmerged);
+  if (!disabled || !merged || PyObject_IsTrue(disabled.o) != 0 || PyObject_IsTrue(merged.o) != 0) return PyErr_Clear(), false;
+  Obj base = member(proj, kmod, kbase);
+  if (!base) return false;
+  if (nf4) {
+    p.parts[0] = member(base.o, kpar, kweight);
+    if (!p.parts[0] || !plain_weight(p.parts[0].o)) return false;
+    PyObject* state = mark(p.parts[0].o, kstate);
+    if (!state || state == Py_None || PyList_Check(state) || PyTuple_Check(state)) return false;
+    p.parts[1] = borrowed(state);
+    p.bias = held(base.o, kbias);
+  } else {
+    const Obj where = attribute(base.o, kmodule);
+    if (!where || !PyUnicode_Check(where.o)) return false;
+    const char* text = PyUnicode_AsUTF8(where.o);
+    if (!text || std::strncmp(text, "auto_gptq", 9) == 0) return PyErr_Clear(), false;  // (those get their zero points' offset there)
+    Obj inner = member(base.o, kmod, kbase);
+    if (inner) base = std::move(inner);
+    for (int i = 0; i < 4; ++i)
+      if (!(p.parts[i] = member(base.o, kbuf, kq[i]))) return false;
+    if (!(p.parts[4] = attribute(base.o, kbits))) return false;
+    p.bias = held(base.o, kbias);
+    if (p.bias.o != Py_None) {  // dropped where it is all zeros, as found once for its version
+      PyObject* known = plain(p.bias.o) ? mark(p.bias.o, knz) : nullptr;
+      if (!known || !PyTuple_CheckExact(known) || PyTuple_GET_SIZE(known) != 2 ||
+          !equals(PyTuple_GET_ITEM(known, 0), (int64_t)THPVariable_Unpack(p.bias.o)._version()))
+        return false;
+      if (PyTuple_GET_ITEM(known, 1) != Py_True) p.bias = borrowed(Py_None);
+    }
+  }
+  Obj active = attribute(proj, kactives);
+  if (active) {
+    active = Obj(PySequence_GetItem(active.o, 0));
+    if (!active) return PyErr_Clear(), false;
+  } else if (!(active = attribute(proj, kactive))) {
+    return false;
+  }
+  const Obj la = member(proj, kmod, kA), lb = member(proj, kmod, kB), scalings = attribute(proj, kscaling), drops = member(proj, kmod, kdrop);
+  if (!la || !lb || !scalings) return false;
+  const Obj ma = active_of(la.o, active.o), mb = active_of(lb.o, active.o);
+  if (!ma || !mb) return false;
+  p.A = member(ma.o, kpar, kweight);
+  p.B = member(mb.o, kpar, kweight);
+  p.scaling = item_of(scalings.o, active.o);
+  p.dropout = !drops || drops.o == Py_None ? borrowed(Py_None) : active_of(drops.o, active.o);
+  return p.A && p.B && p.scaling && p.dropout;
+}
+
+PyObject* gptq_operands(PyObject* const* a, Py_ssize_t) {  // projection
+  Adapted p;
+  if (!read_adapted(a[0], false, p)) Py_RETURN_NONE;
+  Obj* all[10] = {&p.parts[0], &p.parts[1], &p.parts[2], &p.parts[3], &p.parts[4], &p.bias, &p.A, &p.B, &p.scaling, &p.dropout};
+  Ref t(PyTuple_New(10));
+  for (int i = 0; i < 10; ++i) {
+    PyTuple_SET_ITEM(t.o, i, all[i]->o);
+    all[i]->o = nullptr;
+  }
+  return t.release();
+}
+
+PyObject* gptq_prepared(PyObject* const* a, Py_ssize_t) {  // qweight, scales, qzeros, g_idx
+  PyObject* w = prepared_gptq(a[0], a[1], a[2], a[3]);
+  if (!w) Py_RETURN_NONE;
+  Py_INCREF(w);
+  return w;
+}
+
+// One projection of few tokens: what _few_tokens asks of it, and its operands
+bool few_operands(PyObject* proj, bool nf4, const at::Tensor& x, PyObject* dtype, bool& interleaved, Adapted& p, Obj& prepared, fmsa_few_proj& q) {
+  static PyObject *kstruct = key("struct"), *kperm = key("perm"), *kok = key("interleaved_ok");
+  if (!read_adapted(proj, nf4, p)) return false;
+  prepared = borrowed(nf4 ? prepared_nf4(p.parts[0].o, p.parts[1].o) : prepared_gptq(p.parts[0].o, p.parts[1].o, p.parts[2].o, p.parts[3].o));
+  if (!prepared) return false;
+  const Obj perm = attribute(prepared.o, kperm), view = attribute(prepared.o, kstruct);
+  if (!perm || perm.o != Py_None || !view || !plain(p.A.o) || !plain(p.B.o)) return false;
+  if (p.dropout.o != Py_None && reinterpret_cast<PyObject*>(Py_TYPE(p.dropout.o)) != g_identity) return false;
+  q.w = weight(view.o);
+  if (nf4 || x.scalar_type() != at::kHalf) {
+    interleaved = false;
+  } else if (interleaved) {
+    const Obj ok(PyObject_CallMethodObjArgs(prepared.o, kok, dtype, nullptr));
+    if (!ok) return PyErr_Clear(), false;
+    interleaved = ok.o == Py_True;
+  }
+  const at::Tensor &A = THPVariable_Unpack(p.A.o), &B = THPVariable_Unpack(p.B.o);
+  const at::ScalarType t = A.scalar_type();
+  if (q.w.group_size % 64 || x.size(-1) != q.w.K || A.dim() != 2 || B.dim() != 2 || B.scalar_type() != t || (t != at::kFloat && t != x.scalar_type()) ||
+      !A.is_cuda() || !B.is_cuda() || !A.is_contiguous() || !B.is_contiguous() || A.size(0) % 8 || A.size(0) <= 0 || A.size(0) > 128 ||
+      A.size(1) != q.w.K || B.size(0) != q.w.N || B.size(1) != A.size(0) || (address(A) | address(B)) % 16)
+    return false;
+  if (p.bias.o != Py_None) {
+    if (!plain(p.bias.o)) return false;
+    const at::Tensor& b = THPVariable_Unpack(p.bias.o);
+    if (b.scalar_type() != x.scalar_type() || b.numel() != q.w.N || !b.is_contiguous() || !b.is_cuda()) return false;
+    q.bias = ptr(b);
+  }
+  if (!PyFloat_Check(p.scaling.o) && !PyLong_Check(p.scaling.o)) return false;
+  q.A = ptr(A);
+  q.B = ptr(B);
+  q.r = (int)A.size(0);
+  q.s = (float)number(p.scaling.o);
+  q.param_dtype = dtype_enum(t);
+  q.ldy = q.w.N;
+  return true;
+}
+
+struct FewCall {
+  Adapted parts[3];
+  Obj prepared[3];
+  fmsa_few_proj arr[3] = {};
+  int n = 0;
+  bool read(PyObject* const* projs, int count, bool nf4, const at::Tensor& x, PyObject* dtype) {
+    static PyObject* kil = key("struct_interleaved");
+    bool interleaved = true;
+    n = count;
+    for (int i = 0; i < n; ++i)
+      if (!few_operands(projs[i], nf4, x, dtype, interleaved, parts[i], prepared[i], arr[i])) return false;
+    if (interleaved)
+      for (int i = 0; i < n; ++i) {
+        const Obj view = attribute(prepared[i].o, kil);
+        if (!view) return false;
+        arr[i].w = weight(view.o);
+      }
+    return true;
+  }
+  // outputs [.., N] (SwiGLU: h is written)
+  std::vector<at::Tensor> run(const at::Tensor& x, int M, int mode, const at::Tensor& h = at::Tensor()) {
+    auto sizes = x.sizes().vec();
+    std::vector<at::Tensor> outs;
+    for (int i = 0; i < n && mode != FMSA_FWD_SWIGLU; ++i) {
+      sizes.back() = arr[i].w.N;
+      outs.push_back(at::empty(sizes, x.options()));
+      arr[i].Y = ptr(outs[i]);
+    }
+    const int act = act_enum(x.scalar_type());
+    void* st = stream(x);
+    const size_t bytes = fmsa_lora_few_workspace(arr, n, M);
+    const at::Tensor ws = bytes ? workspace(bytes, x) : at::Tensor();
+    check("fmsa_lora_few_fwd", unlocked([&] {
+            return fmsa_lora_few_fwd(arr, n, ptr(x), x.size(-1), M, mode, ptr(h), h.defined() ? arr[0].w.N : 0, act, ptr(ws), bytes, st);
+          }));
+    return outs;
+  }
+};
+
+// Tokens of an input that the calls below take as it is, else 0
+int few_rows(PyObject* X, long most) {
+  if (!plain(X) && !(THPVariable_CheckExact(X) && THPVariable_Unpack(X).is_inference())) return 0;
+  const at::Tensor& x = THPVariable_Unpack(X);
+  if (x.dim() < 1 || x.numel() == 0 || !x.is_cuda() || !x.is_contiguous() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) return 0;
+  const int64_t M = x.numel() / x.size(-1);
+  return M <= most ? (int)M : 0;
+}
+
+// X, projections, whether they are NF4, its dtype, most tokens: their outputs where no graph is built and the kernel for few tokens
+// reads everything as it lies; else None
+PyObject* few_linear(PyObject* const* a, Py_ssize_t) {
+  const int M = few_rows(a[0], integer(a[4]));
+  if (!M) Py_RETURN_NONE;
+  const at::Tensor& x = THPVariable_Unpack(a[0]);
+  Sequence projs(a[1]);
+  need(projs.size() >= 1 && projs.size() <= 3, "few_linear: one to three projections");
+  PyObject* ps[3];
+  for (Py_ssize_t i = 0; i < projs.size(); ++i) ps[i] = projs[i];
+  FewCall call;
+  if (!call.read(ps, (int)projs.size(), truth(a[2]), x, a[3]) || !fmsa_lora_few_is_few(call.arr, call.n, M, FMSA_FWD_LINEAR)) Py_RETURN_NONE;
+  const auto outs = call.run(x, M, FMSA_FWD_LINEAR);
+  Ref t(PyTuple_New((Py_ssize_t)outs.size()));
+  for (size_t i = 0; i < outs.size(); ++i) PyTuple_SET_ITEM(t.o, (Py_ssize_t)i, wrap(outs[i]));
+  return t.release();
+}
+
+// X, (gate, up, down), NF4, dtype, most tokens: the output of the SwiGLU MLP, likewise
+PyObject* few_mlp(PyObject* const* a, Py_ssize_t) {
+  const int M = few_rows(a[0], integer(a[4]));
+  if (!M) Py_RETURN_NONE;
+  const at::Tensor& x = THPVariable_Unpack(a[0]);
+  Sequence projs(a[1]);
+  need(projs.size() == 3, "few_mlp: gate, up, down");
+  PyObject* const ps[3] = {projs[0], projs[1], projs[2]};
+  const bool nf4 = truth(a[2]);
+  FewCall first, second;
+  if (!first.read(ps, 2, nf4, x, a[3]) || first.arr[0].w.N != first.arr[1].w.N || !fmsa_lora_few_is_few(first.arr, 2, M, FMSA_FWD_SWIGLU)) Py_RETURN_NONE;
+  // the second launch is known to follow before the first goes out
+  auto sizes = x.sizes().vec();
+  sizes.back() = first.arr[0].w.N;
+  const at::Tensor h = at::empty(sizes, x.options());
+  if (!second.read(ps + 2, 1, nf4, h, a[3]) || !fmsa_lora_few_is_few(second.arr, 1, M, FMSA_FWD_LINEAR)) Py_RETURN_NONE;
+  first.run(x, M, FMSA_FWD_SWIGLU, h);
+  return wrap(second.run(h, M, FMSA_FWD_LINEAR)[0]);
+}
+
+// X, weight, eps, gemma: the normalised X where no graph is built and both lie as the kernel reads them, else None
+PyObject* rms_layernorm(PyObject* const* a, Py_ssize_t) {
+  if (!THPVariable_CheckExact(a[0]) || !THPVariable_CheckExact(a[1])) Py_RETURN_NONE;
+  const at::Tensor &x = THPVariable_Unpack(a[0]), &w = THPVariable_Unpack(a[1]);
+  if (x.dim() < 1 || x.numel() == 0 || !x.is_cuda() || !w.is_cuda() || !x.is_contiguous() || !w.is_contiguous() || w.numel() != x.size(-1)) Py_RETURN_NONE;
+  for (at::ScalarType t : {x.scalar_type(), w.scalar_type()})
+    if (t != at::kHalf && t != at::kBFloat16 && t != at::kFloat) Py_RETURN_NONE;
+  const float eps = (float)number(a[2]);
+  const int gemma = truth(a[3]), C = (int)x.size(-1), M = (int)(x.numel() / C);
+  at::Tensor y = at::empty(x.sizes(), x.options()), r = empty({M}, x, at::kFloat);
+  void* st = stream(x);
+  check("fmsa_rms_layernorm_fwd", unlocked([&] {
+          return fmsa_rms_layernorm_fwd(ptr(x), C, ptr(w), M, C, eps, gemma, dtype_enum(x.scalar_type()), dtype_enum(w.scalar_type()), ptr(y), C,
+                                        (float*)ptr(r), st);
+        }));
+  return wrap(y);
+}
+
+PyObject* install_types(PyObject* const* a, Py_ssize_t) {  // torch.nn.Identity, torch.nn.ModuleDict, torch.nn.Parameter
+  for (int i = 0; i < 3; ++i) Py_INCREF(a[i]);
+  g_identity = a[0];
+  g_module_dict = a[1];
+  g_parameter = a[2];
+  Py_RETURN_NONE;
+}
+
 // ---- norm and rotary embedding --------------------------------------------------------------------------------------------
 PyObject* rms_layernorm_fwd(PyObject* const* a, Py_ssize_t) {  // x2d, weight, eps, gemma
   const at::Tensor &x = tensor(a[0]), &w = tensor(a[1]);
@@ -641,6 +1020,8 @@ PyMethodDef g_methods[] = {ENTRY(lora_down, 3),           ENTRY(lora_down_batch,
                            ENTRY(lora_few, 3),            ENTRY(rms_layernorm_fwd, 4), ENTRY(rms_layernorm_bwd, 5),
                            ENTRY(rope_embedding_, 6),     ENTRY(rope_embedding_pair_, 5),
                            ENTRY(rope_embedding_strided, 4), ENTRY(install, 1),
+                           ENTRY(install_types, 3),       ENTRY(gptq_operands, 1),     ENTRY(gptq_prepared, 4),
+                           ENTRY(few_linear, 5),          ENTRY(few_mlp, 5),           ENTRY(rms_layernorm, 4),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fmsa_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

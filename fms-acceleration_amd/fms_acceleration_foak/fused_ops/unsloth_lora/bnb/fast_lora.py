@@ -144,6 +144,9 @@ class LoRA_MLP(torch.autograd.Function):
 
 
 def apply_lora_mlp_swiglu(self, X):
+    few = core.few_mlp(X, (self.gate_proj, self.up_proj, self.down_proj), True)
+    if few is not None:
+        return few
     gateW, gateW_quant, gate_bias, gateA, gateB, gateS, dropout_gate = get_lora_parameters(self.gate_proj)
     upW, upW_quant, up_bias, upA, upB, upS, dropout_up = get_lora_parameters(self.up_proj)
     downW, downW_quant, down_bias, downA, downB, downS, dropout_down = get_lora_parameters(self.down_proj)
@@ -156,6 +159,9 @@ def apply_lora_mlp_swiglu(self, X):
 
 
 def apply_lora_qkv(self, X):
+    few = core.few_linear(X, (self.q_proj, self.k_proj, self.v_proj), True)
+    if few is not None:
+        return few
     QW, QW_quant, Q_bias, QA, QB, QS, dropoutQ = get_lora_parameters(self.q_proj)
     KW, KW_quant, K_bias, KA, KB, KS, dropoutK = get_lora_parameters(self.k_proj)
     VW, VW_quant, V_bias, VA, VB, VS, dropoutV = get_lora_parameters(self.v_proj)
@@ -183,11 +189,14 @@ def apply_lora_qkv_rope(self, X, cos, sin):
                     dropoutQ, dropoutK, dropoutV)
 
 
+def _apply_lora_one(proj, X):
+    few = core.few_linear(X, (proj,), True)
+    return few[0] if few is not None else core.run(LoRA_W, X, *get_lora_parameters(proj))
+
+
 def apply_lora_o(self, X):
-    OW, OW_quant, O_bias, OA, OB, OS, dropout = get_lora_parameters(self.o_proj)
-    return core.run(LoRA_W, X, OW, OW_quant, O_bias, OA, OB, OS, dropout)
+    return _apply_lora_one(self.o_proj, X)
 
 
 def apply_lora_o_v2(self, X):
-    OW, OW_quant, O_bias, OA, OB, OS, dropout = get_lora_parameters(self)
-    return core.run(LoRA_W, X, OW, OW_quant, O_bias, OA, OB, OS, dropout)
+    return _apply_lora_one(self, X)

@@ -18,7 +18,7 @@ import torch
 
 import fmsa_hip
 
-from ...autograd import NoGraph, run  # noqa: F401  (run: for the entry points)
+from ...autograd import NoGraph, no_graph, run  # noqa: F401  (run: for the entry points)
 
 
 # ----------------------------------------------------------------------------------------------
@@ -73,6 +73,17 @@ def _few_tokens(ctx, X2, projs, dropouts, mode=fmsa_hip.FWD_LINEAR):
         return None
     il = _interleaved(projs, X2.dtype)
     return fmsa_hip.lora_few(X2, [(p.w.struct_interleaved if il else p.w.struct, p.A_param, p.B_param, p.bias, p.s) for p in projs], mode)
+
+
+def few_linear(X, projs, nf4):
+    """The outputs of adapted projections (modules) that share X where no graph is built, the tokens are few and everything lies as
+    the kernel reads it: what run() would return, the look-ups in native code.  None where that is not so."""
+    return fmsa_hip.native().few_linear(X, projs, nf4, X.dtype, fmsa_hip.FEW_TOKENS) if no_graph() else None
+
+
+def few_mlp(X, projs, nf4):
+    """The output of a SwiGLU MLP of (gate, up, down), likewise."""
+    return fmsa_hip.native().few_mlp(X, projs, nf4, X.dtype, fmsa_hip.FEW_TOKENS) if no_graph() else None
 
 
 class _Proj:

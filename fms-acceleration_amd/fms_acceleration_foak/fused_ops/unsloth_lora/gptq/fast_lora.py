@@ -34,6 +34,7 @@ from typing import Optional
 
 import torch
 
+import fmsa_hip
 from fmsa_hip.gptq_prepared import prepare as _prepare  # per-weight C-ABI view, cached on the qweight tensor
 
 from ....autograd import bwd_as_fwd
@@ -105,6 +106,15 @@ def get_lora_parameters(proj):
         return qstate, bias, None, None, None, None
     return (qstate, bias) + active_adapter_parts(proj)
 
+
+def _operands(proj):
+    """(qweight, scales, qzeros, g_idx, bits, bias, A, B, s, dropout) of get_lora_parameters, from native code where the projection
+    is an ordinary one with an active adapter."""
+    found = fmsa_hip.native().gptq_operands(proj)
+    if found is None:
+        qstate, bias, *adapter = get_lora_parameters(proj)
+        found = (*unpack_gptqstate(qstate), bias, *adapter)
+    return found
 
 
 def _proj(args, dtype):
@@ -239,29 +249,21 @@ class LoRA_MLP(torch.autograd.Function):
 # module-level entry points (bound to modules with MethodType by the model patcher)
 # ----------------------------------------------------------------------------------------------
 def apply_lora_mlp(self, X):
-    gateQstate, gate_bias, gateA, gateB, gateS, dropout_gate = get_lora_parameters(self.gate_proj)
-    upQState, up_bias, upA, upB, upS, dropout_up = get_lora_parameters(self.up_proj)
-    downQState, down_bias, downA, downB, downS, dropout_down = get_lora_parameters(self.down_proj)
-    return core.run(
-        LoRA_MLP, X,
-        *unpack_gptqstate(gateQstate), gate_bias, gateA, gateB, gateS,
-        *unpack_gptqstate(upQState), up_bias, upA, upB, upS,
-        *unpack_gptqstate(downQState), down_bias, downA, downB, downS,
-        dropout_gate, dropout_up, dropout_down,
-    )
+    projs = (self.gate_proj, self.up_proj, self.down_proj)
+    few = core.few_mlp(X, projs, False)
+    if few is not None:
+        return few
+    gate, up, down = map(_operands, projs)
+    return core.run(LoRA_MLP, X, *gate[:9], *up[:9], *down[:9], gate[9], up[9], down[9])
 
 
 def apply_lora_qkv(self, X):
-    Qqstate, Q_bias, QA, QB, QS, Qdropout = get_lora_parameters(self.q_proj)
-    Kqstate, K_bias, KA, KB, KS, Kdropout = get_lora_parameters(self.k_proj)
-    Vqstate, V_bias, VA, VB, VS, Vdropout = get_lora_parameters(self.v_proj)
-    return core.run(
-        LoRA_QKV, X,
-        *unpack_gptqstate(Qqstate), Q_bias, QA, QB, QS,
-        *unpack_gptqstate(Kqstate), K_bias, KA, KB, KS,
-        *unpack_gptqstate(Vqstate), V_bias, VA, VB, VS,
-        Qdropout, Kdropout, Vdropout,
-    )
+    projs = (self.q_proj, self.k_proj, self.v_proj)
+    few = core.few_linear(X, projs, False)
+    if few is not None:
+        return few
+    q, k, v = map(_operands, projs)
+    return core.run(LoRA_QKV, X, *q[:9], *k[:9], *v[:9], q[9], k[9], v[9])
 
 
 def rope_tables(cos, sin, batch, seq_len):
@@ -276,27 +278,22 @@ def rope_tables(cos, sin, batch, seq_len):
 def apply_lora_qkv_rope(self, X, cos, sin):
     """apply_lora_qkv with the rotary embedding of Q and K fused into the projection launch.  X [batch, seq, hidden];
     returns (Q, K, V) as [batch, seq, N]; `self.head_dim` (or config.head_dim) gives the head size."""
-    Qqstate, Q_bias, QA, QB, QS, Qdropout = get_lora_parameters(self.q_proj)
-    Kqstate, K_bias, KA, KB, KS, Kdropout = get_lora_parameters(self.k_proj)
-    Vqstate, V_bias, VA, VB, VS, Vdropout = get_lora_parameters(self.v_proj)
+    q, k, v = map(_operands, (self.q_proj, self.k_proj, self.v_proj))
     batch, seq_len = (X.shape[0], X.shape[1]) if X.dim() == 3 else (1, X.shape[0])
     cos2d, sin2d = rope_tables(cos, sin, batch, seq_len)
     head_dim = getattr(self, "head_dim", None) or self.config.head_dim
-    return core.run(
-        LoRA_QKV_RoPE, X, cos2d, sin2d, head_dim,
-        *unpack_gptqstate(Qqstate), Q_bias, QA, QB, QS,
-        *unpack_gptqstate(Kqstate), K_bias, KA, KB, KS,
-        *unpack_gptqstate(Vqstate), V_bias, VA, VB, VS,
-        Qdropout, Kdropout, Vdropout,
-    )
+    return core.run(LoRA_QKV_RoPE, X, cos2d, sin2d, head_dim, *q[:9], *k[:9], *v[:9], q[9], k[9], v[9])
+
+
+def _apply_lora_one(proj, X):
+    few = core.few_linear(X, (proj,), False)
+    return few[0] if few is not None else core.run(LoRA_W, X, *_operands(proj))
 
 
 def apply_lora_o(self, X):
-    Oqstate, O_bias, OA, OB, OS, dropout = get_lora_parameters(self.o_proj)
-    return core.run(LoRA_W, X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)
+    return _apply_lora_one(self.o_proj, X)
 
 
 def apply_lora_o_v2(self, X):
     """Patched directly on the output linear (`self` is the LoRA layer itself, :856-859)."""
-    Oqstate, O_bias, OA, OB, OS, dropout = get_lora_parameters(self)
-    return core.run(LoRA_W, X, *unpack_gptqstate(Oqstate), O_bias, OA, OB, OS, dropout)
+    return _apply_lora_one(self, X)

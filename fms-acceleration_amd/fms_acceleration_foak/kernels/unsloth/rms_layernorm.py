@@ -6,7 +6,7 @@ import torch
 
 import fmsa_hip
 
-from ...autograd import run
+from ...autograd import no_graph, run
 
 
 class Fast_RMS_Layernorm(torch.autograd.Function):
@@ -37,4 +37,8 @@ class Fast_RMS_Layernorm(torch.autograd.Function):
 def fast_rms_layernorm(layernorm, X, gemma=False):
     W = layernorm.weight
     eps = layernorm.variance_epsilon if hasattr(layernorm, "variance_epsilon") else layernorm.eps
+    if no_graph():
+        Y = fmsa_hip.native().rms_layernorm(X, W, eps, gemma)
+        if Y is not None:
+            return Y
     return run(Fast_RMS_Layernorm, X, W, eps, gemma)

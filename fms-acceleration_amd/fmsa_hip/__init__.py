@@ -363,6 +363,7 @@ def native():
         spec.loader.exec_module(module)
         if module.install(FmsaError) != ABI_VERSION:
             raise RuntimeError(f"{CALLS_PATH} was built for another ABI version than {ABI_VERSION}, that of {LIB_PATH}: rebuild both")
+        module.install_types(torch.nn.Identity, torch.nn.ModuleDict, torch.nn.Parameter)
         _native = module
     return _native
 

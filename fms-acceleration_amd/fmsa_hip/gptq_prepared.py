@@ -118,6 +118,10 @@ class PreparedWeight:
 
 
 def prepare(qweight, scales, qzeros, g_idx, bits) -> PreparedWeight:
+    if fmsa_hip._native is not None:  # the comparison below, where everything is an ordinary tensor
+        known = fmsa_hip._native.gptq_prepared(qweight, scales, qzeros, g_idx)
+        if known is not None:
+            return known
     key = (qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), g_idx.data_ptr(), g_idx._version,
            qweight._version, scales._version, qzeros._version, int(getattr(qzeros, "offset", 0) or 0))
     cached = getattr(qweight, "_fmsa_prepared", None)
