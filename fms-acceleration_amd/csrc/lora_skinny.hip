@@ -857,6 +857,29 @@ __global__ __launch_bounds__(512) void lora_grad_partial_kernel(const LoraGradAr
   }
 }
 
+// Four elements of a gradient from `at` on
+FMSA_DEVI void grad_store4(const LoraGradJobDev& J, size_t at, f32x4 v) {
+  v *= J.scale;
+  const bool aligned = reinterpret_cast<uintptr_t>(J.out) % 16 == 0;
+  if (J.out_dtype == FMSA_F32) {
+    float* out = reinterpret_cast<float*>(J.out) + at;
+    if (aligned) {
+      *reinterpret_cast<f32x4*>(out) = v;
+    } else {
+      for (int i = 0; i < 4; ++i) out[i] = v[i];
+    }
+  } else {
+    uint16_t* out = reinterpret_cast<uint16_t*>(J.out) + at;
+    const u32x2 o = J.out_dtype == FMSA_BF16 ? u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])}
+                                             : u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
+    if (aligned) {
+      *reinterpret_cast<u32x2*>(out) = o;
+    } else {
+      for (int i = 0; i < 4; ++i) out[i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
+    }
+  }
+}
+
 // The sums of a job's splits, in the output's order (which the partial sums are in too), V elements a thread: four, whose loads
 // are whole lines (the transposed outputs were written 4 bytes at a time, r elements apart, 10.5 us where the sums of q, k, v at
 // rank 64 and 1100 tokens take 6), or one, of straight outputs in launches that four leave short of workgroups (below).
@@ -875,29 +898,12 @@ template <int V> FMSA_DEVI void grad_reduce(const LoraGradJobDev& J, int idx) {
   }
 #pragma unroll 4
   for (; sp < J.splits; ++sp) v += *reinterpret_cast<const fv*>(src + (size_t)sp * step);
-  v *= J.scale;
   if constexpr (V == 1) {
+    v *= J.scale;
     if (J.out_dtype == FMSA_F32) reinterpret_cast<float*>(J.out)[idx] = v;
     else reinterpret_cast<uint16_t*>(J.out)[idx] = J.out_dtype == FMSA_BF16 ? pack1<bf16_t>(v) : pack1<f16_t>(v);
   } else {
-    const bool aligned = reinterpret_cast<uintptr_t>(J.out) % 16 == 0;
-    if (J.out_dtype == FMSA_F32) {
-      float* out = reinterpret_cast<float*>(J.out) + idx;
-      if (aligned) {
-        *reinterpret_cast<f32x4*>(out) = v;
-      } else {
-        for (int i = 0; i < 4; ++i) out[i] = v[i];
-      }
-    } else {
-      uint16_t* out = reinterpret_cast<uint16_t*>(J.out) + idx;
-      const u32x2 o = J.out_dtype == FMSA_BF16 ? u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])}
-                                               : u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
-      if (aligned) {
-        *reinterpret_cast<u32x2*>(out) = o;
-      } else {
-        for (int i = 0; i < 4; ++i) out[i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
-      }
-    }
+    grad_store4(J, idx, v);
   }
 }
 
@@ -936,6 +942,121 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGradArg
     if (4 * at < r * C) grad_reduce<4>(J, 4 * at);
   } else if (at < r * C) {
     grad_reduce<1>(J, at);
+  }
+}
+
+// The same gradients in one launch: workgroup = 64 columns of R, its eight waves share the tokens (wave w takes tiles w, w + 8, ..),
+// every wave stages its own tiles through its own part of LDS, and the waves' sums meet there in wave order, so nothing goes
+// through memory and nothing is waited for but a wave's own loads.  The two-pass kernel above gives a gradient of few tokens one
+// workgroup for 256 columns, which walks the tokens tile after tile (2048 columns: 8 workgroups), and a second launch.
+constexpr int LGW_WAVES = 8;
+constexpr int LGW_COLS = 64;
+constexpr int LGW_RSTRIDE = LGW_COLS + 16;  // elements
+constexpr int LGW_SUM = LGW_COLS + 4;       // floats: a rank's row of sums
+template <int RT> constexpr int lgw_lstride() { return RT == 1 ? 16 : RT * 16 + 16; }
+template <int RT> constexpr int lgw_round() { return RT < 2 ? 1 : 2; }  // 16-rank tiles summed at a time
+template <int RT> constexpr int lgw_lds() {
+  constexpr int stage = LGW_WAVES * LG_TM * (LGW_RSTRIDE + lgw_lstride<RT>()) * 2, sums = LGW_WAVES * lgw_round<RT>() * 16 * LGW_SUM * 4;
+  return stage > sums ? stage : sums;
+}
+
+template <typename T, int RT>
+__global__ __launch_bounds__(64 * LGW_WAVES) void lora_grad_waves_kernel(const LoraGradArgs a) {
+  constexpr int LSTRIDE = lgw_lstride<RT>(), ROUND = lgw_round<RT>(), G = LGW_COLS / 16;
+  __shared__ __attribute__((aligned(16))) char lds[lgw_lds<RT>()];
+  const LoraGradJobDev J = select_job<false>(a, blockIdx.x);
+  const int M = a.M, C = J.C, r = J.r, rt = (r + 15) / 16;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
+  const int c0 = (blockIdx.x - J.block_start) * LGW_COLS;
+  const int n_tiles = (M + LG_TM - 1) / LG_TM;
+  uint16_t* r_lds = reinterpret_cast<uint16_t*>(lds) + wave * LG_TM * (LGW_RSTRIDE + LSTRIDE);
+  uint16_t* l_lds = r_lds + LG_TM * LGW_RSTRIDE;
+  // R tile: 32 rows x 8 chunks of 16 B, 4 a lane (8 rows a pass: whole lines); L tile: 32 rows x 2 RT chunks, RT a lane
+  const int r_row = lane >> 3, r_chunk = lane & 7;
+  const bool r_ok = c0 + 8 * r_chunk < C;  // C % 8 == 0
+  u32x4 rst[4], lst[RT];
+  auto load_tile = [&](int tile) {
+    const int m0 = tile * LG_TM;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int m = m0 + r_row + 8 * p;
+      rst[p] = u32x4{0u, 0u, 0u, 0u};
+      if (m < M && r_ok) rst[p] = *reinterpret_cast<const u32x4*>(J.R + (size_t)m * J.ldr + c0 + 8 * r_chunk);
+    }
+#pragma unroll
+    for (int p = 0; p < RT; ++p) {
+      const int ci = lane + 64 * p, row = ci / (2 * RT), chunk = ci % (2 * RT), m = m0 + row;
+      lst[p] = u32x4{0u, 0u, 0u, 0u};
+      if (m < M && 8 * chunk < r) lst[p] = *reinterpret_cast<const u32x4*>(J.L + (size_t)m * J.ldl + 8 * chunk);  // r % 8 == 0
+    }
+  };
+  // a wave's own stage: its lanes exchange data, so neither side of a fence moves past it
+  auto own_stage_fence = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  auto column_frag = [&](const uint16_t* base, int stride, int col0) {  // as in the kernel above
+    const uint16_t* p = base + (8 * kg + (l16 >> 2)) * stride + col0 + 4 * (l16 & 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p + 4 * stride));
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l2[0], l2[1], h2[0], h2[1]};
+  };
+  f32x4 acc[G][RT];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (wave < n_tiles) load_tile(wave);
+  for (int tile = wave; tile < n_tiles; tile += LGW_WAVES) {
+    own_stage_fence();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) *reinterpret_cast<u32x4*>(r_lds + (r_row + 8 * p) * LGW_RSTRIDE + 8 * r_chunk) = rst[p];
+#pragma unroll
+    for (int p = 0; p < RT; ++p) {
+      const int ci = lane + 64 * p;
+      *reinterpret_cast<u32x4*>(l_lds + ci / (2 * RT) * LSTRIDE + 8 * (ci % (2 * RT))) = lst[p];
+    }
+    own_stage_fence();
+    if (tile + LGW_WAVES < n_tiles) load_tile(tile + LGW_WAVES);
+    u32x4 rf[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) rf[g] = column_frag(r_lds, LGW_RSTRIDE, 16 * g);
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+      if (t < rt) {
+        const u32x4 lf = column_frag(l_lds, LSTRIDE, 16 * t);
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][t] = mfma16<T>(rf[g], lf, acc[g][t]);  // D[c][j]
+      }
+  }
+  // ROUND rank tiles at a time: every wave's sums to LDS (rank-major), added in wave order, scaled, rounded once and stored
+  float* sums = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int t0 = 0; t0 < RT; t0 += ROUND) {
+    if (t0 >= rt) break;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < ROUND; ++t)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        *reinterpret_cast<f32x4*>(sums + ((wave * ROUND + t) * 16 + l16) * LGW_SUM + 16 * g + 4 * kg) = acc[g][t0 + t];
+    __syncthreads();
+    // four columns of a rank, or, for a transposed output, four ranks of a column
+    const int quads = ROUND * 16 * LGW_COLS / 4;
+    if (tid < quads) {
+      const bool tr = J.transpose_out;
+      const int j = tr ? 4 * (tid % (ROUND * 4)) : tid / (LGW_COLS / 4), c = tr ? tid / (ROUND * 4) : 4 * (tid % (LGW_COLS / 4));
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < LGW_WAVES; ++w) {
+        const float* src = sums + (w * ROUND * 16 + j) * LGW_SUM + c;
+        v += tr ? f32x4{src[0], src[LGW_SUM], src[2 * LGW_SUM], src[3 * LGW_SUM]} : *reinterpret_cast<const f32x4*>(src);
+      }
+      const int jr = 16 * t0 + j;
+      if (c0 + c < C && jr < r) grad_store4(J, tr ? (size_t)(c0 + c) * r + jr : (size_t)jr * C + c0 + c, v);
+    }
   }
 }
 
@@ -1329,6 +1450,24 @@ namespace {
 size_t job_partial_bytes(const fmsa_lora_grad_job& s, int M) {
   return (size_t)lora_grad_splits(M, s.C) * (size_t)s.r * (size_t)s.C * sizeof(float);
 }
+// Whether a launch's gradients come from one launch (lora_grad_waves_kernel).  us in two passes / there: q, k, v of hidden 2048 at 300
+// tokens, rank 16, 13.2 / 6.3; 14336 and 4096 at 1100, rank 64, 22 / 14; gate and up of 4096 -> 14336 at 3217, rank 64, 87 / 50.  All of
+// 36 forms, 2048 to 28672 columns, ranks 8 to 64: at 64 tokens 342 / 254, 512 706 / 331, 1100 778 / 469, 2048 1012 / 703, 4096 1534 /
+// 1278, 8192 1570 / 1581.  Not where T comes along; above 2048 tokens for ranks that T never comes along with (smaller ones have the
+// sums of a launch with T, and are a copy that takes more bytes in flight: 14336 and 4096 at 3217, rank 8, 23.9 / 25.7), and not
+// where few workgroups hold many ranks (q, k, v of 2048 at 4096, stacked ranks 96, 25.5 / 28.1); and not where the stores of many
+// ranks are all there is to do (8192 -> 28672 at 300, rank 64, 27.8 / 32).
+bool lora_grad_in_one_launch(const fmsa_lora_grad_job* jobs, int n_jobs, int M) {
+  int r_max = 0, blocks = 0;
+  for (int q = 0; q < n_jobs; ++q) {
+    if (jobs[q].Wt) return false;
+    blocks += (jobs[q].C + LGW_COLS - 1) / LGW_COLS;
+    r_max = std::max(r_max, jobs[q].r);
+  }
+  if (M <= 512) return r_max <= 64 || blocks <= 512;
+  if (M <= 2048) return true;
+  return M <= 4096 && r_max > 32 && (r_max <= 64 || blocks >= 128 || M <= 3217);
+}
 size_t job_tpart_bytes(const fmsa_lora_grad_job& s, int M) {
   return s.Wt ? (size_t)((s.C + LG_TC_T - 1) / LG_TC_T) * (size_t)M * (size_t)s.r * sizeof(float) : 0;
 }
@@ -1351,7 +1490,8 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
     any_t = any_t || jobs[q].Wt != nullptr;
     elements += (int64_t)jobs[q].r * jobs[q].C;
   }
-  const int tc = LG_TC_T;
+  const bool waves = lora_grad_in_one_launch(jobs, n_jobs, M);
+  const int tc = waves ? LGW_COLS : LG_TC_T;
   int blocks = 0, rblocks = 0, r_max = 0;
   size_t ws_off = 0;
   for (int q = 0; q < n_jobs; ++q) {
@@ -1373,7 +1513,7 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
     d.transpose_out = s.transpose_out;
     d.out_dtype = s.out_dtype;
     d.scale = s.scale;
-    blocks += ((s.C + tc - 1) / tc) * d.splits;
+    blocks += ((s.C + tc - 1) / tc) * (waves ? 1 : d.splits);
     // one element a thread: straight sums over several splits, in launches of fewer than 1024 workgroups with four (us with four /
     // one; single outputs: 4096 of rank 64 at 3217 tokens 25.2 / 22.8, 14336 of rank 32 at 8192 50.6 / 46.9, of rank 64 at 1100
     // 25.3 / 23.7, of rank 128 at 3217, 1792 workgroups, 58.8 / 60.4; q, k, v of rank 128 at 2048, 2304, 54 / 58; 14336 of rank 128
@@ -1393,6 +1533,20 @@ int launch_lora_grad_batch(const fmsa_lora_grad_job* jobs, int n_jobs, int M, in
   }
   dim3 grid1(blocks), grid2(rblocks), block(256), block1(512);
   const int rt = (r_max + 15) / 16;
+  if (waves) {
+#define LAUNCH(TT)                                                                                                           \
+  do {                                                                                                                      \
+    if (rt == 1) hipLaunchKernelGGL((lora_grad_waves_kernel<TT, 1>), grid1, block1, 0, st, a);                               \
+    else if (rt == 2) hipLaunchKernelGGL((lora_grad_waves_kernel<TT, 2>), grid1, block1, 0, st, a);                          \
+    else if (rt <= 4) hipLaunchKernelGGL((lora_grad_waves_kernel<TT, 4>), grid1, block1, 0, st, a);                          \
+    else hipLaunchKernelGGL((lora_grad_waves_kernel<TT, 8>), grid1, block1, 0, st, a);                                       \
+  } while (0)
+    if (act_dtype == FMSA_BF16) LAUNCH(bf16_t);
+    else LAUNCH(f16_t);
+#undef LAUNCH
+    FMSA_CHECK_LAUNCH();
+    return FMSA_OK;
+  }
 #define LAUNCH(TT, RT, WT) hipLaunchKernelGGL((lora_grad_partial_kernel<TT, RT, WT>), grid1, block1, 0, st, a)
 #define DISPATCH(TT)                                                  \
   switch (rt) {                                                       \
