@@ -100,3 +100,15 @@ def test_rms_layernorm(monkeypatch, shape, dtype, wtype, gemma):
         monkeypatch.setattr(rms_layernorm, "no_graph", lambda: False)
         general = fast_rms_layernorm(norm, x, gemma)
     assert _equal(native, general) and _equal(strided, general)
+
+
+@pytest.mark.parametrize("C", [8, 504, 4096])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rms_layernorm_asks_for_the_weight_early_up_to_64_rows(C, dtype):
+    import fmsa_hip
+
+    x, w = torch.randn(65, C, device="cuda").to(dtype), torch.randn(C, device="cuda").to(dtype)
+    y, r = fmsa_hip.rms_layernorm_fwd(x, w, 1e-5, False)
+    for M in (1, 63, 64):
+        y_few, r_few = fmsa_hip.rms_layernorm_fwd(x[:M], w, 1e-5, False)
+        assert torch.equal(y_few, y[:M]) and torch.equal(r_few, r[:M])
