@@ -74,7 +74,7 @@ template <typename T> FMSA_DEVI u32x4 few_params(const void* base, size_t at, bo
 }
 
 // FMT 0: affine words in the checkpoint's nibble order; 1: interleaved words, packed-half unpack (fp16); 2: code book
-// (the 16 entries sit in lanes 0..15 and are gathered with ds_bpermute: 8 per word).
+// (codes from a table of pairs in LDS, two per 8-byte read).
 template <typename T, int FMT, int NP, int MT, int CT, int NW, int DEPTH, int WPE>
 __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const FewArgs a) {
   static_assert(CT == 1 || CT == 2, "columns per lane");
@@ -88,6 +88,13 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
   __shared__ __attribute__((aligned(1024))) uint16_t st1[NW * MT * FEW_STAGE];
   __shared__ __attribute__((aligned(1024))) uint16_t st2[DEPTH > 2 ? NW * MT * FEW_STAGE : 8];
   __shared__ __attribute__((aligned(1024))) uint16_t st3[DEPTH > 2 ? NW * MT * FEW_STAGE : 8];
+  // Code book: entry [16 hi + lo][copy] = (code[lo], code[hi]) as fp32, a lane's copy by its number: with 16 of them 16 lanes never
+  // meet in a bank.  The LDS pipe bound the launches while every code was a ds_bpermute of its own (16 of them and 36 vector
+  // instructions for the two words of a column, 8 reads and 20 now): the launches of a layer of hidden 4096 at 12 / 64 / 300 tokens, three
+  // ranks, 263 / 500 / 301 -> 213 / 407 / 217 us, of hidden 2048 140 / 256 / 320 -> 131 / 230 / 252; affine words take 204 / 395 / 203.
+  // COPIES leaves as many workgroups on a CU as run there without the table.
+  constexpr int COPIES = FMT == 2 ? (MT == 1 ? 16 : 8) : 0;
+  __shared__ __attribute__((aligned(1024))) u32x2 pairs[FMT == 2 ? 256 * COPIES : 1];
   auto stage = [&](auto d_c) -> char* {
     constexpr int d = decltype(d_c)::value;
     return reinterpret_cast<char*>(d == 0 ? st0 : (d == 1 ? st1 : (d == 2 ? st2 : st3)));
@@ -177,7 +184,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
   __amdgpu_buffer_rsrc_t q_rsrc[NP], s_rsrc[NP], z_rsrc[NP];
   uint32_t q_off[NP], s_off[NP], z_off[NP], q_chunk[NP], q_half[NP];
   int zshift[NP], N[NP];
-  float zoff[NP], lut[NP];
+  float zoff[NP];
   const int n_chunks = (a.K + FEW_BK - 1) / FEW_BK;
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -193,7 +200,6 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
     q_chunk[p] = (uint32_t)N[p] * 32;
     zshift[p] = 4 * (col & 7);
     zoff[p] = (float)P[p].zero_offset;
-    lut[p] = FMT == 2 ? P[p].code[lane & 15] : 0.f;
   }
   // X: the wave's chunk of 16 * MT rows goes through its own 2 KB * MT of a stage buffer by direct loads, 8 rows x 128 B
   // each; a fragment load from global has four rows in every four lanes, which the address path takes one by one (16 B per
@@ -259,6 +265,25 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
       }
     }
   };
+  // The table is written while the first chunks are on their way: the book's entries are asked for ahead of them, and the barrier
+  // waits for the LDS writes alone.  Where the two projections' books differ, each has half of the copies.
+  uint32_t pair_lane[NP];
+  constexpr int PAIR_VEC = 256 * COPIES / 2, PAIR_TURNS = FMT == 2 ? PAIR_VEC / (64 * NW) : 0;  // 16-byte writes, two copies each
+  static_assert(FMT != 2 || PAIR_VEC % (64 * NW) == 0, "every thread writes as many entries");
+  u32x2 entry[FMT == 2 ? PAIR_TURNS : 1];
+  if constexpr (FMT == 2) {
+    const float *c0 = P[0].code, *c1 = P[NP - 1].code;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      pair_lane[p] = c0 == c1 ? (uint32_t)(8 * (lane & (COPIES - 1))) : (uint32_t)(8 * (lane & (COPIES / 2 - 1)) + 4 * COPIES * p);
+#pragma unroll
+    for (int k = 0; k < PAIR_TURNS; ++k) {
+      const int v = tid + 64 * NW * k, e = v / (COPIES / 2);
+      const float* book = v % (COPIES / 2) < COPIES / 4 ? c0 : c1;
+      entry[k] = u32x2{__float_as_uint(book[e & 15]), __float_as_uint(book[e >> 4])};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const uint32_t pk_mask = opaque(0x000F000Fu), pk_bias = opaque(0x64006400u);
   auto multiply = [&](auto d_c) {
     constexpr int d = decltype(d_c)::value;
@@ -277,19 +302,20 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
         u32x4 wf[2];
         if constexpr (FMT == 2) {
           const float bs = __uint_as_float(sc[d][p][j]);
-          const int li = (int)__float_as_uint(lut[p]);
+          u32x2 v[2][4];
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const uint32_t w = qw[d][p][t][j];
-            const uint32_t e = opaque((w << 2) & 0x3C3C3C3Cu);  // byte b: 4 * nibble 2b (a lane's byte address)
-            const uint32_t o = opaque((w >> 2) & 0x3C3C3C3Cu);  // byte b: 4 * nibble 2b + 1
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-              const float v0 = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)((e >> (8 * b)) & 0xffu), li));
-              const float v1 = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)((o >> (8 * b)) & 0xffu), li));
-              wf[t][b] = pack2<T>(v0 * bs, v1 * bs);
-            }
+            static_for<0, 4>([&](auto b_c) {  // the codes of byte b: elements 2b, 2b + 1
+              constexpr int b = decltype(b_c)::value, at = COPIES == 16 ? 7 : 6;
+              const uint32_t byte = 8 * b < at ? w << (at - 8 * b) : w >> (8 * b - at);
+              v[t][b] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const char*>(pairs) + ((byte & (0xFFu << at)) | pair_lane[p]));
+            });
           }
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) wf[t][b] = pack2<T>(__uint_as_float(v[t][b][0]) * bs, __uint_as_float(v[t][b][1]) * bs);
         } else {
           const uint16_t sb = (uint16_t)(sc[d][p][0] >> (16 * j));
           const float z = (float)((zw[d][p] >> (zshift[p] + 4 * j)) & 0xFu) + zoff[p];
@@ -323,6 +349,17 @@ __global__ __launch_bounds__(64 * NW, WPE) void gptq_lora_fwd_few_kernel(const F
     // knows the buffers for separate arrays, from issuing them first
     __builtin_amdgcn_sched_barrier(0);
   });
+  if constexpr (FMT == 2) {
+#pragma unroll
+    for (int k = 0; k < PAIR_TURNS; ++k)
+      reinterpret_cast<u32x4*>(pairs)[tid + 64 * NW * k] = u32x4{entry[k][0], entry[k][1], entry[k][0], entry[k][1]};
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
   for (int it = 0; it < n_it; it += DEPTH)
     static_for<0, DEPTH>([&](auto d_c) {
       constexpr int d = decltype(d_c)::value;
@@ -513,19 +550,19 @@ int few_gemm(FewArgs& a, const fmsa_gptq_weight& w0, int n_proj, int mode, int a
 // linear launch goes in whole rounds of one workgroup per CU (4096 columns and K: 12.2 us at 64 and 12.8 at 128 tokens, one
 // round; 21.7 and 22.4 at 192 and 256, two; 2048 -> 2048 8.0 to 8.7 from 64 to 256 tokens; 14336 -> 4096 28 to 30 a round),
 // two workgroups with the SwiGLU per CU share it more evenly (4096 -> 14336: 43, 72, 101, 130 us at 64, 128, 192, 256 tokens);
-// the code book's gathers take half as long again (17 and 31 us for 4096 columns, one round and two).
+// from a code book 4 to 10 % more.
 float few_us(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {
   if (M <= 64) return 0.f;
   const bool codebook = projs[0].w.format == FMSA_WEIGHT_CODEBOOK;
   const float k = (float)projs[0].w.K, tb = (float)((M + 63) / 64);
   if (mode == FMSA_FWD_SWIGLU) {
     const float rounds = projs[0].w.N / 16 * tb / 512.f;
-    return 4.f + 0.0022f * k + rounds * (4.f + 0.0031f * k) * (codebook ? 1.4f : 1.f);
+    return 4.f + 0.0022f * k + rounds * (4.f + 0.0031f * k) * (codebook ? 1.08f : 1.f);
   }
   int cols = 0;
   for (int p = 0; p < n_proj; ++p) cols += projs[p].w.N;
   const int rounds = (int)((cols / 32 * tb + 255.f) / 256.f);
-  return 2.5f + rounds * (1.9f + 0.00185f * k * (codebook ? 1.6f : 1.f));
+  return 2.5f + rounds * (1.9f + 0.00185f * k * (codebook ? 1.08f : 1.f));
 }
 
 // U given (in the activation type), adapters packed.
