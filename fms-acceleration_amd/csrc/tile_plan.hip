@@ -98,15 +98,15 @@ bool gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int mod
   return few_us(projs, n_proj, M, mode) < (mode == FMSA_FWD_SWIGLU ? 1.2f : 1.1f) * plan.us;
 }
 
-// Whether the rotating flavours, which run whole tiles of 8, are expected to take less time than the plan and a pass over what it wrote.
-// (Cut launches are small: q, k, v of hidden 4096 rotated in the launch / after a cut one 85 / 41 us at 1 token, 88 / 53 at 512.)
+// Whether the rotating flavours, which run whole tiles of 8, are expected to take less time than the plan and the passes over what it
+// wrote (3 us and 0.4 ps an element, out of the caches that it lies in).  q, k, v of hidden 4096 (k, v of 1024) rotated in the launch /
+// after it, us at 512, 1100, 2048, 3217, 4096, 8192 tokens: 87 / 49, 89 / 68, 95 / 106, 195 / 163, 198 / 213, 344 / 357; of hidden 2048
+// (512) at 1100, 3217, 4096, 6000: 50 / 39, 52.3 / 51.3, 54 / 62, 108 / 91.
 bool gptq_lora_fwd_rope_pays(const fmsa_fwd_proj* projs, int n_proj, int M) {
-  const SplitPlan plan = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR);
-  if (plan.s > 1 || plan.mt == 8) return plan.s == 1;
   int64_t columns = 0;
   for (int p = 0; p < n_proj; ++p) columns += projs[p].w.N;
-  const SplitPlan rotating = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR, true);
-  return rotating.us < plan.us + 4.0f + 4.0e-6f * M * columns;
+  const float after = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR).us + 3.0f + 4.0e-7f * M * columns;
+  return plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR, true).us < after;
 }
 
 size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {

@@ -263,10 +263,10 @@ def _lora_down_all(projs, Xds, stack):
 def _rope_in_epilogue(projs, rope, dtype, M):
     """Whether one forward launch over these projections can apply the rotary embedding itself (fmsa_gptq_lora_fwd_rope):
     group sizes and K in whole 64-wide stages, heads that do not straddle its 256-column tiles, tables of the activation
-    type or fp32 whose rows start on 16-byte boundaries.  Where the launch would be cut along K (few tokens), the plain one
-    and the rotating pass over its small outputs are taken: the rotating flavours are not cut.  (q, k, v of hidden 4096
-    rotated in the launch / after it, GPU time: 85 / 41 us at 1 token, 88 / 53 at 512, 88 / 88 at 1280, 192 / 175 at 3217;
-    hidden 1024 at 256 tokens 31 / 30.)"""
+    type or fp32 whose rows start on 16-byte boundaries.  Where the plain launch, cut along K or in lower tiles, and
+    a rotating pass over its outputs are expected to be faster, that way is taken: the rotating flavours run whole tiles of 256.
+    (q, k, v of hidden 4096 rotated in the launch / after it, GPU time: 87 / 49 us at 512 tokens, 89 / 68 at 1100, 95 / 106 at
+    2048, 344 / 357 at 8192.)"""
     cos2d, sin2d, head_dim, mask = rope
     K = projs[0].w.K
     esz = cos2d.element_size()
