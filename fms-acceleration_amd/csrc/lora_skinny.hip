@@ -1454,9 +1454,9 @@ size_t job_partial_bytes(const fmsa_lora_grad_job& s, int M) {
 // tokens, rank 16, 13.2 / 6.3; 14336 and 4096 at 1100, rank 64, 22 / 14; gate and up of 4096 -> 14336 at 3217, rank 64, 87 / 50.  All of
 // 36 forms, 2048 to 28672 columns, ranks 8 to 64: at 64 tokens 342 / 254, 512 706 / 331, 1100 778 / 469, 2048 1012 / 703, 4096 1534 /
 // 1278, 8192 1570 / 1581.  Not where T comes along; above 2048 tokens for ranks that T never comes along with (smaller ones have the
-// sums of a launch with T, and are a copy that takes more bytes in flight: 14336 and 4096 at 3217, rank 8, 23.9 / 25.7), and not
-// where few workgroups hold many ranks (q, k, v of 2048 at 4096, stacked ranks 96, 25.5 / 28.1); and not where the stores of many
-// ranks are all there is to do (8192 -> 28672 at 300, rank 64, 27.8 / 32).
+// sums of a launch with T, and are a copy that takes more bytes in flight: 14336 and 4096 at 3217, rank 8, 23.9 / 25.7), and there
+// not where few workgroups hold many ranks over more than 12 token tiles a wave (q, k, v of 2048 at 4096, stacked ranks 96, 25.5 /
+// 28.1); and not where the stores of many ranks are all there is to do (8192 -> 28672 at 300, rank 64, 27.8 / 32).
 bool lora_grad_in_one_launch(const fmsa_lora_grad_job* jobs, int n_jobs, int M) {
   int r_max = 0, blocks = 0;
   for (int q = 0; q < n_jobs; ++q) {
@@ -1466,7 +1466,7 @@ bool lora_grad_in_one_launch(const fmsa_lora_grad_job* jobs, int n_jobs, int M) 
   }
   if (M <= 512) return r_max <= 64 || blocks <= 512;
   if (M <= 2048) return true;
-  return M <= 4096 && r_max > 32 && (r_max <= 64 || blocks >= 128 || M <= 3217);
+  return M <= 4096 && r_max > 32 && (r_max <= 64 || blocks >= 128 || M <= 3072);
 }
 size_t job_tpart_bytes(const fmsa_lora_grad_job& s, int M) {
   return s.Wt ? (size_t)((s.C + LG_TC_T - 1) / LG_TC_T) * (size_t)M * (size_t)s.r * sizeof(float) : 0;

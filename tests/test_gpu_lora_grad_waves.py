@@ -38,7 +38,7 @@ def test_gradients(M, r, dtype):
         assert torch.equal(g, again)
 
 
-@pytest.mark.parametrize("M,C,r", [(2048, 4096, 16), (2049, 4096, 16), (4096, 4096, 64), (4097, 4096, 64), (4096, 2048, 96), (3217, 2048, 96), (300, 33024, 128), (513, 33024, 128)])
+@pytest.mark.parametrize("M,C,r", [(2048, 4096, 16), (2049, 4096, 16), (4096, 4096, 64), (4097, 4096, 64), (4096, 2048, 96), (3072, 2048, 96), (3073, 2048, 96), (300, 33024, 128), (513, 33024, 128)])
 def test_either_side_of_the_rule(M, C, r):
     import fmsa_hip
 
