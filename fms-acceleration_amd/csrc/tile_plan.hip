@@ -102,14 +102,15 @@ bool gptq_lora_fwd_is_few(const fmsa_fwd_proj* projs, int n_proj, int M, int mod
 // wrote (3 us and 0.4 ps an element, out of the caches that it lies in).  q, k, v of hidden 4096 (k, v of 1024) rotated in the launch /
 // after it, us at 512, 1100, 2048, 3217, 4096, 8192 tokens: 87 / 49, 89 / 68, 95 / 106, 195 / 163, 198 / 213, 344 / 357; of hidden 2048
 // (512) at 1100, 3217, 4096, 6000: 50 / 39, 52.3 / 51.3, 54 / 62, 108 / 91.
-// Launches of a few stages, below the range the estimates are fitted to, keep rotating: they end before the host has issued the one or two
-// launches more (about 5 us each), so the step waits for those (hidden 1024 at 256 tokens, where the two ways meet, 31 / 30 us).
+// Launches of a few stages that run whole either way (the same sums), below the range the estimates are fitted to, keep rotating: they end
+// before the host has issued the one or two launches more (about 5 us each), so the step waits for those (hidden 1024 at 256 tokens, where
+// the two ways meet, 31 / 30 us).
 bool gptq_lora_fwd_rope_pays(const fmsa_fwd_proj* projs, int n_proj, int M) {
   int64_t columns = 0;
   for (int p = 0; p < n_proj; ++p) columns += projs[p].w.N;
-  const float after = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR).us + 3.0f + 4.0e-7f * M * columns;
-  const float rotated = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR, true).us;
-  return rotated < 20.0f || rotated < after;
+  const SplitPlan plan = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR);
+  const float after = plan.us + 3.0f + 4.0e-7f * M * columns, rotated = plan_fwd(projs, n_proj, M, FMSA_FWD_LINEAR, true).us;
+  return rotated < after || (plan.ask == 0 && rotated < 20.0f);
 }
 
 size_t gptq_lora_fwd_workspace(const fmsa_fwd_proj* projs, int n_proj, int M, int mode) {

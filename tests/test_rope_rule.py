@@ -24,7 +24,7 @@ def _pays(M, K, Ns, **kw):
     (8192, (8192, 1024, 1024), 1100, 0), (8192, (8192, 1024, 1024), 2048, 0),  # 185 / 172, 366 / 314
     (8192, (8192, 1024, 1024), 1536, 1), (8192, (8192, 1024, 1024), 2560, 1), (8192, (8192, 1024, 1024), 8192, 1),  # 209 / 220, 372 / 388, 1046 / 1080
     (256, (256, 128, 128), 1, 1), (256, (256, 128, 128), 128, 1), (512, (512, 256, 256), 700, 1),  # a few stages: the launches count
-    (2048, (2048, 512, 512), 64, 0),
+    (512, (512, 128, 192), 140, 0), (2048, (2048, 512, 512), 64, 0),  # the kernel for few tokens
 ])
 @pytest.mark.parametrize("codebook", [False, True])
 def test_the_faster_way_is_taken(K, Ns, M, pays, codebook):
