@@ -41,7 +41,8 @@ TOL_OUT, TOL_GRAD = 1e-2, 2e-2  # max |out - ref| / max |ref| per tensor: output
 # WRITE_SIZE, scaled by a device copy of known size): lines `roofline_traffic_bytes <kernel label> = <bytes>`,
 # and `kernel_sources_sha256 = <digest>` of the two GEMM sources the counters were taken with.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "gptq_lora_gemms_llama3_8b_hbm_traffic_pmc.txt")
-GEMM_SOURCES = [os.path.join(ROOT, "fms-acceleration_amd", "csrc", f) for f in ("gemm_fwd.hip", "gemm_bwd.hip", "gemm_bwd_t.hip", "common.h")]
+GEMM_SOURCES = [os.path.join(ROOT, "fms-acceleration_amd", "csrc", f) for f in ("gemm_fwd.hip", "gemm_fwd_tiles.h", "gemm_bwd.hip", "gemm_bwd_t.hip",
+                                                                               "gemm_bwd_t_tiles.h", "common.h")]
 
 _W_BYTES = HIDDEN * INTER // 2 + (HIDDEN // GROUP) * INTER * 2 + (HIDDEN // GROUP) * INTER // 2  # packed + scales + zeros
 # algorithmic bytes of the launches that can be the dominant one

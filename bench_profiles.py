@@ -58,9 +58,9 @@ def collect(names):
 
 # ---------------------------------------------------------------------------------------------------------------
 def short(n):
-    n = re.sub(r"\(anonymous namespace\)::", "", n)
+    n = re.sub(r"\(anonymous namespace\)::|[fb]wd_tiles::", "", n)
     n = re.sub(r"^void ", "", n)
-    m = re.match(r"_ZN12_GLOBAL__N_1\d+([a-z_0-9]+?)I", n)
+    m = re.match(r"_ZN(?:12_GLOBAL__N_1|9[fb]wd_tiles)\d+([a-z_0-9]+?)I", n)
     if m:
         n = m.group(1)
     return n.split("(")[0].split("<")[0][:44]
