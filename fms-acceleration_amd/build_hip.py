@@ -25,7 +25,7 @@ LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libfmsa_hip.so")
 
 SOURCES = ["api.hip", "dequant.hip", "gemm_fwd.hip", "gemm_few.hip", "gemm_bwd.hip", "gemm_bwd_t.hip", "lora_skinny.hip", "elementwise.hip", "nf4.hip", "norm_rope.hip", "tile_plan.hip"]
-# one source, a translation unit a tile height (the kernels of the low tiles take the longest to compile)
+# one source, a translation unit a tile height, so that they compile side by side
 HEIGHT_SOURCES = ["gemm_bwd_t_low.hip", "gemm_fwd_low.hip"]
 HEIGHTS = (4, 5, 6, 7)
 PROBE_SOURCE = "probe.hip"
@@ -77,8 +77,8 @@ def build(verbose: bool = False, extra_flags=()) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     hipcc = _hipcc()
-    units = [(s, os.path.join(OBJ_DIR, s.replace(".hip", f"_{h}.o")), [f"-DFMSA_TILE_HEIGHT={h}"]) for s in HEIGHT_SOURCES for h in HEIGHTS]
-    units += [(s, os.path.join(OBJ_DIR, s.replace(".hip", ".o")), []) for s in SOURCES]
+    units = [(s, os.path.join(OBJ_DIR, s.replace(".hip", ".o")), []) for s in SOURCES]  # first: gemm_fwd and gemm_bwd_t take the longest
+    units += [(s, os.path.join(OBJ_DIR, s.replace(".hip", f"_{h}.o")), [f"-DFMSA_TILE_HEIGHT={h}"]) for s in HEIGHT_SOURCES for h in HEIGHTS]
     objs = [obj for _, obj, _ in units]
 
     def compile_one(unit):
